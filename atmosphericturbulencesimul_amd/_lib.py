@@ -104,6 +104,9 @@ _SIGS = {
                                      C.c_void_p, C.c_long, C.c_long, C.c_long,
                                      C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_float,
                                      C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_void_p, C.c_void_p, C.c_int]),
+    "atsim_nn_pointwise": (C.c_int, [C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_long, C.c_void_p,
+                                     C.c_void_p, C.c_long, C.c_long, C.c_void_p, C.c_long, C.c_void_p, C.c_long,
+                                     C.c_long, C.c_void_p, C.c_void_p, C.c_int]),
     "atsim_nn_add_bias_act": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                         C.c_long, C.c_long, C.c_long, C.c_int]),
     "atsim_nn_gelu_bwd": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long]),

@@ -2119,6 +2119,20 @@ int atsim_gemm_bf16_ex(atsim_ctx* c, long M, long N, long K, long batch, float a
     return ATSIM_OK;
 }
 
+int atsim_nn_pointwise(atsim_ctx* c, const float* W, long swm, long swk, long Cout, long Cin, const float* h, float* out,
+                       long nrows, long rowlen, const float* U, long K2, const float* F, long sfk, long sfx,
+                       const float* bias, float* pre, int act) {
+    if (!c || !W || !h || !out || Cout <= 0 || Cin <= 0 || nrows <= 0 || rowlen <= 0) return ATSIM_EINVAL;
+    if (swm < 0 || swk < 0 || act < 0 || act > 2 || (act == 2 && !pre) || (U && (!F || sfk < 0 || sfx < 0)))
+        return fail(c, ATSIM_EINVAL, "pointwise: invalid operands");
+    if (!pointwise_supported(h, out, pre, U, Cout, Cin, nrows, rowlen, K2))
+        return fail(c, ATSIM_EUNSUPPORTED, "pointwise: %ld x %ld channels over rows of %ld", Cout, Cin, rowlen);
+    c->work_gen++;
+    HIPCHK(c, launch_pointwise(W, swm, swk, (int)Cout, (int)Cin, h, out, nrows, (int)rowlen, U, (int)K2, F, sfk, sfx,
+                               bias, pre, act, c->stream));
+    return ATSIM_OK;
+}
+
 int atsim_nn_add_bias_act(atsim_ctx* c, const float* a, const float* b, const float* bias, float* pre, float* y,
                           long C, long P, long n, int gelu) {
     if (!c || !a || !y || C <= 0 || P <= 0 || n < 0 || n % (C * P)) return ATSIM_EINVAL;

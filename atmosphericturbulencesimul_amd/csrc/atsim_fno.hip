@@ -182,6 +182,260 @@ hipError_t launch_gemm_bf16(const GemmArgs& g0, hipStream_t st) {
     return k32 ? gemm_launch<64, 64, 32, 2>(g, st) : gemm_launch<64, 64, 64, 2>(g, st);
 }
 
+// ------------------------------------------------------------------ channel maps
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// float pairs to BF16, round to nearest even (v_cvt_pk_bf16_f32; the values
+// of to_bf16)
+__device__ __forceinline__ bf16x8 to_bf16x8(const float (&x)[8]) {
+    bf16x8 h;
+#pragma unroll
+    for (int j = 0; j < 8; j++) h[j] = (__bf16)x[j];
+    return h;
+}
+
+// out[c][p] = act( sum_i W[c][i] h[i][p]  (+ sum_k U[c][row(p)][k] F[k][x(p)])  (+ bias[c]) )
+// over channel-major images [C][nrows][rowlen]: a 1x1 channel map with, in the
+// same pass, the spectral path's inverse transform along x (U: the rows'
+// retained spectrum, F: the transform's table).  act 0: none, 1: GELU (pre,
+// if given, keeps its argument), 2: times GELU'(pre).
+//
+// Bound: HBM (h read and out written once, U and pre when given).  A wave
+// takes 64 pixels: lane l loads float4s of 8 channels at pixels
+// 4 (l % 16) .. + 3, so that pixel t of every lane's four is one MFMA column
+// and the operand is made in registers, without LDS; the four tiles' outputs
+// of a lane are again four neighbouring pixels, stored as float4.  The
+// products of one output are summed by the MFMAs in k_gemm_bf16's order (k
+// steps of 32, zero padded), the two sums added last: the same results as
+// its passes.
+// A block's map at 32 channels, 50 images of 256^2 (839 MB + 52 MB of U):
+// 194 us, 4.6 TB/s, where the inverse x transform and the map with its bias and
+// GELU took 340 + 1 016 us as two k_gemm_bf16 passes (staging through LDS in
+// 2-byte stores, the image written, read and written again).
+struct PointArgs {
+    const float* W;
+    long swm, swk;
+    int Cout, Cin;
+    const float* h;
+    float* out;
+    long nrows;
+    int rowlen;
+    const float* U;  // [Cout][nrows][K2], or null
+    int K2;
+    const float* F;
+    long sfk, sfx;
+    const float* bias;
+    float* pre;
+    int act;
+};
+
+template <int RT, int KT, int KU>
+__global__ void __launch_bounds__(256) k_pointwise(PointArgs g) {
+    extern __shared__ __attribute__((aligned(16))) __bf16 Fs[];  // F as MFMA operands: [KU][64-pixel group][4][lane][8]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lm = lane & 15, lk = (lane >> 4) * 8;
+    const long SP = g.nrows * g.rowlen;
+    const int ngrp = (g.rowlen + 63) / 64;
+    if constexpr (KU > 0) {
+        for (int e = threadIdx.x; e < KU * ngrp * 256; e += 256) {
+            const int ln = e & 63, t = (e >> 6) & 3, kg = e >> 8;
+            const int x = (kg % ngrp) * 64 + 4 * (ln & 15) + t, k = (kg / ngrp) * 32 + (ln >> 4) * 8;
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                v[j] = g.F[min(k + j, g.K2 - 1) * g.sfk + min(x, g.rowlen - 1) * g.sfx];
+                if (k + j >= g.K2) v[j] = 0.f;
+            }
+            *reinterpret_cast<bf16x8*>(Fs + (size_t)e * 8) = to_bf16x8(v);
+        }
+        __syncthreads();
+    }
+    bf16x8 wa[RT][KT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int c = rt * 16 + lm, i = kt * 32 + lk + j;
+                v[j] = g.W[min(c, g.Cout - 1) * g.swm + min(i, g.Cin - 1) * g.swk];
+                if (i >= g.Cin) v[j] = 0.f;
+            }
+            wa[rt][kt] = to_bf16x8(v);
+        }
+    float bias[RT][4];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            bias[rt][q] = g.bias ? g.bias[min(rt * 16 + (lane >> 4) * 4 + q, g.Cout - 1)] : 0.f;
+    const long units = g.nrows * ngrp;
+    for (long u = (long)blockIdx.x * 4 + wave; u < units; u += (long)gridDim.x * 4) {
+        const long r = u / ngrp;
+        const int x0 = (int)(u - r * ngrp) * 64;
+        bf16x8 ua[RT][KU > 0 ? KU : 1];
+        if constexpr (KU > 0) {
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int ku = 0; ku < KU; ku++) {
+                    const int c = rt * 16 + lm, k = ku * 32 + lk;
+                    const float* up = g.U + ((long)min(c, g.Cout - 1) * g.nrows + r) * g.K2;
+                    const float4 a = *reinterpret_cast<const float4*>(up + min(k, g.K2 - 4));
+                    const float4 b = *reinterpret_cast<const float4*>(up + min(k + 4, g.K2 - 4));
+                    float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+                        if (k + j >= g.K2) v[j] = 0.f;
+                    ua[rt][ku] = to_bf16x8(v);
+                }
+        }
+        const bool in = x0 + 4 * lm < g.rowlen;
+        const long p = r * g.rowlen + min(x0 + 4 * lm, g.rowlen - 4);
+        // every load unconditional, at a clamped channel and pixel: a load
+        // under a lane's own condition is waited for before the next one
+        float4 hv[KT][8];
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int i = kt * 32 + lk + j;
+                hv[kt][j] = *reinterpret_cast<const float4*>(g.h + min(i, g.Cin - 1) * SP + p);
+            }
+        f32x4 res[RT][4];  // [row tile][pixel t]: rows 4 (l / 16) .. + 3
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            bf16x8 hb[KT];
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    v[j] = t == 0 ? hv[kt][j].x : t == 1 ? hv[kt][j].y : t == 2 ? hv[kt][j].z : hv[kt][j].w;
+                    if (kt * 32 + lk + j >= g.Cin) v[j] = 0.f;
+                }
+                hb[kt] = to_bf16x8(v);
+            }
+            bf16x8 fb[KU > 0 ? KU : 1];
+            if constexpr (KU > 0) {
+#pragma unroll
+                for (int ku = 0; ku < KU; ku++)
+                    fb[ku] = *reinterpret_cast<const bf16x8*>(
+                        Fs + ((size_t)((ku * ngrp + (x0 >> 6)) * 4 + t) * 64 + lane) * 8);
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[rt][kt], hb[kt], acc, 0, 0, 0);
+                if constexpr (KU > 0) {
+                    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int ku = 0; ku < KU; ku++)
+                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua[rt][ku], fb[ku], s, 0, 0, 0);
+                    acc += s;
+                }
+                res[rt][t] = acc;
+            }
+        }
+        if (!in) continue;
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int c = rt * 16 + (lane >> 4) * 4 + q;
+                if (c >= g.Cout) continue;
+                const long o = c * SP + p;
+                const float b = bias[rt][q];
+                float4 v;
+                v.x = res[rt][0][q];
+                v.y = res[rt][1][q];
+                v.z = res[rt][2][q];
+                v.w = res[rt][3][q];
+                if (g.bias) {  // (the sum of a null bias could turn -0 into 0)
+                    v.x += b;
+                    v.y += b;
+                    v.z += b;
+                    v.w += b;
+                }
+                if (g.act == 1) {
+                    if (g.pre) *reinterpret_cast<float4*>(g.pre + o) = v;
+                    v.x = gelu_t(v.x, nullptr);
+                    v.y = gelu_t(v.y, nullptr);
+                    v.z = gelu_t(v.z, nullptr);
+                    v.w = gelu_t(v.w, nullptr);
+                } else if (g.act == 2) {
+                    const float4 z = *reinterpret_cast<const float4*>(g.pre + o);
+                    float d;
+                    gelu_t(z.x, &d);
+                    v.x *= d;
+                    gelu_t(z.y, &d);
+                    v.y *= d;
+                    gelu_t(z.z, &d);
+                    v.z *= d;
+                    gelu_t(z.w, &d);
+                    v.w *= d;
+                } else if (g.pre) {
+                    *reinterpret_cast<float4*>(g.pre + o) = v;
+                }
+                *reinterpret_cast<float4*>(g.out + o) = v;
+            }
+    }
+}
+
+template <int RT, int KT, int KU>
+static hipError_t point_launch(const PointArgs& g, hipStream_t st) {
+    const long wg = (g.nrows * ((g.rowlen + 63) / 64) + 3) / 4;
+    // as many workgroups as can be resident (each stages F once)
+    const unsigned grid = (unsigned)(wg < 1024 ? (wg > 0 ? wg : 1) : 1024);
+    const size_t lds = (size_t)KU * ((g.rowlen + 63) / 64) * 256 * 8 * sizeof(__bf16);
+    k_pointwise<RT, KT, KU><<<grid, 256, lds, st>>>(g);
+    return hipGetLastError();
+}
+
+template <int RT, int KT>
+static hipError_t point_ku(const PointArgs& g, hipStream_t st) {
+    if (!g.U) return point_launch<RT, KT, 0>(g, st);
+    return g.K2 <= 32 ? point_launch<RT, KT, 1>(g, st) : point_launch<RT, KT, 2>(g, st);
+}
+template <int RT>
+static hipError_t point_kt(const PointArgs& g, hipStream_t st) {
+    return g.Cin <= 32 ? point_ku<RT, 1>(g, st) : point_ku<RT, 2>(g, st);
+}
+
+// Channel maps of at most 64 in and out channels over rows of a multiple of 4
+// pixels at 16-byte aligned addresses (rows of at most 512 pixels and 64
+// spectrum values with U); anything else takes k_gemm_bf16.
+bool pointwise_supported(const float* h, const float* out, const float* pre, const float* U, long Cout, long Cin,
+                         long nrows, long rowlen, long K2) {
+    const uintptr_t a = (uintptr_t)h | (uintptr_t)out | (uintptr_t)pre | (uintptr_t)U;
+    return Cout >= 1 && Cout <= 64 && Cin >= 1 && Cin <= 64 && nrows >= 1 && rowlen >= 4 && rowlen % 4 == 0 &&
+           (a & 15) == 0 && nrows * (rowlen / 4) < (1L << 40) && rowlen < (1L << 30) &&
+           (!U || (rowlen <= 512 && K2 >= 4 && K2 <= 64 && K2 % 4 == 0));
+}
+
+hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Cin, const float* h, float* out,
+                            long nrows, int rowlen, const float* U, int K2, const float* F, long sfk, long sfx,
+                            const float* bias, float* pre, int act, hipStream_t st) {
+    if (!pointwise_supported(h, out, pre, U, Cout, Cin, nrows, rowlen, K2)) return hipErrorInvalidValue;
+    if (!U) {  // no rows to tell apart: the image as rows of 64 pixels
+        const long SP = nrows * rowlen;
+        if (SP % 64 == 0) {
+            nrows = SP / 64;
+            rowlen = 64;
+        }
+    }
+    const PointArgs g{W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U, K2, F, sfk, sfx, bias, pre, act};
+    switch ((Cout + 15) / 16) {
+        case 1: return point_kt<1>(g, st);
+        case 2: return point_kt<2>(g, st);
+        case 3: return point_kt<3>(g, st);
+        default: return point_kt<4>(g, st);
+    }
+}
+
 // ------------------------------------------------------------------ elementwise
 
 // y = act(a + b + bias[channel]) over [S][C][P]; pre (optional) keeps a + b + bias

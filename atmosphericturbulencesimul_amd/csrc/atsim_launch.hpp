@@ -133,6 +133,13 @@ struct GemmArgs {
     int avec, bvec;     // staging modes, set by launch_gemm_bf16
 };
 hipError_t launch_gemm_bf16(const GemmArgs& g, hipStream_t st);
+// 1x1 channel map of [C][nrows][rowlen] images, with (U) the inverse transform
+// along x of the rows' retained spectrum added; see k_pointwise
+bool pointwise_supported(const float* h, const float* out, const float* pre, const float* U, long Cout, long Cin,
+                         long nrows, long rowlen, long K2);
+hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Cin, const float* h, float* out,
+                            long nrows, int rowlen, const float* U, int K2, const float* F, long sfk, long sfx,
+                            const float* bias, float* pre, int act, hipStream_t st);
 hipError_t launch_add_bias_act(const float* a, const float* b, const float* bias, float* pre, float* y, long C,
                                long P, long n, int gelu, hipStream_t st);
 hipError_t launch_gelu_bwd(const float* pre, const float* dy, float* dx, long n, hipStream_t st);

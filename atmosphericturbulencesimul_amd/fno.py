@@ -76,6 +76,27 @@ class Ops:
             self.ctx._chk(L.atsim_gemm_bf16_ex(self.ctx.h, M, N, K, batch, alpha, pa, sab, sam, sak, pb, sbb, sbk,
                                                sbn, beta, pc, scb, scm, scn, _p(bias), pp, int(gelu)))
 
+    @staticmethod
+    def pointwise_ok(Cout, Cin, rowlen, tensors, K2=0):
+        """the sizes and alignments atsim_nn_pointwise takes (K2 > 0: with the
+        inverse x transform); the others go through gemm"""
+        return (Cout <= 64 and Cin <= 64 and rowlen % 4 == 0
+                and all(t.data_ptr() % 16 == 0 for t in tensors if t is not None)
+                and (K2 == 0 or (rowlen <= 512 and K2 <= 64 and K2 % 4 == 0)))
+
+    def pointwise(self, W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U=None, K2=0, F=None, sfk=0, sfx=0, bias=None,
+                  pre=None, act=0):
+        """out = act(W h [+ U F] [+ bias]) over [C][nrows][rowlen] images; act 0
+        identity, 1 GELU (pre keeps its argument), 2 times GELU'(pre)"""
+        n = nrows * rowlen
+        if (h.numel() < Cin * n or out.numel() < Cout * n or W.numel() <= (Cout - 1) * swm + (Cin - 1) * swk
+                or (bias is not None and bias.numel() < Cout) or (pre is not None and pre.numel() != out.numel())
+                or (U is not None and (U.numel() < Cout * nrows * K2
+                                       or F.numel() <= (K2 - 1) * sfk + (rowlen - 1) * sfx))):
+            raise ValueError(f"pointwise operands out of bounds ({Cout} x {Cin} channels, {nrows} rows of {rowlen})")
+        self.ctx._chk(self.L.atsim_nn_pointwise(self.ctx.h, _p(W), swm, swk, Cout, Cin, _p(h), _p(out), nrows, rowlen,
+                                                _p(U), K2, _p(F), sfk, sfx, _p(bias), _p(pre), act))
+
     def add_bias_act(self, a, b, bias, pre, y, Cc, P, gelu):
         n = a.numel()
         if any(t is not None and t.numel() != n for t in (b, pre, y)) or (bias is not None and bias.numel() != Cc):
@@ -176,14 +197,23 @@ class FNO:
         self.Fx, self.Gre, self.Gim, self.Fxi = f(Fx), f(np.cos(ay)), f(-np.sin(ay)), f(Fxi)
 
     # ---------------------------------------------------------------- building blocks
-    def _pointwise(self, Wt, h, out, Cout, Cin, SP, beta=0.0, bias=None, pre=None, gelu=False):
-        # out[o][q] = act(sum_i W[o][i] h[i][q] + beta out[o][q] + bias[o])
-        self.ops.gemm(Cout, SP, Cin, 1, Wt, 0, 0, Cin, 1, h, 0, 0, SP, 1, out, 0, 0, SP, 1, beta=beta, bias=bias,
-                      pre=pre, gelu=gelu)
+    def _pointwise(self, Wt, h, out, Cout, Cin, SP, bias=None, pre=None, gelu=False):
+        # out[o][q] = act(sum_i W[o][i] h[i][q] + bias[o])
+        if self.ops.pointwise_ok(Cout, Cin, self.N, (h, out, pre)):
+            self.ops.pointwise(Wt, Cin, 1, Cout, Cin, h, out, SP // self.N, self.N, bias=bias, pre=pre, act=int(gelu))
+            return
+        self.ops.gemm(Cout, SP, Cin, 1, Wt, 0, 0, Cin, 1, h, 0, 0, SP, 1, out, 0, 0, SP, 1, bias=bias, pre=pre,
+                      gelu=gelu)
 
-    def _pointwise_t(self, Wt, dy, out, Cout, Cin, SP, beta=0.0):
-        # out[i][q] = sum_o W[o][i] dy[o][q]
-        self.ops.gemm(Cin, SP, Cout, 1, Wt, 0, 0, 1, Cin, dy, 0, 0, SP, 1, out, 0, 0, SP, 1, beta=beta)
+    def _pointwise_t(self, Wt, dy, out, Cout, Cin, SP, pre=None):
+        # out[i][q] = sum_o W[o][i] dy[o][q], times GELU'(pre[i][q]) if pre is given
+        if self.ops.pointwise_ok(Cin, Cout, self.N, (dy, out, pre)):
+            self.ops.pointwise(Wt, 1, Cin, Cin, Cout, dy, out, SP // self.N, self.N, pre=pre,
+                               act=2 if pre is not None else 0)
+            return
+        self.ops.gemm(Cin, SP, Cout, 1, Wt, 0, 0, 1, Cin, dy, 0, 0, SP, 1, out, 0, 0, SP, 1)
+        if pre is not None:
+            self.ops.gelu_bwd(pre, out, out)
 
     def _weight_grad(self, dy, h, gW, Cout, Cin, SP):
         # gW[o][i] = sum_q dy[o][q] h[i][q], split over K chunks, partials summed in order
@@ -194,8 +224,9 @@ class FNO:
         self.ops.gemm(Cout, Cin, kc, nb, dy, 0, kc, SP, 1, h, 0, kc, 1, SP, part, 0, Cout * Cin, Cin, 1)
         self.ops.reduce(part, gW, nb, Cout * Cin)
 
-    def _spectral(self, h, R, S, out):
-        """out [C][S][N][N] = K h; returns the retained spectrum B [C][S][2m][m][2]"""
+    def _spectral(self, h, R, S):
+        """U [C][S][N][2m], the retained spectrum of K h transformed back along y,
+        and the retained spectrum B [C][S][2m][m][2] of h"""
         torch = _torch()
         N, m, Cw = self.N, self.m, self.width
         rows = Cw * S * N
@@ -208,8 +239,22 @@ class FNO:
         self._mix(R, B, O, S)
         U = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
         self._cmat_left_inv(O, U, cs)
-        self.ops.gemm(rows, N, 2 * m, 1, U, 0, 0, 2 * m, 1, self.Fxi, 0, 0, N, 1, out, 0, 0, N, 1)
-        return B
+        return U, B
+
+    def _map_add(self, W, swm, swk, h, U, F, sfk, sfx, out, SP, bias=None, pre=None, act=0):
+        """out = act(W h + U F + bias): a block's 1x1 map with the inverse x
+        transform of its spectral path (U, table F) in the same pass; act as
+        Ops.pointwise"""
+        N, K2, Cw = self.N, 2 * self.m, self.width
+        if self.ops.pointwise_ok(Cw, Cw, N, (h, out, pre, U), K2):
+            self.ops.pointwise(W, swm, swk, Cw, Cw, h, out, SP // N, N, U, K2, F, sfk, sfx, bias, pre, act)
+            return
+        g = self.ops.gemm
+        g(Cw * SP // N, N, K2, 1, U, 0, 0, K2, 1, F, 0, 0, sfk, sfx, out, 0, 0, N, 1)
+        g(Cw, SP, Cw, 1, W, 0, 0, swm, swk, h, 0, 0, SP, 1, out, 0, 0, SP, 1, beta=1.0, bias=bias,
+          pre=pre if act < 2 else None, gelu=act == 1)
+        if act == 2:
+            self.ops.gelu_bwd(pre, out, out)
 
     def _cmat_left(self, Gre, Gim, T, Bout, batch, transpose):
         """Bout[b] (2m x m complex) = G (2m x N complex) T[b] (N x m complex, interleaved columns)"""
@@ -245,8 +290,9 @@ class FNO:
         g(Cw, S, Cw, nm, R, 0, *ra, B, 1, *bb, O, 1, *cc)
         g(Cw, S, Cw, nm, R, 1, *ra, B, 0, *bb, O, 1, *cc, beta=1.0)
 
-    def _spectral_backward(self, g_out, R, B, S, dh, dR):
-        """dh (written) and dR (written) from the upstream gradient g_out [C][S][N][N]"""
+    def _spectral_backward(self, g_out, R, B, S, dR):
+        """dR (written) from the upstream gradient g_out [C][S][N][N]; returns dT1
+        [C][S][N][2m], whose product with Fx^T is the gradient of h"""
         torch = _torch()
         N, m, Cw = self.N, self.m, self.width
         rows, cs, nm = Cw * S * N, Cw * S, 2 * m * m
@@ -276,29 +322,27 @@ class FNO:
         # dT1re = Gre^T dBre + Gim^T dBim ; dT1im = Gre^T dBim - Gim^T dBre  (the inverse-y form)
         dT1 = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
         self._cmat_left_inv(dB, dT1, cs)
-        # dh = dT1 Fx^T
-        gm(rows, N, 2 * m, 1, dT1, 0, 0, 2 * m, 1, self.Fx, 0, 0, 1, 2 * m, dh, 0, 0, N, 1)
+        return dT1
 
     # ---------------------------------------------------------------- forward / backward
     @on_ctx_stream
     def forward(self, x, keep=True):
         """x [cin][S][N][N] float32 -> y [cout][S][N][N]"""
         torch = _torch()
-        P = self.N * self.N
-        S = x.shape[1]
-        SP = S * P
+        N, S = self.N, x.shape[1]
+        SP = S * N * N
         Cw, p, ops = self.width, self.param, self.ops
         cache = {"x": x, "S": S}
         h = torch.empty((Cw, S, self.N, self.N), dtype=torch.float32, device=self.dev)
         self._pointwise(p["Lw"], x, h, Cw, self.cin, SP, bias=p["Lb"])
         for b in range(self.blocks):
-            # hn = act(W h + K h + B): the spectral path writes K h, the 1x1 map
-            # adds onto it with its bias and activation in one GEMM epilogue
+            # hn = act(W h + K h + B): the 1x1 map adds the spectral path's
+            # inverse x transform, its bias and activation in one pass
             hn = torch.empty_like(h)
-            B = self._spectral(h, p[f"R{b}"], S, hn)
+            U, B = self._spectral(h, p[f"R{b}"], S)
             pre = torch.empty_like(h) if keep else None
-            self._pointwise(p[f"W{b}"], h, hn, Cw, Cw, SP, beta=1.0, bias=p[f"B{b}"], pre=pre,
-                            gelu=b < self.blocks - 1)
+            self._map_add(p[f"W{b}"], Cw, 1, h, U, self.Fxi, N, 1, hn, SP, bias=p[f"B{b}"], pre=pre,
+                          act=int(b < self.blocks - 1))
             if keep:
                 cache[f"h{b}"], cache[f"pre{b}"], cache[f"B{b}"] = h, pre, B
             h = hn
@@ -329,22 +373,21 @@ class FNO:
         self._weight_grad(dy, c["q1"], g["Q2"], self.cout, H, SP)
         ops.bias_grad(dy, g["q2b"], self.cout, SP)
         dq1 = torch.empty_like(c["q1"])
-        self._pointwise_t(p["Q2"], dy, dq1, self.cout, H, SP)
-        ops.gelu_bwd(c["preq"], dq1, dq1)
+        self._pointwise_t(p["Q2"], dy, dq1, self.cout, H, SP, pre=c["preq"])
         self._weight_grad(dq1, c["hL"], g["Q1"], H, Cw, SP)
         ops.bias_grad(dq1, g["q1b"], H, SP)
         dh = torch.empty_like(c["hL"])
         self._pointwise_t(p["Q1"], dq1, dh, H, Cw, SP)
         for b in reversed(range(self.blocks)):
-            if b < self.blocks - 1:
-                ops.gelu_bwd(c[f"pre{b}"], dh, dh)
-            dpre = dh
+            dpre = dh  # times GELU' already: by the pass that wrote it
             h = c[f"h{b}"]
             ops.bias_grad(dpre, g[f"B{b}"], Cw, SP)
             self._weight_grad(dpre, h, g[f"W{b}"], Cw, Cw, SP)
             dhn = torch.empty_like(h)
-            self._spectral_backward(dpre, p[f"R{b}"], c[f"B{b}"], S, dhn, g[f"R{b}"])
-            self._pointwise_t(p[f"W{b}"], dpre, dhn, Cw, Cw, SP, beta=1.0)
+            dT1 = self._spectral_backward(dpre, p[f"R{b}"], c[f"B{b}"], S, g[f"R{b}"])
+            # W^T dpre + dT1 Fx^T, times the GELU' of the block before
+            self._map_add(p[f"W{b}"], 1, Cw, dpre, dT1, self.Fx, 1, 2 * self.m, dhn, SP,
+                          pre=c[f"pre{b - 1}"] if b > 0 else None, act=2 if b > 0 else 0)
             dh = dhn
         self._weight_grad(dh, c["x"], g["Lw"], Cw, self.cin, SP)
         ops.bias_grad(dh, g["Lb"], Cw, SP)

@@ -381,6 +381,19 @@ int atsim_gemm_bf16_ex(atsim_ctx *ctx, long M, long N, long K, long batch, float
                        const float *A, long sab, long sam, long sak,
                        const float *B, long sbb, long sbk, long sbn, float beta,
                        float *C, long scb, long scm, long scn, const float *bias, float *pre, int gelu);
+/* A 1x1 channel map in one pass: out[c][p] = act(sum_i W[c swm + i swk]
+ * h[i][p] + sum_k U[c][r][k] F[k sfk + x sfx] + bias[c]) over channel-major
+ * images of nrows rows of rowlen pixels (p = r rowlen + x); U (with K2 values
+ * per row and the table F: the inverse transform of a row's retained spectrum)
+ * and bias may be NULL.  act 0: identity (pre, if given, receives the value
+ * too), 1: GELU (pre receives its argument), 2: times GELU'(pre).  Products and
+ * order as atsim_gemm_bf16 (BF16 operands, FP32 accumulation).  At most 64
+ * channels in and out, rowlen a multiple of 4, h / out / pre / U 16-byte
+ * aligned, and with U rows of at most 512 pixels and K2 <= 64, a multiple of 4
+ * (ATSIM_EUNSUPPORTED otherwise); out must not overlap h. */
+int atsim_nn_pointwise(atsim_ctx *ctx, const float *W, long swm, long swk, long Cout, long Cin, const float *h,
+                       float *out, long nrows, long rowlen, const float *U, long K2, const float *F, long sfk,
+                       long sfx, const float *bias, float *pre, int act);
 /* y = act(a + b + bias[c]) over n = S*C*P elements laid out [S][C][P]; b, bias
  * and pre may be NULL; pre keeps the activation's input; act = GELU (tanh
  * form) if gelu != 0, else identity. */

@@ -2133,6 +2133,31 @@ int atsim_nn_pointwise(atsim_ctx* c, const float* W, long swm, long swk, long Co
     return ATSIM_OK;
 }
 
+int atsim_nn_spectral_fwd(atsim_ctx* c, const float* h, const float* F, long sfk, long sfn, const float* Gre,
+                          const float* Gim, const float* R, int adjoint, float* B, float* O, float* U, long C, long S,
+                          long N, long m) {
+    if (!c || !h || !F || !Gre || !Gim || !R || !B || !O || !U || C <= 0 || S <= 0 || N <= 0 || m <= 0 || sfk < 0 ||
+        sfn < 0)
+        return ATSIM_EINVAL;
+    const long images = C * S;
+    if (!spectral_supported(h, U, B, O, R, images, N, m, C, S))
+        return fail(c, ATSIM_EUNSUPPORTED, "spectral: %ld channels, %ld samples of %ld^2, %ld modes", C, S, N, m);
+    c->work_gen++;
+    HIPCHK(c, launch_dft2(h, F, sfk, sfn, Gre, Gim, B, images, (int)N, (int)m, c->stream));
+    HIPCHK(c, launch_mix(R, B, O, (int)C, (int)S, (int)(2 * m * m), adjoint != 0, c->stream));
+    HIPCHK(c, launch_idft_y(Gre, Gim, O, U, images, (int)N, (int)m, c->stream));
+    return ATSIM_OK;
+}
+
+int atsim_nn_mix_grad(atsim_ctx* c, const float* dO, const float* B, float* dR, long C, long S, long m) {
+    if (!c || !dO || !B || !dR || C <= 0 || S <= 0 || m <= 0) return ATSIM_EINVAL;
+    if (C > 64 || S > (1L << 24) || m > 4096 || (((uintptr_t)dO | (uintptr_t)B | (uintptr_t)dR) & 7))
+        return fail(c, ATSIM_EUNSUPPORTED, "mix_grad: %ld channels, %ld samples, %ld modes", C, S, m);
+    c->work_gen++;
+    HIPCHK(c, launch_mix_grad(dO, B, dR, (int)C, (int)S, (int)(2 * m * m), c->stream));
+    return ATSIM_OK;
+}
+
 int atsim_nn_add_bias_act(atsim_ctx* c, const float* a, const float* b, const float* bias, float* pre, float* y,
                           long C, long P, long n, int gelu) {
     if (!c || !a || !y || C <= 0 || P <= 0 || n < 0 || n % (C * P)) return ATSIM_EINVAL;

@@ -436,6 +436,339 @@ hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Ci
     }
 }
 
+// ------------------------------------------------------------------ spectral path
+// The products of a block's spectral path, forward and backward, each complex
+// product in one pass: the four real products in accumulators of their own, in
+// k_gemm_bf16's order (k steps of 32, zero padded), and added last in the order
+// its passes added them (first product kept, second added with its sign): the
+// same results.  As k_gemm_bf16 passes a complex product read its operands
+// and its half-written output four times over, in 4-byte loads.
+
+// the 8 values X[k + j] (j < 8) of one operand row, zero past K
+__device__ __forceinline__ bf16x8 operand8(const float* __restrict__ X, long sk, int k, int K) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        v[j] = X[min(k + j, K - 1) * sk];
+        if (k + j >= K) v[j] = 0.f;
+    }
+    return to_bf16x8(v);
+}
+// the same from interleaved complex values: real and imaginary operands
+__device__ __forceinline__ void operand8c(const float* __restrict__ X, long sk, int k, int K, bf16x8& re, bf16x8& im) {
+    float a[8], b[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float2 z = *reinterpret_cast<const float2*>(X + min(k + j, K - 1) * sk);
+        a[j] = z.x;
+        b[j] = z.y;
+        if (k + j >= K) a[j] = b[j] = 0.f;
+    }
+    re = to_bf16x8(a);
+    im = to_bf16x8(b);
+}
+#define MFMA16(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16((a), (b), (c), 0, 0, 0)
+
+// Retained spectrum of real N x N images: T = h F along x (F[x sfk + c sfn],
+// 2m columns: re and im of m modes), then out[ky][kx] = sum_y G[ky][y] T[y][kx]
+// (complex) for 2m ky.  One workgroup takes one image at a time: a wave
+// transforms 16 rows from float4 loads, T stays in LDS as the BF16 operand of the
+// second product (N + 8 values per column), and F and G are staged once per
+// workgroup as MFMA operands.  Bound: HBM (the image read once).  1 600 images
+// of 256^2, 16 modes (419 MB): 113 us, 3.7 TB/s, where the x product (292 us)
+// and the four real y products (49 us each) took 489 us.
+constexpr int DFT_T = 512;
+template <int NT>
+__global__ void __launch_bounds__(DFT_T) k_dft2(const float* __restrict__ h, const float* __restrict__ F, long sfk,
+                                                long sfn, const float* __restrict__ Gre,
+                                                const float* __restrict__ Gim, float* __restrict__ out, long images,
+                                                int N, int m) {
+    extern __shared__ __attribute__((aligned(16))) __bf16 sm[];
+    const int KS = N / 32, M2 = 2 * m, NX = (m + 15) / 16, TS = N + 8;
+    __bf16* Fs = sm;                                  // [KS][NT][lane][8]
+    __bf16* Gs = Fs + (size_t)KS * NT * 512;          // [re, im][NT][KS][lane][8]
+    __bf16* Tt = Gs + (size_t)2 * NT * KS * 512;      // [column 2 kx + (re, im)][TS]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lm = lane & 15, lk = (lane >> 4) * 8;
+    for (int e = threadIdx.x; e < KS * NT * 64; e += DFT_T) {
+        const int ln = e & 63, t = e >> 6, nt = t % NT, ks = t / NT;
+        const int n = nt * 16 + (ln & 15), k = ks * 32 + (ln >> 4) * 8;
+        bf16x8 v = operand8(F + min(n, M2 - 1) * sfn, sfk, k, N);
+        *reinterpret_cast<bf16x8*>(Fs + (size_t)e * 8) = v;
+    }
+    for (int e = threadIdx.x; e < 2 * NT * KS * 64; e += DFT_T) {
+        const int ln = e & 63, t = e >> 6, ks = t % KS, mt = (t / KS) % NT, ri = t / (KS * NT);
+        const int r = min(mt * 16 + (ln & 15), M2 - 1), k = ks * 32 + (ln >> 4) * 8;
+        *reinterpret_cast<bf16x8*>(Gs + (size_t)e * 8) = operand8((ri ? Gim : Gre) + (long)r * N, 1, k, N);
+    }
+    for (long img = blockIdx.x; img < images; img += gridDim.x) {
+        __syncthreads();  // the tables are staged / the previous image's T is read
+        const float* hi = h + img * N * N;
+        for (int y0 = wave * 16; y0 < N; y0 += DFT_T / 64 * 16) {
+            const float* row = hi + (long)(y0 + lm) * N + lk;
+            f32x4 acc[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int k0 = 0; k0 < KS; k0 += 4) {
+                float4 a[4][2];  // the loads of 4 k steps together
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const float* p = row + min(k0 + q, KS - 1) * 32;
+                    a[q][0] = *reinterpret_cast<const float4*>(p);
+                    a[q][1] = *reinterpret_cast<const float4*>(p + 4);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (k0 + q >= KS) break;
+                    const float v[8] = {a[q][0].x, a[q][0].y, a[q][0].z, a[q][0].w,
+                                        a[q][1].x, a[q][1].y, a[q][1].z, a[q][1].w};
+                    const bf16x8 av = to_bf16x8(v);
+#pragma unroll
+                    for (int nt = 0; nt < NT; nt++)
+                        acc[nt] = MFMA16(av, *reinterpret_cast<const bf16x8*>(Fs + ((size_t)((k0 + q) * NT + nt) * 64 + lane) * 8),
+                                         acc[nt]);
+                }
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const bf16x4 t = {(__bf16)acc[nt][0], (__bf16)acc[nt][1], (__bf16)acc[nt][2], (__bf16)acc[nt][3]};
+                *reinterpret_cast<bf16x4*>(Tt + (nt * 16 + lm) * TS + y0 + (lane >> 4) * 4) = t;
+            }
+        }
+        __syncthreads();
+        // one (ky tile, kx tile, re or im) per wave
+        for (int task = wave; task < NT * NX * 2; task += DFT_T / 64) {
+            const int ri = task & 1, nx = (task >> 1) % NX, mt = (task >> 1) / NX;
+            f32x4 p = {0.f, 0.f, 0.f, 0.f}, s = {0.f, 0.f, 0.f, 0.f};
+            const __bf16* tr = Tt + (2 * (nx * 16 + lm) + ri) * TS + lk;        // multiplied by Gre
+            const __bf16* ti = Tt + (2 * (nx * 16 + lm) + 1 - ri) * TS + lk;    // multiplied by Gim
+            for (int ks = 0; ks < KS; ks++) {
+                const bf16x8 gr = *reinterpret_cast<const bf16x8*>(Gs + ((size_t)(mt * KS + ks) * 64 + lane) * 8);
+                const bf16x8 gi = *reinterpret_cast<const bf16x8*>(Gs + ((size_t)((NT + mt) * KS + ks) * 64 + lane) * 8);
+                p = MFMA16(gr, *reinterpret_cast<const bf16x8*>(tr + ks * 32), p);
+                s = MFMA16(gi, *reinterpret_cast<const bf16x8*>(ti + ks * 32), s);
+            }
+            const int kx = nx * 16 + lm;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int ky = mt * 16 + (lane >> 4) * 4 + q;
+                if (ky < M2 && kx < m) out[((img * M2 + ky) * m + kx) * 2 + ri] = ri ? p[q] + s[q] : p[q] - s[q];
+            }
+        }
+    }
+}
+
+// U[y][kx] = sum_ky conj(G[ky][y]) O[ky][kx] (complex): the spectra back along
+// y.  A workgroup stages G once as MFMA operands; a wave keeps an image's
+// spectrum operands and makes its 16-row tiles.  Bound: HBM (U written).
+template <int KT>
+__global__ void __launch_bounds__(256) k_idft_y(const float* __restrict__ Gre, const float* __restrict__ Gim,
+                                                const float* __restrict__ O, float* __restrict__ U, long images,
+                                                int N, int m) {
+    extern __shared__ __attribute__((aligned(16))) __bf16 sm[];
+    const int M2 = 2 * m, YT = N / 16, NX = (m + 15) / 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lm = lane & 15, lk = (lane >> 4) * 8;
+    // [re, im][YT][KT][lane][8]: row y, k = ky
+    for (int e = threadIdx.x; e < 2 * YT * KT * 64; e += 256) {
+        const int ln = e & 63, t = e >> 6, kt = t % KT, yt = (t / KT) % YT, ri = t / (KT * YT);
+        *reinterpret_cast<bf16x8*>(sm + (size_t)e * 8) =
+            operand8((ri ? Gim : Gre) + yt * 16 + (ln & 15), N, kt * 32 + (ln >> 4) * 8, M2);
+    }
+    __syncthreads();
+    for (long img = blockIdx.x; img < images; img += gridDim.x)
+        for (int nx = 0; nx < NX; nx++) {
+            const int kx = nx * 16 + lm;
+            bf16x8 ore[KT], oim[KT];
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+                operand8c(O + (img * M2 * m + min(kx, m - 1)) * 2, 2 * m, kt * 32 + lk, M2, ore[kt], oim[kt]);
+            for (int yt = wave; yt < YT; yt += 4) {
+                f32x4 rr = {0.f, 0.f, 0.f, 0.f}, ii = rr, ri = rr, ir = rr;
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+                    const bf16x8 gr = *reinterpret_cast<const bf16x8*>(sm + ((size_t)(yt * KT + kt) * 64 + lane) * 8);
+                    const bf16x8 gi =
+                        *reinterpret_cast<const bf16x8*>(sm + ((size_t)((YT + yt) * KT + kt) * 64 + lane) * 8);
+                    rr = MFMA16(gr, ore[kt], rr);
+                    ii = MFMA16(gi, oim[kt], ii);
+                    ri = MFMA16(gr, oim[kt], ri);
+                    ir = MFMA16(gi, ore[kt], ir);
+                }
+                if (kx < m)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const long y = img * N + yt * 16 + (lane >> 4) * 4 + q;
+                        *reinterpret_cast<float2*>(U + y * M2 + 2 * kx) = make_float2(rr[q] + ii[q], ri[q] - ir[q]);
+                    }
+            }
+        }
+}
+
+// Per retained mode (one wave each): out[o][s] = sum_i R[o][i] B[i][s], or with
+// ADJ out[i][s] = sum_o conj(R[o][i]) B[o][s].  R [mode][C][C], B and out
+// [C][S][mode], complex; the four waves of a workgroup take adjacent modes.
+template <int RT, int KT, bool ADJ>
+__global__ void __launch_bounds__(256) k_mix(const float* __restrict__ R, const float* __restrict__ B,
+                                             float* __restrict__ out, int C, int S, int nm) {
+    const int lane = threadIdx.x & 63, lm = lane & 15, lk = (lane >> 4) * 8;
+    const int mode = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (mode >= nm) return;
+    bf16x8 are[RT][KT], aim[RT][KT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            const int r = min(rt * 16 + lm, C - 1);
+            operand8c(R + ((long)mode * C * C + (ADJ ? r : r * C)) * 2, ADJ ? 2 * C : 2, kt * 32 + lk, C, are[rt][kt],
+                      aim[rt][kt]);
+        }
+    for (int s0 = blockIdx.y * 16; s0 < S; s0 += gridDim.y * 16) {
+        bf16x8 bre[KT], bim[KT];
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++)
+            operand8c(B + ((long)min(s0 + lm, S - 1) * nm + mode) * 2, 2L * S * nm, kt * 32 + lk, C, bre[kt], bim[kt]);
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            f32x4 rr = {0.f, 0.f, 0.f, 0.f}, ii = rr, ri = rr, ir = rr;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+                rr = MFMA16(are[rt][kt], bre[kt], rr);
+                ii = MFMA16(aim[rt][kt], bim[kt], ii);
+                ri = MFMA16(are[rt][kt], bim[kt], ri);
+                ir = MFMA16(aim[rt][kt], bre[kt], ir);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = rt * 16 + (lane >> 4) * 4 + q;
+                if (r < C && s0 + lm < S)
+                    *reinterpret_cast<float2*>(out + (((long)r * S + s0 + lm) * nm + mode) * 2) =
+                        ADJ ? make_float2(rr[q] + ii[q], ri[q] - ir[q]) : make_float2(rr[q] - ii[q], ri[q] + ir[q]);
+            }
+        }
+    }
+}
+
+// Gradient of the mixing matrices, one wave per mode and 16 rows:
+// dR[o][i] = sum_s dO[o][s] conj(B[i][s]).
+template <int CT>
+__global__ void __launch_bounds__(256) k_mix_grad(const float* __restrict__ dO, const float* __restrict__ B,
+                                                  float* __restrict__ dR, int C, int S, int nm) {
+    const int lane = threadIdx.x & 63, lm = lane & 15, lk = (lane >> 4) * 8;
+    const int mode = blockIdx.x * 4 + (threadIdx.x >> 6), rt = blockIdx.y;
+    if (mode >= nm) return;
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    f32x4 rr[CT], ii[CT], ri[CT], ir[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) rr[ct] = ii[ct] = ri[ct] = ir[ct] = z;
+    for (int k0 = 0; k0 < S; k0 += 32) {
+        bf16x8 are, aim;
+        operand8c(dO + ((long)min(rt * 16 + lm, C - 1) * S * nm + mode) * 2, 2L * nm, k0 + lk, S, are, aim);
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+            bf16x8 bre, bim;
+            operand8c(B + ((long)min(ct * 16 + lm, C - 1) * S * nm + mode) * 2, 2L * nm, k0 + lk, S, bre, bim);
+            rr[ct] = MFMA16(are, bre, rr[ct]);
+            ii[ct] = MFMA16(aim, bim, ii[ct]);
+            ir[ct] = MFMA16(aim, bre, ir[ct]);
+            ri[ct] = MFMA16(are, bim, ri[ct]);
+        }
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int r = rt * 16 + (lane >> 4) * 4 + q, i = ct * 16 + lm;
+            if (r < C && i < C)
+                *reinterpret_cast<float2*>(dR + (((long)mode * C + r) * C + i) * 2) =
+                    make_float2(rr[ct][q] + ii[ct][q], ir[ct][q] - ri[ct][q]);
+        }
+}
+
+static size_t dft2_lds(long N, long m) {
+    const long nt = (2 * m + 15) / 16, ks = N / 32;
+    return (size_t)(3 * nt * ks * 512 + 32 * ((m + 15) / 16) * (N + 8)) * sizeof(__bf16);
+}
+// images of N x N, N a multiple of 32, at most 32 modes, at 16-byte aligned
+// addresses (spectra at 8), channels of at most 64, within the LDS of a CU
+bool spectral_supported(const float* h, const float* U, const float* B, const float* O, const float* R, long images,
+                        long N, long m, long C, long S) {
+    return N >= 32 && N % 32 == 0 && N <= 1024 && m >= 1 && 2 * m <= N && m <= 32 && C >= 1 && C <= 64 && S >= 1 &&
+           S <= (1L << 24) && images < (1L << 31) && (((uintptr_t)h | (uintptr_t)U) & 15) == 0 &&
+           (((uintptr_t)B | (uintptr_t)O | (uintptr_t)R) & 7) == 0 && dft2_lds(N, m) <= 160 * 1024;
+}
+
+template <int NT>
+static hipError_t dft2_launch(const float* h, const float* F, long sfk, long sfn, const float* Gre, const float* Gim,
+                              float* out, long images, int N, int m, hipStream_t st) {
+    const size_t lds = dft2_lds(N, m);
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void*)k_dft2<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const long res = 256 * (lds <= 80 * 1024 ? 2 : 1);  // resident workgroups
+    k_dft2<NT><<<(unsigned)(images < res ? images : res), DFT_T, lds, st>>>(h, F, sfk, sfn, Gre, Gim, out, images, N, m);
+    return hipGetLastError();
+}
+hipError_t launch_dft2(const float* h, const float* F, long sfk, long sfn, const float* Gre, const float* Gim,
+                       float* out, long images, int N, int m, hipStream_t st) {
+    if (images <= 0) return hipSuccess;
+    switch ((2 * m + 15) / 16) {
+        case 1: return dft2_launch<1>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
+        case 2: return dft2_launch<2>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
+        case 3: return dft2_launch<3>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
+        default: return dft2_launch<4>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
+    }
+}
+
+template <int KT>
+static hipError_t idft_y_launch(const float* Gre, const float* Gim, const float* O, float* U, long images, int N,
+                                int m, hipStream_t st) {
+    const size_t lds = (size_t)2 * (N / 16) * KT * 512 * sizeof(__bf16);
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void*)k_idft_y<KT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const long res = 256 * (lds <= 40 * 1024 ? 4 : lds <= 80 * 1024 ? 2 : 1);
+    k_idft_y<KT><<<(unsigned)(images < res ? images : res), 256, lds, st>>>(Gre, Gim, O, U, images, N, m);
+    return hipGetLastError();
+}
+hipError_t launch_idft_y(const float* Gre, const float* Gim, const float* O, float* U, long images, int N, int m,
+                         hipStream_t st) {
+    if (images <= 0) return hipSuccess;
+    return 2 * m <= 32 ? idft_y_launch<1>(Gre, Gim, O, U, images, N, m, st)
+                       : idft_y_launch<2>(Gre, Gim, O, U, images, N, m, st);
+}
+
+template <int RT, int KT>
+static hipError_t mix_launch(const float* R, const float* B, float* out, int C, int S, int nm, bool adj,
+                             hipStream_t st) {
+    const int gy = (S + 15) / 16;
+    dim3 grid((nm + 3) / 4, gy < 64 ? gy : 64);
+    if (adj) k_mix<RT, KT, true><<<grid, 256, 0, st>>>(R, B, out, C, S, nm);
+    else k_mix<RT, KT, false><<<grid, 256, 0, st>>>(R, B, out, C, S, nm);
+    return hipGetLastError();
+}
+hipError_t launch_mix(const float* R, const float* B, float* out, int C, int S, int nm, bool adj, hipStream_t st) {
+    switch ((C + 15) / 16) {
+        case 1: return mix_launch<1, 1>(R, B, out, C, S, nm, adj, st);
+        case 2: return mix_launch<2, 1>(R, B, out, C, S, nm, adj, st);
+        case 3: return mix_launch<3, 2>(R, B, out, C, S, nm, adj, st);
+        default: return mix_launch<4, 2>(R, B, out, C, S, nm, adj, st);
+    }
+}
+hipError_t launch_mix_grad(const float* dO, const float* B, float* dR, int C, int S, int nm, hipStream_t st) {
+    const int ct = (C + 15) / 16;
+    dim3 grid((nm + 3) / 4, ct);
+    switch (ct) {
+        case 1: k_mix_grad<1><<<grid, 256, 0, st>>>(dO, B, dR, C, S, nm); break;
+        case 2: k_mix_grad<2><<<grid, 256, 0, st>>>(dO, B, dR, C, S, nm); break;
+        case 3: k_mix_grad<3><<<grid, 256, 0, st>>>(dO, B, dR, C, S, nm); break;
+        default: k_mix_grad<4><<<grid, 256, 0, st>>>(dO, B, dR, C, S, nm); break;
+    }
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------------------ elementwise
 
 // y = act(a + b + bias[channel]) over [S][C][P]; pre (optional) keeps a + b + bias

@@ -140,6 +140,16 @@ bool pointwise_supported(const float* h, const float* out, const float* pre, con
 hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Cin, const float* h, float* out,
                             long nrows, int rowlen, const float* U, int K2, const float* F, long sfk, long sfx,
                             const float* bias, float* pre, int act, hipStream_t st);
+// the spectral path: see k_dft2, k_idft_y, k_mix, k_mix_grad (spectral_supported
+// sizes only)
+bool spectral_supported(const float* h, const float* U, const float* B, const float* O, const float* R, long images,
+                        long N, long m, long C, long S);
+hipError_t launch_dft2(const float* h, const float* F, long sfk, long sfn, const float* Gre, const float* Gim,
+                       float* out, long images, int N, int m, hipStream_t st);
+hipError_t launch_idft_y(const float* Gre, const float* Gim, const float* O, float* U, long images, int N, int m,
+                         hipStream_t st);
+hipError_t launch_mix(const float* R, const float* B, float* out, int C, int S, int nm, bool adj, hipStream_t st);
+hipError_t launch_mix_grad(const float* dO, const float* B, float* dR, int C, int S, int nm, hipStream_t st);
 hipError_t launch_add_bias_act(const float* a, const float* b, const float* bias, float* pre, float* y, long C,
                                long P, long n, int gelu, hipStream_t st);
 hipError_t launch_gelu_bwd(const float* pre, const float* dy, float* dx, long n, hipStream_t st);

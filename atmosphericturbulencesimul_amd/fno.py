@@ -97,6 +97,31 @@ class Ops:
         self.ctx._chk(self.L.atsim_nn_pointwise(self.ctx.h, _p(W), swm, swk, Cout, Cin, _p(h), _p(out), nrows, rowlen,
                                                 _p(U), K2, _p(F), sfk, sfx, _p(bias), _p(pre), act))
 
+    @staticmethod
+    def spectral_ok(C_, N, m, h, R):
+        """the sizes and alignments atsim_nn_spectral_fwd takes; the others go
+        through gemm"""
+        nt, ks = (2 * m + 15) // 16, N // 32
+        lds = 2 * (3 * nt * ks * 512 + 32 * ((m + 15) // 16) * (N + 8))
+        return (C_ <= 64 and N % 32 == 0 and 2 * m <= N <= 1024 and m <= 32 and lds <= 160 * 1024
+                and h.data_ptr() % 16 == 0 and R.data_ptr() % 8 == 0)
+
+    def spectral(self, h, F, sfk, sfn, Gre, Gim, R, adjoint, B, O, U, C_, S, N, m):
+        """B = G (h F), O = R B per mode (adjoint: R^H B), U = G^H O"""
+        sp = C_ * S * 4 * m * m
+        if (h.numel() < C_ * S * N * N or F.numel() <= (N - 1) * sfk + (2 * m - 1) * sfn or Gre.numel() < 2 * m * N
+                or Gim.numel() < 2 * m * N or R.numel() < 4 * m * m * C_ * C_ or B.numel() < sp or O.numel() < sp
+                or U.numel() < C_ * S * N * 2 * m):
+            raise ValueError(f"spectral operands out of bounds ({C_} channels, {S} samples of {N}^2, {m} modes)")
+        self.ctx._chk(self.L.atsim_nn_spectral_fwd(self.ctx.h, _p(h), _p(F), sfk, sfn, _p(Gre), _p(Gim), _p(R),
+                                                   int(adjoint), _p(B), _p(O), _p(U), C_, S, N, m))
+
+    def mix_grad(self, dO, B, dR, C_, S, m):
+        """dR = dO B^H per mode over the samples"""
+        if min(dO.numel(), B.numel()) < C_ * S * 4 * m * m or dR.numel() < 4 * m * m * C_ * C_:
+            raise ValueError("mix_grad: operands too small")
+        self.ctx._chk(self.L.atsim_nn_mix_grad(self.ctx.h, _p(dO), _p(B), _p(dR), C_, S, m))
+
     def add_bias_act(self, a, b, bias, pre, y, Cc, P, gelu):
         n = a.numel()
         if any(t is not None and t.numel() != n for t in (b, pre, y)) or (bias is not None and bias.numel() != Cc):
@@ -231,13 +256,16 @@ class FNO:
         N, m, Cw = self.N, self.m, self.width
         rows = Cw * S * N
         cs = Cw * S
+        B = torch.empty((Cw, S, 2 * m, m, 2), dtype=torch.float32, device=self.dev)
+        O = torch.empty_like(B)
+        U = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
+        if self.ops.spectral_ok(Cw, N, m, h, R):
+            self.ops.spectral(h, self.Fx, 2 * m, 1, self.Gre, self.Gim, R, False, B, O, U, Cw, S, N, m)
+            return U, B
         T1 = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
         self.ops.gemm(rows, 2 * m, N, 1, h, 0, 0, N, 1, self.Fx, 0, 0, 2 * m, 1, T1, 0, 0, 2 * m, 1)
-        B = torch.empty((Cw, S, 2 * m, m, 2), dtype=torch.float32, device=self.dev)
         self._cmat_left(self.Gre, self.Gim, T1, B, cs, transpose=False)
-        O = torch.empty_like(B)
         self._mix(R, B, O, S)
-        U = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
         self._cmat_left_inv(O, U, cs)
         return U, B
 
@@ -297,6 +325,15 @@ class FNO:
         N, m, Cw = self.N, self.m, self.width
         rows, cs, nm = Cw * S * N, Cw * S, 2 * m * m
         gm = self.ops.gemm
+        if self.ops.spectral_ok(Cw, N, m, g_out, R) and dR.data_ptr() % 8 == 0:
+            # the adjoint has the forward path's form: dO = G (g Fxi^T), dB = R^H dO,
+            # dT1 = G^H dB
+            dO = torch.empty((Cw, S, 2 * m, m, 2), dtype=torch.float32, device=self.dev)
+            dB = torch.empty_like(dO)
+            dT1 = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
+            self.ops.spectral(g_out, self.Fxi, 1, N, self.Gre, self.Gim, R, True, dO, dB, dT1, Cw, S, N, m)
+            self.ops.mix_grad(dO, B, dR, Cw, S, m)
+            return dT1
         dU = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
         gm(rows, 2 * m, N, 1, g_out, 0, 0, N, 1, self.Fxi, 0, 0, 1, N, dU, 0, 0, 2 * m, 1)
         dO = torch.empty((Cw, S, 2 * m, m, 2), dtype=torch.float32, device=self.dev)

@@ -394,6 +394,22 @@ int atsim_gemm_bf16_ex(atsim_ctx *ctx, long M, long N, long K, long batch, float
 int atsim_nn_pointwise(atsim_ctx *ctx, const float *W, long swm, long swk, long Cout, long Cin, const float *h,
                        float *out, long nrows, long rowlen, const float *U, long K2, const float *F, long sfk,
                        long sfx, const float *bias, float *pre, int act);
+/* The spectral path of one block up to its inverse x transform, on images h
+ * [C][S][N][N]: B = G (h F) the retained spectrum ([C][S][2m][m] complex; F[x
+ * sfk + c sfn] the table along x with 2m columns, re and im of m modes; G =
+ * Gre + i Gim [2m][N]), O = R B per mode (R [2m m][C][C] complex; adjoint != 0:
+ * its conjugate transpose) and U = G^H O ([C][S][N][2m]).  B, O and U receive
+ * the three.  Products and order as atsim_gemm_bf16.  N a multiple of 32, m <=
+ * 32, C <= 64, h and U 16-byte and B, O, R 8-byte aligned, tables within the
+ * LDS (N = 256 takes m <= 32, N = 512 m <= 16) (ATSIM_EUNSUPPORTED
+ * otherwise). */
+int atsim_nn_spectral_fwd(atsim_ctx *ctx, const float *h, const float *F, long sfk, long sfn, const float *Gre,
+                          const float *Gim, const float *R, int adjoint, float *B, float *O, float *U, long C,
+                          long S, long N, long m);
+/* dR = dO B^H per mode over the samples: dO and B [C][S][2m][m], dR
+ * [2m m][C][C], complex.  C <= 64, 8-byte aligned (ATSIM_EUNSUPPORTED
+ * otherwise). */
+int atsim_nn_mix_grad(atsim_ctx *ctx, const float *dO, const float *B, float *dR, long C, long S, long m);
 /* y = act(a + b + bias[c]) over n = S*C*P elements laid out [S][C][P]; b, bias
  * and pre may be NULL; pre keeps the activation's input; act = GELU (tanh
  * form) if gelu != 0, else identity. */

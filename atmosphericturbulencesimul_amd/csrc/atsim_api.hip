@@ -2158,6 +2158,17 @@ int atsim_nn_mix_grad(atsim_ctx* c, const float* dO, const float* B, float* dR, 
     return ATSIM_OK;
 }
 
+int atsim_nn_weight_grad(atsim_ctx* c, const float* dy, const float* h, float* part, float* gW, long Cout, long Cin,
+                         long SP, long kc) {
+    if (!c || !dy || !h || !part || !gW || Cout <= 0 || Cin <= 0 || SP <= 0 || kc <= 0) return ATSIM_EINVAL;
+    if (!weight_grad_supported(dy, h, Cout, Cin, SP, kc))
+        return fail(c, ATSIM_EUNSUPPORTED, "weight_grad: %ld x %ld channels, %ld pixels by %ld", Cout, Cin, SP, kc);
+    c->work_gen++;
+    HIPCHK(c, launch_weight_grad(dy, h, part, (int)Cout, (int)Cin, SP, (int)kc, c->stream));
+    HIPCHK(c, launch_reduce_batches(part, gW, SP / kc, Cout * Cin, 0, c->stream));
+    return ATSIM_OK;
+}
+
 int atsim_nn_add_bias_act(atsim_ctx* c, const float* a, const float* b, const float* bias, float* pre, float* y,
                           long C, long P, long n, int gelu) {
     if (!c || !a || !y || C <= 0 || P <= 0 || n < 0 || n % (C * P)) return ATSIM_EINVAL;

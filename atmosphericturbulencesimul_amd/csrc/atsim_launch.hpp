@@ -150,6 +150,9 @@ hipError_t launch_idft_y(const float* Gre, const float* Gim, const float* O, flo
                          hipStream_t st);
 hipError_t launch_mix(const float* R, const float* B, float* out, int C, int S, int nm, bool adj, hipStream_t st);
 hipError_t launch_mix_grad(const float* dO, const float* B, float* dR, int C, int S, int nm, hipStream_t st);
+bool weight_grad_supported(const float* dy, const float* h, long Cout, long Cin, long SP, long kc);
+hipError_t launch_weight_grad(const float* dy, const float* h, float* part, int Cout, int Cin, long SP, int kc,
+                              hipStream_t st);
 hipError_t launch_add_bias_act(const float* a, const float* b, const float* bias, float* pre, float* y, long C,
                                long P, long n, int gelu, hipStream_t st);
 hipError_t launch_gelu_bwd(const float* pre, const float* dy, float* dx, long n, hipStream_t st);

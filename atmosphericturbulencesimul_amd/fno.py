@@ -122,6 +122,20 @@ class Ops:
             raise ValueError("mix_grad: operands too small")
         self.ctx._chk(self.L.atsim_nn_mix_grad(self.ctx.h, _p(dO), _p(B), _p(dR), C_, S, m))
 
+    @staticmethod
+    def weight_grad_ok(Cout, Cin, SP, kc, dy, h):
+        """the sizes and alignments atsim_nn_weight_grad takes; the others go
+        through gemm and reduce"""
+        return (Cout <= 64 and Cin <= 64 and kc % 128 == 0 and SP % kc == 0
+                and dy.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
+
+    def weight_grad(self, dy, h, part, gW, Cout, Cin, SP, kc):
+        """gW = dy h^T over SP pixels, in chunks of kc"""
+        if (dy.numel() < Cout * SP or h.numel() < Cin * SP or part.numel() < SP // kc * Cout * Cin
+                or gW.numel() < Cout * Cin):
+            raise ValueError("weight_grad: operands too small")
+        self.ctx._chk(self.L.atsim_nn_weight_grad(self.ctx.h, _p(dy), _p(h), _p(part), _p(gW), Cout, Cin, SP, kc))
+
     def add_bias_act(self, a, b, bias, pre, y, Cc, P, gelu):
         n = a.numel()
         if any(t is not None and t.numel() != n for t in (b, pre, y)) or (bias is not None and bias.numel() != Cc):
@@ -246,6 +260,9 @@ class FNO:
         kc = 1024 if SP % 1024 == 0 else SP
         nb = SP // kc
         part = torch.empty((nb, Cout, Cin), dtype=torch.float32, device=self.dev)
+        if self.ops.weight_grad_ok(Cout, Cin, SP, kc, dy, h):
+            self.ops.weight_grad(dy, h, part, gW, Cout, Cin, SP, kc)
+            return
         self.ops.gemm(Cout, Cin, kc, nb, dy, 0, kc, SP, 1, h, 0, kc, 1, SP, part, 0, Cout * Cin, Cin, 1)
         self.ops.reduce(part, gW, nb, Cout * Cin)
 

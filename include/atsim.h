@@ -410,6 +410,13 @@ int atsim_nn_spectral_fwd(atsim_ctx *ctx, const float *h, const float *F, long s
  * [2m m][C][C], complex.  C <= 64, 8-byte aligned (ATSIM_EUNSUPPORTED
  * otherwise). */
 int atsim_nn_mix_grad(atsim_ctx *ctx, const float *dO, const float *B, float *dR, long C, long S, long m);
+/* Weight gradient of a channel map: gW[o][i] = sum_q dy[o][q] h[i][q] over SP
+ * pixels, in chunks of kc whose partial sums (part, SP / kc x Cout x Cin) are
+ * added in order.  Products as atsim_gemm_bf16.  At most 64 channels each way,
+ * kc a multiple of 128 that divides SP, dy and h 16-byte aligned
+ * (ATSIM_EUNSUPPORTED otherwise). */
+int atsim_nn_weight_grad(atsim_ctx *ctx, const float *dy, const float *h, float *part, float *gW, long Cout, long Cin,
+                         long SP, long kc);
 /* y = act(a + b + bias[c]) over n = S*C*P elements laid out [S][C][P]; b, bias
  * and pre may be NULL; pre keeps the activation's input; act = GELU (tanh
  * form) if gelu != 0, else identity. */

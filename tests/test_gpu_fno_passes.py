@@ -93,7 +93,38 @@ def test_network_matches_the_general_path(ctx, monkeypatch, N, m, width, S, hidd
     assert used
     monkeypatch.setattr(fno.Ops, "spectral_ok", staticmethod(lambda *a: False))
     monkeypatch.setattr(fno.Ops, "pointwise_ok", staticmethod(lambda *a: False))
+    monkeypatch.setattr(fno.Ops, "weight_grad_ok", staticmethod(lambda *a: False))
     loss0, g0 = step()
     assert loss == loss0
     for k in g0:
         assert np.array_equal(g[k], g0[k]), k
+
+
+@pytest.mark.parametrize("nb", [1, 2, 127, 128, 129, 512])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_reduce_batches_sums_in_order(ctx, nb, n, accumulate):
+    rng = np.random.default_rng(nb + n)
+    part, out = rng.standard_normal((nb, n)).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    tp, to = _dev(part, out)
+    assert ctx.L.atsim_nn_reduce_batches(ctx.h, tp.data_ptr(), to.data_ptr(), nb, n, accumulate) == 0
+    ctx.sync()
+    want = out.copy() if accumulate else np.zeros(n, np.float32)
+    for b in range(nb):
+        want = want + part[b]  # float32, ascending
+    assert np.array_equal(to.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("S,C,P", [(1, 3, 4096), (1, 2, 131072 + 1), (1, 1, 5), (3, 2, 1000)])
+def test_bias_grad(ctx, S, C, P):
+    rng = np.random.default_rng(P)
+    dy = rng.standard_normal((S, C, P)).astype(np.float32)
+    t, = _dev(dy)
+    db = torch.empty(C, device="cuda")
+    torch.cuda.synchronize()
+    assert ctx.L.atsim_nn_bias_grad(ctx.h, t.data_ptr(), db.data_ptr(), S, C, P, 0) == 0
+    ctx.sync()
+    # FP64 chunks rounded to float and 64 of them added: 65 roundings of at most
+    # half an ulp of the chunks' magnitudes
+    got, want = db.cpu().numpy().astype(np.float64), dy.astype(np.float64).sum((0, 2))
+    assert np.all(np.abs(got - want) <= 65 * 2.0 ** -24 * np.abs(dy).astype(np.float64).sum((0, 2)))

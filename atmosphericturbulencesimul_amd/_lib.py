@@ -113,6 +113,9 @@ _SIGS = {
     "atsim_nn_mix_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long]),
     "atsim_nn_weight_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long,
                                        C.c_long, C.c_long]),
+    "atsim_nn_tail": (C.c_int, [C.c_void_p, C.c_void_p, C.c_long, C.c_void_p, C.c_long, C.c_long, C.c_void_p, C.c_long,
+                                C.c_void_p, C.c_long, C.c_long, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long,
+                                C.c_void_p, C.c_void_p, C.c_long, C.c_void_p]),
     "atsim_nn_add_bias_act": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                         C.c_long, C.c_long, C.c_long, C.c_int]),
     "atsim_nn_gelu_bwd": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long]),

@@ -2169,6 +2169,20 @@ int atsim_nn_weight_grad(atsim_ctx* c, const float* dy, const float* h, float* p
     return ATSIM_OK;
 }
 
+int atsim_nn_tail(atsim_ctx* c, const float* W, long C, const float* h, long nrows, long rowlen, const float* U,
+                  long K2, const float* F, long sfk, long sfx, const float* bias, const float* Q1, const float* q1b,
+                  long H, const float* Q2, const float* q2b, long cout, float* y) {
+    if (!c || !W || !h || !U || !F || !bias || !Q1 || !q1b || !Q2 || !q2b || !y || C <= 0 || H <= 0 || cout <= 0 ||
+        nrows <= 0 || rowlen <= 0 || sfk < 0 || sfx < 0)
+        return ATSIM_EINVAL;
+    if (!pointwise_supported(h, y, nullptr, U, C, C, nrows, rowlen, K2) || H > 64 || cout > 16)
+        return fail(c, ATSIM_EUNSUPPORTED, "tail: %ld, %ld and %ld channels over rows of %ld", C, H, cout, rowlen);
+    c->work_gen++;
+    HIPCHK(c, launch_tail(W, (int)C, h, nrows, (int)rowlen, U, (int)K2, F, sfk, sfx, bias, Q1, q1b, (int)H, Q2, q2b,
+                          (int)cout, y, c->stream));
+    return ATSIM_OK;
+}
+
 int atsim_nn_add_bias_act(atsim_ctx* c, const float* a, const float* b, const float* bias, float* pre, float* y,
                           long C, long P, long n, int gelu) {
     if (!c || !a || !y || C <= 0 || P <= 0 || n < 0 || n % (C * P)) return ATSIM_EINVAL;

@@ -229,6 +229,85 @@ struct PointArgs {
     int act;
 };
 
+// F [K2][rowlen] staged as MFMA operands [KU][64-pixel group][t][lane][8]
+template <int KU>
+__device__ __forceinline__ void stage_xtable(__bf16* Fs, const float* __restrict__ F, long sfk, long sfx, int K2,
+                                             int rowlen) {
+    const int ngrp = (rowlen + 63) / 64;
+    for (int e = threadIdx.x; e < KU * ngrp * 256; e += 256) {
+        const int ln = e & 63, t = (e >> 6) & 3, kg = e >> 8;
+        const int x = (kg % ngrp) * 64 + 4 * (ln & 15) + t, k = (kg / ngrp) * 32 + (ln >> 4) * 8;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            v[j] = F[min(k + j, K2 - 1) * sfk + min(x, rowlen - 1) * sfx];
+            if (k + j >= K2) v[j] = 0.f;
+        }
+        *reinterpret_cast<bf16x8*>(Fs + (size_t)e * 8) = to_bf16x8(v);
+    }
+}
+// a wave's operands of an M x K matrix (element strides sm, sk)
+template <int RT, int KT>
+__device__ __forceinline__ void matrix_operands(bf16x8 (&wa)[RT][KT], const float* __restrict__ W, long sm, long sk,
+                                                int M, int K, int lm, int lk) {
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                v[j] = W[min(rt * 16 + lm, M - 1) * sm + min(kt * 32 + lk + j, K - 1) * sk];
+                if (kt * 32 + lk + j >= K) v[j] = 0.f;
+            }
+            wa[rt][kt] = to_bf16x8(v);
+        }
+}
+// the spectrum operands of row r of every channel
+template <int RT, int KU>
+__device__ __forceinline__ void spectrum_operands(bf16x8 (&ua)[RT][KU], const float* __restrict__ U, long nrows,
+                                                  long r, int C, int K2, int lm, int lk) {
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int ku = 0; ku < KU; ku++) {
+            const int k = ku * 32 + lk;
+            const float* up = U + ((long)min(rt * 16 + lm, C - 1) * nrows + r) * K2;
+            const float4 a = *reinterpret_cast<const float4*>(up + min(k, K2 - 4));
+            const float4 b = *reinterpret_cast<const float4*>(up + min(k + 4, K2 - 4));
+            float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (k + j >= K2) v[j] = 0.f;
+            ua[rt][ku] = to_bf16x8(v);
+        }
+}
+// the operands of pixel t of a lane's four, from its 8 KT loaded channels
+template <int KT>
+__device__ __forceinline__ void pixel_operands(bf16x8 (&hb)[KT], const float4 (&hv)[KT][8], int t, int C, int lk) {
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            v[j] = t == 0 ? hv[kt][j].x : t == 1 ? hv[kt][j].y : t == 2 ? hv[kt][j].z : hv[kt][j].w;
+            if (kt * 32 + lk + j >= C) v[j] = 0.f;
+        }
+        hb[kt] = to_bf16x8(v);
+    }
+}
+// every load unconditional, at a clamped channel and pixel: a load under a
+// lane's own condition is waited for before the next one
+template <int KT>
+__device__ __forceinline__ void load_channels(float4 (&hv)[KT][8], const float* __restrict__ h, long SP, long p,
+                                              int C, int lk) {
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            hv[kt][j] = *reinterpret_cast<const float4*>(h + min(kt * 32 + lk + j, C - 1) * SP + p);
+}
+
 template <int RT, int KT, int KU>
 __global__ void __launch_bounds__(256) k_pointwise(PointArgs g) {
     extern __shared__ __attribute__((aligned(16))) __bf16 Fs[];  // F as MFMA operands: [KU][64-pixel group][4][lane][8]
@@ -237,33 +316,11 @@ __global__ void __launch_bounds__(256) k_pointwise(PointArgs g) {
     const long SP = g.nrows * g.rowlen;
     const int ngrp = (g.rowlen + 63) / 64;
     if constexpr (KU > 0) {
-        for (int e = threadIdx.x; e < KU * ngrp * 256; e += 256) {
-            const int ln = e & 63, t = (e >> 6) & 3, kg = e >> 8;
-            const int x = (kg % ngrp) * 64 + 4 * (ln & 15) + t, k = (kg / ngrp) * 32 + (ln >> 4) * 8;
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                v[j] = g.F[min(k + j, g.K2 - 1) * g.sfk + min(x, g.rowlen - 1) * g.sfx];
-                if (k + j >= g.K2) v[j] = 0.f;
-            }
-            *reinterpret_cast<bf16x8*>(Fs + (size_t)e * 8) = to_bf16x8(v);
-        }
+        stage_xtable<KU>(Fs, g.F, g.sfk, g.sfx, g.K2, g.rowlen);
         __syncthreads();
     }
     bf16x8 wa[RT][KT];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-        for (int kt = 0; kt < KT; kt++) {
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int c = rt * 16 + lm, i = kt * 32 + lk + j;
-                v[j] = g.W[min(c, g.Cout - 1) * g.swm + min(i, g.Cin - 1) * g.swk];
-                if (i >= g.Cin) v[j] = 0.f;
-            }
-            wa[rt][kt] = to_bf16x8(v);
-        }
+    matrix_operands<RT, KT>(wa, g.W, g.swm, g.swk, g.Cout, g.Cin, lm, lk);
     float bias[RT][4];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
@@ -275,48 +332,16 @@ __global__ void __launch_bounds__(256) k_pointwise(PointArgs g) {
         const long r = u / ngrp;
         const int x0 = (int)(u - r * ngrp) * 64;
         bf16x8 ua[RT][KU > 0 ? KU : 1];
-        if constexpr (KU > 0) {
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-                for (int ku = 0; ku < KU; ku++) {
-                    const int c = rt * 16 + lm, k = ku * 32 + lk;
-                    const float* up = g.U + ((long)min(c, g.Cout - 1) * g.nrows + r) * g.K2;
-                    const float4 a = *reinterpret_cast<const float4*>(up + min(k, g.K2 - 4));
-                    const float4 b = *reinterpret_cast<const float4*>(up + min(k + 4, g.K2 - 4));
-                    float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-                    for (int j = 0; j < 8; j++)
-                        if (k + j >= g.K2) v[j] = 0.f;
-                    ua[rt][ku] = to_bf16x8(v);
-                }
-        }
+        if constexpr (KU > 0) spectrum_operands<RT, KU>(ua, g.U, g.nrows, r, g.Cout, g.K2, lm, lk);
         const bool in = x0 + 4 * lm < g.rowlen;
         const long p = r * g.rowlen + min(x0 + 4 * lm, g.rowlen - 4);
-        // every load unconditional, at a clamped channel and pixel: a load
-        // under a lane's own condition is waited for before the next one
         float4 hv[KT][8];
-#pragma unroll
-        for (int kt = 0; kt < KT; kt++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int i = kt * 32 + lk + j;
-                hv[kt][j] = *reinterpret_cast<const float4*>(g.h + min(i, g.Cin - 1) * SP + p);
-            }
+        load_channels<KT>(hv, g.h, SP, p, g.Cin, lk);
         f32x4 res[RT][4];  // [row tile][pixel t]: rows 4 (l / 16) .. + 3
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             bf16x8 hb[KT];
-#pragma unroll
-            for (int kt = 0; kt < KT; kt++) {
-                float v[8];
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    v[j] = t == 0 ? hv[kt][j].x : t == 1 ? hv[kt][j].y : t == 2 ? hv[kt][j].z : hv[kt][j].w;
-                    if (kt * 32 + lk + j >= g.Cin) v[j] = 0.f;
-                }
-                hb[kt] = to_bf16x8(v);
-            }
+            pixel_operands<KT>(hb, hv, t, g.Cin, lk);
             bf16x8 fb[KU > 0 ? KU : 1];
             if constexpr (KU > 0) {
 #pragma unroll
@@ -403,6 +428,169 @@ static hipError_t point_ku(const PointArgs& g, hipStream_t st) {
 template <int RT>
 static hipError_t point_kt(const PointArgs& g, hipStream_t st) {
     return g.Cin <= 32 ? point_ku<RT, 1>(g, st) : point_ku<RT, 2>(g, st);
+}
+
+// The network's tail for inference, in one pass over the pixels: the last
+// block's map h' = W h + U F + bias (no activation), q = GELU(Q1 h' + q1b),
+// y = Q2 q + q2b, without writing h' and q.  Per pixel t of its lanes' fours a
+// wave passes h' and q through its own LDS rows (BF16, as the next product's
+// operand).  Products, sums and roundings as the three k_pointwise passes: the
+// same results.  Bound: VALU (64 GELUs a pixel).  50 images of 256^2, 32 and 64
+// channels: 248 us, where the three passes took 194 + 276 + 207 us and wrote and
+// read 1.3 GB between them.
+struct TailArgs {
+    PointArgs b;     // the block's map (act 0, no pre; out unused)
+    const float *Q1, *q1b, *Q2, *q2b;
+    int H, cout;
+    float* y;        // [cout][nrows][rowlen]
+};
+template <int RT, int RH, int KU>
+__global__ void __launch_bounds__(256) k_tail(TailArgs g) {
+    constexpr int KT = (RT + 1) / 2, KH = (RH + 1) / 2, PS = 64 + 8;
+    extern __shared__ __attribute__((aligned(16))) __bf16 Fs[];
+    __shared__ __attribute__((aligned(16))) __bf16 X[4][16][PS];  // [wave][pixel][channel]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lm = lane & 15, lk = (lane >> 4) * 8, lr = (lane >> 4) * 4;
+    const int C = g.b.Cout;
+    const long SP = g.b.nrows * g.b.rowlen;
+    const int ngrp = (g.b.rowlen + 63) / 64;
+    stage_xtable<KU>(Fs, g.b.F, g.b.sfk, g.b.sfx, g.b.K2, g.b.rowlen);
+    for (int e = threadIdx.x; e < 4 * 16 * PS; e += 256) (&X[0][0][0])[e] = (__bf16)0.f;  // channels past the last stay 0
+    __syncthreads();
+    bf16x8 wa[RT][KT], q1[RH][KT], q2[1][KH];
+    matrix_operands<RT, KT>(wa, g.b.W, g.b.swm, g.b.swk, C, g.b.Cin, lm, lk);
+    matrix_operands<RH, KT>(q1, g.Q1, C, 1, g.H, C, lm, lk);
+    matrix_operands<1, KH>(q2, g.Q2, g.H, 1, g.cout, g.H, lm, lk);
+    float b0[RT][4], b1[RH][4], b2[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) b0[rt][q] = g.b.bias[min(rt * 16 + lr + q, C - 1)];
+#pragma unroll
+        for (int rt = 0; rt < RH; rt++) b1[rt][q] = g.q1b[min(rt * 16 + lr + q, g.H - 1)];
+        b2[q] = g.q2b[min(lr + q, g.cout - 1)];
+    }
+    // the D layout's 4 channels of one pixel into the wave's rows, and back as
+    // an operand of the next product.  Channels past n stay zero.
+    auto put = [&](int c, int n, const float (&v)[4]) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (c + q < n) X[wave][lm][c + q] = (__bf16)v[q];
+    };
+    auto put4 = [&](int c, const float (&v)[4]) {
+        const bf16x4 t = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+        *reinterpret_cast<bf16x4*>(&X[wave][lm][c]) = t;
+    };
+    auto wave_fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    const long units = g.b.nrows * ngrp;
+    for (long u = (long)blockIdx.x * 4 + wave; u < units; u += (long)gridDim.x * 4) {
+        const long r = u / ngrp;
+        const int x0 = (int)(u - r * ngrp) * 64;
+        bf16x8 ua[RT][KU];
+        spectrum_operands<RT, KU>(ua, g.b.U, g.b.nrows, r, C, g.b.K2, lm, lk);
+        const bool in = x0 + 4 * lm < g.b.rowlen;
+        const long p = r * g.b.rowlen + min(x0 + 4 * lm, g.b.rowlen - 4);
+        float4 hv[KT][8];
+        load_channels<KT>(hv, g.b.h, SP, p, g.b.Cin, lk);
+        float yv[4][4];  // [t][row]
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            bf16x8 hb[KT];
+            pixel_operands<KT>(hb, hv, t, g.b.Cin, lk);
+            wave_fence();
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f}, sp = acc;
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[rt][kt], hb[kt], acc, 0, 0, 0);
+#pragma unroll
+                for (int ku = 0; ku < KU; ku++)
+                    sp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        ua[rt][ku],
+                        *reinterpret_cast<const bf16x8*>(Fs + ((size_t)((ku * ngrp + (x0 >> 6)) * 4 + t) * 64 + lane) * 8),
+                        sp, 0, 0, 0);
+                acc += sp;
+                const float v[4] = {acc[0] + b0[rt][0], acc[1] + b0[rt][1], acc[2] + b0[rt][2], acc[3] + b0[rt][3]};
+                if (C == RT * 16) put4(rt * 16 + lr, v);
+                else put(rt * 16 + lr, C, v);
+            }
+            // channels C .. 32 KT - 1 hold q's of the pixel before: their products must be zero
+            if (C < KT * 32)
+                for (int c = C + (lane >> 4); c < KT * 32; c += 4) X[wave][lm][c] = (__bf16)0.f;
+            wave_fence();
+            bf16x8 xb[KT];
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) xb[kt] = *reinterpret_cast<const bf16x8*>(&X[wave][lm][kt * 32 + lk]);
+            wave_fence();
+#pragma unroll
+            for (int rt = 0; rt < RH; rt++) {
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q1[rt][kt], xb[kt], acc, 0, 0, 0);
+                float v[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[q] = gelu_t(acc[q] + b1[rt][q], nullptr);
+                if (g.H == RH * 16) put4(rt * 16 + lr, v);
+                else put(rt * 16 + lr, g.H, v);
+            }
+            if (g.H < KH * 32)
+                for (int c = g.H + (lane >> 4); c < KH * 32; c += 4) X[wave][lm][c] = (__bf16)0.f;
+            wave_fence();
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kt = 0; kt < KH; kt++)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    q2[0][kt], *reinterpret_cast<const bf16x8*>(&X[wave][lm][kt * 32 + lk]), acc, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; q++) yv[t][q] = acc[q] + b2[q];
+        }
+        if (!in) continue;
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (lr + q < g.cout)
+                *reinterpret_cast<float4*>(g.y + (lr + q) * SP + p) =
+                    make_float4(yv[0][q], yv[1][q], yv[2][q], yv[3][q]);
+    }
+}
+
+template <int RT, int RH, int KU>
+static hipError_t tail_launch(const TailArgs& g, hipStream_t st) {
+    const long wg = (g.b.nrows * ((g.b.rowlen + 63) / 64) + 3) / 4;
+    const size_t lds = (size_t)KU * ((g.b.rowlen + 63) / 64) * 256 * 8 * sizeof(__bf16);
+    if (lds + sizeof(__bf16) * 4 * 16 * 72 > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void*)k_tail<RT, RH, KU>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    k_tail<RT, RH, KU><<<(unsigned)(wg < 1024 ? wg : 1024), 256, lds, st>>>(g);
+    return hipGetLastError();
+}
+template <int RT>
+static hipError_t tail_rt(const TailArgs& g, hipStream_t st) {
+    if (g.b.K2 <= 32) return g.H <= 32 ? tail_launch<RT, 2, 1>(g, st) : tail_launch<RT, 4, 1>(g, st);
+    return g.H <= 32 ? tail_launch<RT, 2, 2>(g, st) : tail_launch<RT, 4, 2>(g, st);
+}
+hipError_t launch_tail(const float* W, int C, const float* h, long nrows, int rowlen, const float* U, int K2,
+                       const float* F, long sfk, long sfx, const float* bias, const float* Q1, const float* q1b, int H,
+                       const float* Q2, const float* q2b, int cout, float* y, hipStream_t st) {
+    TailArgs g{};
+    g.b = PointArgs{W, C, 1, C, C, h, nullptr, nrows, rowlen, U, K2, F, sfk, sfx, bias, nullptr, 0};
+    g.Q1 = Q1;
+    g.q1b = q1b;
+    g.Q2 = Q2;
+    g.q2b = q2b;
+    g.H = H;
+    g.cout = cout;
+    g.y = y;
+    switch ((C + 15) / 16) {
+        case 1: return tail_rt<1>(g, st);
+        case 2: return tail_rt<2>(g, st);
+        case 3: return tail_rt<3>(g, st);
+        default: return tail_rt<4>(g, st);
+    }
 }
 
 // Channel maps of at most 64 in and out channels over rows of a multiple of 4

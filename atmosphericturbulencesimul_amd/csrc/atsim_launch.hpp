@@ -140,6 +140,11 @@ bool pointwise_supported(const float* h, const float* out, const float* pre, con
 hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Cin, const float* h, float* out,
                             long nrows, int rowlen, const float* U, int K2, const float* F, long sfk, long sfx,
                             const float* bias, float* pre, int act, hipStream_t st);
+// the last block's map and the two projection maps in one pass; see k_tail
+// (pointwise_supported sizes for both maps, cout <= 16)
+hipError_t launch_tail(const float* W, int C, const float* h, long nrows, int rowlen, const float* U, int K2,
+                       const float* F, long sfk, long sfx, const float* bias, const float* Q1, const float* q1b, int H,
+                       const float* Q2, const float* q2b, int cout, float* y, hipStream_t st);
 // the spectral path: see k_dft2, k_idft_y, k_mix, k_mix_grad (spectral_supported
 // sizes only)
 bool spectral_supported(const float* h, const float* U, const float* B, const float* O, const float* R, long images,

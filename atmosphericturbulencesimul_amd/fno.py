@@ -97,6 +97,16 @@ class Ops:
         self.ctx._chk(self.L.atsim_nn_pointwise(self.ctx.h, _p(W), swm, swk, Cout, Cin, _p(h), _p(out), nrows, rowlen,
                                                 _p(U), K2, _p(F), sfk, sfx, _p(bias), _p(pre), act))
 
+    def tail(self, W, C_, h, nrows, rowlen, U, K2, F, sfk, sfx, bias, Q1, q1b, H, Q2, q2b, cout, y):
+        """y = Q2 GELU(Q1 (W h + U F + bias) + q1b) + q2b (row-major matrices)"""
+        n = nrows * rowlen
+        if (h.numel() < C_ * n or y.numel() < cout * n or W.numel() < C_ * C_ or U.numel() < C_ * nrows * K2
+                or F.numel() <= (K2 - 1) * sfk + (rowlen - 1) * sfx or bias.numel() < C_ or Q1.numel() < H * C_
+                or q1b.numel() < H or Q2.numel() < cout * H or q2b.numel() < cout):
+            raise ValueError(f"tail operands out of bounds ({C_}, {H}, {cout} channels, {nrows} rows of {rowlen})")
+        self.ctx._chk(self.L.atsim_nn_tail(self.ctx.h, _p(W), C_, _p(h), nrows, rowlen, _p(U), K2, _p(F), sfk, sfx,
+                                           _p(bias), _p(Q1), _p(q1b), H, _p(Q2), _p(q2b), cout, _p(y)))
+
     @staticmethod
     def spectral_ok(C_, N, m, h, R):
         """the sizes and alignments atsim_nn_spectral_fwd takes; the others go
@@ -392,8 +402,15 @@ class FNO:
         for b in range(self.blocks):
             # hn = act(W h + K h + B): the 1x1 map adds the spectral path's
             # inverse x transform, its bias and activation in one pass
-            hn = torch.empty_like(h)
             U, B = self._spectral(h, p[f"R{b}"], S)
+            if not keep and b == self.blocks - 1 and self.cout <= 16 and self.hidden <= 64 \
+                    and ops.pointwise_ok(Cw, Cw, N, (h, U), 2 * self.m):
+                # nothing is kept: the last map and both projections in one pass
+                y = torch.empty((self.cout, S, N, N), dtype=torch.float32, device=self.dev)
+                ops.tail(p[f"W{b}"], Cw, h, S * N, N, U, 2 * self.m, self.Fxi, N, 1, p[f"B{b}"], p["Q1"], p["q1b"],
+                         self.hidden, p["Q2"], p["q2b"], self.cout, y)
+                return y
+            hn = torch.empty_like(h)
             pre = torch.empty_like(h) if keep else None
             self._map_add(p[f"W{b}"], Cw, 1, h, U, self.Fxi, N, 1, hn, SP, bias=p[f"B{b}"], pre=pre,
                           act=int(b < self.blocks - 1))

@@ -394,6 +394,14 @@ int atsim_gemm_bf16_ex(atsim_ctx *ctx, long M, long N, long K, long batch, float
 int atsim_nn_pointwise(atsim_ctx *ctx, const float *W, long swm, long swk, long Cout, long Cin, const float *h,
                        float *out, long nrows, long rowlen, const float *U, long K2, const float *F, long sfk,
                        long sfx, const float *bias, float *pre, int act);
+/* The network after its last spectral path, in one pass: h' = W h + U F + bias
+ * (C x C, as atsim_nn_pointwise with act 0), q = GELU(Q1 h' + q1b) (H x C),
+ * y = Q2 q + q2b (cout x H), matrices row-major.  Sizes and alignments as
+ * atsim_nn_pointwise for each map, cout <= 16 (ATSIM_EUNSUPPORTED otherwise);
+ * y must not overlap h. */
+int atsim_nn_tail(atsim_ctx *ctx, const float *W, long C, const float *h, long nrows, long rowlen, const float *U,
+                  long K2, const float *F, long sfk, long sfx, const float *bias, const float *Q1, const float *q1b,
+                  long H, const float *Q2, const float *q2b, long cout, float *y);
 /* The spectral path of one block up to its inverse x transform, on images h
  * [C][S][N][N]: B = G (h F) the retained spectrum ([C][S][2m][m] complex; F[x
  * sfk + c sfn] the table along x with 2m columns, re and im of m modes; G =

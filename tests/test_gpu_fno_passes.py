@@ -83,8 +83,9 @@ def test_network_matches_the_general_path(ctx, monkeypatch, N, m, width, S, hidd
     def step():
         net = fno.FNO(ctx, N, cin, 2, width=width, modes=m, blocks=2, hidden=hidden, seed=3)
         loss = net.loss_and_grads(x, t)
+        y = net.forward(x, keep=False)
         ctx.sync()
-        return loss, {k: v.cpu().numpy() for k, v in net.grad.items()}
+        return loss, {**{k: v.cpu().numpy() for k, v in net.grad.items()}, "y": y.cpu().numpy()}
 
     used = []
     spectral = fno.Ops.spectral

@@ -27,6 +27,14 @@ struct atsim_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     std::map<long, float2*> twiddles;
+    // Bluestein plans of (length, sign): chirp [L], then filter spectrum [M];
+    // at most MAX_LINE_PLANS, the least recently used given back
+    struct LineTables {
+        float2* d = nullptr;
+        unsigned long used = 0;
+    };
+    std::map<std::pair<long, int>, LineTables> line_plans;
+    unsigned long line_use = 0;
     // launch-shape tuning (0 = built-in default)
     int row_mw = 0;  // wavelengths per row-pass workgroup
     int col_c = 0;   // columns per column-pass workgroup
@@ -148,11 +156,16 @@ static void host_fft(std::vector<double>& re, std::vector<double>& im, int sign)
             std::swap(im[i], im[j]);
         }
     }
+    std::vector<double> c(n / 2), s(n / 2);  // e^{sign 2 pi i k / n}
+    for (size_t k = 0; k < n / 2; k++) {
+        const double a = sign * 2.0 * M_PI * (double)k / (double)n;
+        c[k] = cos(a);
+        s[k] = sin(a);
+    }
     for (size_t len = 2; len <= n; len <<= 1) {
         for (size_t i = 0; i < n; i += len)
             for (size_t k = 0; k < len / 2; k++) {
-                const double a = sign * 2.0 * M_PI * (double)k / (double)len;
-                const double wr = cos(a), wi = sin(a);
+                const double wr = c[k * (n / len)], wi = s[k * (n / len)];
                 const size_t p = i + k, q = i + k + len / 2;
                 const double xr = re[q] * wr - im[q] * wi, xi = re[q] * wi + im[q] * wr;
                 re[q] = re[p] - xr;
@@ -161,19 +174,6 @@ static void host_fft(std::vector<double>& re, std::vector<double>& im, int sign)
                 im[p] += xi;
             }
     }
-}
-
-// gather map of the reference's permut (fft.c:570-792) on an n0 x n1 image:
-// after the swap loops, element p holds what was at sigma[p]
-static std::vector<int> permut_sigma(long n0, long n1) {
-    std::vector<int> idx((size_t)(n0 * n1));
-    for (long k = 0; k < n0 * n1; k++) idx[(size_t)k] = (int)k;
-    const long xh = n0 / 2, yh = n1 / 2;
-    for (long jj = 0; jj < yh; jj++)
-        for (long ii = 0; ii < xh; ii++) std::swap(idx[(size_t)(jj * n0 + ii)], idx[(size_t)((jj + yh) * n0 + ii + xh)]);
-    for (long jj = yh; jj < n1; jj++)
-        for (long ii = 0; ii < xh; ii++) std::swap(idx[(size_t)(jj * n0 + ii)], idx[(size_t)((jj - yh) * n0 + ii + xh)]);
-    return idx;
 }
 
 static long next_pow2(long n) {
@@ -235,6 +235,7 @@ void atsim_ctx_destroy(atsim_ctx* c) {
     hipSetDevice(c->device);
     hipStreamSynchronize(c->stream);
     for (auto& kv : c->twiddles) hipFree(kv.second);
+    for (auto& kv : c->line_plans) hipFree(kv.second.d);
     if (c->mg_fork) hipEventDestroy(c->mg_fork);
     if (c->nn_part) hipFree(c->nn_part);
     if (c->nn_bias) hipFree(c->nn_bias);
@@ -466,96 +467,79 @@ int atsim_permut(atsim_ctx* c, void* d_data, long n0, long n1, long nbatch) {
         HIPCHK(c, launch_permut((float2*)d_data, n0, n1, nbatch, c->stream));
         return ATSIM_OK;
     }
-    // odd sizes: the swap loops are no longer a half-size shift; their
-    // gather map is built on the host and applied on the device
+    // odd sizes: the swap loops are no longer a half-size shift but a gather
     if (n0 * n1 > (1L << 30)) return fail(c, ATSIM_EUNSUPPORTED, "permut: image too large");
-    const std::vector<int> sig = permut_sigma(n0, n1);
-    int* d_sig = nullptr;
     float2* tmp = nullptr;
     const size_t bytes = sizeof(float2) * n0 * n1 * nbatch;
-    HIPCHK(c, hipMallocAsync((void**)&d_sig, sizeof(int) * sig.size(), c->stream));
+    if (hipMallocAsync((void**)&tmp, bytes, c->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(c, ATSIM_ENOMEM, "permut: no memory");
+    }
     int r = ATSIM_OK;
-    if (hipMallocAsync((void**)&tmp, bytes, c->stream) != hipSuccess) r = fail(c, ATSIM_ENOMEM, "permut: no memory");
-    if (r == ATSIM_OK && (hipMemcpyAsync(d_sig, sig.data(), sizeof(int) * sig.size(), hipMemcpyHostToDevice, c->stream) !=
-                              hipSuccess ||
-                          hipMemcpyAsync(tmp, d_data, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
-                          launch_index_gather(tmp, (float2*)d_data, d_sig, n0 * n1, nbatch, c->stream) != hipSuccess))
+    if (hipMemcpyAsync(tmp, d_data, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
+        launch_permut_any(tmp, (float2*)d_data, n0, n1, nbatch, c->stream) != hipSuccess)
         r = fail(c, ATSIM_EHIP, "permut: device gather failed");
-    if (tmp) hipFreeAsync(tmp, c->stream);
-    hipFreeAsync(d_sig, c->stream);
-    HIPCHK(c, hipStreamSynchronize(c->stream));  // the host map must outlive its copy
+    hipFreeAsync(tmp, c->stream);
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     return r;
 }
 
-// One 1D transform of length L (unnormalised, sign) over nlines lines of a
-// batch of images (line base (l / per_img) img_size + (l % per_img) lstep,
-// elements estride apart), in place.  Power-of-two L: gather into padded
-// rows, row FFT, scatter.  Other L: Bluestein -- with c_n = e^{s i pi n^2 / L}
-// and d_m = e^{-s i pi m^2 / L}, X_k = c_k sum_n (x_n c_n) d_{k-n}, the
-// convolution taken by FFTs of length M >= 2L - 1 (filter spectrum built on
-// the host in FP64, 1/M folded in).  Chirp angles use n^2 mod 2L (exact).
-static int axis_transform(atsim_ctx* c, float2* data, long L, long nlines, long per_img, long img_size, long lstep,
-                          long estride, int sign) {
-    if (L == 1) return ATSIM_OK;
+// The plan of one axis: a power-of-two length >= 16 directly, any other by
+// Bluestein through transforms of length M >= 2 L - 1 (>= 16, the shortest the
+// device has), with c_n = e^{s i pi n^2 / L} and the spectrum of d_m = conj c_m
+// over M (in FP64 on the host, 1 / M folded in).  Chirp angles use n^2 mod 2L
+// (exact).  The tables of a length depend on nothing else, and stay with the
+// context as its twiddles do.
+static constexpr size_t MAX_LINE_PLANS = 64;  // at most 96 KB each
+static int line_plan(atsim_ctx* c, long L, long nlines, int sign, LinePlan* out) {
     const bool p2 = pow2(L);
-    const long M = p2 ? L : next_pow2(2 * L - 1);
-    // the device row transforms start at 16: shorter lines take the padded
-    // (Bluestein) path at length 16 >= 2 L - 1
-    const long Mf = std::max<long>(M, 16);
-    if (Mf > 8192)
-        return fail(c, ATSIM_EUNSUPPORTED, "fft: axis length %ld needs a transform of %ld > 8192", L, Mf);
-    const bool blue = !p2 || M < 16;
-    const long F = (nlines + Mf - 1) / Mf;
-    if (F > 65535) return fail(c, ATSIM_EUNSUPPORTED, "fft: %ld lines of length %ld are too many", nlines, L);
+    const long M = std::max<long>(p2 ? L : next_pow2(2 * L - 1), 16);
+    if (M > 8192) return fail(c, ATSIM_EUNSUPPORTED, "fft: axis length %ld needs a transform of %ld > 8192", L, M);
+    if ((nlines + M - 1) / M > 65535)
+        return fail(c, ATSIM_EUNSUPPORTED, "fft: %ld lines of length %ld are too many", nlines, L);
     float2* tw = nullptr;
-    if (int r = get_twiddles(c, Mf, &tw)) return r;
-    float2 *scr = nullptr, *d_c = nullptr, *d_h = nullptr;
-    HIPCHK(c, hipMallocAsync((void**)&scr, sizeof(float2) * F * Mf * Mf, c->stream));
-    std::vector<float2> hc, hh;
-    int r = ATSIM_OK;
-    if (blue) {
-        hc.resize((size_t)L);
-        std::vector<double> dr((size_t)Mf, 0.0), di((size_t)Mf, 0.0);
+    if (int r = get_twiddles(c, M, &tw)) return r;
+    *out = LinePlan{(int)L, (int)M, nullptr, nullptr, tw};
+    if (p2 && L >= 16) return ATSIM_OK;
+    const auto key = std::make_pair(L, sign);
+    auto it = c->line_plans.find(key);
+    if (it == c->line_plans.end()) {
+        if (c->line_plans.size() >= MAX_LINE_PLANS) {
+            auto old = c->line_plans.begin();
+            for (auto k = c->line_plans.begin(); k != c->line_plans.end(); ++k)
+                if (k->second.used < old->second.used) old = k;
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            hipFree(old->second.d);
+            c->line_plans.erase(old);
+        }
+        std::vector<float2> h((size_t)(L + M));
+        std::vector<double> dr((size_t)M, 0.0), di((size_t)M, 0.0);
         for (long n = 0; n < L; n++) {
             const long q = (long)(((unsigned long long)n * (unsigned long long)n) % (unsigned long long)(2 * L));
             const double a = M_PI * (double)q / (double)L;
-            hc[(size_t)n] = make_float2((float)cos(a), (float)(sign * sin(a)));
+            h[(size_t)n] = make_float2((float)cos(a), (float)(sign * sin(a)));
             dr[(size_t)n] = cos(a);
             di[(size_t)n] = -sign * sin(a);
             if (n > 0) {
-                dr[(size_t)(Mf - n)] = cos(a);
-                di[(size_t)(Mf - n)] = -sign * sin(a);
+                dr[(size_t)(M - n)] = dr[(size_t)n];
+                di[(size_t)(M - n)] = di[(size_t)n];
             }
         }
         host_fft(dr, di, -1);
-        hh.resize((size_t)Mf);
-        for (long k = 0; k < Mf; k++) hh[(size_t)k] = make_float2((float)(dr[(size_t)k] / Mf), (float)(di[(size_t)k] / Mf));
-        if (hipMallocAsync((void**)&d_c, sizeof(float2) * L, c->stream) != hipSuccess ||
-            hipMallocAsync((void**)&d_h, sizeof(float2) * Mf, c->stream) != hipSuccess ||
-            hipMemcpyAsync(d_c, hc.data(), sizeof(float2) * L, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-            hipMemcpyAsync(d_h, hh.data(), sizeof(float2) * Mf, hipMemcpyHostToDevice, c->stream) != hipSuccess)
-            r = fail(c, ATSIM_EHIP, "fft: table upload failed");
-    }
-    ScreenArgs none{};
-    auto ok = [](hipError_t e) { return e == hipSuccess; };
-    if (r == ATSIM_OK) {
-        bool good = ok(launch_line_gather(data, scr, nlines, L, Mf, per_img, img_size, lstep, estride, d_c, c->stream));
-        if (blue) {
-            good = good && ok(launch_row(Mf, OP_FFT, -1, false, scr, F, nullptr, tw, none, c->stream)) &&
-                   ok(launch_row_mul(scr, d_h, F * Mf, Mf, c->stream)) &&
-                   ok(launch_row(Mf, OP_FFT, +1, false, scr, F, nullptr, tw, none, c->stream));
-        } else {
-            good = good && ok(launch_row(Mf, OP_FFT, sign, false, scr, F, nullptr, tw, none, c->stream));
+        for (long k = 0; k < M; k++)
+            h[(size_t)(L + k)] = make_float2((float)(dr[(size_t)k] / M), (float)(di[(size_t)k] / M));
+        float2* d = nullptr;
+        HIPCHK(c, hipMalloc(&d, sizeof(float2) * h.size()));
+        if (hipError_t e = copy_on_stream(c, d, h.data(), sizeof(float2) * h.size())) {
+            hipFree(d);
+            return fail(c, ATSIM_EHIP, "fft: table upload: %s", hipGetErrorString(e));
         }
-        good = good && ok(launch_line_scatter(scr, data, nlines, L, Mf, per_img, img_size, lstep, estride, d_c,
-                                              c->stream));
-        if (!good) r = fail(c, ATSIM_EHIP, "fft: launch failed for length %ld", L);
+        it = c->line_plans.emplace(key, atsim_ctx::LineTables{d, 0}).first;
     }
-    hipFreeAsync(scr, c->stream);
-    if (d_c) hipFreeAsync(d_c, c->stream);
-    if (d_h) hipFreeAsync(d_h, c->stream);
-    HIPCHK(c, hipStreamSynchronize(c->stream));  // host tables must outlive their copies
-    return r;
+    it->second.used = ++c->line_use;
+    out->chirp = it->second.d;
+    out->filt = it->second.d + L;
+    return ATSIM_OK;
 }
 
 int atsim_fft2d_nm(atsim_ctx* c, void* d_data, long n0, long n1, long nbatch, int sign) {
@@ -565,10 +549,18 @@ int atsim_fft2d_nm(atsim_ctx* c, void* d_data, long n0, long n1, long nbatch, in
     if (sign != -1 && sign != 1) return fail(c, ATSIM_EINVAL, "fft2d_nm: sign must be -1 or +1");
     if (n0 == n1 && supported_n(n0) && nbatch <= 65535) return atsim_fft2d(c, d_data, n0, nbatch, sign);
     float2* d = (float2*)d_data;
-    // along x: lines are the rows, n1 per image
-    if (int r = axis_transform(c, d, n0, n1 * nbatch, n1, n0 * n1, n0, 1, sign)) return r;
-    // along y: lines are the columns, n0 per image
-    return axis_transform(c, d, n1, n0 * nbatch, n0, n0 * n1, 1, n0, sign);
+    // along x, then along y (a length of 1 is its own transform)
+    LinePlan p;
+    if (n0 > 1) {
+        if (int r = line_plan(c, n0, n1 * nbatch, sign, &p)) return r;
+        HIPCHK(c, launch_any_row(p, sign, d, d, n1 * nbatch, c->stream));
+    }
+    if (n1 > 1) {
+        if (int r = line_plan(c, n1, n0 * nbatch, sign, &p)) return r;
+        HIPCHK(c, launch_any_col(p, nullptr, sign, d, n0, nbatch, nullptr, nullptr, c->stream));
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return ATSIM_OK;
 }
 
 // ------------------------------------------------------------------ Fresnel
@@ -609,30 +601,42 @@ int atsim_fresnel_nm(atsim_ctx* c, const void* d_in, void* d_out, long n0, long 
     if (n0 <= 0 || n1 <= 0 || nbatch <= 0) return fail(c, ATSIM_EINVAL, "fresnel_nm: sizes must be > 0");
     if (!(dx > 0.0)) return fail(c, ATSIM_EINVAL, "fresnel_nm: pupil scale must be > 0");
     if (n0 == n1 && supported_n(n0) && nbatch <= 65535) return atsim_fresnel(c, d_in, d_out, n0, nbatch, dx, z, lambda);
-    const size_t bytes = sizeof(float2) * n0 * n1 * nbatch;
-    float2* tmp = nullptr;
-    int* d_sig = nullptr;
-    std::vector<int> sig;
-    HIPCHK(c, hipMallocAsync((void**)&tmp, bytes, c->stream));
-    int r = ATSIM_OK;
-    if (hipMemcpyAsync(tmp, d_in, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
-        r = fail(c, ATSIM_EHIP, "fresnel_nm: copy failed");
-    if (r == ATSIM_OK) r = atsim_fft2d_nm(c, tmp, n0, n1, nbatch, -1);
-    if (r == ATSIM_OK && ((n0 & 1) || (n1 & 1))) {
-        sig = permut_sigma(n0, n1);
-        if (hipMallocAsync((void**)&d_sig, sizeof(int) * sig.size(), c->stream) != hipSuccess ||
-            hipMemcpyAsync(d_sig, sig.data(), sizeof(int) * sig.size(), hipMemcpyHostToDevice, c->stream) != hipSuccess)
-            r = fail(c, ATSIM_EHIP, "fresnel_nm: permut map upload failed");
-    }
     // WFpropagate.c:97: the coefficient uses naxes[0] for both axes
     const double coeff = M_PI * z * lambda / (dx * n0) / (dx * n0);
-    if (r == ATSIM_OK && launch_fresnel_any(tmp, (float2*)d_out, n0, n1, nbatch, coeff, d_sig, c->stream) != hipSuccess)
-        r = fail(c, ATSIM_EHIP, "fresnel_nm: launch failed");
-    if (r == ATSIM_OK) r = atsim_fft2d_nm(c, d_out, n0, n1, nbatch, +1);
-    hipFreeAsync(tmp, c->stream);
-    if (d_sig) hipFreeAsync(d_sig, c->stream);
+    float2* out = (float2*)d_out;
+    if ((n0 & 1) || (n1 & 1)) {
+        // odd sides: the reference's permut pair is no shift, so the factor is a
+        // pass of its own between the transforms
+        float2* tmp = nullptr;
+        const size_t bytes = sizeof(float2) * n0 * n1 * nbatch;
+        HIPCHK(c, hipMallocAsync((void**)&tmp, bytes, c->stream));
+        int r = ATSIM_OK;
+        if (hipMemcpyAsync(tmp, d_in, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+            r = fail(c, ATSIM_EHIP, "fresnel_nm: copy failed");
+        if (r == ATSIM_OK) r = atsim_fft2d_nm(c, tmp, n0, n1, nbatch, -1);
+        if (r == ATSIM_OK && launch_fresnel_odd(tmp, out, n0, n1, nbatch, coeff, c->stream) != hipSuccess)
+            r = fail(c, ATSIM_EHIP, "fresnel_nm: launch failed");
+        if (r == ATSIM_OK) r = atsim_fft2d_nm(c, out, n0, n1, nbatch, +1);
+        hipFreeAsync(tmp, c->stream);
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return r;
+    }
+    // even sides: rows, then columns with the factor and back, then rows back
+    LinePlan xf, xb, yf, yb;
+    if (int r = line_plan(c, n0, n1 * nbatch, -1, &xf)) return r;
+    if (int r = line_plan(c, n0, n1 * nbatch, +1, &xb)) return r;
+    if (int r = line_plan(c, n1, n0 * nbatch, -1, &yf)) return r;
+    if (int r = line_plan(c, n1, n0 * nbatch, +1, &yb)) return r;
+    double2* h = nullptr;
+    HIPCHK(c, hipMallocAsync((void**)&h, sizeof(double2) * (n0 + n1), c->stream));
+    hipError_t e = launch_any_factor(h, h + n0, n0, n1, coeff, c->stream);
+    if (e == hipSuccess) e = launch_any_row(xf, -1, (const float2*)d_in, out, n1 * nbatch, c->stream);
+    if (e == hipSuccess) e = launch_any_col(yf, &yb, 0, out, n0, nbatch, h, h + n0, c->stream);
+    if (e == hipSuccess) e = launch_any_row(xb, +1, out, out, n1 * nbatch, c->stream);
+    hipFreeAsync(h, c->stream);
+    if (e != hipSuccess) return fail(c, ATSIM_EHIP, "fresnel_nm: %s", hipGetErrorString(e));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    return r;
+    return ATSIM_OK;
 }
 
 int atsim_fresnel_noalloc(atsim_ctx* c, const void* d_in, void* d_out, long n, long nbatch, double dx, double z,

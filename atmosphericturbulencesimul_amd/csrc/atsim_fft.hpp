@@ -33,6 +33,14 @@ __device__ __forceinline__ float2 mul_qi(float2 a) {
     return DIR < 0 ? make_float2(a.y, -a.x) : make_float2(-a.y, a.x);
 }
 
+// the value of x, opaque to the optimiser: index arithmetic derived from it
+// is recomputed instead of kept live from an earlier use of x (an empty asm
+// statement with no instructions)
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 // cos / sin of pi*m/8, m = 0..9
 __device__ __forceinline__ float2 w16(int m, int dir) {
     constexpr float C1 = 0.92387953251128674f, S1 = 0.38268343236508978f, H = 0.70710678118654752f;

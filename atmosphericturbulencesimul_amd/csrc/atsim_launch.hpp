@@ -55,20 +55,28 @@ bool fft_mfma_supported(long n);
 hipError_t launch_row_fft_mfma(float2* data, long nrows, int dir, const float2* tw, hipStream_t st);
 // out[b][x][y] = in[b][y][x], n a multiple of 32
 hipError_t launch_transpose(const float2* in, float2* out, long n, long nbatch, hipStream_t st);
-// transforms of any size: lines of length L (< = M) between strided images and
-// a padded scratch [nlines][M]; base of line l = (l / per_img) img_size +
-// (l % per_img) lstep, elements estride apart; chirp (nullable) multiplies
-hipError_t launch_line_gather(const float2* src, float2* dst, long nlines, long L, long M, long per_img, long img_size,
-                              long lstep, long estride, const float2* chirp, hipStream_t st);
-hipError_t launch_line_scatter(const float2* src, float2* dst, long nlines, long L, long M, long per_img,
-                               long img_size, long lstep, long estride, const float2* chirp, hipStream_t st);
-hipError_t launch_row_mul(float2* data, const float2* h, long nrows, long M, hipStream_t st);
-// out[b][p] = in[b][sigma[p]] (images of n elements)
-hipError_t launch_index_gather(const float2* in, float2* out, const int* sigma, long n, long nbatch, hipStream_t st);
-// Fresnel factor of any n0 x n1 spectrum with the reference's permut pair
-// (sigma: gather map of one permut, null for even sizes); out != in
-hipError_t launch_fresnel_any(const float2* in, float2* out, long n0, long n1, long nbatch, double coeff,
-                              const int* sigma, hipStream_t st);
+// transforms of any length along one axis (atsim_fft_any.hip): length L through
+// transforms of length M, with the chirp and filter of one sign (Bluestein), or
+// directly (chirp null, L = M)
+struct LinePlan {
+    int L, M;
+    const float2* chirp;  // [L]
+    const float2* filt;   // [M]
+    const float2* tw;     // twiddles of M, with the per-stage tables
+};
+// nrows contiguous rows; in may equal out
+hipError_t launch_any_row(const LinePlan& p, int sign, const float2* in, float2* out, long nrows, hipStream_t st);
+// the columns of nbatch n0-wide images of p.L rows, in place.  back (the plan
+// of sign +1): forward transform, times hx[column] hy[row], inverse transform.
+hipError_t launch_any_col(const LinePlan& p, const LinePlan* back, int sign, float2* data, long n0, long nbatch,
+                          const double2* hx, const double2* hy, hipStream_t st);
+// Fresnel factors of even sides: hx [n0], hy [n1] (with 1 / (n0 n1))
+hipError_t launch_any_factor(double2* hx, double2* hy, long n0, long n1, double coeff, hipStream_t st);
+// the Fresnel factor between the reference's permut pair, any sides; out != in
+hipError_t launch_fresnel_odd(const float2* in, float2* out, long n0, long n1, long nbatch, double coeff,
+                              hipStream_t st);
+// permut on any sides; out != in
+hipError_t launch_permut_any(const float2* in, float2* out, long n0, long n1, long nbatch, hipStream_t st);
 hipError_t launch_noise(float2* out, long n, uint64_t seed, uint32_t stream, hipStream_t st);
 hipError_t launch_synth_filter(const float2* noise, float2* out, long size, double f0, double fi,
                                double rlim, hipStream_t st);

@@ -65,6 +65,10 @@ struct atsim_ctx {
     // frames of several simulations in one call (atsim_sims_frame)
     long mg_frames = 0;
     hipEvent_t mg_fork = nullptr;
+    float2* fresnel_tab = nullptr;  // [8192] transfer factor of the running Fresnel step
+    // work space of calls on the context stream (ctx_scratch), kept between them
+    void* scratch = nullptr;
+    size_t scratch_cap = 0;
     double* nn_part = nullptr;  // 256 partial sums of the network's loss reduction
     float* nn_bias = nullptr;   // per-chunk partial sums of bias gradients
     size_t nn_bias_cap = 0;
@@ -95,6 +99,44 @@ static int fail(atsim_ctx* c, int code, const char* fmt, ...) {
         hipError_t e_ = (expr);                                                                   \
         if (e_ != hipSuccess) return fail((ctx), ATSIM_EHIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
+
+// Work space of one call, used on the context stream only (the next call's
+// kernels follow this one's): the context's own block, grown as needed and kept
+// up to SCRATCH_KEEP bytes (an 8192^2 master), so that a call does not wait for
+// an allocation; more than that is allocated for the call alone.
+static constexpr size_t SCRATCH_KEEP = (size_t)640 << 20;
+struct Scratch {
+    atsim_ctx* c;
+    void* p = nullptr;
+    bool own = false;
+    explicit Scratch(atsim_ctx* ctx) : c(ctx) {}
+    ~Scratch() {
+        if (own && p) (void)hipFreeAsync(p, c->stream);
+    }
+    hipError_t get(size_t bytes) {
+        if (bytes > SCRATCH_KEEP) {
+            own = true;
+            hipError_t e = hipMallocAsync(&p, bytes, c->stream);
+            if (e != hipSuccess) p = nullptr;
+            return e;
+        }
+        if (bytes > c->scratch_cap) {
+            hipError_t e = hipStreamSynchronize(c->stream);
+            if (e != hipSuccess) return e;
+            if (c->scratch) (void)hipFree(c->scratch);
+            c->scratch = nullptr;
+            c->scratch_cap = 0;
+            e = hipMalloc(&c->scratch, bytes);
+            if (e != hipSuccess) {
+                c->scratch = nullptr;
+                return e;
+            }
+            c->scratch_cap = bytes;
+        }
+        p = c->scratch;
+        return hipSuccess;
+    }
+};
 
 static bool pow2(long n) { return n > 0 && (n & (n - 1)) == 0; }
 
@@ -194,16 +236,29 @@ static __device__ __align__(256) float2 scratch[2 * ATSIM_NOALLOC_MAX_N];
 // first context on that device (the host-side name is only a stand-in)
 static float2* g_scratch[ATSIM_MAX_DEVICES];
 
-// tab[k] = h(k) as fresnel_table builds it, tw[m] = e^{-2 pi i m / n} as
-// get_twiddles builds it, both in FP64 and rounded to float
-__global__ void k_fresnel_tables(float2* __restrict__ tab, float2* __restrict__ tw, long n, double coeff) {
+// Tables of nz propagation distances z_j = zstart + (zend - zstart) j / nz (j =
+// blockIdx.y): tab[j n + k] = h(k) as fresnel_table builds it, with coeff(z) = co z,
+// and (tw not null) tw[m] = e^{-2 pi i m / n} as get_twiddles builds it, in FP64
+// and rounded to float
+__global__ void k_fresnel_tables(float2* __restrict__ tab, float2* __restrict__ tw, long n, double co, double zstart,
+                                 double zend, long j0, long nz) {
     const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const double kt = (double)(k < n / 2 ? k : k - n);
-    const double ang = -coeff * kt * kt;
-    tab[k] = make_float2((float)(cos(ang) / n), (float)(sin(ang) / n));
-    const double a = -2.0 * M_PI * (double)k / (double)n;
-    tw[k] = make_float2((float)cos(a), (float)sin(a));
+    const double ang = -(co * (zstart + (zend - zstart) * (double)(j0 + blockIdx.y) / (double)nz)) * kt * kt;
+    double sn, cs;
+    sincos(ang, &sn, &cs);
+    tab[(size_t)blockIdx.y * n + k] = make_float2((float)(cs / n), (float)(sn / n));
+    if (tw == nullptr || blockIdx.y > 0) return;
+    sincos(-2.0 * M_PI * (double)k / (double)n, &sn, &cs);
+    tw[k] = make_float2((float)cs, (float)sn);
+}
+static hipError_t launch_fresnel_tables(float2* tab, float2* tw, long n, double dx, double lambda, double zstart,
+                                        double zend, long j0, long cnt, long nz, hipStream_t st) {
+    const double co = M_PI * lambda / (dx * n) / (dx * n);
+    k_fresnel_tables<<<dim3((unsigned)((n + 255) / 256), (unsigned)cnt), 256, 0, st>>>(tab, tw, n, co, zstart, zend, j0,
+                                                                                      nz);
+    return hipGetLastError();
 }
 
 extern "C" {
@@ -237,6 +292,8 @@ void atsim_ctx_destroy(atsim_ctx* c) {
     for (auto& kv : c->twiddles) hipFree(kv.second);
     for (auto& kv : c->line_plans) hipFree(kv.second.d);
     if (c->mg_fork) hipEventDestroy(c->mg_fork);
+    if (c->fresnel_tab) hipFree(c->fresnel_tab);
+    if (c->scratch) hipFree(c->scratch);
     if (c->nn_part) hipFree(c->nn_part);
     if (c->nn_bias) hipFree(c->nn_bias);
     if (c->copy_stream) {
@@ -409,9 +466,9 @@ int atsim_fft2d(atsim_ctx* c, void* d_data, long n, long nbatch, int sign) {
     if (sign != -1 && sign != 1) return fail(c, ATSIM_EINVAL, "fft2d: sign must be -1 or +1");
     float2* tw;
     if (int r = get_twiddles(c, n, &tw)) return r;
-    ScreenArgs none{};
-    HIPCHK(c, launch_row(n, OP_FFT, sign, false, (float2*)d_data, nbatch, nullptr, tw, none, c->stream));
-    HIPCHK(c, launch_col(n, OP_FFT, sign, (float2*)d_data, nbatch, nullptr, 1, tw, c->stream));
+    float2* d = (float2*)d_data;
+    HIPCHK(c, launch_row(n, OP_FFT, sign, d, n * n, d, nbatch, nullptr, 1, tw, c->stream));
+    HIPCHK(c, launch_col(n, OP_FFT, sign, d, nbatch, nullptr, 1, tw, c->stream));
     return ATSIM_OK;
 }
 
@@ -449,8 +506,8 @@ int atsim_row_fft_variant(atsim_ctx* c, void* d_data, long n, long nrows, int si
     if (int r = get_twiddles(c, n, &tw)) return r;
     if (variant == 0) {
         if (!supported_n(n)) return fail(c, ATSIM_EUNSUPPORTED, "row_fft_variant: size %ld unsupported", n);
-        ScreenArgs none{};
-        HIPCHK(c, launch_row(n, OP_FFT, sign, false, (float2*)d_data, nrows / n, nullptr, tw, none, c->stream));
+        float2* d = (float2*)d_data;
+        HIPCHK(c, launch_row(n, OP_FFT, sign, d, n * n, d, nrows / n, nullptr, 1, tw, c->stream));
         return ATSIM_OK;
     }
     if (variant != 1 || !fft_mfma_supported(n))
@@ -469,17 +526,17 @@ int atsim_permut(atsim_ctx* c, void* d_data, long n0, long n1, long nbatch) {
     }
     // odd sizes: the swap loops are no longer a half-size shift but a gather
     if (n0 * n1 > (1L << 30)) return fail(c, ATSIM_EUNSUPPORTED, "permut: image too large");
-    float2* tmp = nullptr;
     const size_t bytes = sizeof(float2) * n0 * n1 * nbatch;
-    if (hipMallocAsync((void**)&tmp, bytes, c->stream) != hipSuccess) {
+    Scratch work(c);
+    if (work.get(bytes) != hipSuccess) {
         (void)hipGetLastError();
         return fail(c, ATSIM_ENOMEM, "permut: no memory");
     }
+    float2* tmp = (float2*)work.p;
     int r = ATSIM_OK;
     if (hipMemcpyAsync(tmp, d_data, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
         launch_permut_any(tmp, (float2*)d_data, n0, n1, nbatch, c->stream) != hipSuccess)
         r = fail(c, ATSIM_EHIP, "permut: device gather failed");
-    hipFreeAsync(tmp, c->stream);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return r;
 }
@@ -564,16 +621,6 @@ int atsim_fft2d_nm(atsim_ctx* c, void* d_data, long n0, long n1, long nbatch, in
 }
 
 // ------------------------------------------------------------------ Fresnel
-static int fresnel_run(atsim_ctx* c, float2* d, long n, long nbatch, const float2* d_tab) {
-    float2* tw;
-    if (int r = get_twiddles(c, n, &tw)) return r;
-    ScreenArgs none{};
-    none.W = 1;
-    HIPCHK(c, launch_row(n, OP_FRESNEL, 0, false, d, nbatch, d_tab, tw, none, c->stream));
-    HIPCHK(c, launch_col(n, OP_FRESNEL, 0, d, nbatch, d_tab, 1, tw, c->stream));
-    return ATSIM_OK;
-}
-
 int atsim_fresnel(atsim_ctx* c, const void* d_in, void* d_out, long n, long nbatch, double dx, double z,
                   double lambda) {
     if (!c || !d_in || !d_out) return ATSIM_EINVAL;
@@ -581,17 +628,17 @@ int atsim_fresnel(atsim_ctx* c, const void* d_in, void* d_out, long n, long nbat
     if (!supported_n(n)) return fail(c, ATSIM_EUNSUPPORTED, "fresnel: size %ld is not a power of two in [16, 8192]", n);
     if (nbatch <= 0 || nbatch > 65535) return fail(c, ATSIM_EINVAL, "fresnel: nbatch %ld out of range", nbatch);
     if (!(dx > 0.0)) return fail(c, ATSIM_EINVAL, "fresnel: pupil scale must be > 0");
-    std::vector<float2> h(n);
-    fresnel_table(h.data(), n, dx, z, lambda);
-    float2* d_tab = nullptr;
-    HIPCHK(c, hipMallocAsync((void**)&d_tab, sizeof(float2) * n, c->stream));
-    HIPCHK(c, hipMemcpyAsync(d_tab, h.data(), sizeof(float2) * n, hipMemcpyHostToDevice, c->stream));
-    if (d_in != d_out)
-        HIPCHK(c, hipMemcpyAsync(d_out, d_in, sizeof(float2) * n * n * nbatch, hipMemcpyDeviceToDevice, c->stream));
-    int r = fresnel_run(c, (float2*)d_out, n, nbatch, d_tab);
-    hipFreeAsync(d_tab, c->stream);
-    HIPCHK(c, hipStreamSynchronize(c->stream));  // host table must outlive the copy
-    return r;
+    float2* tw;
+    if (int r = get_twiddles(c, n, &tw)) return r;
+    // the transfer factor is made on the device, in the context's own table (one
+    // call's kernels follow the other's on the stream); the row pass reads d_in
+    if (!c->fresnel_tab) HIPCHK(c, hipMalloc(&c->fresnel_tab, sizeof(float2) * 8192));
+    HIPCHK(c, launch_fresnel_tables(c->fresnel_tab, nullptr, n, dx, lambda, z, z, 0, 1, 1, c->stream));
+    HIPCHK(c, launch_row(n, OP_FRESNEL, 0, (const float2*)d_in, n * n, (float2*)d_out, nbatch, c->fresnel_tab, 1, tw,
+                         c->stream));
+    HIPCHK(c, launch_col(n, OP_FRESNEL, 0, (float2*)d_out, nbatch, c->fresnel_tab, 1, tw, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return ATSIM_OK;
 }
 
 int atsim_fresnel_nm(atsim_ctx* c, const void* d_in, void* d_out, long n0, long n1, long nbatch, double dx,
@@ -607,9 +654,10 @@ int atsim_fresnel_nm(atsim_ctx* c, const void* d_in, void* d_out, long n0, long 
     if ((n0 & 1) || (n1 & 1)) {
         // odd sides: the reference's permut pair is no shift, so the factor is a
         // pass of its own between the transforms
-        float2* tmp = nullptr;
         const size_t bytes = sizeof(float2) * n0 * n1 * nbatch;
-        HIPCHK(c, hipMallocAsync((void**)&tmp, bytes, c->stream));
+        Scratch work(c);
+        HIPCHK(c, work.get(bytes));
+        float2* tmp = (float2*)work.p;
         int r = ATSIM_OK;
         if (hipMemcpyAsync(tmp, d_in, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
             r = fail(c, ATSIM_EHIP, "fresnel_nm: copy failed");
@@ -617,7 +665,6 @@ int atsim_fresnel_nm(atsim_ctx* c, const void* d_in, void* d_out, long n0, long 
         if (r == ATSIM_OK && launch_fresnel_odd(tmp, out, n0, n1, nbatch, coeff, c->stream) != hipSuccess)
             r = fail(c, ATSIM_EHIP, "fresnel_nm: launch failed");
         if (r == ATSIM_OK) r = atsim_fft2d_nm(c, out, n0, n1, nbatch, +1);
-        hipFreeAsync(tmp, c->stream);
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return r;
     }
@@ -627,13 +674,13 @@ int atsim_fresnel_nm(atsim_ctx* c, const void* d_in, void* d_out, long n0, long 
     if (int r = line_plan(c, n0, n1 * nbatch, +1, &xb)) return r;
     if (int r = line_plan(c, n1, n0 * nbatch, -1, &yf)) return r;
     if (int r = line_plan(c, n1, n0 * nbatch, +1, &yb)) return r;
-    double2* h = nullptr;
-    HIPCHK(c, hipMallocAsync((void**)&h, sizeof(double2) * (n0 + n1), c->stream));
+    Scratch work(c);
+    HIPCHK(c, work.get(sizeof(double2) * (n0 + n1)));
+    double2* h = (double2*)work.p;
     hipError_t e = launch_any_factor(h, h + n0, n0, n1, coeff, c->stream);
     if (e == hipSuccess) e = launch_any_row(xf, -1, (const float2*)d_in, out, n1 * nbatch, c->stream);
     if (e == hipSuccess) e = launch_any_col(yf, &yb, 0, out, n0, nbatch, h, h + n0, c->stream);
     if (e == hipSuccess) e = launch_any_row(xb, +1, out, out, n1 * nbatch, c->stream);
-    hipFreeAsync(h, c->stream);
     if (e != hipSuccess) return fail(c, ATSIM_EHIP, "fresnel_nm: %s", hipGetErrorString(e));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return ATSIM_OK;
@@ -654,14 +701,9 @@ int atsim_fresnel_noalloc(atsim_ctx* c, const void* d_in, void* d_out, long n, l
     float2* d_tab = base;
     float2* d_tw = base + ATSIM_NOALLOC_MAX_N;
     HIPCHK(c, hipSetDevice(c->device));
-    const double coeff = M_PI * z * lambda / (dx * n) / (dx * n);
-    k_fresnel_tables<<<(unsigned)((n + 255) / 256), 256, 0, c->stream>>>(d_tab, d_tw, n, coeff);
-    HIPCHK(c, hipGetLastError());
-    if (d_in != d_out)
-        HIPCHK(c, hipMemcpyAsync(d_out, d_in, sizeof(float2) * n * n * nbatch, hipMemcpyDeviceToDevice, c->stream));
-    ScreenArgs none{};
-    none.W = 1;
-    HIPCHK(c, launch_row(n, OP_FRESNEL, 0, false, (float2*)d_out, nbatch, d_tab, d_tw, none, c->stream));
+    HIPCHK(c, launch_fresnel_tables(d_tab, d_tw, n, dx, lambda, z, z, 0, 1, 1, c->stream));
+    HIPCHK(c, launch_row(n, OP_FRESNEL, 0, (const float2*)d_in, n * n, (float2*)d_out, nbatch, d_tab, 1, d_tw,
+                         c->stream));
     HIPCHK(c, launch_col(n, OP_FRESNEL, 0, (float2*)d_out, nbatch, d_tab, 1, d_tw, c->stream));
     return ATSIM_OK;
 }
@@ -692,20 +734,30 @@ int atsim_fresnel_cube(atsim_ctx* c, const void* d_in, float* d_amp, float* d_ph
     c->work_gen++;
     if (!supported_n(n)) return fail(c, ATSIM_EUNSUPPORTED, "fresnel_cube: size %ld unsupported", n);
     if (nz <= 0) return fail(c, ATSIM_EINVAL, "fresnel_cube: nz must be > 0");
-    float2* tmp = nullptr;
-    HIPCHK(c, hipMalloc(&tmp, sizeof(float2) * n * n));
-    int r = ATSIM_OK;
-    for (long k = 0; k < nz && r == ATSIM_OK; k++) {
-        const double zp = zstart + (zend - zstart) * k / nz;
-        r = atsim_fresnel(c, d_in, tmp, n, 1, dx, zp, lambda);
-        if (r == ATSIM_OK) {
-            hipError_t e = launch_amp_pha(tmp, d_amp + k * n * n, d_pha + k * n * n, n * n, c->stream);
-            if (e != hipSuccess) r = fail(c, ATSIM_EHIP, "amp_pha: %s", hipGetErrorString(e));
-        }
+    if (!(dx > 0.0)) return fail(c, ATSIM_EINVAL, "fresnel_cube: pupil scale must be > 0");
+    float2* tw;
+    if (int r = get_twiddles(c, n, &tw)) return r;
+    // the planes in chunks of up to 256 MB of fields: one row pass from the same
+    // input with each plane's factor, one column pass that writes the amplitudes
+    // and phases
+    const long most = std::min<long>(std::max<long>(1, (256L << 20) / (long)(sizeof(float2) * n * n)), 32768);
+    const long cz = std::min(nz, most);
+    Scratch work(c);
+    HIPCHK(c, work.get(sizeof(float2) * (n * n + n) * cz));
+    float2* tmp = (float2*)work.p;
+    float2* tab = tmp + (size_t)n * n * cz;
+    hipError_t e = hipSuccess;
+    for (long k = 0; k < nz && e == hipSuccess; k += cz) {
+        const long cnt = std::min(cz, nz - k);
+        e = launch_fresnel_tables(tab, nullptr, n, dx, lambda, zstart, zend, k, cnt, nz, c->stream);
+        if (e == hipSuccess)
+            e = launch_row(n, OP_FRESNEL, 0, (const float2*)d_in, 0, tmp, cnt, tab, (int)cnt, tw, c->stream);
+        if (e == hipSuccess)
+            e = launch_col_amp(n, tmp, cnt, tab, tw, d_amp + k * n * n, d_pha + k * n * n, c->stream);
     }
-    hipStreamSynchronize(c->stream);
-    hipFree(tmp);
-    return r;
+    if (e != hipSuccess) return fail(c, ATSIM_EHIP, "fresnel_cube: %s", hipGetErrorString(e));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return ATSIM_OK;
 }
 
 // ------------------------------------------------------------------ noise

@@ -3,9 +3,7 @@
 //  k_row / k_col   LDS Stockham FFT passes along x / y.  OP_FRESNEL fuses
 //                  FFT -> transfer-function multiply -> IFFT in one pass
 //                  (the separable form of Fresnel_propagate_wavefront,
-//                  WFpropagate.c:68-152); k_row can also multiply the field by
-//                  the screen phase of a group of layers first, sampling the
-//                  master screens itself (AtmosphericTurbulence.c:2759-3412).
+//                  WFpropagate.c:68-152).
 //  k_row_fresnel   the frame's x pass over several wavelengths of one row:
 //                  optionally the x factor of the gap before a layer group,
 //                  the group's screen, the x factor of the gap after it.
@@ -121,17 +119,6 @@ __device__ __forceinline__ float2 expi_q(double qt) {
     if (qi & 2) sr = -sr;
     if ((qi + 1) & 2) cr = -cr;
     return make_float2(cr, sr);
-}
-
-__device__ __forceinline__ double screen_phase(const ScreenArgs& sa, int d, int w, int i, int j) {
-    double ph = 0.0;
-    for (int q = 0; q < sa.lcount; q++) {
-        const int l = sa.lfirst + q;
-        const LayerSample p = sa.ls[d * sa.L + l];
-        const float* m = sa.masters + (size_t)l * sa.M * sa.M;
-        ph = fma(sa.s[w * sa.L + l], sample_layer(m, (int)sa.M, p, i, j), ph);
-    }
-    return ph;
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (blockIdx b runs on
@@ -271,18 +258,27 @@ struct RowCfg {
     static constexpr int ROWS = ROWS0 < N ? ROWS0 : N;
     static constexpr int THREADS = ROWS * T;
 };
+// columns per workgroup of a column pass with 16 elements per thread.  8 up to
+// 2048: from 512 on two workgroups then share a CU (one Fresnel call on 8 fields
+// of 1024^2: 82 us against 92 with 16 columns, 64 of 512^2: 117 against 124).
 template <int N>
 struct ColCfg {
-    static constexpr int C0 = N <= 1024 ? 16 : (N == 2048 ? 8 : (N == 4096 ? 4 : 2));
+    static constexpr int C = N <= 2048 ? 8 : (N == 4096 ? 4 : 2);
+};
+// the same for the pass with a screen
+template <int N>
+struct ColScreenCfg {
+    static constexpr int C0 = N <= 1024 ? 16 : (N == 2048 ? 8 : 4);
     static constexpr int C = C0 < N ? C0 : N;
-    static constexpr int THREADS = C * (N / 16);
 };
 
 // ------------------------------------------------------------------ passes
-template <int N, int OP, int DIR, bool GEN>
+// Rows of F fields: read from in (field f at in + f istride: the fields
+// themselves, or with istride 0 one field for all), written to out.
+template <int N, int OP, int DIR>
 __global__ void __launch_bounds__(RowCfg<N>::THREADS)
-k_row(float2* __restrict__ data, const float2* __restrict__ tf, int W, const float2* __restrict__ tw,
-      ScreenArgs sa) {
+k_row(const float2* in, long istride, float2* out, const float2* __restrict__ tf, int W,
+      const float2* __restrict__ tw) {
     using P = Plan<N>;
     constexpr int T = P::T, ROWS = RowCfg<N>::ROWS;
     constexpr int RI = (OP == OP_FRESNEL) ? P::first(-1) : P::first(DIR);
@@ -291,18 +287,10 @@ k_row(float2* __restrict__ data, const float2* __restrict__ tf, int W, const flo
     const int lr = threadIdx.x / T, t = threadIdx.x - lr * T;
     const int row = blockIdx.x * ROWS + lr;
     const int f = blockIdx.y;
-    float2* rowp = data + ((size_t)f * N + row) * N;
+    const float2* ip = in + f * istride + (size_t)row * N;
     float2 v[16];
 #pragma unroll
-    for (int q = 0; q < 16; q++) v[q] = GEN ? make_float2(1.f, 0.f) : rowp[reg_index<N, RI>(t, q)];
-    if (sa.lcount > 0) {
-        const int w = f % sa.W, d = f / sa.W;
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const double ph = screen_phase(sa, d, w, reg_index<N, RI>(t, q), row);
-            v[q] = cmul(v[q], expi_d(ph));
-        }
-    }
+    for (int q = 0; q < 16; q++) v[q] = ip[reg_index<N, RI>(t, q)];
     float2* L = lds + lr * P::LDS;
     if constexpr (OP == OP_FRESNEL) {
         fft_regs<N, -1, 1>(v, L, t, 0, tw);
@@ -314,14 +302,18 @@ k_row(float2* __restrict__ data, const float2* __restrict__ tf, int W, const flo
     } else {
         fft_regs<N, DIR, 1>(v, L, t, 0, tw);
     }
+    float2* rowp = out + ((size_t)f * N + row) * N;
 #pragma unroll
     for (int q = 0; q < 16; q++) rowp[reg_index<N, RO>(t, q)] = v[q];
 }
 
-template <int N, int OP, int DIR, int C>
+// AMP (Fresnel only): the fields' amplitude and phase are written instead of
+// the fields (Fresnel_propagate_cube, WFpropagate.c:337-401; both from the float
+// field in FP64).
+template <int N, int OP, int DIR, int C, bool AMP = false>
 __global__ void __launch_bounds__(C * (N / 16))
 k_col(float2* __restrict__ data, const float2* __restrict__ tf, int W, const float2* __restrict__ tw, int wlo,
-      int wcnt) {
+      int wcnt, float* __restrict__ amp, float* __restrict__ pha) {
     using P = Plan<N>;
     constexpr int RI = (OP == OP_FRESNEL) ? P::first(-1) : P::first(DIR);
     constexpr int RO = (OP == OP_FRESNEL) ? P::last(+1) : P::last(DIR);
@@ -347,21 +339,33 @@ k_col(float2* __restrict__ data, const float2* __restrict__ tf, int W, const flo
     } else {
         fft_regs<N, DIR, C>(v, lds, t, c, tw);
     }
+    if constexpr (AMP) {
+        const size_t o = (size_t)f * N * N + col;
 #pragma unroll
-    for (int q = 0; q < 16; q++) base[(size_t)reg_index<N, RO>(t, q) * N] = v[q];
+        for (int q = 0; q < 16; q++) {
+            const double re = v[q].x, im = v[q].y;
+            const size_t p = o + (size_t)reg_index<N, RO>(t, q) * N;
+            amp[p] = (float)sqrt(re * re + im * im);
+            pha[p] = (float)atan2(im, re);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 16; q++) base[(size_t)reg_index<N, RO>(t, q) * N] = v[q];
+    }
 }
 
-// Column Fresnel pass with E = 32 elements per thread (N / 32 threads per
+// Column pass with E = 32 elements per thread (N / 32 threads per
 // column, C * N / 32 per workgroup) and float exchanges: C columns take
 // C * Plan::LDSC * 4 B of LDS.  C = 8 (72 KB at N = 2048) lets two
 // workgroups share a CU; C = 16 (144 KB) reads 128-byte row segments.  At
 // most 128 VGPRs (4 waves per SIMD).
-template <int N, int C, int E>
+template <int N, int OP, int DIR, int C, int E>
 __global__ void __launch_bounds__(C * (N / E)) __attribute__((amdgpu_waves_per_eu(4)))
 k_col_split(float2* __restrict__ data, const float2* __restrict__ tf, int W, const float2* __restrict__ tw, int wlo,
             int wcnt) {
     using P = Plan<N>;
-    constexpr int RI = P::first(-1), RO = P::last(+1), RL = P::last(-1);
+    constexpr int RI = (OP == OP_FRESNEL) ? P::first(-1) : P::first(DIR);
+    constexpr int RO = (OP == OP_FRESNEL) ? P::last(+1) : P::last(DIR), RL = P::last(-1);
     __shared__ float lds[C * P::LDSC];
     const int c = threadIdx.x % C, t = threadIdx.x / C;
     const int ntile = N / C;
@@ -376,11 +380,15 @@ k_col_split(float2* __restrict__ data, const float2* __restrict__ tf, int W, con
     float2 v[E];
 #pragma unroll
     for (int q = 0; q < E; q++) v[q] = buf_load2(fr, lo, (reg_index<N, RI, E>(0, q) * N) * 8);
-    fft_regs_split<N, -1, C, E>(v, lds, t, c, tw);
-    const auto hr = buf_rsrc(tf + (size_t)(f % W) * N, (uint32_t)N * 8);
+    if constexpr (OP == OP_FRESNEL) {
+        fft_regs_split<N, -1, C, E>(v, lds, t, c, tw);
+        const auto hr = buf_rsrc(tf + (size_t)(f % W) * N, (uint32_t)N * 8);
 #pragma unroll
-    for (int q = 0; q < E; q++) v[q] = cmul(v[q], buf_load2(hr, (uint32_t)t * 8, reg_index<N, RL, E>(0, q) * 8));
-    fft_regs_split<N, +1, C, E>(v, lds, t, c, tw);
+        for (int q = 0; q < E; q++) v[q] = cmul(v[q], buf_load2(hr, (uint32_t)t * 8, reg_index<N, RL, E>(0, q) * 8));
+        fft_regs_split<N, +1, C, E>(v, lds, t, c, tw);
+    } else {
+        fft_regs_split<N, DIR, C, E>(v, lds, t, c, tw);
+    }
 #pragma unroll
     for (int q = 0; q < E; q++) buf_store2(v[q], fr, lo, (reg_index<N, RO, E>(0, q) * N) * 8);
 }
@@ -721,17 +729,12 @@ static hipError_t row_fresnel_dispatch(bool gen, float2* data, int D, const floa
 }
 
 template <int N>
-static hipError_t row_dispatch(int op, int dir, bool gen, float2* data, long F, const float2* tf, int W,
-                               const float2* tw, const ScreenArgs& sa, hipStream_t st) {
+static hipError_t row_dispatch(int op, int dir, const float2* in, long istride, float2* out, long F, const float2* tf,
+                               int W, const float2* tw, hipStream_t st) {
     dim3 grid(N / RowCfg<N>::ROWS, (unsigned)F), block(RowCfg<N>::THREADS);
-    if (op == OP_FRESNEL) {
-        if (gen) k_row<N, OP_FRESNEL, 0, true><<<grid, block, 0, st>>>(data, tf, W, tw, sa);
-        else k_row<N, OP_FRESNEL, 0, false><<<grid, block, 0, st>>>(data, tf, W, tw, sa);
-    } else if (dir < 0) {
-        k_row<N, OP_FFT, -1, false><<<grid, block, 0, st>>>(data, tf, W, tw, sa);
-    } else {
-        k_row<N, OP_FFT, +1, false><<<grid, block, 0, st>>>(data, tf, W, tw, sa);
-    }
+    if (op == OP_FRESNEL) k_row<N, OP_FRESNEL, 0><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw);
+    else if (dir < 0) k_row<N, OP_FFT, -1><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw);
+    else k_row<N, OP_FFT, +1><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw);
     return hipGetLastError();
 }
 
@@ -748,32 +751,44 @@ static hipError_t col_launch(int op, int dir, float2* data, long F, const float2
         return hipErrorInvalidValue;
     } else {
         dim3 grid(N / C, (unsigned)F), block(C * (N / 16));
-        if (op == OP_FRESNEL) k_col<N, OP_FRESNEL, 0, C><<<grid, block, 0, st>>>(data, tf, W, tw, wlo, wcnt);
-        else if (dir < 0) k_col<N, OP_FFT, -1, C><<<grid, block, 0, st>>>(data, tf, W, tw, 0, 0);
-        else k_col<N, OP_FFT, +1, C><<<grid, block, 0, st>>>(data, tf, W, tw, 0, 0);
+        if (op == OP_FRESNEL) k_col<N, OP_FRESNEL, 0, C><<<grid, block, 0, st>>>(data, tf, W, tw, wlo, wcnt, nullptr, nullptr);
+        else if (dir < 0) k_col<N, OP_FFT, -1, C><<<grid, block, 0, st>>>(data, tf, W, tw, 0, 0, nullptr, nullptr);
+        else k_col<N, OP_FFT, +1, C><<<grid, block, 0, st>>>(data, tf, W, tw, 0, 0, nullptr, nullptr);
         return hipGetLastError();
     }
 }
 
-template <int N>
-static int col_default_c() { return ColCfg<N>::C; }
+template <int N, int C>
+static hipError_t col_split_launch(int op, int dir, float2* data, long F, const float2* tf, int W, const float2* tw,
+                                   int wlo, int wcnt, hipStream_t st) {
+    dim3 grid(N / C, (unsigned)F), block(C * (N / 32));
+    if (op == OP_FRESNEL) k_col_split<N, OP_FRESNEL, 0, C, 32><<<grid, block, 0, st>>>(data, tf, W, tw, wlo, wcnt);
+    else if (dir < 0) k_col_split<N, OP_FFT, -1, C, 32><<<grid, block, 0, st>>>(data, tf, W, tw, 0, 0);
+    else k_col_split<N, OP_FFT, +1, C, 32><<<grid, block, 0, st>>>(data, tf, W, tw, 0, 0);
+    return hipGetLastError();
+}
 
 template <int N>
 static hipError_t col_dispatch(int op, int dir, float2* data, long F, const float2* tf, int W, const float2* tw,
                                int c, int e, int wlo, int wcnt, hipStream_t st) {
     if constexpr (N >= 256 && N <= 2048) {
-        if (e == 32 && op == OP_FRESNEL && (c <= 0 || c == 8)) {
-            dim3 grid(N / 8, (unsigned)F), block(8 * (N / 32));
-            k_col_split<N, 8, 32><<<grid, block, 0, st>>>(data, tf, W, tw, wlo, wcnt);
-            return hipGetLastError();
-        }
+        if (e == 32 && op == OP_FRESNEL && (c <= 0 || c == 8))
+            return col_split_launch<N, 8>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
         if (e == 32 && op == OP_FRESNEL && c == 16) {
             dim3 grid(N / 16, (unsigned)F), block(16 * (N / 32));
-            k_col_split<N, 16, 32><<<grid, block, 0, st>>>(data, tf, W, tw, wlo, wcnt);
+            k_col_split<N, OP_FRESNEL, 0, 16, 32><<<grid, block, 0, st>>>(data, tf, W, tw, wlo, wcnt);
             return hipGetLastError();
         }
     }
-    if (c <= 0) c = col_default_c<N>();
+    if constexpr (N >= 4096) {
+        // 32 elements per thread exchanging through half the LDS: twice the
+        // columns (64 and 32 bytes of a row) in a workgroup (one Fresnel call on
+        // 4 fields of 4096^2: 684 against 792 us; 8192^2: 966 against 1 038)
+        if (c <= 0) return col_split_launch<N, N == 4096 ? 8 : 4>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
+    }
+    // 4 columns where 8 leave CUs without a workgroup (one field of 1024^2: 37
+    // against 39 us a call, 512^2: 31 against 32)
+    if (c <= 0) c = (ColCfg<N>::C == 8 && N / 8 * F < 256) ? 4 : ColCfg<N>::C;
     switch (c) {
         case 2: return col_launch<N, 2>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
         case 4: return col_launch<N, 4>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
@@ -787,12 +802,30 @@ bool supported_n(long n) { return n >= 16 && n <= 8192 && (n & (n - 1)) == 0; }
 
 #define ATSIM_FOR_EACH_N(X) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192)
 
-hipError_t launch_row(long n, int op, int dir, bool gen, float2* data, long F, const float2* tf,
-                      const float2* tw, const ScreenArgs& sa, hipStream_t st) {
-    const int W = sa.W > 0 ? sa.W : 1;
+hipError_t launch_row(long n, int op, int dir, const float2* in, long istride, float2* out, long F, const float2* tf,
+                      int W, const float2* tw, hipStream_t st) {
     switch (n) {
 #define X(NN) \
-    case NN: return row_dispatch<NN>(op, dir, gen, data, F, tf, W, tw, sa, st);
+    case NN: return row_dispatch<NN>(op, dir, in, istride, out, F, tf, W, tw, st);
+        ATSIM_FOR_EACH_N(X)
+#undef X
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <int N>
+static hipError_t col_amp(float2* data, long F, const float2* tf, const float2* tw, float* amp, float* pha,
+                          hipStream_t st) {
+    constexpr int C = ColCfg<N>::C;
+    dim3 grid(N / C, (unsigned)F), block(C * (N / 16));
+    k_col<N, OP_FRESNEL, 0, C, true><<<grid, block, 0, st>>>(data, tf, (int)F, tw, 0, 0, amp, pha);
+    return hipGetLastError();
+}
+hipError_t launch_col_amp(long n, float2* data, long F, const float2* tf, const float2* tw, float* amp, float* pha,
+                          hipStream_t st) {
+    switch (n) {
+#define X(NN) \
+    case NN: return col_amp<NN>(data, F, tf, tw, amp, pha, st);
         ATSIM_FOR_EACH_N(X)
 #undef X
         default: return hipErrorInvalidValue;
@@ -862,7 +895,7 @@ hipError_t launch_col_screen(long n, float2* data, int D, const float2* tfp, con
     switch (n) {
 #define X(NN)                                                                                         \
     case NN: {                                                                                        \
-        constexpr int C = ColCfg<NN>::C;                                                              \
+        constexpr int C = ColScreenCfg<NN>::C;                                                        \
         dim3 grid(NN / C, (unsigned)(D * nw)), block(C * (NN / 16));                                  \
         k_col_screen<NN, C><<<grid, block, 0, st>>>(data, tfp, tf, tw, sa, vq, slot0);                \
         return hipGetLastError();                                                                     \
@@ -1070,21 +1103,6 @@ hipError_t launch_cmul(float2* a, const float2* b, long n, long nbatch, hipStrea
     int blocks = (int)((tot + 255) / 256 < 16384 ? (tot + 255) / 256 : 16384);
     if (blocks < 1) blocks = 1;
     k_cmul<<<blocks, 256, 0, st>>>(a, b, n, nbatch);
-    return hipGetLastError();
-}
-
-__global__ void k_amp_pha(const float2* __restrict__ e, float* __restrict__ amp, float* __restrict__ pha, long n) {
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const double re = e[i].x, im = e[i].y;
-        amp[i] = (float)sqrt(re * re + im * im);
-        pha[i] = (float)atan2(im, re);
-    }
-}
-
-hipError_t launch_amp_pha(const float2* e, float* amp, float* pha, long n, hipStream_t st) {
-    int blocks = (int)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
-    if (blocks < 1) blocks = 1;
-    k_amp_pha<<<blocks, 256, 0, st>>>(e, amp, pha, n);
     return hipGetLastError();
 }
 

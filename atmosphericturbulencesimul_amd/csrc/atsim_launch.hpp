@@ -11,12 +11,11 @@ enum { OP_FFT = 0, OP_FRESNEL = 1 };
 
 bool supported_n(long n);
 
-// Row pass over F fields of n x n: optional screen multiply (sa.lcount > 0)
-// before the transform; op OP_FRESNEL = FFT_x, x h(kx) (table tf + (f % W) n),
-// IFFT_x; OP_FFT = one transform of sign dir.  gen: the input field is 1
-// (nothing is read).
-hipError_t launch_row(long n, int op, int dir, bool gen, float2* data, long F, const float2* tf,
-                      const float2* tw, const ScreenArgs& sa, hipStream_t st);
+// Row pass over F fields of n x n, from in (field f at in + f istride; istride
+// 0: one field for all) to out (may be in): op OP_FRESNEL = FFT_x, x h(kx)
+// (table tf + (f % W) n), IFFT_x; OP_FFT = one transform of sign dir.
+hipError_t launch_row(long n, int op, int dir, const float2* in, long istride, float2* out, long F, const float2* tf,
+                      int W, const float2* tw, hipStream_t st);
 // Fresnel x pass of every (direction, wavelength) field with the screen
 // phase of the layer group sa.lfirst .. + sa.lcount (sampled once per pixel
 // and direction); gen: the incoming field is 1.  Tables tf + w n.
@@ -46,6 +45,11 @@ bool col_screen_supported(long n);
 // holds 32 elements per thread and exchanges through float LDS (256 <= n <= 2048)
 hipError_t launch_col(long n, int op, int dir, float2* data, long F, const float2* tf, int W,
                       const float2* tw, hipStream_t st, int c = 0, int e = 0, int wlo = 0, int wcnt = 0);
+
+// Fresnel column pass of F fields (tables tf + f n) that writes their amplitude
+// and phase ([F][n][n]) instead of the fields
+hipError_t launch_col_amp(long n, float2* data, long F, const float2* tf, const float2* tw, float* amp, float* pha,
+                          hipStream_t st);
 
 hipError_t launch_permut(float2* data, long n0, long n1, long nbatch, hipStream_t st);
 // mixed-precision row transforms (atsim_fft_mfma.hip): length 2048, radix-16
@@ -89,7 +93,6 @@ hipError_t launch_strfn(const float* s, long size, long a, long b, int circular,
                         int nblocks, hipStream_t st);
 hipError_t launch_scale(float* s, long n, double scale, hipStream_t st);
 hipError_t launch_cmul(float2* a, const float2* b, long n, long nbatch, hipStream_t st);
-hipError_t launch_amp_pha(const float2* e, float* amp, float* pha, long n, hipStream_t st);
 hipError_t launch_tf_init(float2* C, long size, double coeff, double fpmaskrad, hipStream_t st);
 
 // the planes a.vr, a.vl of the factored geometric phase, and with vq the

@@ -787,56 +787,38 @@ int atsim_make_master(atsim_ctx* c, const void* d_noise, long size, double outer
     if (!(outerscale_px > 0) || !(innerscale_px > 0)) return fail(c, ATSIM_EINVAL, "make_master: scales must be > 0");
     const double f0 = 1.0 * size / outerscale_px;                        // AT.c:679
     const double fi = (5.92 / (2.0 * M_PI)) * size / innerscale_px;       // AT.c:680
-    float2* buf = nullptr;
-    const int nblocks = 1024;
-    double* part = nullptr;
-    HIPCHK(c, hipMalloc(&buf, sizeof(float2) * size * size));
-    if (hipMalloc(&part, sizeof(double) * nblocks * 8) != hipSuccess) {
-        hipFree(buf);
+    float2* tw;
+    if (int r = get_twiddles(c, size, &tw)) return r;
+    const size_t nn = (size_t)size * size;
+    Scratch work(c);
+    if (work.get(sizeof(float2) * nn + sizeof(double) * (8 * (size_t)lag_blocks(size) + 4)) != hipSuccess) {
+        (void)hipGetLastError();
         return fail(c, ATSIM_ENOMEM, "make_master: allocation failed");
     }
-    int r = ATSIM_OK;
-    std::vector<double> s;
-    hipError_t e = launch_synth_filter((const float2*)d_noise, buf, size, f0, fi, rlim, c->stream);
-    if (e != hipSuccess) r = fail(c, ATSIM_EHIP, "synth_filter: %s", hipGetErrorString(e));
-    if (r == ATSIM_OK) r = atsim_fft2d(c, buf, size, 1, -1);
-    if (r == ATSIM_OK) {
-        e = launch_lag_sums(buf, size, part, nblocks, c->stream);
-        if (e != hipSuccess) r = fail(c, ATSIM_EHIP, "lag_sums: %s", hipGetErrorString(e));
-    }
-    if (r == ATSIM_OK) r = reduce_partials(c, part, nblocks, 8, s);
-    if (r == ATSIM_OK) {
-        // AT.c:794-847: lags (ii, jj) in {1,2}^2, ii outer; sums ordered (1,1) (1,2) (2,1) (2,2)
-        const double n2 = (double)size * (double)size;
-        const int la[4] = {1, 1, 2, 2}, lb[4] = {1, 2, 1, 2};
-        double v1 = 0.0, v2 = 0.0;
-        for (int q = 0; q < 4; q++) {
-            const double lg = 5.0 / 3.0 * log10(sqrt((double)(la[q] * la[q] + lb[q] * lb[q])));
-            v1 += log10(s[q] / n2) - lg;
-            v2 += log10(s[4 + q] / n2) - lg;
-        }
-        const double c1 = pow(10.0, v1 / 4.0), c2 = pow(10.0, v2 / 4.0);
-        if (C1) *C1 = c1;
-        if (C2) *C2 = c2;
-        e = launch_split_scale(buf, d_out1, d_out2, size * size, 1.0 / sqrt(c1), 1.0 / sqrt(c2), c->stream);
-        if (e != hipSuccess) r = fail(c, ATSIM_EHIP, "split_scale: %s", hipGetErrorString(e));
-    }
-    hipStreamSynchronize(c->stream);
-    hipFree(part);
-    hipFree(buf);
-    return r;
+    float2* buf = (float2*)work.p;
+    double* fit = (double*)(buf + nn);  // C1, C2, 1/sqrt(C1), 1/sqrt(C2)
+    HIPCHK(c, launch_synth_row((const float2*)d_noise, buf, size, f0, fi, rlim, tw, c->stream));
+    HIPCHK(c, launch_col(size, OP_FFT, -1, buf, 1, nullptr, 1, tw, c->stream));
+    HIPCHK(c, launch_lag_fit(buf, size, fit + 4, fit, c->stream));
+    HIPCHK(c, launch_split_scale(buf, d_out1, d_out2, (long)nn, fit + 2, c->stream));
+    double h[2];
+    if (C1 || C2) HIPCHK(c, hipMemcpyAsync(h, fit, sizeof h, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (C1) *C1 = h[0];
+    if (C2) *C2 = h[1];
+    return ATSIM_OK;
 }
 
 int atsim_strfn(atsim_ctx* c, const float* d_screen, long size, long a, long b, double* out) {
     if (!c || !d_screen || !out || size <= 0) return ATSIM_EINVAL;
     const int nblocks = 512;
-    double* part = nullptr;
-    HIPCHK(c, hipMalloc(&part, sizeof(double) * nblocks));
+    Scratch work(c);
+    HIPCHK(c, work.get(sizeof(double) * nblocks));
+    double* part = (double*)work.p;
     long aa = ((a % size) + size) % size;
     hipError_t e = launch_strfn(d_screen, size, aa, b, 1, part, nblocks, c->stream);
     std::vector<double> s;
     int r = e == hipSuccess ? reduce_partials(c, part, nblocks, 1, s) : fail(c, ATSIM_EHIP, "strfn launch");
-    hipFree(part);
     if (r) return r;
     *out = s[0] / ((double)size * (double)size);
     return ATSIM_OK;
@@ -845,12 +827,12 @@ int atsim_strfn(atsim_ctx* c, const float* d_screen, long size, long a, long b, 
 int atsim_r0_measure(atsim_ctx* c, const float* d_screen, long size, long dpix, double* r0) {
     if (!c || !d_screen || !r0 || dpix <= 0 || dpix >= size) return ATSIM_EINVAL;
     const int nblocks = 512;
-    double* part = nullptr;
-    HIPCHK(c, hipMalloc(&part, sizeof(double) * nblocks));
+    Scratch work(c);
+    HIPCHK(c, work.get(sizeof(double) * nblocks));
+    double* part = (double*)work.p;
     hipError_t e = launch_strfn(d_screen, size, dpix, 0, 0, part, nblocks, c->stream);
     std::vector<double> s;
     int r = e == hipSuccess ? reduce_partials(c, part, nblocks, 1, s) : fail(c, ATSIM_EHIP, "r0 launch");
-    hipFree(part);
     if (r) return r;
     const double cnt = (double)(size - dpix) * (double)size;
     *r0 = 1.0 * dpix * pow((s[0] / cnt) / 6.88, -3.0 / 5.0);  // AT.c:2269

@@ -14,8 +14,9 @@
 //  k_layer_phase   FP64 phase planes of the layers column passes apply.
 //  k_permut        quadrant swap (fft.c:570-792).
 //  k_noise         Philox4x32-10 + Box-Muller complex Gaussian noise.
-//  k_synth_filter  von Karman spectral filter on the noise, written in the
-//                  quadrant-swapped layout (AtmosphericTurbulence.c:643-784).
+//  k_synth_row     von Karman spectral filter on the noise in the
+//                  quadrant-swapped layout (AtmosphericTurbulence.c:643-784) and
+//                  its transform along x.
 //  k_lag_sums, k_strfn  FP64 structure-function reductions
 //                  (AT.c:790-847, 2246-2270).
 //  k_extract       crop, amplitude, phase, geometric-phase unwrap
@@ -970,31 +971,73 @@ hipError_t launch_noise(float2* out, long n, uint64_t seed, uint32_t stream, hip
 }
 
 // ------------------------------------------------------------------ synthesis
-// storage index p holds centred index (p + s/2) mod s after the quadrant swap
-__global__ void k_synth_filter(const float2* __restrict__ noise, float2* __restrict__ out, long size,
-                               double f0, double fi, double rlim) {
-    const long n = size * size, h = size / 2;
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
-        const long py = e / size, px = e - py * size;
-        const long cx = (px + h) % size, cy = (py + h) % size;
-        const double dx = (double)(cx - h), dy = (double)(cy - h);
-        const double r2 = dx * dx + dy * dy;
-        double A = 0.0;
-        const double tmpd = sqrt(r2 + f0 * f0);
-        const bool inside = rlim > 0.0 && sqrt(r2) < rlim;
-        if (!inside && tmpd > 0.0) A = sqrt(exp(-r2 / fi / fi)) / pow(tmpd, 11.0 / 6.0);
-        if (cx == h && cy == h) A = 0.0;
-        const float2 z = noise[cy * size + cx];
-        out[e] = make_float2((float)(A * (double)z.x), (float)(A * (double)z.y));
+// The von Karman filter (AtmosphericTurbulence.c:671-784) on the noise and the
+// spectrum's transform along x in one pass.  Storage index p holds the centred
+// index (p + s/2) mod s (the quadrant swap).  The amplitude depends on |dx| and
+// |dy| alone, and its FP64 exponential and power cost more than the pass moves:
+// a workgroup takes the rows y and s - y (one |dy|; rows 0 and s/2 share the
+// first workgroup) and makes each of the s/2 + 1 amplitudes once, in LDS, for
+// the four pixels that use it.  4096^2: 79 us (268 MB), where the filter alone
+// took 198 us and the transform 44.
+template <int N>
+__global__ void __launch_bounds__(2 * (N / 16))
+k_synth_row(const float2* __restrict__ noise, float2* __restrict__ out, double f0, double fi, double rlim,
+            const float2* __restrict__ tw) {
+    using P = Plan<N>;
+    constexpr int T = P::T, H = N / 2, RI = P::first(-1), RO = P::last(-1);
+    constexpr int AL = H + 1;  // amplitudes of |dx| = 0 .. H
+    __shared__ union {
+        float2 lds[2 * P::LDS];
+        double A[AL];
+    } sh;
+    const int lr = threadIdx.x / T, t = threadIdx.x - lr * T;
+    const int b = blockIdx.x;
+    const int row = lr == 0 ? b : (b == 0 ? H : N - b);
+    const float2* src = noise + (size_t)((row + H) % N) * N;
+    float2 v[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) v[q] = src[(reg_index<N, RI>(t, q) + H) % N];
+    for (int part = 0; part < (b == 0 ? 2 : 1); part++) {
+        // |dy| of this part's rows (both rows when b > 0)
+        const double dy = b == 0 ? (double)(part * H) : (double)b;
+        __syncthreads();
+        for (int i = threadIdx.x; i < AL; i += 2 * T) {
+            const double dx = (double)i, r2 = dx * dx + dy * dy;
+            double a = 0.0;
+            const double tmpd = sqrt(r2 + f0 * f0);
+            const bool inside = rlim > 0.0 && sqrt(r2) < rlim;
+            if (!inside && tmpd > 0.0) a = sqrt(exp(-r2 / fi / fi)) / pow(tmpd, 11.0 / 6.0);
+            if (i == 0 && dy == 0.0) a = 0.0;
+            sh.A[i] = a;
+        }
+        __syncthreads();
+        if (b > 0 || lr == part) {
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const int px = reg_index<N, RI>(t, q);
+                const double a = sh.A[px < H ? px : N - px];
+                v[q] = make_float2((float)(a * (double)v[q].x), (float)(a * (double)v[q].y));
+            }
+        }
     }
+    __syncthreads();
+    fft_regs<N, -1, 1, true>(v, sh.lds + lr * P::LDS, t, 0, tw);
+    float2* dst = out + (size_t)row * N;
+#pragma unroll
+    for (int q = 0; q < 16; q++) dst[reg_index<N, RO>(t, q)] = v[q];
 }
 
-hipError_t launch_synth_filter(const float2* noise, float2* out, long size, double f0, double fi, double rlim,
-                               hipStream_t st) {
-    long n = size * size;
-    int blocks = (int)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
-    k_synth_filter<<<blocks, 256, 0, st>>>(noise, out, size, f0, fi, rlim);
-    return hipGetLastError();
+hipError_t launch_synth_row(const float2* noise, float2* out, long size, double f0, double fi, double rlim,
+                            const float2* tw, hipStream_t st) {
+    switch (size) {
+#define X(NN)                                                                                                 \
+    case NN:                                                                                                  \
+        k_synth_row<NN><<<NN / 2, 2 * (NN / 16), 0, st>>>(noise, out, f0, fi, rlim, tw);                      \
+        return hipGetLastError();
+        ATSIM_FOR_EACH_N(X)
+#undef X
+        default: return hipErrorInvalidValue;
+    }
 }
 
 template <int NV>
@@ -1015,32 +1058,78 @@ __device__ __forceinline__ void block_reduce_store(double (&acc)[NV], double* __
     }
 }
 
-__global__ void __launch_bounds__(256) k_lag_sums(const float2* __restrict__ c, long size, double* partial) {
+// Sums of squared differences of Re and Im at the lags (1,1) (1,2) (2,1) (2,2)
+// (AT.c:790-847; x lag first), circular, in FP64: partial[block][8].  A thread
+// walks LAG_R rows down one column; the two pixels to the right of each later
+// row are loaded once and serve both y lags from registers.  4096^2: 30 us (134
+// MB), against 83 with the four neighbours of every pixel looked up.
+constexpr int LAG_R = 64;
+__global__ void __launch_bounds__(256) k_lag_sums(const float2* __restrict__ c, int size, double* __restrict__ partial) {
     double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const long n = size * size;
-    const int la[4] = {1, 1, 2, 2}, lb[4] = {1, 2, 1, 2};
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
-        const long y = e / size, x = e - y * size;
-        const float2 p = c[e];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const long x2 = (x + la[q]) % size, y2 = (y + lb[q]) % size;
-            const float2 o = c[y2 * size + x2];
+    const int x = min(blockIdx.x * 256 + (int)threadIdx.x, size - 1);
+    const bool in = blockIdx.x * 256 + (int)threadIdx.x < size;
+    const int x1 = x + 1 < size ? x + 1 : x + 1 - size, x2 = x + 2 < size ? x + 2 : x + 2 - size;
+    const int y0 = blockIdx.y * LAG_R, y1 = min(y0 + LAG_R, size);
+    auto row = [&](int y) { return c + (size_t)(y < size ? y : y - size) * size; };
+    float2 a1 = row(y0 + 1)[x1], a2 = row(y0 + 1)[x2];  // row y + 1
+#pragma unroll 4
+    for (int y = y0; y < y1; y++) {
+        const float2 p = row(y)[x];
+        const float2 b1 = row(y + 2)[x1], b2 = row(y + 2)[x2];
+        auto add = [&](int q, float2 o) {
             const double dr = (double)p.x - (double)o.x, di = (double)p.y - (double)o.y;
             acc[q] = fma(dr, dr, acc[q]);
             acc[4 + q] = fma(di, di, acc[4 + q]);
-        }
+        };
+        add(0, a1);
+        add(1, b1);
+        add(2, a2);
+        add(3, b2);
+        a1 = b1;
+        a2 = b2;
     }
-    block_reduce_store<8>(acc, partial + (size_t)blockIdx.x * 8);
+    if (!in)
+#pragma unroll
+        for (int q = 0; q < 8; q++) acc[q] = 0.0;
+    block_reduce_store<8>(acc, partial + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 8);
 }
 
-hipError_t launch_lag_sums(const float2* c, long size, double* partial, int nblocks, hipStream_t st) {
-    k_lag_sums<<<nblocks, 256, 0, st>>>(c, size, partial);
+// The structure function's fit at the four lags (AT.c:790-847): C_k is ten to the
+// mean over the lags of log10(D_k) - 5/3 log10(lag), k = Re, Im; out: C_1, C_2,
+// 1/sqrt(C_1), 1/sqrt(C_2).  One workgroup; the blocks are added in a fixed order.
+__global__ void __launch_bounds__(256) k_lag_fit(const double* __restrict__ partial, int nblocks, double n2,
+                                                 double* __restrict__ out) {
+    __shared__ double red[32][8];
+    const int v = threadIdx.x & 7, s = threadIdx.x >> 3;
+    double acc = 0.0;
+    for (int b = s; b < nblocks; b += 32) acc += partial[(size_t)b * 8 + v];
+    red[s][v] = acc;
+    __syncthreads();
+    if (threadIdx.x >= 2) return;
+    const int la[4] = {1, 1, 2, 2}, lb[4] = {1, 2, 1, 2};
+    double f = 0.0;
+    for (int q = 0; q < 4; q++) {
+        double t = 0.0;
+        for (int g = 0; g < 32; g++) t += red[g][threadIdx.x * 4 + q];
+        f += log10(t / n2) - 5.0 / 3.0 * log10(sqrt((double)(la[q] * la[q] + lb[q] * lb[q])));
+    }
+    const double c = pow(10.0, f / 4.0);
+    out[threadIdx.x] = c;
+    out[2 + threadIdx.x] = 1.0 / sqrt(c);
+}
+
+int lag_blocks(long size) { return (int)((size + 255) / 256) * (int)((size + LAG_R - 1) / LAG_R); }
+hipError_t launch_lag_fit(const float2* c, long size, double* partial, double* out, hipStream_t st) {
+    dim3 grid((unsigned)((size + 255) / 256), (unsigned)((size + LAG_R - 1) / LAG_R));
+    k_lag_sums<<<grid, 256, 0, st>>>(c, (int)size, partial);
+    k_lag_fit<<<1, 256, 0, st>>>(partial, lag_blocks(size), (double)size * (double)size, out);
     return hipGetLastError();
 }
 
-__global__ void k_split_scale(const float2* __restrict__ c, float* __restrict__ o1, float* __restrict__ o2,
-                              long n, double s1, double s2) {
+// the two screens of a complex one, scaled by sc[0] and sc[1]
+__global__ void __launch_bounds__(256) k_split_scale(const float2* __restrict__ c, float* __restrict__ o1,
+                                                     float* __restrict__ o2, long n, const double* __restrict__ sc) {
+    const double s1 = sc[0], s2 = sc[1];
     for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
         const float2 p = c[e];
         o1[e] = (float)((double)p.x * s1);
@@ -1048,10 +1137,9 @@ __global__ void k_split_scale(const float2* __restrict__ c, float* __restrict__ 
     }
 }
 
-hipError_t launch_split_scale(const float2* c, float* o1, float* o2, long n, double s1, double s2,
-                              hipStream_t st) {
+hipError_t launch_split_scale(const float2* c, float* o1, float* o2, long n, const double* sc, hipStream_t st) {
     int blocks = (int)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
-    k_split_scale<<<blocks, 256, 0, st>>>(c, o1, o2, n, s1, s2);
+    k_split_scale<<<blocks, 256, 0, st>>>(c, o1, o2, n, sc);
     return hipGetLastError();
 }
 

@@ -82,13 +82,15 @@ hipError_t launch_fresnel_odd(const float2* in, float2* out, long n0, long n1, l
 // permut on any sides; out != in
 hipError_t launch_permut_any(const float2* in, float2* out, long n0, long n1, long nbatch, hipStream_t st);
 hipError_t launch_noise(float2* out, long n, uint64_t seed, uint32_t stream, hipStream_t st);
-hipError_t launch_synth_filter(const float2* noise, float2* out, long size, double f0, double fi,
-                               double rlim, hipStream_t st);
-// partial sums of squared differences at lags (1,1),(1,2),(2,1),(2,2) of Re
-// and Im: partial[block][8]
-hipError_t launch_lag_sums(const float2* c, long size, double* partial, int nblocks, hipStream_t st);
-hipError_t launch_split_scale(const float2* c, float* o1, float* o2, long n, double s1, double s2,
-                              hipStream_t st);
+// the filtered noise spectrum transformed along x (tw with the per-stage tables)
+hipError_t launch_synth_row(const float2* noise, float2* out, long size, double f0, double fi, double rlim,
+                            const float2* tw, hipStream_t st);
+// the structure function's fit of Re and Im: partial holds 8 lag_blocks(size)
+// doubles, out receives C1, C2, 1/sqrt(C1), 1/sqrt(C2)
+int lag_blocks(long size);
+hipError_t launch_lag_fit(const float2* c, long size, double* partial, double* out, hipStream_t st);
+// o1 = sc[0] Re c, o2 (may be null) = sc[1] Im c
+hipError_t launch_split_scale(const float2* c, float* o1, float* o2, long n, const double* sc, hipStream_t st);
 hipError_t launch_strfn(const float* s, long size, long a, long b, int circular, double* partial,
                         int nblocks, hipStream_t st);
 hipError_t launch_scale(float* s, long n, double scale, hipStream_t st);

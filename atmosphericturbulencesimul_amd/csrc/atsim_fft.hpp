@@ -250,42 +250,6 @@ __host__ __device__ constexpr int tw_stage_off(int n, int dir, int s) {
 }
 __host__ __device__ constexpr int tw_tables_size(int n) { return tw_stage_off(n, +1, (ilog2c(n) + 3) / 4); }
 
-// stage_compute with the twiddles from the stage's table (tw: the N-entry
-// table followed by the per-stage tables): w^1, w^2, w^4, w^8 loaded, the
-// others composed as stage_compute does -- the same values, so the same
-// results.  (Loading all R - 1 twiddles of a butterfly from [r][k] tables
-// instead saves the 11 products but costs more than it saves: 2048^2 fused
-// row pass 272 us against 242 us.)
-template <int N, int R, int NS, int DIR, int E, int S>
-__device__ __forceinline__ void stage_compute_tab(float2* v, int t, const float2* __restrict__ tw) {
-    constexpr int T = N / E;
-    constexpr int OFF = N + tw_stage_off(N, DIR, S);
-#pragma unroll
-    for (int b = 0; b < E / R; b++) {
-        if constexpr (NS > 1) {
-            const int k = (t + b * T) % NS;
-            float2 p[4];  // w^1, w^2, w^4, w^8
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if ((1 << e) < R) p[e] = twiddle<N, DIR>(tw, OFF + e * NS + k);
-#pragma unroll
-            for (int r = 1; r < R; r++) {
-                float2 w = make_float2(1.f, 0.f);
-                bool first = true;
-#pragma unroll
-                for (int e = 3; e >= 0; e--)
-                    if (r & (1 << e)) {
-                        w = first ? p[e] : cmul(w, p[e]);
-                        first = false;
-                    }
-                v[b * R + r] = cmul(v[b * R + r], w);
-            }
-        }
-        dftR<R, DIR>(v + b * R);
-        if constexpr (E > 16) __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
 // Padded LDS positions (one pad slot every 2^PS elements) as one per-thread
 // base plus compile-time offsets (immediate offsets of the LDS instructions,
 // no per-element address registers).  For every plan here (all N, E = 16 or
@@ -326,12 +290,56 @@ __device__ __forceinline__ void stage_load(float2* v, const float2* lds, int t, 
         for (int r = 0; r < R; r++) v[b * R + r] = p[load_off<N, R, E, PS>(b, r) * C];
 }
 
-// stage s >= 1 of a transform: twiddles from the N-entry table, or (TAB) from
-// the stage's own table that follows it
+// The twiddles w^1, w^2, w^4, w^8 of the butterflies of stage s >= 1, from the
+// N-entry table or (TAB) from the stage's own table that follows it.
 template <int N, int R, int NS, int DIR, int E, int S, bool TAB>
-__device__ __forceinline__ void stage_compute_sel(float2* v, int t, const float2* __restrict__ tw) {
-    if constexpr (TAB) stage_compute_tab<N, R, NS, DIR, E, S>(v, t, tw);
-    else stage_compute<N, R, NS, DIR, E>(v, t, tw);
+__device__ __forceinline__ void stage_twiddles(float2 (&p)[E / R][4], int t, const float2* __restrict__ tw) {
+    constexpr int T = N / E, STEP = N / (NS * R), OFF = N + tw_stage_off(N, DIR, S);
+#pragma unroll
+    for (int b = 0; b < E / R; b++) {
+        const int k = (t + b * T) % NS;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if ((1 << e) < R) p[b][e] = twiddle<N, DIR>(tw, TAB ? OFF + e * NS + k : (1 << e) * k * STEP);
+    }
+}
+// the twiddled butterflies of a stage (the other 11 twiddles of a radix-16
+// butterfly composed as stage_compute does)
+template <int R, int DIR, int E>
+__device__ __forceinline__ void stage_butterflies(float2* v, const float2 (&p)[E / R][4]) {
+#pragma unroll
+    for (int b = 0; b < E / R; b++) {
+#pragma unroll
+        for (int r = 1; r < R; r++) {
+            float2 w = make_float2(1.f, 0.f);
+            bool first = true;
+#pragma unroll
+            for (int e = 3; e >= 0; e--)
+                if (r & (1 << e)) {
+                    w = first ? p[b][e] : cmul(w, p[b][e]);
+                    first = false;
+                }
+            v[b * R + r] = cmul(v[b * R + r], w);
+        }
+        dftR<R, DIR>(v + b * R);
+        if constexpr (E > 16) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// Exchange after stage S and stage S + 1.  The next stage's twiddles are loaded
+// before the exchange, whose barriers the compiler moves no load over, so that
+// their latency runs beside it.
+template <int N, int DIR, int C, int S, bool TAB>
+__device__ __forceinline__ void exchange_stage(float2* v, float2* lds, int t, int c, const float2* __restrict__ tw) {
+    using P = Plan<N>;
+    constexpr int PS = xpad<N, DIR, C, S>(), R = P::radix(S + 1, DIR);
+    float2 p[16 / R][4];
+    stage_twiddles<N, R, P::ns(S + 1, DIR), DIR, 16, S + 1, TAB>(p, t, tw);
+    __syncthreads();
+    stage_store<N, P::radix(S, DIR), P::ns(S, DIR), C, 16, PS>(v, lds, t, c);
+    __syncthreads();
+    stage_load<N, R, C, 16, PS>(v, lds, t, c);
+    stage_butterflies<R, DIR, 16>(v, p);
 }
 
 // Full transform on registers.  All threads of the workgroup must call it
@@ -341,27 +349,9 @@ template <int N, int DIR, int C, bool TAB = false>
 __device__ __forceinline__ void fft_regs(float2* v, float2* lds, int t, int c, const float2* __restrict__ tw) {
     using P = Plan<N>;
     stage_compute<N, P::radix(0, DIR), P::ns(0, DIR), DIR>(v, t, tw);
-    if constexpr (P::S > 1) {
-        __syncthreads();
-        stage_store<N, P::radix(0, DIR), P::ns(0, DIR), C, 16, xpad<N, DIR, C, 0>()>(v, lds, t, c);
-        __syncthreads();
-        stage_load<N, P::radix(1, DIR), C, 16, xpad<N, DIR, C, 0>()>(v, lds, t, c);
-        stage_compute_sel<N, P::radix(1, DIR), P::ns(1, DIR), DIR, 16, 1, TAB>(v, t, tw);
-    }
-    if constexpr (P::S > 2) {
-        __syncthreads();
-        stage_store<N, P::radix(1, DIR), P::ns(1, DIR), C, 16, xpad<N, DIR, C, 1>()>(v, lds, t, c);
-        __syncthreads();
-        stage_load<N, P::radix(2, DIR), C, 16, xpad<N, DIR, C, 1>()>(v, lds, t, c);
-        stage_compute_sel<N, P::radix(2, DIR), P::ns(2, DIR), DIR, 16, 2, TAB>(v, t, tw);
-    }
-    if constexpr (P::S > 3) {
-        __syncthreads();
-        stage_store<N, P::radix(2, DIR), P::ns(2, DIR), C, 16, xpad<N, DIR, C, 2>()>(v, lds, t, c);
-        __syncthreads();
-        stage_load<N, P::radix(3, DIR), C, 16, xpad<N, DIR, C, 2>()>(v, lds, t, c);
-        stage_compute_sel<N, P::radix(3, DIR), P::ns(3, DIR), DIR, 16, 3, TAB>(v, t, tw);
-    }
+    if constexpr (P::S > 1) exchange_stage<N, DIR, C, 0, TAB>(v, lds, t, c, tw);
+    if constexpr (P::S > 2) exchange_stage<N, DIR, C, 1, TAB>(v, lds, t, c, tw);
+    if constexpr (P::S > 3) exchange_stage<N, DIR, C, 2, TAB>(v, lds, t, c, tw);
 }
 
 // index held by register slot q = b*R + r in the layout of a stage of radix R
@@ -410,24 +400,26 @@ __device__ __forceinline__ void exchange_split(float2* v, float* lds, int t, int
     stage_load_part<N, P::radix(S + 1, DIR), C, E, 1, PS>(v, lds, t, c);
 }
 
+template <int N, int DIR, int C, int E, int S, bool TAB>
+__device__ __forceinline__ void exchange_split_stage(float2* v, float* lds, int t, int c,
+                                                     const float2* __restrict__ tw) {
+    using P = Plan<N>;
+    constexpr int R = P::radix(S + 1, DIR);
+    float2 p[E / R][4];
+    stage_twiddles<N, R, P::ns(S + 1, DIR), DIR, E, S + 1, TAB>(p, t, tw);
+    exchange_split<N, DIR, C, E, S>(v, lds, t, c);
+    stage_butterflies<R, DIR, E>(v, p);
+}
+
 // Full transform on registers, E elements per thread, exchanges through a
 // float LDS region of C interleaved transforms (C * Plan<N>::LDS floats).
 template <int N, int DIR, int C, int E, bool TAB = false>
 __device__ __forceinline__ void fft_regs_split(float2* v, float* lds, int t, int c, const float2* __restrict__ tw) {
     using P = Plan<N>;
     stage_compute<N, P::radix(0, DIR), P::ns(0, DIR), DIR, E>(v, t, tw);
-    if constexpr (P::S > 1) {
-        exchange_split<N, DIR, C, E, 0>(v, lds, t, c);
-        stage_compute_sel<N, P::radix(1, DIR), P::ns(1, DIR), DIR, E, 1, TAB>(v, t, tw);
-    }
-    if constexpr (P::S > 2) {
-        exchange_split<N, DIR, C, E, 1>(v, lds, t, c);
-        stage_compute_sel<N, P::radix(2, DIR), P::ns(2, DIR), DIR, E, 2, TAB>(v, t, tw);
-    }
-    if constexpr (P::S > 3) {
-        exchange_split<N, DIR, C, E, 2>(v, lds, t, c);
-        stage_compute_sel<N, P::radix(3, DIR), P::ns(3, DIR), DIR, E, 3, TAB>(v, t, tw);
-    }
+    if constexpr (P::S > 1) exchange_split_stage<N, DIR, C, E, 0, TAB>(v, lds, t, c, tw);
+    if constexpr (P::S > 2) exchange_split_stage<N, DIR, C, E, 1, TAB>(v, lds, t, c, tw);
+    if constexpr (P::S > 3) exchange_split_stage<N, DIR, C, E, 2, TAB>(v, lds, t, c, tw);
 }
 
 }  // namespace atsim

@@ -888,7 +888,7 @@ long atsim_superlayers(const double* alt, const double* cn2, long L, double bin,
 struct Group {
     int lfirst, lcount;  // layers [lfirst, lfirst + lcount)
     double dz;           // propagation distance before this group (0 for the top group)
-    int slot0 = 0;       // first phase plane of its layers (groups applied by column passes)
+    int slot0 = 0;       // first phase plane of its layers
 };
 
 struct atsim_sim {
@@ -933,9 +933,11 @@ struct atsim_sim {
     double* ch = nullptr;
     unsigned* cmax = nullptr;  // [F] largest first-round count of each block-rule field (in bsum's allocation)
     int* flist_dev = nullptr;
-    // sampled phase planes of the layers whose screens column passes apply
-    // (one pass per gap): [nslots][D][N][N] FP64 quarter turns
+    // sampled phase planes of the layers whose screens the passes between two
+    // gaps apply (one pass per gap; row_planes false: only the column passes):
+    // [nslots][D][N][N] FP64 quarter turns
     double* vq = nullptr;
+    bool row_planes = false;
     int* slot_layer_dev = nullptr;
     int nslots = 0;
     int nblockfields = 0;
@@ -1251,17 +1253,28 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
         for (long w = 0; w < s->W; w++)
             if (s->unwrap[w] != 0 && s->amplitude) flist.push_back((int)(dd * s->W + w));
     s->nblockfields = (int)flist.size();
-    // one pass per gap: column pass k (odd, 1 <= k < G) applies group k
+    // one pass per gap: pass k (1 <= k < G; columns for odd k) applies group k
+    // from its layers' phase planes.  Without the memory for every group's planes
+    // only the column passes have them and the row passes sample the layers.
     std::vector<int> slot_layer;
-    if (s->propagate && col_screen_supported(s->N) && G >= 2) {
-        for (long k = 1; k < G; k += 2) {
+    auto make_slots = [&](long step) {
+        slot_layer.clear();
+        for (long k = 1; k < G; k += step) {
             s->groups[k].slot0 = (int)slot_layer.size();
             for (int q = 0; q < s->groups[k].lcount; q++) slot_layer.push_back(s->groups[k].lfirst + q);
         }
-    }
-    s->nslots = (int)slot_layer.size();
-    if (s->nslots > 0) {
-        SIMALLOC(s->vq, sizeof(double) * s->nslots * s->D * nn);
+        s->nslots = (int)slot_layer.size();
+    };
+    if (r == ATSIM_OK && s->propagate && col_screen_supported(s->N) && G >= 2) {
+        make_slots(1);
+        s->row_planes = true;
+        if (hipMalloc((void**)&s->vq, sizeof(double) * s->nslots * s->D * nn) != hipSuccess) {
+            (void)hipGetLastError();
+            s->vq = nullptr;
+            s->row_planes = false;
+            make_slots(2);
+            SIMALLOC(s->vq, sizeof(double) * s->nslots * s->D * nn);
+        }
         SIMALLOC(s->slot_layer_dev, sizeof(int) * s->nslots);
     }
     s->xs = (int)(s->Nout / 20);
@@ -1455,6 +1468,8 @@ static hipError_t launch_step(atsim_sim* s, bool fused, long step, ScreenArgs sa
                           sa.wlo, sa.wcnt);
     }
     group(k);
+    if (rows && s->row_planes)
+        return launch_row_screen(N, s->fields, (int)D, tab(k - 1), tab(k), s->tw, sa, s->vq, s->groups[k].slot0, st);
     if (rows)
         return launch_row_fresnel(N, false, s->fields, (int)D, tab(k), s->tw, sa, st, c->row_mw, tab(k - 1));
     return launch_col_screen(N, s->fields, (int)D, tab(k - 1), tab(k), s->tw, sa, s->vq, s->groups[k].slot0, st,

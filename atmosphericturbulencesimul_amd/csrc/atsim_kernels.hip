@@ -266,12 +266,6 @@ template <int N>
 struct ColCfg {
     static constexpr int C = N <= 2048 ? 8 : (N == 4096 ? 4 : 2);
 };
-// the same for the pass with a screen
-template <int N>
-struct ColScreenCfg {
-    static constexpr int C0 = N <= 1024 ? 16 : (N == 2048 ? 8 : 4);
-    static constexpr int C = C0 < N ? C0 : N;
-};
 
 // ------------------------------------------------------------------ passes
 // Rows of F fields: read from in (field f at in + f istride: the fields
@@ -412,11 +406,12 @@ k_col_screen(float2* __restrict__ data, const float2* __restrict__ tfp, const fl
     static_assert(P::first(-1) == P::last(+1), "the inverse plan must end in the forward plan's layout");
     const int c = threadIdx.x % C, t = threadIdx.x / C;
     const int nf = gridDim.y;
-    // 16 consecutive launch indices per XCD: with 8 fields, both 64-byte
-    // halves of a 128-byte line of every field and of the phase planes are
-    // read on one XCD
-    const int lin = xcd_chunk<16>(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
-    const int ct = lin / nf, fi = lin - ct * nf;
+    // adjacent column tiles (256 bytes of every row) of one field, fields next,
+    // an eighth of them to an XCD, as k_col_screen_split
+    constexpr int TG = 32 / C < N / C ? 32 / C : N / C;
+    const int lin = xcd_slab(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
+    const int h = lin % TG, rest = lin / TG;
+    const int fi = rest % nf, ct = (rest / nf) * TG + h;
     const int nw = sa.wcnt > 0 ? sa.wcnt : sa.W;
     const int d = fi / nw, w = (sa.wcnt > 0 ? sa.wlo : 0) + (fi - d * nw);
     const int f = d * sa.W + w;
@@ -430,13 +425,13 @@ k_col_screen(float2* __restrict__ data, const float2* __restrict__ tfp, const fl
     float2 v[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) v[q] = buf_load2(fr, lo, (reg_index<N, RI>(0, q) * N) * 8);
-    fft_regs<N, -1, C>(v, lds, t, c, tw);
+    fft_regs<N, -1, C, true>(v, lds, t, c, tw);
     {
         const auto hr = buf_rsrc(tfp + (size_t)w * N, (uint32_t)N * 8);
 #pragma unroll
         for (int q = 0; q < 16; q++) v[q] = cmul(v[q], buf_load2(hr, (uint32_t)t * 8, reg_index<N, RL>(0, q) * 8));
     }
-    fft_regs<N, +1, C>(v, lds, t, c, tw);
+    fft_regs<N, +1, C, true>(v, lds, t, c, tw);
     if (sa.lcount > 0) {
         double ph[16];
 #pragma unroll
@@ -453,13 +448,13 @@ k_col_screen(float2* __restrict__ data, const float2* __restrict__ tfp, const fl
     // the second factor's twiddle and LDS indices are recomputed, not kept
     // live through the screen from the first factor
     const int t2 = opaque(t), c2 = opaque(c);
-    fft_regs<N, -1, C>(v, lds, t2, c2, tw);
+    fft_regs<N, -1, C, true>(v, lds, t2, c2, tw);
     {
         const auto hr = buf_rsrc(tfc + (size_t)w * N, (uint32_t)N * 8);
 #pragma unroll
         for (int q = 0; q < 16; q++) v[q] = cmul(v[q], buf_load2(hr, (uint32_t)t2 * 8, reg_index<N, RL>(0, q) * 8));
     }
-    fft_regs<N, +1, C>(v, lds, t2, c2, tw);
+    fft_regs<N, +1, C, true>(v, lds, t2, c2, tw);
 #pragma unroll
     for (int q = 0; q < 16; q++) buf_store2(v[q], fr, lo, (reg_index<N, RI>(0, q) * N) * 8);
 }
@@ -486,7 +481,7 @@ k_col_screen_split(float2* __restrict__ data, const float2* __restrict__ tfp, co
     // time (2048^2 x 8 fields: 262-265 us and 1.20-1.22 x the algorithmic
     // bytes, against 266 us and 1.27 x with single tiles and 285 us with
     // 16-index chunks)
-    constexpr int TG = 4;
+    constexpr int TG = 32 / C;
     static_assert((N / C) % TG == 0, "column tiles come in groups of 4");
     const int lin = xcd_slab(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
     const int h = lin % TG, rest = lin / TG;
@@ -704,6 +699,88 @@ k_row_fresnel(float2* __restrict__ data, const float2* __restrict__ tf, const fl
     }
 }
 
+// Row pass around a layer group, the x counterpart of k_col_screen: x factor tfp
+// of the gap before the group, the group's phase from the layers' planes (made
+// once per frame by the sweep that makes the column passes'), x factor tfc of the
+// gap after it.  Bound: VALU issue, as far as the exchanges leave waves to issue
+// from: a workgroup is MW (row, wavelength) pairs, one wave up to 1024 (no wave
+// waits for another) and two rows at 2048, where k_row_fresnel, which samples the
+// layers for 8192 / N wavelengths at a time, has 8 waves at every barrier and 70 KB
+// of LDS.  Frames: 2048^2 x 8 2 381 -> 2 326 us (2 335 with one row, 2 366 with
+// four), 1024^2 x 5 319 -> 301 (306 with two rows), 512^2 x 128 2 111 -> 2 050 (2 083
+// with two waves).
+template <int N, int MW>
+__global__ void __launch_bounds__(MW * (N / 16)) __attribute__((amdgpu_waves_per_eu(4)))
+k_row_screen(float2* __restrict__ data, const float2* __restrict__ tfp, const float2* __restrict__ tfc,
+             const float2* __restrict__ tw, ScreenArgs sa, const double* __restrict__ vq, int slot0) {
+    using P = Plan<N>;
+    constexpr int T = P::T, RI = P::first(-1), RL = P::last(-1);
+    static_assert(RI == P::last(+1), "the inverse plan must end in the forward plan's layout");
+    __shared__ float2 lds[MW * P::LDS];
+    const int lw = threadIdx.x / T, t = threadIdx.x - lw * T;
+    const int nw = sa.wcnt > 0 ? sa.wcnt : sa.W, D = gridDim.y, d = blockIdx.y;
+    // (row, wavelength) pairs in order, the wavelengths of a row next to each
+    // other: they read its phase planes at about the same time through one L2
+    const int item = xcd_chunk<16>(blockIdx.x, gridDim.x) * MW + lw;
+    const bool active = item < N * nw;
+    const int j = min(item / nw, N - 1);
+    const int w = (sa.wcnt > 0 ? sa.wlo : 0) + item % nw;
+    float2* rowp = data + ((size_t)(d * sa.W + w) * N + j) * N;
+    float2* L = lds + lw * P::LDS;
+    float2 v[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) v[q] = rowp[reg_index<N, RI>(t, q)];
+    fft_regs<N, -1, 1, true>(v, L, t, 0, tw);
+    {
+        const float2* h = tfp + (size_t)w * N;
+#pragma unroll
+        for (int q = 0; q < 16; q++) v[q] = cmul(v[q], h[reg_index<N, RL>(t, q)]);
+    }
+    fft_regs<N, +1, 1, true>(v, L, t, 0, tw);
+    // the group's phase sum_l s_wl V_l, 8 register slots at a time
+#pragma unroll
+    for (int q0 = 0; q0 < 16; q0 += 8) {
+        double ph[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) ph[u] = 0.0;
+        for (int k = 0; k < sa.lcount; k++) {
+            const double sw = sa.s[(size_t)w * sa.L + sa.lfirst + k];
+            const double* vp = vq + (((size_t)(slot0 + k) * D + d) * N + j) * N;
+#pragma unroll
+            for (int u = 0; u < 8; u++) ph[u] = fma(sw, vp[reg_index<N, RI>(t, q0 + u)], ph[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[q0 + u] = cmul(v[q0 + u], expi_q(ph[u]));
+    }
+    const int t2 = opaque(t);  // indices recomputed, not kept live through the screen
+    fft_regs<N, -1, 1, true>(v, L, t2, 0, tw);
+    {
+        const float2* h = tfc + (size_t)w * N;
+#pragma unroll
+        for (int q = 0; q < 16; q++) v[q] = cmul(v[q], h[reg_index<N, RL>(t2, q)]);
+    }
+    fft_regs<N, +1, 1, true>(v, L, t2, 0, tw);
+    if (active) {
+#pragma unroll
+        for (int q = 0; q < 16; q++) rowp[reg_index<N, RI>(t2, q)] = v[q];
+    }
+}
+
+template <int N, int MW>
+static hipError_t row_screen_mw(float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
+                                const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st) {
+    const int nw = sa.wcnt > 0 ? sa.wcnt : sa.W;
+    dim3 grid((N * nw + MW - 1) / MW, D);
+    k_row_screen<N, MW><<<grid, MW * (N / 16), 0, st>>>(data, tfp, tf, tw, sa, vq, slot0);
+    return hipGetLastError();
+}
+template <int N>
+static hipError_t row_screen(float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
+                             const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st) {
+    constexpr int MW = N < 2048 ? 1024 / N : N == 2048 ? 2 : 1;
+    return row_screen_mw<N, MW>(data, D, tfp, tf, tw, sa, vq, slot0, st);
+}
+
 template <int N>
 static hipError_t row_fresnel_dispatch(bool gen, float2* data, int D, const float2* tf, const float2* tw,
                                        const ScreenArgs& sa, int mw, hipStream_t st, const float2* tfp) {
@@ -872,6 +949,27 @@ hipError_t launch_layer_phase(double* vq, const float* masters, const LayerSampl
     return hipGetLastError();
 }
 
+hipError_t launch_row_screen(long n, float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
+                             const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st) {
+    if (!tfp || !tf || D <= 0 || (sa.lcount > 0 && !vq)) return hipErrorInvalidValue;
+    switch (n) {
+#define X(NN) \
+    case NN: return row_screen<NN>(data, D, tfp, tf, tw, sa, vq, slot0, st);
+        X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096)
+#undef X
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <int N, int C>
+static hipError_t col_screen(float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
+                             const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st) {
+    const int nw = sa.wcnt > 0 ? sa.wcnt : sa.W;
+    dim3 grid(N / C, (unsigned)(D * nw)), block(C * (N / 16));
+    k_col_screen<N, C><<<grid, block, 0, st>>>(data, tfp, tf, tw, sa, vq, slot0);
+    return hipGetLastError();
+}
+
 template <int N>
 static hipError_t col_screen_split(float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
                                    const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st) {
@@ -885,23 +983,38 @@ hipError_t launch_col_screen(long n, float2* data, int D, const float2* tfp, con
                              const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st, int e) {
     if (!tfp || !tf || D <= 0 || (sa.lcount > 0 && !vq)) return hipErrorInvalidValue;
     const int nw = sa.wcnt > 0 ? sa.wcnt : sa.W;
-    if (e != 16 && n >= 256 && n <= 2048) {
+    const long F = (long)D * nw;
+    // 32 elements per thread: asked for, or where the field is largest (4096), or
+    // at 2048 from 2 fields on (8 fields: 2 321 us a frame against 2 365 with 16
+    // elements and 8 columns, 2 425 with 4; one field: 591 against 528)
+    const bool split = n >= 256 && e != 16 && (e == 32 || n >= 4096 || (n == 2048 && F > 1));
+    if (split) {
         switch (n) {
             case 256: return col_screen_split<256>(data, D, tfp, tf, tw, sa, vq, slot0, st);
             case 512: return col_screen_split<512>(data, D, tfp, tf, tw, sa, vq, slot0, st);
             case 1024: return col_screen_split<1024>(data, D, tfp, tf, tw, sa, vq, slot0, st);
-            default: return col_screen_split<2048>(data, D, tfp, tf, tw, sa, vq, slot0, st);
+            case 2048: return col_screen_split<2048>(data, D, tfp, tf, tw, sa, vq, slot0, st);
+            case 4096: return col_screen_split<4096>(data, D, tfp, tf, tw, sa, vq, slot0, st);
+            default: return hipErrorInvalidValue;
+        }
+    }
+    // columns per workgroup with 16 elements per thread: 8 (more, smaller
+    // workgroups than 16 for the barriers), and 4 where 8 leave CUs without a
+    // workgroup or, at 1024, give a CU no more than two of its 8-wave ones.  Frames,
+    // with 32 elements / 8 / 4 columns: 256^2 x 256 fields 868 / 818 / 914 us,
+    // x 1 163 / 128 / 128; 512^2 x 32 568 / 478 / 495, x 1 240 / 175 / 166; 1024^2 x
+    // 32 2 152 / 2 110 / 2 213, x 8 594 / 536 / 522, x 1 303 / 249 / 236.
+    const bool few = n / 8 * F < 256 || (n == 1024 && n / 8 * F <= 512);
+#define X(NN, CC)                                                                                     \
+    case NN: return col_screen<NN, CC>(data, D, tfp, tf, tw, sa, vq, slot0, st);
+    if (few) {
+        switch (n) {
+            X(256, 4) X(512, 4) X(1024, 4)
+            default: break;
         }
     }
     switch (n) {
-#define X(NN)                                                                                         \
-    case NN: {                                                                                        \
-        constexpr int C = ColScreenCfg<NN>::C;                                                        \
-        dim3 grid(NN / C, (unsigned)(D * nw)), block(C * (NN / 16));                                  \
-        k_col_screen<NN, C><<<grid, block, 0, st>>>(data, tfp, tf, tw, sa, vq, slot0);                \
-        return hipGetLastError();                                                                     \
-    }
-        X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096)
+        X(16, 16) X(32, 16) X(64, 16) X(128, 8) X(256, 8) X(512, 8) X(1024, 8) X(2048, 8) X(4096, 4)
 #undef X
         default: return hipErrorInvalidValue;
     }

@@ -29,11 +29,14 @@ hipError_t launch_row_fresnel(long n, bool gen, float2* data, int D, const float
 // group, the group's screen phase (layers sa.lfirst .. + sa.lcount, their
 // sampled phases in planes slot0 .. of vq), y factor tf of the gap after it;
 // every field of the wavelength range of sa (tables + w n).  n <= 4096.
-// e: elements per thread (0 = default: 32 with float exchanges for
-// 256 <= n <= 2048, else 16; 16 forces 16).  tw as for launch_row_fresnel
-// (the 32-element passes read the per-stage tables).
+// e: elements per thread (0 = by size and fields, 16 or 32 forced where built).
+// tw as for launch_row_fresnel (with the per-stage tables).
 hipError_t launch_col_screen(long n, float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
                              const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st, int e = 0);
+// The row pass around a layer group whose phases are in planes, as
+// launch_col_screen along x.
+hipError_t launch_row_screen(long n, float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
+                             const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st);
 // Sampled phase planes (FP64 quarter turns) of layers slot_layer[0 ..
 // nslots) for every direction: vq[((slot D + d) n + j) n + i].
 hipError_t launch_layer_phase(double* vq, const float* masters, const LayerSample* ls, const int* slot_layer,

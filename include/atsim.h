@@ -60,8 +60,8 @@ int atsim_copy_async(atsim_ctx *ctx, int slot, void *dst, const void *src, size_
 int atsim_copy_wait(atsim_ctx *ctx, int slot);
 int atsim_stream_wait_copy(atsim_ctx *ctx, int slot);
 /* Launch-shape tuning of this context (0 restores the built-in default):
- *   "row_mw"  wavelength fields per row-pass workgroup (1..8; default
- *             8192 / n, at most 8: two workgroups per CU)
+ *   "row_mw"  wavelength fields per workgroup of the row passes that sample
+ *             the layers or apply none (1..8; default 8192 / n, at most 8)
  *   "col_c"   columns per column-pass workgroup (2, 4, 8, 16)
  *   "col_e"   elements per thread of the column Fresnel pass (16, or 32:
  *             8 columns per workgroup exchanging through half the LDS).
@@ -81,11 +81,12 @@ int atsim_stream_wait_copy(atsim_ctx *ctx, int slot);
  *             screen and the x (y) factor of the gap after it (n <= 4096,
  *             at least 2 gaps; the screens of the column passes' layers are
  *             sampled once per frame and direction into FP64 planes of
- *             n^2 x 8 bytes each); 2: a row pass (screen, x factor) and a
+ *             n^2 x 8 bytes each, those of the row passes between two gaps
+ *             too where the memory allows); 2: a row pass (screen, x factor) and a
  *             column pass (y factor) per gap
  *   "col2_e"  elements per thread of the column passes that apply a screen
  *             (16, or 32: 8 columns per workgroup exchanging through half
- *             the LDS, the default for 256 <= n <= 2048)
+ *             the LDS, for 256 <= n <= 4096; default by size and fields)
  *   "graph"   1: atsim_sim_frame replays a HIP graph of the frame's kernels,
  *             captured at the second frame (and again when the output
  *             pointers change, or at the second frame after a tuning

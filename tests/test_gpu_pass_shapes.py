@@ -1,0 +1,56 @@
+"""GPU checks of the frame's passes at every shape the dispatch picks: grid
+sizes from 16 to 4096, few and many fields, layer groups of one and several
+layers, against the same frame with a row and a column pass per gap (other
+kernels, each checked against the oracle elsewhere).
+
+Tolerance: 3 gaps of 4 FP32 transforms of at most 12 radix-2 levels in each
+arrangement; with a rounding of 6e-8 a level, adding as random errors do,
+2 x sqrt(3 x 4 x 12) x 6e-8 = 1.5e-6 relative L2, and 5e-6 leaves a margin for
+the factors and exponentials."""
+import numpy as np
+import pytest
+
+from tests.conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def _frame(ctx, N, W, D, factored, **tuning):
+    from atmosphericturbulencesimul_amd.api import Simulation
+    L = 6
+    alt = np.array([0.0, 4000.0, 8000.0, 12000.0])
+    sli = np.array([0, 0, 1, 2, 2, 3])  # groups of 2, 1, 2 and 1 layers
+    lam = np.linspace(0.6e-6, 2.0e-6, W)
+    sc = np.array([[0.5e-6 / m * (1.0 if factored else 1.0 + 1e-3 * l * w) for l in range(L)]
+                   for w, m in enumerate(lam)])
+    x0 = np.array([[10.3 + 3.7 * d + l for l in range(L)] for d in range(D)])
+    keys = {k: ctx.get_tuning(k) for k in tuning}
+    for k, v in tuning.items():
+        ctx.set_tuning(k, v)
+    M = max(N, 256)
+    s = Simulation(ctx, N, N, M, alt, sli, lam, sc, [1] * W, x0, x0[:, ::-1], np.linspace(100.0, 900.0, L),
+                   np.linspace(-500.0, 700.0, L), 0.02, 0.001)
+    s.synth_masters(7, 400.0, 1.0)
+    s.normalize_masters(6.0, np.array([0.4, 0.2, 0.15, 0.1, 0.1, 0.05]))
+    s.frame()
+    pha, amp = s.frame()
+    out = (amp * torch.exp(1j * pha.double())).cpu().numpy()
+    s.close()
+    for k, v in keys.items():
+        ctx.set_tuning(k, v)
+    return out
+
+
+@pytest.mark.parametrize("N,W,D", [(16, 1, 1), (16, 5, 3), (32, 3, 1), (64, 1, 1), (64, 8, 2), (128, 3, 1),
+                                   (128, 8, 16), (256, 1, 1), (256, 5, 4), (512, 1, 1), (512, 8, 1), (512, 3, 5),
+                                   (1024, 1, 1), (1024, 5, 1), (1024, 7, 2), (2048, 1, 1), (2048, 3, 1),
+                                   (4096, 1, 1)])
+@pytest.mark.parametrize("factored", [True, False])
+def test_one_pass_per_gap(ctx, N, W, D, factored):
+    print(f"pass shapes N={N} W={W} D={D} factored={factored}", flush=True)
+    want = _frame(ctx, N, W, D, factored, gap_passes=2, streams=1)
+    got = _frame(ctx, N, W, D, factored)
+    assert rel_l2(got, want) < 5e-6
+    for e in (16, 32):
+        assert rel_l2(_frame(ctx, N, W, D, factored, col2_e=e), want) < 5e-6

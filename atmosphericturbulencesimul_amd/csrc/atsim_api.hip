@@ -937,7 +937,7 @@ struct atsim_sim {
     // gaps apply (one pass per gap; row_planes false: only the column passes):
     // [nslots][D][N][N] FP64 quarter turns
     double* vq = nullptr;
-    bool row_planes = false;
+    bool row_planes = false, gen_planes = false;
     int* slot_layer_dev = nullptr;
     int nslots = 0;
     int nblockfields = 0;
@@ -1253,13 +1253,15 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
         for (long w = 0; w < s->W; w++)
             if (s->unwrap[w] != 0 && s->amplitude) flist.push_back((int)(dd * s->W + w));
     s->nblockfields = (int)flist.size();
-    // one pass per gap: pass k (1 <= k < G; columns for odd k) applies group k
+    // one pass per gap: pass k (0 <= k < G; columns for odd k) applies group k
     // from its layers' phase planes.  Without the memory for every group's planes
     // only the column passes have them and the row passes sample the layers.
     std::vector<int> slot_layer;
     auto make_slots = [&](long step) {
         slot_layer.clear();
-        for (long k = 1; k < G; k += step) {
+        // one wavelength (one chain of passes, after the planes): group 0's too
+        s->gen_planes = step == 1 && s->W == 1;
+        for (long k = s->gen_planes ? 0 : 1; k < G; k += step) {
             s->groups[k].slot0 = (int)slot_layer.size();
             for (int q = 0; q < s->groups[k].lcount; q++) slot_layer.push_back(s->groups[k].lfirst + q);
         }
@@ -1438,7 +1440,8 @@ static int step_kind(bool fused, long step, long G) {
 }
 
 // one step of the chain for the wavelength range of sa (wcnt 0: all)
-static hipError_t launch_step(atsim_sim* s, bool fused, long step, ScreenArgs sa, hipStream_t st) {
+static hipError_t launch_step(atsim_sim* s, bool fused, long step, ScreenArgs sa, hipStream_t st,
+                              bool planes_first = false) {
     atsim_ctx* c = s->ctx;
     const long G = (long)s->groups.size() - 1, W = s->W, N = s->N, D = s->D;
     auto tab = [&](long g) { return (const float2*)(s->tf + (size_t)g * W * N); };
@@ -1458,12 +1461,18 @@ static hipError_t launch_step(atsim_sim* s, bool fused, long step, ScreenArgs sa
     const bool rows = k % 2 == 0;
     if (k == 0) {
         group(0);
+        // with one chain the planes are ready before the first pass; beside it
+        // (several wavelength sets) it samples its layers
+        if (s->gen_planes && planes_first)
+            return launch_row_screen(N, s->fields, (int)D, nullptr, tab(0), s->tw, sa, s->vq, s->groups[0].slot0, st);
         return launch_row_fresnel(N, true, s->fields, (int)D, tab(0), s->tw, sa, st, c->row_mw);
     }
     if (k == G) {
         sa.lfirst = 0;
         sa.lcount = 0;
-        if (rows) return launch_row_fresnel(N, false, s->fields, (int)D, tab(G - 1), s->tw, sa, st, c->row_mw);
+        if (rows)
+            return launch_row(N, OP_FRESNEL, 0, s->fields, N * N, s->fields, nfields, tab(G - 1), (int)W, s->tw, st,
+                              sa.wlo, sa.wcnt);
         return launch_col(N, OP_FRESNEL, 0, s->fields, nfields, tab(G - 1), (int)W, s->tw, st, c->col_c, c->col_e,
                           sa.wlo, sa.wcnt);
     }
@@ -1613,7 +1622,7 @@ static int enqueue_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field
             }
             for (long step = 0; step < nsteps; step++) {
                 long pr = prof_begin(s, step_kind(fused, step, G));
-                HIPCHK(c, launch_step(s, fused, step, sa, ms));
+                HIPCHK(c, launch_step(s, fused, step, sa, ms, true));
                 prof_end(s, pr);
             }
         }

@@ -255,7 +255,7 @@ __device__ __forceinline__ void stage_tail(float* S, int stride, const float* __
 template <int N>
 struct RowCfg {
     static constexpr int T = N / 16;
-    static constexpr int ROWS0 = 256 / T > 0 ? 256 / T : 1;
+    static constexpr int ROWS0 = 64 / T > 0 ? 64 / T : 1;  // one wave, or one row
     static constexpr int ROWS = ROWS0 < N ? ROWS0 : N;
     static constexpr int THREADS = ROWS * T;
 };
@@ -273,7 +273,7 @@ struct ColCfg {
 template <int N, int OP, int DIR>
 __global__ void __launch_bounds__(RowCfg<N>::THREADS)
 k_row(const float2* in, long istride, float2* out, const float2* __restrict__ tf, int W,
-      const float2* __restrict__ tw) {
+      const float2* __restrict__ tw, int wlo, int wcnt) {
     using P = Plan<N>;
     constexpr int T = P::T, ROWS = RowCfg<N>::ROWS;
     constexpr int RI = (OP == OP_FRESNEL) ? P::first(-1) : P::first(DIR);
@@ -281,7 +281,8 @@ k_row(const float2* in, long istride, float2* out, const float2* __restrict__ tf
     __shared__ float2 lds[ROWS * P::LDS];
     const int lr = threadIdx.x / T, t = threadIdx.x - lr * T;
     const int row = blockIdx.x * ROWS + lr;
-    const int f = blockIdx.y;
+    // all fields, or wavelengths wlo .. of every direction
+    const int f = wcnt > 0 ? ((int)blockIdx.y / wcnt) * W + wlo + (int)blockIdx.y % wcnt : (int)blockIdx.y;
     const float2* ip = in + f * istride + (size_t)row * N;
     float2 v[16];
 #pragma unroll
@@ -709,7 +710,9 @@ k_row_fresnel(float2* __restrict__ data, const float2* __restrict__ tf, const fl
 // of LDS.  Frames: 2048^2 x 8 2 381 -> 2 326 us (2 335 with one row, 2 366 with
 // four), 1024^2 x 5 319 -> 301 (306 with two rows), 512^2 x 128 2 111 -> 2 050 (2 083
 // with two waves).
-template <int N, int MW>
+// GEN: the first pass of a frame whose planes are ready (no factor before the
+// group; the incoming field is 1).
+template <int N, int MW, bool GEN>
 __global__ void __launch_bounds__(MW * (N / 16)) __attribute__((amdgpu_waves_per_eu(4)))
 k_row_screen(float2* __restrict__ data, const float2* __restrict__ tfp, const float2* __restrict__ tfc,
              const float2* __restrict__ tw, ScreenArgs sa, const double* __restrict__ vq, int slot0) {
@@ -728,15 +731,15 @@ k_row_screen(float2* __restrict__ data, const float2* __restrict__ tfp, const fl
     float2* rowp = data + ((size_t)(d * sa.W + w) * N + j) * N;
     float2* L = lds + lw * P::LDS;
     float2 v[16];
+    if constexpr (!GEN) {
 #pragma unroll
-    for (int q = 0; q < 16; q++) v[q] = rowp[reg_index<N, RI>(t, q)];
-    fft_regs<N, -1, 1, true>(v, L, t, 0, tw);
-    {
+        for (int q = 0; q < 16; q++) v[q] = rowp[reg_index<N, RI>(t, q)];
+        fft_regs<N, -1, 1, true>(v, L, t, 0, tw);
         const float2* h = tfp + (size_t)w * N;
 #pragma unroll
         for (int q = 0; q < 16; q++) v[q] = cmul(v[q], h[reg_index<N, RL>(t, q)]);
+        fft_regs<N, +1, 1, true>(v, L, t, 0, tw);
     }
-    fft_regs<N, +1, 1, true>(v, L, t, 0, tw);
     // the group's phase sum_l s_wl V_l, 8 register slots at a time
 #pragma unroll
     for (int q0 = 0; q0 < 16; q0 += 8) {
@@ -750,7 +753,7 @@ k_row_screen(float2* __restrict__ data, const float2* __restrict__ tfp, const fl
             for (int u = 0; u < 8; u++) ph[u] = fma(sw, vp[reg_index<N, RI>(t, q0 + u)], ph[u]);
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[q0 + u] = cmul(v[q0 + u], expi_q(ph[u]));
+        for (int u = 0; u < 8; u++) v[q0 + u] = GEN ? expi_q(ph[u]) : cmul(v[q0 + u], expi_q(ph[u]));
     }
     const int t2 = opaque(t);  // indices recomputed, not kept live through the screen
     fft_regs<N, -1, 1, true>(v, L, t2, 0, tw);
@@ -771,7 +774,8 @@ static hipError_t row_screen_mw(float2* data, int D, const float2* tfp, const fl
                                 const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st) {
     const int nw = sa.wcnt > 0 ? sa.wcnt : sa.W;
     dim3 grid((N * nw + MW - 1) / MW, D);
-    k_row_screen<N, MW><<<grid, MW * (N / 16), 0, st>>>(data, tfp, tf, tw, sa, vq, slot0);
+    if (tfp) k_row_screen<N, MW, false><<<grid, MW * (N / 16), 0, st>>>(data, tfp, tf, tw, sa, vq, slot0);
+    else k_row_screen<N, MW, true><<<grid, MW * (N / 16), 0, st>>>(data, nullptr, tf, tw, sa, vq, slot0);
     return hipGetLastError();
 }
 template <int N>
@@ -808,11 +812,11 @@ static hipError_t row_fresnel_dispatch(bool gen, float2* data, int D, const floa
 
 template <int N>
 static hipError_t row_dispatch(int op, int dir, const float2* in, long istride, float2* out, long F, const float2* tf,
-                               int W, const float2* tw, hipStream_t st) {
+                               int W, const float2* tw, int wlo, int wcnt, hipStream_t st) {
     dim3 grid(N / RowCfg<N>::ROWS, (unsigned)F), block(RowCfg<N>::THREADS);
-    if (op == OP_FRESNEL) k_row<N, OP_FRESNEL, 0><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw);
-    else if (dir < 0) k_row<N, OP_FFT, -1><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw);
-    else k_row<N, OP_FFT, +1><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw);
+    if (op == OP_FRESNEL) k_row<N, OP_FRESNEL, 0><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw, wlo, wcnt);
+    else if (dir < 0) k_row<N, OP_FFT, -1><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw, 0, 0);
+    else k_row<N, OP_FFT, +1><<<grid, block, 0, st>>>(in, istride, out, tf, W, tw, 0, 0);
     return hipGetLastError();
 }
 
@@ -864,6 +868,11 @@ static hipError_t col_dispatch(int op, int dir, float2* data, long F, const floa
         // 4 fields of 4096^2: 684 against 792 us; 8192^2: 966 against 1 038)
         if (c <= 0) return col_split_launch<N, N == 4096 ? 8 : 4>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
     }
+    if constexpr (N == 2048) {
+        // two workgroups a CU instead of one (forward and backward transform of 4
+        // images: 327 us with the copies, against 344)
+        if (c <= 0 && e != 16 && F > 1) return col_split_launch<N, 8>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
+    }
     // 4 columns where 8 leave CUs without a workgroup (one field of 1024^2: 37
     // against 39 us a call, 512^2: 31 against 32)
     if (c <= 0) c = (ColCfg<N>::C == 8 && N / 8 * F < 256) ? 4 : ColCfg<N>::C;
@@ -881,10 +890,10 @@ bool supported_n(long n) { return n >= 16 && n <= 8192 && (n & (n - 1)) == 0; }
 #define ATSIM_FOR_EACH_N(X) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192)
 
 hipError_t launch_row(long n, int op, int dir, const float2* in, long istride, float2* out, long F, const float2* tf,
-                      int W, const float2* tw, hipStream_t st) {
+                      int W, const float2* tw, hipStream_t st, int wlo, int wcnt) {
     switch (n) {
 #define X(NN) \
-    case NN: return row_dispatch<NN>(op, dir, in, istride, out, F, tf, W, tw, st);
+    case NN: return row_dispatch<NN>(op, dir, in, istride, out, F, tf, W, tw, wlo, wcnt, st);
         ATSIM_FOR_EACH_N(X)
 #undef X
         default: return hipErrorInvalidValue;
@@ -951,7 +960,7 @@ hipError_t launch_layer_phase(double* vq, const float* masters, const LayerSampl
 
 hipError_t launch_row_screen(long n, float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
                              const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st) {
-    if (!tfp || !tf || D <= 0 || (sa.lcount > 0 && !vq)) return hipErrorInvalidValue;
+    if (!tf || D <= 0 || (sa.lcount > 0 && !vq)) return hipErrorInvalidValue;
     switch (n) {
 #define X(NN) \
     case NN: return row_screen<NN>(data, D, tfp, tf, tw, sa, vq, slot0, st);

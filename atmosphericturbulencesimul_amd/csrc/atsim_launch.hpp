@@ -13,9 +13,10 @@ bool supported_n(long n);
 
 // Row pass over F fields of n x n, from in (field f at in + f istride; istride
 // 0: one field for all) to out (may be in): op OP_FRESNEL = FFT_x, x h(kx)
-// (table tf + (f % W) n), IFFT_x; OP_FFT = one transform of sign dir.
+// (table tf + (f % W) n), IFFT_x; OP_FFT = one transform of sign dir.  wcnt > 0
+// (Fresnel): F = D * wcnt fields, wavelengths wlo .. of each direction.
 hipError_t launch_row(long n, int op, int dir, const float2* in, long istride, float2* out, long F, const float2* tf,
-                      int W, const float2* tw, hipStream_t st);
+                      int W, const float2* tw, hipStream_t st, int wlo = 0, int wcnt = 0);
 // Fresnel x pass of every (direction, wavelength) field with the screen
 // phase of the layer group sa.lfirst .. + sa.lcount (sampled once per pixel
 // and direction); gen: the incoming field is 1.  Tables tf + w n.
@@ -34,7 +35,7 @@ hipError_t launch_row_fresnel(long n, bool gen, float2* data, int D, const float
 hipError_t launch_col_screen(long n, float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
                              const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st, int e = 0);
 // The row pass around a layer group whose phases are in planes, as
-// launch_col_screen along x.
+// launch_col_screen along x; tfp null: the first pass (the incoming field is 1).
 hipError_t launch_row_screen(long n, float2* data, int D, const float2* tfp, const float2* tf, const float2* tw,
                              const ScreenArgs& sa, const double* vq, int slot0, hipStream_t st);
 // Sampled phase planes (FP64 quarter turns) of layers slot_layer[0 ..

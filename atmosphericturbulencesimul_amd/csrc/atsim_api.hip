@@ -939,7 +939,11 @@ struct atsim_sim {
     double* vq = nullptr;
     bool row_planes = false, gen_planes = false;
     int* slot_layer_dev = nullptr;
-    int nslots = 0;
+    // nslots planes, the first pass_slots of them for the passes; the others (with
+    // layer_slot_dev [L], the plane of each layer) for the extraction of
+    // multipliers that do not factor
+    int nslots = 0, pass_slots = 0;
+    int* layer_slot_dev = nullptr;
     int nblockfields = 0;
     int xs = 0;
     // per-frame output statistics (atsim_sim_stats_enable): partial sums and
@@ -1090,6 +1094,7 @@ static void sim_free(atsim_sim* s) {
     hipFree(s->flist_dev);
     hipFree(s->vq);
     hipFree(s->slot_layer_dev);
+    hipFree(s->layer_slot_dev);
     hipFree(s->st_part);
     hipFree(s->st_out);
     for (auto e : s->ev_pool) (void)hipEventDestroy(e);
@@ -1256,7 +1261,20 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
     // one pass per gap: pass k (0 <= k < G; columns for odd k) applies group k
     // from its layers' phase planes.  Without the memory for every group's planes
     // only the column passes have them and the row passes sample the layers.
-    std::vector<int> slot_layer;
+    std::vector<int> slot_layer, layer_slot;
+    // multipliers that do not factor: a plane of every layer, those of the top and
+    // the last group after the others, for the extraction
+    auto make_extra = [&] {
+        s->pass_slots = s->nslots;
+        layer_slot.assign((size_t)s->L, -1);
+        for (size_t q = 0; q < slot_layer.size(); q++) layer_slot[slot_layer[q]] = (int)q;
+        for (long l = 0; l < s->L; l++)
+            if (layer_slot[l] < 0) {
+                layer_slot[l] = (int)slot_layer.size();
+                slot_layer.push_back((int)l);
+            }
+        s->nslots = (int)slot_layer.size();
+    };
     auto make_slots = [&](long step) {
         slot_layer.clear();
         // one wavelength (one chain of passes, after the planes): group 0's too
@@ -1270,14 +1288,18 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
     if (r == ATSIM_OK && s->propagate && col_screen_supported(s->N) && G >= 2) {
         make_slots(1);
         s->row_planes = true;
+        if (!s->factored) make_extra();
         if (hipMalloc((void**)&s->vq, sizeof(double) * s->nslots * s->D * nn) != hipSuccess) {
             (void)hipGetLastError();
             s->vq = nullptr;
             s->row_planes = false;
+            layer_slot.clear();
             make_slots(2);
             SIMALLOC(s->vq, sizeof(double) * s->nslots * s->D * nn);
         }
         SIMALLOC(s->slot_layer_dev, sizeof(int) * s->nslots);
+        if (!layer_slot.empty()) SIMALLOC(s->layer_slot_dev, sizeof(int) * s->L);
+        else s->pass_slots = s->nslots;
     }
     s->xs = (int)(s->Nout / 20);
     if (s->nblockfields > 0) {
@@ -1320,6 +1342,8 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
             (s->nblockfields > 0 &&
              (copy_on_stream(c, s->flist_dev, flist.data(), sizeof(int) * flist.size()) != hipSuccess ||
               copy_on_stream(c, s->bstart, bstart.data(), sizeof(int) * bstart.size()) != hipSuccess)) ||
+            (s->layer_slot_dev &&
+             copy_on_stream(c, s->layer_slot_dev, layer_slot.data(), sizeof(int) * layer_slot.size()) != hipSuccess) ||
             (s->nslots > 0 &&
              copy_on_stream(c, s->slot_layer_dev, slot_layer.data(), sizeof(int) * slot_layer.size()) != hipSuccess))
             r = fail(c, ATSIM_EHIP, "sim: parameter upload failed");
@@ -1540,6 +1564,13 @@ static int enqueue_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field
     // passes on the second set's stream (or before the extraction on one)
     const bool planes = s->factored && c->extract_planes == 1;
     const bool full = d_field != nullptr;
+    // other multipliers: the extraction reads the layers' planes (one set of
+    // them: not when the next frame's passes run beside it)
+    const bool layers = !s->factored && c->extract_planes == 1 && fused && s->layer_slot_dev && part == FRAME_ALL;
+    if (layers) {
+        a.lv = s->vq;
+        a.lslot = s->layer_slot_dev;
+    }
     if (planes) {
         a.geo_a = s->geo_a;
         a.geo_b = s->geo_b;
@@ -1559,8 +1590,11 @@ static int enqueue_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field
         rsrc = RemainderSource{s->fields, a.vr, a.vl, s->geo_a, (int)s->N, (int)W, (int)(s->N - s->Nout) / 2,
                                a.amplitude && a.last_count > 0};
     }
-    auto phase = [&](hipStream_t st) {
-        return launch_layer_phase(s->vq, s->masters, s->ls_dev, s->slot_layer_dev, s->nslots, s->N, M, L, D, st);
+    // the planes that the passes read, and those that only the extraction reads
+    auto phase = [&](hipStream_t st, bool extra) {
+        const int s0 = extra ? s->pass_slots : 0, n = extra ? s->nslots - s->pass_slots : s->pass_slots;
+        return launch_layer_phase(s->vq + (size_t)s0 * D * s->N * s->N, s->masters, s->ls_dev, s->slot_layer_dev + s0,
+                                  n, s->N, M, L, D, st);
     };
     if (part & FRAME_PASSES) {
         if (s->propagate && nsets >= 2 && !s->prof) {
@@ -1583,8 +1617,9 @@ static int enqueue_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field
                 geometry_done = true;
             } else {
                 if (fused) {
-                    HIPCHK(c, phase(s->xs_stream[0]));
+                    HIPCHK(c, phase(s->xs_stream[0], false));
                     HIPCHK(c, hipEventRecord(s->ev_phase, s->xs_stream[0]));
+                    if (layers) HIPCHK(c, phase(s->xs_stream[0], true));
                 }
                 if (planes) {
                     HIPCHK(c, launch_extract_geometry(a, full, s->xs_stream[0], nullptr, nullptr, 0, zp, zn));
@@ -1617,7 +1652,8 @@ static int enqueue_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field
                 geometry_done = true;
             } else if (fused) {
                 long pp = prof_begin(s, PROF_PHASE);
-                HIPCHK(c, phase(ms));
+                HIPCHK(c, phase(ms, false));
+                if (layers) HIPCHK(c, phase(ms, true));
                 prof_end(s, pp);
             }
             for (long step = 0; step < nsteps; step++) {

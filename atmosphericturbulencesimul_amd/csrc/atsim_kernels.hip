@@ -1389,6 +1389,13 @@ __device__ __forceinline__ void planes_phase(double a, double vr, double vl, dou
     pl = a * vl;
     phi = fma(a, vr, pl);
 }
+// The same from the layers' phase planes (quarter turns): the sums of s_wl V_l
+// over the layers before the last group (other) and over it (last).
+__device__ __forceinline__ void layers_phase(double other, double last, double& phi, double& pl) {
+#pragma clang fp contract(off)
+    pl = last * 1.57079632679489661923;
+    phi = (other + last) * 1.57079632679489661923;
+}
 // arg of the field rotated by the last group's screen, not yet in (-pi, pi]
 __device__ __forceinline__ double rotated_arg(float2 E, double rot) {
 #pragma clang fp contract(off)
@@ -1432,7 +1439,10 @@ __device__ __forceinline__ float wave_inclusive_sum(float x) {
 // and the screen of the last layer group, applied here after the last
 // Fresnel gap.
 //
-// MODE 0 does all of that.  When the phase multipliers factor as
+// MODE 0 does all of that.  MODE 1 reads the pixel's samples from the layers'
+// phase planes, made beside the first pass, when every layer has one and the
+// multipliers do not factor (1024^2, 7 layers, 5 wavelengths: 42 us against 62).  When
+// the phase multipliers factor as
 // s_wl = a_w b_l, the sums need the layers only through two planes per
 // direction, Vr = sum b_l v_l over the layers before the last group and Vl
 // over the last group: k_geo_planes writes them, and MODE 2 reads them
@@ -1446,7 +1456,7 @@ constexpr int EXT_LC = 5;              // layers staged per LDS fill
 constexpr int EXT_BC = 8;              // block columns a tile row can touch (blocks are >= 20 pixels wide)
 template <bool FULL, int MODE>
 __global__ void __launch_bounds__(EXT_T) k_extract(ExtractArgs a) {
-    static_assert(MODE == 0 || MODE == 2, "sampling or planes");
+    static_assert(MODE == 0 || MODE == 1 || MODE == 2, "sampling, layer planes or summed planes");
     constexpr bool SAMPLE = MODE == 0;
     __shared__ float S[EXT_LC][EXT_SR][EXT_SW];   // staged master rows
     __shared__ double H[EXT_LC][EXT_SR][EXT_W];   // their x-filtered values
@@ -1511,11 +1521,12 @@ __global__ void __launch_bounds__(EXT_T) k_extract(ExtractArgs a) {
             ysq[k] = mod_m(p.y0 + jf0 - 1, M);
             xsq[k] = mod_m(p.x0 + xfirst - 1, M);
         }
+    }
+    if (MODE != 2)
         for (int k = threadIdx.x; k < 8 * L; k += EXT_T) {
             const int w = k / L, l = k - w * L;
             ss[l][w] = w < Wc ? a.all.s[(w_begin + w) * L + l] : 0.0;
         }
-    }
     {
         if (threadIdx.x < 8) um[threadIdx.x] = threadIdx.x < Wc ? a.unwrap_mode[w_begin + threadIdx.x] : 0;
         for (int k = threadIdx.x; k < 2 * 8 * 2 * EXT_BC; k += EXT_T) (&bs[0][0][0][0])[k] = 0.0;
@@ -1538,6 +1549,31 @@ __global__ void __launch_bounds__(EXT_T) k_extract(ExtractArgs a) {
         const double vr = a.vr[gi], vl = a.vl[gi];
 #pragma unroll
         for (int w = 0; w < 8; w++) planes_phase(w < Wc ? a.geo_a[w_begin + w] : 0.0, vr, vl, PHI[w], PL[w]);
+    }
+    if (MODE == 1) {
+        // layers lo .. hi - 1 are the last group's; 4 planes' loads in flight
+        // (clamped addresses: a load under a lane's condition is waited for)
+        const size_t gc = ((size_t)d * a.N + min(jf, a.N - 1)) * a.N + min(ifl, a.N - 1);
+        auto sum = [&](int l0, int l1, double(&acc)[8]) {
+            for (int l = l0; l < l1; l += 4) {
+                double V[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    V[u] = a.lv[(size_t)a.lslot[min(l + u, l1 - 1)] * a.D * a.N * a.N + gc];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (l + u >= l1) break;
+                    const double* sl = ss[l + u];
+#pragma unroll
+                    for (int w = 0; w < 8; w++) acc[w] = fma(sl[w], V[u], acc[w]);
+                }
+            }
+        };
+        sum(0, a.last_first, PHI);
+        sum(a.last_first + a.last_count, L, PHI);
+        sum(a.last_first, a.last_first + a.last_count, PL);
+#pragma unroll
+        for (int w = 0; w < 8; w++) layers_phase(PHI[w], PL[w], PHI[w], PL[w]);
     }
     for (int l0 = 0; SAMPLE && l0 < L; l0 += EXT_LC) {
         const int nl = min(EXT_LC, L - l0);
@@ -1858,7 +1894,10 @@ hipError_t launch_extract(const ExtractArgs& a, bool full, hipStream_t st) {
     const long tiles = (long)((n + EXT_W - 1) / EXT_W) * ((n + EXT_R - 1) / EXT_R);
     if (tiles > 0x7fffffffL) return hipErrorInvalidValue;
     dim3 grid((unsigned)tiles, a.D * ((a.W + 7) / 8)), block(EXT_T);
-    if (a.vr == nullptr) {
+    if (a.vr == nullptr && a.lv != nullptr) {
+        if (full) k_extract<true, 1><<<grid, block, 0, st>>>(a);
+        else k_extract<false, 1><<<grid, block, 0, st>>>(a);
+    } else if (a.vr == nullptr) {
         if (full) k_extract<true, 0><<<grid, block, 0, st>>>(a);
         else k_extract<false, 0><<<grid, block, 0, st>>>(a);
     } else {
@@ -2163,25 +2202,42 @@ __global__ void __launch_bounds__(64) k_block_apply_sparse(float* __restrict__ p
         const int r0 = bstart[by], c0 = bstart[bx];
         const int w = bstart[bx + 1] - c0, n = (bstart[by + 1] - r0) * w;
         const double peak = bin[(size_t)f * nb + bb];
-        for (int e = lane; e < n; e += 64) {
-            const int q = e / w, jj = r0 + q, ii = c0 + (e - q * w);
-            const size_t o = ((size_t)f * Nout + jj) * Nout + ii;
-            float rf;
-            if (rs.fields) {
-                // the extraction's remainder again, from the final field and
-                // the geometric phase's planes at the full-grid pixel
-                const int dd = f / rs.W, jf = jj + rs.o, ifl = ii + rs.o;
-                const size_t gi = ((size_t)dd * rs.N + jf) * rs.N + ifl;
-                double phi, pl, r;
-                planes_phase(rs.geo_a[f - dd * rs.W], rs.vr[gi], rs.vl[gi], phi, pl);
-                const float2 E = rs.fields[((size_t)f * rs.N + jf) * rs.N + ifl];
-                block_turns(phi, rotated_arg(E, rs.rot ? pl : 0.0), r);
-                rf = (float)r;
-            } else {
-                rf = dres[o];
+        // 4 pixels of a lane at a time, their loads together (clamped to the
+        // block's last pixel; a block of 20 x 20 is two rounds instead of seven)
+        for (int e0 = lane; e0 < n; e0 += 256) {
+            size_t o[4];
+            float rf[4];
+            double vr[4], vl[4];
+            float2 E[4];
+            const int dd = f / max(rs.W, 1);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int e = min(e0 + u * 64, n - 1), q = e / w, jj = r0 + q, ii = c0 + (e - q * w);
+                o[u] = ((size_t)f * Nout + jj) * Nout + ii;
+                if (rs.fields) {
+                    // the extraction's remainder again, from the final field and
+                    // the geometric phase's planes at the full-grid pixel
+                    const int jf = jj + rs.o, ifl = ii + rs.o;
+                    const size_t gi = ((size_t)dd * rs.N + jf) * rs.N + ifl;
+                    vr[u] = rs.vr[gi];
+                    vl[u] = rs.vl[gi];
+                    E[u] = rs.fields[((size_t)f * rs.N + jf) * rs.N + ifl];
+                } else {
+                    rf[u] = dres[o[u]];
+                }
             }
-            const double cnt = apply_count(rf, peak);
-            if (cnt != 0.0) pha[o] = (float)fma(2.0 * M_PI, cnt, (double)pha[o]);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                if (e0 + u * 64 >= n) continue;
+                if (rs.fields) {
+                    double phi, pl, r;
+                    planes_phase(rs.geo_a[f - dd * rs.W], vr[u], vl[u], phi, pl);
+                    block_turns(phi, rotated_arg(E[u], rs.rot ? pl : 0.0), r);
+                    rf[u] = (float)r;
+                }
+                const double cnt = apply_count(rf[u], peak);
+                if (cnt != 0.0) pha[o[u]] = (float)fma(2.0 * M_PI, cnt, (double)pha[o[u]]);
+            }
         }
     }
 }

@@ -55,6 +55,10 @@ struct ExtractArgs {
     const double* geo_b;     // [L]
     double* vr;
     double* vl;
+    // the layers' phase planes (FP64 quarter turns, layer l at plane lslot[l] of
+    // [slots][D][N][N]) when every layer has one; lv null: not used
+    const double* lv;
+    const int* lslot;        // [L]
     int w_begin;             // first field of this chunk of <= 8 wavelengths
 };
 

@@ -98,7 +98,10 @@ int atsim_stream_wait_copy(atsim_ctx *ctx, int slot);
  *             layers before the last group and over the last group, 16 n^2
  *             bytes) by a kernel that runs beside the Fresnel passes, and
  *             the extraction reads them (PHI_w = a_w Vr + a_w Vl) instead of
- *             sampling every layer; 2: the extraction samples the layers
+ *             sampling every layer; with other multipliers and one pass per
+ *             gap every layer is sampled into a phase plane and the extraction
+ *             reads those (where the memory allows, and not in pipelined
+ *             frames); 2: the extraction samples the layers
  *   "block_apply" 1 (default): the final update of the block unwrap rule
  *             visits only the blocks where a count can be non-zero (from
  *             each block's largest |r|, kept by the extraction); 2: every

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-def _frame(ctx, N, W, D, factored, **tuning):
+def _frame(ctx, N, W, D, factored, field=False, Nout=None, **tuning):
     from atmosphericturbulencesimul_amd.api import Simulation
     L = 6
     alt = np.array([0.0, 4000.0, 8000.0, 12000.0])
@@ -29,13 +29,16 @@ def _frame(ctx, N, W, D, factored, **tuning):
     for k, v in tuning.items():
         ctx.set_tuning(k, v)
     M = max(N, 256)
-    s = Simulation(ctx, N, N, M, alt, sli, lam, sc, [1] * W, x0, x0[:, ::-1], np.linspace(100.0, 900.0, L),
+    s = Simulation(ctx, N, Nout or N, M, alt, sli, lam, sc, [1] * W, x0, x0[:, ::-1], np.linspace(100.0, 900.0, L),
                    np.linspace(-500.0, 700.0, L), 0.02, 0.001)
     s.synth_masters(7, 400.0, 1.0)
     s.normalize_masters(6.0, np.array([0.4, 0.2, 0.15, 0.1, 0.1, 0.05]))
     s.frame()
-    pha, amp = s.frame()
+    f = torch.empty((D, W, N, N), dtype=torch.complex64, device="cuda") if field else None
+    pha, amp = s.frame(f)
     out = (amp * torch.exp(1j * pha.double())).cpu().numpy()
+    if field:
+        out = np.concatenate([out.ravel(), f.cpu().numpy().ravel()])
     s.close()
     for k, v in keys.items():
         ctx.set_tuning(k, v)
@@ -54,3 +57,15 @@ def test_one_pass_per_gap(ctx, N, W, D, factored):
     assert rel_l2(got, want) < 5e-6
     for e in (16, 32):
         assert rel_l2(_frame(ctx, N, W, D, factored, col2_e=e), want) < 5e-6
+
+
+# cropped outputs and the full field, from summed planes and from layer planes;
+# one wavelength per chunk edge (9 fields are two chunks of the extraction)
+@pytest.mark.parametrize("N,Nout,W", [(64, 41, 9), (256, 250, 3), (512, 333, 1)])
+@pytest.mark.parametrize("factored", [True, False])
+@pytest.mark.parametrize("field", [False, True])
+def test_outputs(ctx, N, Nout, W, factored, field):
+    want = _frame(ctx, N, W, 2, factored, field, Nout, gap_passes=2, streams=1, extract_planes=2)
+    assert rel_l2(_frame(ctx, N, W, 2, factored, field, Nout), want) < 5e-6
+    assert rel_l2(_frame(ctx, N, W, 2, factored, field, Nout, extract_planes=2), want) < 5e-6
+    assert rel_l2(_frame(ctx, N, W, 2, factored, field, Nout, pipeline=1), want) < 5e-6

@@ -121,12 +121,17 @@ _SIGS = {
     "atsim_nn_gelu_bwd": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long]),
     "atsim_nn_bias_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_int]),
     "atsim_nn_mse": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.POINTER(C.c_double)]),
+    "atsim_nn_mse_begin": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long]),
+    "atsim_nn_mse_end": (C.c_int, [C.c_void_p, C.c_long, C.POINTER(C.c_double)]),
     "atsim_nn_reduce_batches": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_int]),
     "atsim_nn_make_pairs": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long,
                                       C.c_long, C.c_long, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_double,
                                       C.c_double, C.c_double, C.c_double]),
     "atsim_nn_unpack": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_double,
                                   C.c_double, C.c_double, C.c_void_p, C.c_void_p]),
+    "atsim_nn_adam_many": (C.c_int, [C.c_void_p, C.c_long, C.POINTER(C.c_void_p), C.POINTER(C.c_void_p),
+                                     C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.POINTER(C.c_long), C.c_float,
+                                     C.c_float, C.c_float, C.c_float, C.c_long]),
     "atsim_nn_adam": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_float,
                                 C.c_float, C.c_float, C.c_float, C.c_long]),
 }

@@ -69,6 +69,8 @@ struct atsim_ctx {
     // work space of calls on the context stream (ctx_scratch), kept between them
     void* scratch = nullptr;
     size_t scratch_cap = 0;
+    double* nn_loss_host = nullptr;  // pinned: partial sums of a loss read later
+    hipEvent_t nn_loss_ev = nullptr;
     double* nn_part = nullptr;  // 256 partial sums of the network's loss reduction
     float* nn_bias = nullptr;   // per-chunk partial sums of bias gradients
     size_t nn_bias_cap = 0;
@@ -295,6 +297,8 @@ void atsim_ctx_destroy(atsim_ctx* c) {
     if (c->fresnel_tab) hipFree(c->fresnel_tab);
     if (c->scratch) hipFree(c->scratch);
     if (c->nn_part) hipFree(c->nn_part);
+    if (c->nn_loss_host) hipHostFree(c->nn_loss_host);
+    if (c->nn_loss_ev) hipEventDestroy(c->nn_loss_ev);
     if (c->nn_bias) hipFree(c->nn_bias);
     if (c->copy_stream) {
         hipStreamSynchronize(c->copy_stream);
@@ -2328,6 +2332,31 @@ int atsim_nn_mse(atsim_ctx* c, const float* pred, const float* target, float* gr
     return ATSIM_OK;
 }
 
+int atsim_nn_mse_begin(atsim_ctx* c, const float* pred, const float* target, float* grad, long n) {
+    if (!c || !pred || !target || n <= 0) return ATSIM_EINVAL;
+    if (!c->nn_loss_host) {
+        if (hipHostMalloc((void**)&c->nn_loss_host, sizeof(double) * 256, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            c->nn_loss_host = nullptr;
+            return fail(c, ATSIM_ENOMEM, "mse: cannot allocate pinned host memory");
+        }
+    }
+    if (!c->nn_loss_ev) HIPCHK(c, hipEventCreateWithFlags(&c->nn_loss_ev, hipEventDisableTiming));
+    if (int r = atsim_nn_mse(c, pred, target, grad, n, nullptr)) return r;
+    HIPCHK(c, hipMemcpyAsync(c->nn_loss_host, c->nn_part, sizeof(double) * 256, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipEventRecord(c->nn_loss_ev, c->stream));
+    return ATSIM_OK;
+}
+
+int atsim_nn_mse_end(atsim_ctx* c, long n, double* loss) {
+    if (!c || !loss || n <= 0 || !c->nn_loss_ev) return ATSIM_EINVAL;
+    HIPCHK(c, hipEventSynchronize(c->nn_loss_ev));
+    double t = 0.0;
+    for (int b = 0; b < 256; b++) t += c->nn_loss_host[b];
+    *loss = t / (double)n;
+    return ATSIM_OK;
+}
+
 int atsim_nn_reduce_batches(atsim_ctx* c, const float* part, float* out, long nb, long n, int accumulate) {
     if (!c || !part || !out || nb <= 0 || n <= 0) return ATSIM_EINVAL;
     c->work_gen++;
@@ -2350,6 +2379,28 @@ int atsim_nn_unpack(atsim_ctx* c, const float* y, const float* x, long L, long S
     if (!c || !y || !x || !amp || !pha || L <= 0 || S <= 0 || P <= 0) return ATSIM_EINVAL;
     c->work_gen++;
     HIPCHK(c, launch_nn_unpack(y, x, L, S, P, xs, cs, ps, amp, pha, c->stream));
+    return ATSIM_OK;
+}
+
+int atsim_nn_adam_many(atsim_ctx* c, long count, float* const* w, const float* const* g, float* const* m,
+                       float* const* v, const long* n, float lr, float b1, float b2, float eps, long step) {
+    if (!c || count < 0 || !w || !g || !m || !v || !n || step < 1) return ATSIM_EINVAL;
+    for (long k = 0; k < count; k++)
+        if (!w[k] || !g[k] || !m[k] || !v[k] || n[k] < 0) return fail(c, ATSIM_EINVAL, "adam: tensor %ld is invalid", k);
+    c->work_gen++;
+    const float c1 = (float)(1.0 - pow((double)b1, (double)step)), c2 = (float)(1.0 - pow((double)b2, (double)step));
+    for (long k0 = 0; k0 < count; k0 += ADAM_MOST) {
+        AdamTensors t{};
+        const int cnt = (int)std::min<long>(ADAM_MOST, count - k0);
+        for (int k = 0; k < cnt; k++) {
+            t.w[k] = w[k0 + k];
+            t.g[k] = g[k0 + k];
+            t.m[k] = m[k0 + k];
+            t.v[k] = v[k0 + k];
+            t.n[k] = n[k0 + k];
+        }
+        HIPCHK(c, launch_adam_many(t, cnt, lr, b1, b2, eps, c1, c2, c->stream));
+    }
     return ATSIM_OK;
 }
 

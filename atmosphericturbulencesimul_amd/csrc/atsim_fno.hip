@@ -665,8 +665,7 @@ __device__ __forceinline__ void operand8c(const float* __restrict__ X, long sk, 
 // workgroup as MFMA operands.  Bound: HBM (the image read once).  1 600 images
 // of 256^2, 16 modes (419 MB): 113 us, 3.7 TB/s, where the x product (292 us)
 // and the four real y products (49 us each) took 489 us.
-constexpr int DFT_T = 512;
-template <int NT>
+template <int NT, int DFT_T>
 __global__ void __launch_bounds__(DFT_T) k_dft2(const float* __restrict__ h, const float* __restrict__ F, long sfk,
                                                 long sfn, const float* __restrict__ Gre,
                                                 const float* __restrict__ Gim, float* __restrict__ out, long images,
@@ -874,42 +873,66 @@ __global__ void __launch_bounds__(256) k_mix_grad(const float* __restrict__ dO, 
 }
 
 // Weight gradient of a channel map, part[chunk][o][i] = sum over the chunk's
-// kc pixels of dy[o][q] h[i][q]: a workgroup takes one chunk, each wave one 16 x
-// 16 tile of (o, i) straight from float4 loads (both operands are contiguous
-// along the sum; the tiles of a workgroup share their rows through L1), 4 k
-// steps of loads in flight.  Order and results as k_gemm_bf16.  Bound: HBM.
-// 32 x 32 channels over 524 288 pixels: 45 us against 53 through
-// k_gemm_bf16's LDS staging.
-__global__ void __launch_bounds__(1024) k_weight_grad(const float* __restrict__ dy, const float* __restrict__ h,
-                                                      float* __restrict__ part, int Cout, int Cin, long SP, int kc) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lm = lane & 15, lk = (lane >> 4) * 8;
-    const int CT = (Cin + 15) / 16, rt = wave / CT, ct = wave % CT;
-    const float* a = dy + min(rt * 16 + lm, Cout - 1) * SP + (long)blockIdx.x * kc + lk;
-    const float* bq = h + min(ct * 16 + lm, Cin - 1) * SP + (long)blockIdx.x * kc + lk;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < kc; k0 += 128) {  // kc is a multiple of 128
-        float4 av[4][2], bv[4][2];
+// kc pixels of dy[o][q] h[i][q]: one wave takes a chunk and every 16 x 16 tile of
+// (o, i), so that each value is loaded and rounded once, straight from float4 loads
+// (both operands are contiguous along the sum), the loads of UN k steps in flight.
+// Order and results as k_gemm_bf16.  Bound: HBM.  32 x 32 channels over 524 288
+// pixels (134 MB): 34 us, 64 x 32 76 us, against 45 and 92 with one tile a wave
+// and 53 through k_gemm_bf16's LDS staging.
+template <int RT, int CT>
+__global__ void __launch_bounds__(64) k_weight_grad(const float* __restrict__ dy, const float* __restrict__ h,
+                                                    float* __restrict__ part, int Cout, int Cin, long SP, int kc) {
+    constexpr int UN = RT + CT <= 4 ? 4 : RT + CT <= 6 ? 2 : 1;
+    const int lane = threadIdx.x, lm = lane & 15, lk = (lane >> 4) * 8;
+    const float *a[RT], *b[CT];
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+    for (int r = 0; r < RT; r++) a[r] = dy + min(r * 16 + lm, Cout - 1) * SP + (long)blockIdx.x * kc + lk;
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                av[q][u] = *reinterpret_cast<const float4*>(a + k0 + q * 32 + u * 4);
-                bv[q][u] = *reinterpret_cast<const float4*>(bq + k0 + q * 32 + u * 4);
+    for (int q = 0; q < CT; q++) b[q] = h + min(q * 16 + lm, Cin - 1) * SP + (long)blockIdx.x * kc + lk;
+    f32x4 acc[RT][CT];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int q = 0; q < CT; q++) acc[r][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float4 v[UN][RT + CT][2];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int s = 0; s < UN; s++)
+#pragma unroll
+            for (int t = 0; t < RT + CT; t++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    v[s][t][u] = *reinterpret_cast<const float4*>((t < RT ? a[t < RT ? t : 0] : b[t < RT ? 0 : t - RT]) +
+                                                                  k0 + s * 32 + u * 4);
+    };
+    fetch(0);
+    for (int k0 = 0; k0 < kc; k0 += 32 * UN) {  // kc is a multiple of 128
+        bf16x8 o[UN][RT + CT];
+#pragma unroll
+        for (int s = 0; s < UN; s++)
+#pragma unroll
+            for (int t = 0; t < RT + CT; t++) {
+                const float x[8] = {v[s][t][0].x, v[s][t][0].y, v[s][t][0].z, v[s][t][0].w,
+                                    v[s][t][1].x, v[s][t][1].y, v[s][t][1].z, v[s][t][1].w};
+                o[s][t] = to_bf16x8(x);
             }
+        fetch(min(k0 + 32 * UN, kc - 32 * UN));  // the next steps' loads beside the products
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float x[8] = {av[q][0].x, av[q][0].y, av[q][0].z, av[q][0].w,
-                                av[q][1].x, av[q][1].y, av[q][1].z, av[q][1].w};
-            const float y[8] = {bv[q][0].x, bv[q][0].y, bv[q][0].z, bv[q][0].w,
-                                bv[q][1].x, bv[q][1].y, bv[q][1].z, bv[q][1].w};
-            acc = MFMA16(to_bf16x8(x), to_bf16x8(y), acc);
-        }
+        for (int s = 0; s < UN; s++)
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int q = 0; q < CT; q++) acc[r][q] = MFMA16(o[s][r], o[s][RT + q], acc[r][q]);
     }
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int o = rt * 16 + (lane >> 4) * 4 + q, i = ct * 16 + lm;
-        if (o < Cout && i < Cin) part[((long)blockIdx.x * Cout + o) * Cin + i] = acc[q];
-    }
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int oo = r * 16 + (lane >> 4) * 4 + q, i = c * 16 + lm;
+                if (oo < Cout && i < Cin) part[((long)blockIdx.x * Cout + oo) * Cin + i] = acc[r][c][q];
+            }
 }
 
 // at most 64 channels each way, chunks of a multiple of 128 pixels, 16-byte
@@ -920,9 +943,17 @@ bool weight_grad_supported(const float* dy, const float* h, long Cout, long Cin,
 }
 hipError_t launch_weight_grad(const float* dy, const float* h, float* part, int Cout, int Cin, long SP, int kc,
                               hipStream_t st) {
-    const int waves = ((Cout + 15) / 16) * ((Cin + 15) / 16);
-    k_weight_grad<<<(unsigned)(SP / kc), 64 * waves, 0, st>>>(dy, h, part, Cout, Cin, SP, kc);
-    return hipGetLastError();
+    const unsigned grid = (unsigned)(SP / kc);
+    switch ((Cout + 15) / 16 * 4 + (Cin + 15) / 16 - 5) {
+#define X(RT, CT)                                                                       \
+    case (RT - 1) * 4 + CT - 1:                                                         \
+        k_weight_grad<RT, CT><<<grid, 64, 0, st>>>(dy, h, part, Cout, Cin, SP, kc);     \
+        return hipGetLastError();
+        X(1, 1) X(1, 2) X(1, 3) X(1, 4) X(2, 1) X(2, 2) X(2, 3) X(2, 4)
+        X(3, 1) X(3, 2) X(3, 3) X(3, 4) X(4, 1) X(4, 2) X(4, 3) X(4, 4)
+#undef X
+        default: return hipErrorInvalidValue;
+    }
 }
 
 static size_t dft2_lds(long N, long m) {
@@ -938,17 +969,25 @@ bool spectral_supported(const float* h, const float* U, const float* B, const fl
            (((uintptr_t)B | (uintptr_t)O | (uintptr_t)R) & 7) == 0 && dft2_lds(N, m) <= 160 * 1024;
 }
 
+template <int NT, int TH>
+static hipError_t dft2_launch_t(const float* h, const float* F, long sfk, long sfn, const float* Gre, const float* Gim,
+                                float* out, long images, int N, int m, hipStream_t st) {
+    const size_t lds = dft2_lds(N, m);
+    if (lds > 64 * 1024) {
+        hipError_t e =
+            hipFuncSetAttribute((const void*)k_dft2<NT, TH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const long res = 256 * (TH == 512 && lds <= 80 * 1024 ? 2 : 1);  // resident workgroups
+    k_dft2<NT, TH><<<(unsigned)(images < res ? images : res), TH, lds, st>>>(h, F, sfk, sfn, Gre, Gim, out, images, N, m);
+    return hipGetLastError();
+}
 template <int NT>
 static hipError_t dft2_launch(const float* h, const float* F, long sfk, long sfn, const float* Gre, const float* Gim,
                               float* out, long images, int N, int m, hipStream_t st) {
-    const size_t lds = dft2_lds(N, m);
-    if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_dft2<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    const long res = 256 * (lds <= 80 * 1024 ? 2 : 1);  // resident workgroups
-    k_dft2<NT><<<(unsigned)(images < res ? images : res), DFT_T, lds, st>>>(h, F, sfk, sfn, Gre, Gim, out, images, N, m);
-    return hipGetLastError();
+    // few images: 16 waves on a CU's one image (256 of 256^2: 22 us against 25)
+    if (images <= 256) return dft2_launch_t<NT, 1024>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
+    return dft2_launch_t<NT, 512>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
 }
 hipError_t launch_dft2(const float* h, const float* F, long sfk, long sfn, const float* Gre, const float* Gim,
                        float* out, long images, int N, int m, hipStream_t st) {
@@ -1103,6 +1142,23 @@ __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float
     }
 }
 
+// The same step on up to ADAM_MOST tensors (blockIdx.y), one launch for a
+// network's parameters: most of its tensors are a few hundred values, and each
+// launch of its own costs more than they do.
+__global__ void k_adam_many(AdamTensors p, float lr, float b1, float b2, float eps, float c1, float c2) {
+    const int k = blockIdx.y;
+    float *__restrict__ w = p.w[k], *__restrict__ m = p.m[k], *__restrict__ v = p.v[k];
+    const float* __restrict__ g = p.g[k];
+    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < p.n[k]; e += (long)gridDim.x * blockDim.x) {
+        const float ge = g[e];
+        const float me = fmaf(b1, m[e] - ge, ge);
+        const float ve = fmaf(b2, v[e] - ge * ge, ge * ge);
+        m[e] = me;
+        v[e] = ve;
+        w[e] -= lr * (me / c1) / (sqrtf(ve / c2) + eps);
+    }
+}
+
 // out[i] (+)= sum_b part[b n + i]: the split-K partial products of the
 // weight gradients, summed in a fixed order (b ascending, one accumulator).
 // A workgroup takes 64 outputs: all four waves load 128 partials of each ahead
@@ -1230,6 +1286,14 @@ hipError_t launch_nn_pairs(const float* screens, const double* sc, const float* 
 hipError_t launch_nn_unpack(const float* y, const float* x, long L, long S, long P, double xs, double cs, double ps,
                             float* amp, float* pha, hipStream_t st) {
     k_nn_unpack<<<grid_for(S * P), 256, 0, st>>>(y, x, (int)L, S, P, xs, cs, ps, amp, pha);
+    return hipGetLastError();
+}
+hipError_t launch_adam_many(const AdamTensors& p, int count, float lr, float b1, float b2, float eps, float c1,
+                            float c2, hipStream_t st) {
+    long most = 1;
+    for (int k = 0; k < count; k++) most = p.n[k] > most ? p.n[k] : most;
+    const unsigned gx = grid_for(most) < 1024 ? grid_for(most) : 1024;
+    k_adam_many<<<dim3(gx, count), 256, 0, st>>>(p, lr, b1, b2, eps, c1, c2);
     return hipGetLastError();
 }
 hipError_t launch_adam(float* w, const float* g, float* m, float* v, long n, float lr, float b1, float b2, float eps,

@@ -187,6 +187,16 @@ hipError_t launch_nn_pairs(const float* screens, const double* sc, const float* 
                            hipStream_t st);
 hipError_t launch_nn_unpack(const float* y, const float* x, long L, long S, long P, double xs, double cs, double ps,
                             float* amp, float* pha, hipStream_t st);
+constexpr int ADAM_MOST = 32;
+struct AdamTensors {
+    float* w[ADAM_MOST];
+    const float* g[ADAM_MOST];
+    float* m[ADAM_MOST];
+    float* v[ADAM_MOST];
+    long n[ADAM_MOST];
+};
+hipError_t launch_adam_many(const AdamTensors& p, int count, float lr, float b1, float b2, float eps, float c1,
+                            float c2, hipStream_t st);
 hipError_t launch_adam(float* w, const float* g, float* m, float* v, long n, float lr, float b1, float b2, float eps,
                        float c1, float c2, hipStream_t st);
 

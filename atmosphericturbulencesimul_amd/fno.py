@@ -171,6 +171,17 @@ class Ops:
                                           C.byref(loss) if want_loss else None))
         return loss.value if want_loss else None
 
+    def mse_begin(self, pred, target, grad):
+        """queue the loss; mse_end waits for it alone and returns it"""
+        if target.numel() != pred.numel() or grad.numel() != pred.numel():
+            raise ValueError("mse: operand sizes differ")
+        self.ctx._chk(self.L.atsim_nn_mse_begin(self.ctx.h, _p(pred), _p(target), _p(grad), pred.numel()))
+
+    def mse_end(self, n):
+        loss = C.c_double()
+        self.ctx._chk(self.L.atsim_nn_mse_end(self.ctx.h, n, C.byref(loss)))
+        return loss.value
+
     def reduce(self, part, out, nb, n):
         if part.numel() < nb * n or out.numel() < n:
             raise ValueError("reduce: operands too small")
@@ -181,6 +192,16 @@ class Ops:
             raise ValueError("adam: operand sizes differ")
         self.ctx._chk(self.L.atsim_nn_adam(self.ctx.h, _p(w), _p(g), _p(m), _p(v), w.numel(), lr, b1, b2, eps,
                                            step))
+
+
+    def adam_many(self, tensors, lr, b1, b2, eps, step):
+        """one Adam step on every (w, g, m, v) of tensors"""
+        if any(not w.numel() == g.numel() == m.numel() == v.numel() for w, g, m, v in tensors):
+            raise ValueError("adam: operand sizes differ")
+        k = len(tensors)
+        ptrs = [(C.c_void_p * k)(*[t[q].data_ptr() for t in tensors]) for q in range(4)]
+        n = (C.c_long * k)(*[t[0].numel() for t in tensors])
+        self.ctx._chk(self.L.atsim_nn_adam_many(self.ctx.h, k, *ptrs, n, lr, b1, b2, eps, step))
 
 
 def init_params(cin, cout, width, modes, blocks, hidden, seed=0):
@@ -440,7 +461,10 @@ class FNO:
         SP = S * P
         Cw, H = self.width, self.hidden
         dy = torch.empty_like(y)
-        loss = ops.mse(y, t, dy, want_loss)
+        if want_loss:  # read after the backward pass is queued, so that it does not wait for the host
+            ops.mse_begin(y, t, dy)
+        else:
+            ops.mse(y, t, dy, False)
         self._weight_grad(dy, c["q1"], g["Q2"], self.cout, H, SP)
         ops.bias_grad(dy, g["q2b"], self.cout, SP)
         dq1 = torch.empty_like(c["q1"])
@@ -462,13 +486,13 @@ class FNO:
             dh = dhn
         self._weight_grad(dh, c["x"], g["Lw"], Cw, self.cin, SP)
         ops.bias_grad(dh, g["Lb"], Cw, SP)
-        return loss
+        return ops.mse_end(y.numel()) if want_loss else None
 
     @on_ctx_stream
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         self.step += 1
-        for k in self.param:
-            self.ops.adam(self.param[k], self.grad[k], self.adam_m[k], self.adam_v[k], lr, b1, b2, eps, self.step)
+        self.ops.adam_many([(self.param[k], self.grad[k], self.adam_m[k], self.adam_v[k]) for k in self.param], lr, b1,
+                           b2, eps, self.step)
 
     @on_ctx_stream
     def params_numpy(self):

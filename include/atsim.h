@@ -441,6 +441,11 @@ int atsim_nn_bias_grad(atsim_ctx *ctx, const float *dy, float *db, long S, long 
 /* mean squared error; grad (may be NULL) = 2 (pred - target) / n; loss (may
  * be NULL; synchronises the stream) = mean of (pred - target)^2 */
 int atsim_nn_mse(atsim_ctx *ctx, const float *pred, const float *target, float *grad, long n, double *loss);
+/* atsim_nn_mse without waiting: _begin queues the loss and its copy to the host,
+ * _end (same n) waits for that copy alone, so that work queued between the two
+ * does not wait for the host.  One loss at a time per context. */
+int atsim_nn_mse_begin(atsim_ctx *ctx, const float *pred, const float *target, float *grad, long n);
+int atsim_nn_mse_end(atsim_ctx *ctx, long n, double *loss);
 /* Pairs of the surrogate from one simulator step: screens [D][L][N*N] (from
  * atsim_sim_layer_screens), d_scoeff [L] (device, FP64) the wavelength's
  * phase multipliers; writes samples s0 .. s0+D-1 of Stot, channel-major
@@ -457,6 +462,10 @@ int atsim_nn_unpack(atsim_ctx *ctx, const float *y, const float *x, long L, long
                     double ps, float *amp, float *pha);
 /* out[i] = sum_{b < nb} part[b n + i] (added to out if accumulate) */
 int atsim_nn_reduce_batches(atsim_ctx *ctx, const float *part, float *out, long nb, long n, int accumulate);
+/* one Adam step on count parameter tensors (atsim_nn_adam of each, 32 tensors a
+ * launch); the arrays of pointers and lengths are host memory */
+int atsim_nn_adam_many(atsim_ctx *ctx, long count, float *const *w, const float *const *g, float *const *m,
+                       float *const *v, const long *n, float lr, float b1, float b2, float eps, long step);
 /* one Adam step (bias-corrected, step >= 1) on n parameters */
 int atsim_nn_adam(atsim_ctx *ctx, float *w, const float *g, float *m, float *v, long n, float lr, float b1,
                   float b2, float eps, long step);

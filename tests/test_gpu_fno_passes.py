@@ -129,3 +129,38 @@ def test_bias_grad(ctx, S, C, P):
     # half an ulp of the chunks' magnitudes
     got, want = db.cpu().numpy().astype(np.float64), dy.astype(np.float64).sum((0, 2))
     assert np.all(np.abs(got - want) <= 65 * 2.0 ** -24 * np.abs(dy).astype(np.float64).sum((0, 2)))
+
+
+# 1, 32 (one launch) and 33 tensors of sizes about a workgroup
+@pytest.mark.parametrize("count", [1, 32, 33])
+def test_adam_many_is_adam_of_each(ctx, count):
+    from atmosphericturbulencesimul_amd.fno import Ops
+    ops = Ops(ctx)
+    rng = np.random.default_rng(count)
+    sizes = [1, 255, 256, 257, 5000][:count] * (count // 5 + 1)
+    sets = [[_dev(*(rng.standard_normal(n) for _ in range(4))) for n in sizes[:count]]]
+    for t in sets[0]:
+        t[3].abs_()
+    sets.append([[x.clone() for x in t] for t in sets[0]])
+    torch.cuda.synchronize()
+    ops.adam_many([tuple(t) for t in sets[0]], 1e-3, 0.9, 0.999, 1e-8, 3)
+    for t in sets[1]:
+        ops.adam(*t, 1e-3, 0.9, 0.999, 1e-8, 3)
+    ctx.sync()
+    for a, b in zip(*sets):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("n", [1, 1000, 70000])
+def test_loss_read_later_is_the_same(ctx, n):
+    from atmosphericturbulencesimul_amd.fno import Ops
+    ops = Ops(ctx)
+    rng = np.random.default_rng(n)
+    p, t = _dev(rng.standard_normal(n), rng.standard_normal(n))
+    g, g2 = torch.empty_like(p), torch.empty_like(p)
+    torch.cuda.synchronize()
+    want = ops.mse(p, t, g)
+    ops.mse_begin(p, t, g2)
+    assert ops.mse_end(n) == want
+    ctx.sync()
+    assert torch.equal(g, g2)

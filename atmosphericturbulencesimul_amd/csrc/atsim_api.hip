@@ -2235,6 +2235,37 @@ int atsim_nn_pointwise(atsim_ctx* c, const float* W, long swm, long swk, long Co
     return ATSIM_OK;
 }
 
+int atsim_nn_map_dft(atsim_ctx* c, const float* W, long swm, long swk, long Cout, long Cin, const float* h, float* out,
+                     long nrows, long rowlen, const float* U, long K2, const float* F, long sfk, long sfx,
+                     const float* bias, float* pre, int act, const float* D, long dsk, long dsn, long m, void* T) {
+    if (!c || !W || !h || !out || !D || !T || Cout <= 0 || Cin <= 0 || nrows <= 0 || rowlen <= 0 || m <= 0)
+        return ATSIM_EINVAL;
+    if (swm < 0 || swk < 0 || act < 0 || act > 2 || (act == 2 && !pre) || (U && (!F || sfk < 0 || sfx < 0)) || dsk < 0 ||
+        dsn < 0)
+        return fail(c, ATSIM_EINVAL, "map and transform: invalid operands");
+    if (!pointwise_supported(h, out, pre, U, Cout, Cin, nrows, rowlen, K2) ||
+        !point_dft_supported(T, Cout, rowlen, m, U ? K2 : 0))
+        return fail(c, ATSIM_EUNSUPPORTED, "map and transform: %ld x %ld channels over rows of %ld, %ld modes", Cout, Cin,
+                    rowlen, m);
+    c->work_gen++;
+    HIPCHK(c, launch_pointwise(W, swm, swk, (int)Cout, (int)Cin, h, out, nrows, (int)rowlen, U, U ? (int)K2 : 0, F, sfk,
+                               sfx, bias, pre, act, c->stream, D, dsk, dsn, (int)m, T));
+    return ATSIM_OK;
+}
+
+int atsim_nn_spectral_rows(atsim_ctx* c, const void* T, const float* Gre, const float* Gim, const float* R, int adjoint,
+                           float* B, float* O, float* U, long C, long S, long N, long m) {
+    if (!c || !T || !Gre || !Gim || !R || !B || !O || !U || C <= 0 || S <= 0 || N <= 0 || m <= 0) return ATSIM_EINVAL;
+    const long images = C * S;
+    if (!spectral_supported((const float*)T, U, B, O, R, images, N, m, C, S) || !point_dft_supported(T, C, N, m, 0))
+        return fail(c, ATSIM_EUNSUPPORTED, "spectral: %ld channels, %ld samples of %ld^2, %ld modes", C, S, N, m);
+    c->work_gen++;
+    HIPCHK(c, launch_dft_y(T, Gre, Gim, B, images, (int)N, (int)m, c->stream));
+    HIPCHK(c, launch_mix(R, B, O, (int)C, (int)S, (int)(2 * m * m), adjoint != 0, c->stream));
+    HIPCHK(c, launch_idft_y(Gre, Gim, O, U, images, (int)N, (int)m, c->stream));
+    return ATSIM_OK;
+}
+
 int atsim_nn_spectral_fwd(atsim_ctx* c, const float* h, const float* F, long sfk, long sfn, const float* Gre,
                           const float* Gim, const float* R, int adjoint, float* B, float* O, float* U, long C, long S,
                           long N, long m) {

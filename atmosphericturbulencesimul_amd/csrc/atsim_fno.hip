@@ -227,6 +227,10 @@ struct PointArgs {
     const float* bias;
     float* pre;
     int act;
+    const float* D;  // table of the transform of out along x (NT > 0): D[x dsk + c dsn], dm modes
+    long dsk, dsn;
+    int dm;
+    __bf16* T;       // its result [Cout][nrows][16 NT]
 };
 
 // F [K2][rowlen] staged as MFMA operands [KU][64-pixel group][t][lane][8]
@@ -245,6 +249,24 @@ __device__ __forceinline__ void stage_xtable(__bf16* Fs, const float* __restrict
         }
         *reinterpret_cast<bf16x8*>(Fs + (size_t)e * 8) = to_bf16x8(v);
     }
+}
+// F [x][n] (x sfk + n sfn) staged as MFMA operands [k step][NT][lane][8] by TH threads
+template <int NT>
+__device__ __forceinline__ void stage_dtable(__bf16* Ds, const float* __restrict__ F, long sfk, long sfn, int N, int M2,
+                                             int TH) {
+    for (int e = threadIdx.x; e < N / 32 * NT * 64; e += TH) {
+        const int ln = e & 63, t = e >> 6, nt = t % NT, ks = t / NT;
+        const float* p = F + min(nt * 16 + (ln & 15), M2 - 1) * sfn + (long)(ks * 32 + (ln >> 4) * 8) * sfk;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = p[j * sfk];
+        *reinterpret_cast<bf16x8*>(Ds + (size_t)e * 8) = to_bf16x8(v);
+    }
+}
+// orders a wave's own LDS writes before its reads
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 // a wave's operands of an M x K matrix (element strides sm, sk)
 template <int RT, int KT>
@@ -308,17 +330,35 @@ __device__ __forceinline__ void load_channels(float4 (&hv)[KT][8], const float* 
             hv[kt][j] = *reinterpret_cast<const float4*>(h + min(kt * 32 + lk + j, C - 1) * SP + p);
 }
 
-template <int RT, int KT, int KU>
-__global__ void __launch_bounds__(256) k_pointwise(PointArgs g) {
+// waves a SIMD that the registers allow without scratch
+constexpr int point_waves(int RT, int KT, int KU) {
+    return KT == 1 ? (KU == 0 || RT <= 2 ? 3 : 2) : RT == 4 && KU == 2 ? 1 : 2;
+}
+// NT > 0: with the transform of out along x that the next spectral path begins
+// with (k_dft2's first product, 16 NT columns), so that out is not read again
+// for it.  A wave takes whole rows then; 64 pixels of all channels pass through
+// its own LDS rows as the BF16 operand of k steps of 32 in k_dft2's order, and
+// T keeps what k_dft2 keeps in LDS: the same results.  50 images of 256^2, 32
+// channels, 16 modes: 232 us + 19 us for k_dft_y, where the map alone takes 190
+// and k_dft2 114 (8 images: 60 + 8 us against 55 + 24).  Bound: VALU (tanhf) and
+// HBM about equally; channel tiles one after the other, 16 of them live at a time,
+// leave room for 3 waves a SIMD (all tiles at once: 2 waves, 264 us; the
+// next pixels loaded ahead: scratch, 254 us).
+template <int RT, int KT, int KU, int NT>
+__global__ void __launch_bounds__(256, point_waves(RT, KT, KU)) k_pointwise(PointArgs g) {
     extern __shared__ __attribute__((aligned(16))) __bf16 Fs[];  // F as MFMA operands: [KU][64-pixel group][4][lane][8]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int XS = 64 + 8;
+    __bf16* Ds = Fs + (size_t)KU * ((g.rowlen + 63) / 64) * 2048;                       // [k step][NT][lane][8]
+    __bf16* Xs = Ds + (size_t)(g.rowlen / 32) * NT * 512 + (threadIdx.x >> 6) * RT * 16 * XS;  // [channel][XS]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lm = lane & 15, lk = (lane >> 4) * 8;
     const long SP = g.nrows * g.rowlen;
     const int ngrp = (g.rowlen + 63) / 64;
     if constexpr (KU > 0) {
         stage_xtable<KU>(Fs, g.F, g.sfk, g.sfx, g.K2, g.rowlen);
-        __syncthreads();
     }
+    if constexpr (NT > 0) stage_dtable<NT>(Ds, g.D, g.dsk, g.dsn, g.rowlen, 2 * g.dm, 256);
+    if constexpr (KU > 0 || NT > 0) __syncthreads();
     bf16x8 wa[RT][KT];
     matrix_operands<RT, KT>(wa, g.W, g.swm, g.swk, g.Cout, g.Cin, lm, lk);
     float bias[RT][4];
@@ -327,58 +367,65 @@ __global__ void __launch_bounds__(256) k_pointwise(PointArgs g) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
             bias[rt][q] = g.bias ? g.bias[min(rt * 16 + (lane >> 4) * 4 + q, g.Cout - 1)] : 0.f;
-    const long units = g.nrows * ngrp;
-    for (long u = (long)blockIdx.x * 4 + wave; u < units; u += (long)gridDim.x * 4) {
-        const long r = u / ngrp;
-        const int x0 = (int)(u - r * ngrp) * 64;
-        bf16x8 ua[RT][KU > 0 ? KU : 1];
-        if constexpr (KU > 0) spectrum_operands<RT, KU>(ua, g.U, g.nrows, r, g.Cout, g.K2, lm, lk);
+    f32x4 tx[RT][NT > 0 ? NT : 1];  // the row's transform: columns 4 (l / 16) .. + 3, channel l % 16
+    bf16x8 ua[RT][KU > 0 ? KU : 1];
+    const long units = NT > 0 ? g.nrows : g.nrows * ngrp, stride = (long)gridDim.x * 4;
+    long u = (long)blockIdx.x * 4 + wave;
+    if (u >= units) return;
+    auto row_of = [&](long v) { return NT > 0 ? v : v / ngrp; };
+    auto x_of = [&](long v, int gr) { return NT > 0 ? gr * 64 : (int)(v - v / ngrp * ngrp) * 64; };
+    for (int grp = 0;;) {
+        const long r = row_of(u);
+        const int x0 = x_of(u, grp);
         const bool in = x0 + 4 * lm < g.rowlen;
         const long p = r * g.rowlen + min(x0 + 4 * lm, g.rowlen - 4);
         float4 hv[KT][8];
         load_channels<KT>(hv, g.h, SP, p, g.Cin, lk);
-        f32x4 res[RT][4];  // [row tile][pixel t]: rows 4 (l / 16) .. + 3
+        bf16x8 hb[4][KT];
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            bf16x8 hb[KT];
-            pixel_operands<KT>(hb, hv, t, g.Cin, lk);
-            bf16x8 fb[KU > 0 ? KU : 1];
-            if constexpr (KU > 0) {
+        for (int t = 0; t < 4; t++) pixel_operands<KT>(hb[t], hv, t, g.Cin, lk);
+        if (NT == 0 || grp == 0) {
+            if constexpr (KU > 0) spectrum_operands<RT, KU>(ua, g.U, g.nrows, r, g.Cout, g.K2, lm, lk);
 #pragma unroll
-                for (int ku = 0; ku < KU; ku++)
-                    fb[ku] = *reinterpret_cast<const bf16x8*>(
-                        Fs + ((size_t)((ku * ngrp + (x0 >> 6)) * 4 + t) * 64 + lane) * 8);
-            }
+            for (int i = 0; i < RT * NT; i++) tx[i / (NT > 0 ? NT : 1)][i % (NT > 0 ? NT : 1)] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        const bool last = NT == 0 || grp == ngrp - 1;
+        const long un = last ? u + stride : u;
+        const int gn = last ? 0 : grp + 1;
+        if constexpr (NT > 0) wave_fence();  // the operands of the group before are read
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
+        for (int rt = 0; rt < RT; rt++) {
+            const int c0 = rt * 16 + (lane >> 4) * 4;
+            f32x4 res[4];  // [pixel t]: channels c0 .. + 3
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[rt][kt], hb[kt], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[rt][kt], hb[t][kt], acc, 0, 0, 0);
                 if constexpr (KU > 0) {
                     f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int ku = 0; ku < KU; ku++)
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua[rt][ku], fb[ku], s, 0, 0, 0);
+                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            ua[rt][ku],
+                            *reinterpret_cast<const bf16x8*>(Fs + ((size_t)((ku * ngrp + (x0 >> 6)) * 4 + t) * 64 + lane) * 8),
+                            s, 0, 0, 0);
                     acc += s;
                 }
-                res[rt][t] = acc;
+                res[t] = acc;
             }
-        }
-        if (!in) continue;
-#pragma unroll
-        for (int rt = 0; rt < RT; rt++)
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const int c = rt * 16 + (lane >> 4) * 4 + q;
-                if (c >= g.Cout) continue;
+                const int c = c0 + q;
+                if (c >= g.Cout || !in) continue;
                 const long o = c * SP + p;
                 const float b = bias[rt][q];
                 float4 v;
-                v.x = res[rt][0][q];
-                v.y = res[rt][1][q];
-                v.z = res[rt][2][q];
-                v.w = res[rt][3][q];
+                v.x = res[0][q];
+                v.y = res[1][q];
+                v.z = res[2][q];
+                v.w = res[3][q];
                 if (g.bias) {  // (the sum of a null bias could turn -0 into 0)
                     v.x += b;
                     v.y += b;
@@ -406,17 +453,69 @@ __global__ void __launch_bounds__(256) k_pointwise(PointArgs g) {
                     *reinterpret_cast<float4*>(g.pre + o) = v;
                 }
                 *reinterpret_cast<float4*>(g.out + o) = v;
+                if constexpr (NT > 0) {
+                    const bf16x4 t = {(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
+                    *reinterpret_cast<bf16x4*>(Xs + c * XS + 4 * lm) = t;
+                }
             }
+        }
+        if constexpr (NT > 0) {
+            wave_fence();
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                if (x0 + ks * 32 >= g.rowlen) break;
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) {
+                    const bf16x8 d = *reinterpret_cast<const bf16x8*>(Ds + ((size_t)((x0 / 32 + ks) * NT + nt) * 64 + lane) * 8);
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++)
+                        tx[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            d, *reinterpret_cast<const bf16x8*>(Xs + (rt * 16 + lm) * XS + ks * 32 + lk), tx[rt][nt], 0, 0, 0);
+                }
+            }
+            if (last)
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                    for (int nt = 0; nt < NT; nt++) {
+                        const f32x4 a = tx[rt][nt];
+                        const bf16x4 t = {(__bf16)a[0], (__bf16)a[1], (__bf16)a[2], (__bf16)a[3]};
+                        if (rt * 16 + lm < g.Cout)
+                            *reinterpret_cast<bf16x4*>(g.T + ((rt * 16 + lm) * g.nrows + r) * (NT * 16) + nt * 16 +
+                                                       (lane >> 4) * 4) = t;
+                    }
+        }
+        if (un >= units) break;
+        u = un;
+        grp = gn;
     }
 }
 
+template <int RT, int KT, int KU, int NT>
+static hipError_t point_dft_launch(const PointArgs& g, hipStream_t st) {
+    const size_t lds = ((size_t)KU * ((g.rowlen + 63) / 64) * 2048 + (size_t)(g.rowlen / 32) * NT * 512 +
+                        4 * RT * 16 * (64 + 8)) * sizeof(__bf16);
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void*)k_pointwise<RT, KT, KU, NT>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    // the resident workgroups, each with the same number of rows a wave
+    const long wg = (g.nrows + 3) / 4, res = 256 * (160 * 1024 / (long)lds < 4 ? 160 * 1024 / (long)lds : 4);
+    const long turns = (wg + res - 1) / res;
+    k_pointwise<RT, KT, KU, NT><<<(unsigned)((wg + turns - 1) / turns), 256, lds, st>>>(g);
+    return hipGetLastError();
+}
 template <int RT, int KT, int KU>
 static hipError_t point_launch(const PointArgs& g, hipStream_t st) {
+    if constexpr (RT <= 2 && KU <= 1) {
+        if (g.T) return g.dm <= 8 ? point_dft_launch<RT, KT, KU, 1>(g, st) : point_dft_launch<RT, KT, KU, 2>(g, st);
+    }
     const long wg = (g.nrows * ((g.rowlen + 63) / 64) + 3) / 4;
     // as many workgroups as can be resident (each stages F once)
     const unsigned grid = (unsigned)(wg < 1024 ? (wg > 0 ? wg : 1) : 1024);
     const size_t lds = (size_t)KU * ((g.rowlen + 63) / 64) * 256 * 8 * sizeof(__bf16);
-    k_pointwise<RT, KT, KU><<<grid, 256, lds, st>>>(g);
+    k_pointwise<RT, KT, KU, 0><<<grid, 256, lds, st>>>(g);
     return hipGetLastError();
 }
 
@@ -480,10 +579,6 @@ __global__ void __launch_bounds__(256) k_tail(TailArgs g) {
     auto put4 = [&](int c, const float (&v)[4]) {
         const bf16x4 t = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
         *reinterpret_cast<bf16x4*>(&X[wave][lm][c]) = t;
-    };
-    auto wave_fence = [] {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
     };
     const long units = g.b.nrows * ngrp;
     for (long u = (long)blockIdx.x * 4 + wave; u < units; u += (long)gridDim.x * 4) {
@@ -604,18 +699,28 @@ bool pointwise_supported(const float* h, const float* out, const float* pre, con
            (!U || (rowlen <= 512 && K2 >= 4 && K2 <= 64 && K2 % 4 == 0));
 }
 
+// With the transform of out: at most 32 channels and 16 modes (more accumulators
+// and LDS rows than a wave has room for beside the map's own) over rows of a
+// multiple of 32 pixels that the tables' LDS holds.
+bool point_dft_supported(const void* T, long Cout, long rowlen, long dm, long K2) {
+    return Cout <= 32 && rowlen % 32 == 0 && rowlen <= 512 && dm >= 1 && dm <= 16 && K2 <= 32 && ((uintptr_t)T & 15) == 0;
+}
+
 hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Cin, const float* h, float* out,
                             long nrows, int rowlen, const float* U, int K2, const float* F, long sfk, long sfx,
-                            const float* bias, float* pre, int act, hipStream_t st) {
+                            const float* bias, float* pre, int act, hipStream_t st, const float* D, long dsk, long dsn,
+                            int dm, void* T) {
     if (!pointwise_supported(h, out, pre, U, Cout, Cin, nrows, rowlen, K2)) return hipErrorInvalidValue;
-    if (!U) {  // no rows to tell apart: the image as rows of 64 pixels
+    if (T && !point_dft_supported(T, Cout, rowlen, dm, K2)) return hipErrorInvalidValue;
+    if (!U && !T) {  // no rows to tell apart: the image as rows of 64 pixels
         const long SP = nrows * rowlen;
         if (SP % 64 == 0) {
             nrows = SP / 64;
             rowlen = 64;
         }
     }
-    const PointArgs g{W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U, K2, F, sfk, sfx, bias, pre, act};
+    const PointArgs g{W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U, K2, F, sfk, sfx, bias, pre, act,
+                      D, dsk, dsn, dm, (__bf16*)T};
     switch ((Cout + 15) / 16) {
         case 1: return point_kt<1>(g, st);
         case 2: return point_kt<2>(g, st);
@@ -657,6 +762,48 @@ __device__ __forceinline__ void operand8c(const float* __restrict__ X, long sk, 
 }
 #define MFMA16(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16((a), (b), (c), 0, 0, 0)
 
+// G [2m][N] staged as MFMA operands [re, im][NT][k step][lane][8] by TH threads
+template <int NT>
+__device__ __forceinline__ void stage_gtable(__bf16* Gs, const float* __restrict__ Gre, const float* __restrict__ Gim,
+                                             int N, int M2, int TH) {
+    const int KS = N / 32;
+    for (int e = threadIdx.x; e < 2 * NT * KS * 64; e += TH) {
+        const int ln = e & 63, t = e >> 6, ks = t % KS, mt = (t / KS) % NT, ri = t / (KS * NT);
+        const int r = min(mt * 16 + (ln & 15), M2 - 1), k = ks * 32 + (ln >> 4) * 8;
+        const float* p = (ri ? Gim : Gre) + (long)r * N + k;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = p[j];
+        *reinterpret_cast<bf16x8*>(Gs + (size_t)e * 8) = to_bf16x8(v);
+    }
+}
+// out[ky][kx] = sum_y G[ky][y] T[y][kx] (complex) of one image, T as columns of
+// y in LDS (Tt[2 kx + (re, im)][TS])
+template <int NT>
+__device__ __forceinline__ void ydft_tasks(const __bf16* Gs, const __bf16* Tt, float* __restrict__ out, int KS, int TS,
+                                           int m, int wave, int nwave, int lane) {
+    const int lm = lane & 15, lk = (lane >> 4) * 8, M2 = 2 * m, NX = (m + 15) / 16;
+    // one (ky tile, kx tile, re or im) per wave
+    for (int task = wave; task < NT * NX * 2; task += nwave) {
+        const int ri = task & 1, nx = (task >> 1) % NX, mt = (task >> 1) / NX;
+        f32x4 p = {0.f, 0.f, 0.f, 0.f}, s = {0.f, 0.f, 0.f, 0.f};
+        const __bf16* tr = Tt + (2 * (nx * 16 + lm) + ri) * TS + lk;        // multiplied by Gre
+        const __bf16* ti = Tt + (2 * (nx * 16 + lm) + 1 - ri) * TS + lk;    // multiplied by Gim
+        for (int ks = 0; ks < KS; ks++) {
+            const bf16x8 gr = *reinterpret_cast<const bf16x8*>(Gs + ((size_t)(mt * KS + ks) * 64 + lane) * 8);
+            const bf16x8 gi = *reinterpret_cast<const bf16x8*>(Gs + ((size_t)((NT + mt) * KS + ks) * 64 + lane) * 8);
+            p = MFMA16(gr, *reinterpret_cast<const bf16x8*>(tr + ks * 32), p);
+            s = MFMA16(gi, *reinterpret_cast<const bf16x8*>(ti + ks * 32), s);
+        }
+        const int kx = nx * 16 + lm;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int ky = mt * 16 + (lane >> 4) * 4 + q;
+            if (ky < M2 && kx < m) out[((long)ky * m + kx) * 2 + ri] = ri ? p[q] + s[q] : p[q] - s[q];
+        }
+    }
+}
+
 // Retained spectrum of real N x N images: T = h F along x (F[x sfk + c sfn],
 // 2m columns: re and im of m modes), then out[ky][kx] = sum_y G[ky][y] T[y][kx]
 // (complex) for 2m ky.  One workgroup takes one image at a time: a wave
@@ -671,23 +818,14 @@ __global__ void __launch_bounds__(DFT_T) k_dft2(const float* __restrict__ h, con
                                                 const float* __restrict__ Gim, float* __restrict__ out, long images,
                                                 int N, int m) {
     extern __shared__ __attribute__((aligned(16))) __bf16 sm[];
-    const int KS = N / 32, M2 = 2 * m, NX = (m + 15) / 16, TS = N + 8;
+    const int KS = N / 32, M2 = 2 * m, TS = N + 8;
     __bf16* Fs = sm;                                  // [KS][NT][lane][8]
     __bf16* Gs = Fs + (size_t)KS * NT * 512;          // [re, im][NT][KS][lane][8]
     __bf16* Tt = Gs + (size_t)2 * NT * KS * 512;      // [column 2 kx + (re, im)][TS]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lm = lane & 15, lk = (lane >> 4) * 8;
-    for (int e = threadIdx.x; e < KS * NT * 64; e += DFT_T) {
-        const int ln = e & 63, t = e >> 6, nt = t % NT, ks = t / NT;
-        const int n = nt * 16 + (ln & 15), k = ks * 32 + (ln >> 4) * 8;
-        bf16x8 v = operand8(F + min(n, M2 - 1) * sfn, sfk, k, N);
-        *reinterpret_cast<bf16x8*>(Fs + (size_t)e * 8) = v;
-    }
-    for (int e = threadIdx.x; e < 2 * NT * KS * 64; e += DFT_T) {
-        const int ln = e & 63, t = e >> 6, ks = t % KS, mt = (t / KS) % NT, ri = t / (KS * NT);
-        const int r = min(mt * 16 + (ln & 15), M2 - 1), k = ks * 32 + (ln >> 4) * 8;
-        *reinterpret_cast<bf16x8*>(Gs + (size_t)e * 8) = operand8((ri ? Gim : Gre) + (long)r * N, 1, k, N);
-    }
+    stage_dtable<NT>(Fs, F, sfk, sfn, N, M2, DFT_T);
+    stage_gtable<NT>(Gs, Gre, Gim, N, M2, DFT_T);
     for (long img = blockIdx.x; img < images; img += gridDim.x) {
         __syncthreads();  // the tables are staged / the previous image's T is read
         const float* hi = h + img * N * N;
@@ -723,25 +861,33 @@ __global__ void __launch_bounds__(DFT_T) k_dft2(const float* __restrict__ h, con
             }
         }
         __syncthreads();
-        // one (ky tile, kx tile, re or im) per wave
-        for (int task = wave; task < NT * NX * 2; task += DFT_T / 64) {
-            const int ri = task & 1, nx = (task >> 1) % NX, mt = (task >> 1) / NX;
-            f32x4 p = {0.f, 0.f, 0.f, 0.f}, s = {0.f, 0.f, 0.f, 0.f};
-            const __bf16* tr = Tt + (2 * (nx * 16 + lm) + ri) * TS + lk;        // multiplied by Gre
-            const __bf16* ti = Tt + (2 * (nx * 16 + lm) + 1 - ri) * TS + lk;    // multiplied by Gim
-            for (int ks = 0; ks < KS; ks++) {
-                const bf16x8 gr = *reinterpret_cast<const bf16x8*>(Gs + ((size_t)(mt * KS + ks) * 64 + lane) * 8);
-                const bf16x8 gi = *reinterpret_cast<const bf16x8*>(Gs + ((size_t)((NT + mt) * KS + ks) * 64 + lane) * 8);
-                p = MFMA16(gr, *reinterpret_cast<const bf16x8*>(tr + ks * 32), p);
-                s = MFMA16(gi, *reinterpret_cast<const bf16x8*>(ti + ks * 32), s);
-            }
-            const int kx = nx * 16 + lm;
+        ydft_tasks<NT>(Gs, Tt, out + img * M2 * m * 2, KS, TS, m, wave, DFT_T / 64, lane);
+    }
+}
+
+// The retained spectrum from T [images][N][16 NT] (BF16), the images' transform
+// along x as k_pointwise leaves it: k_dft2's second half.  Bound: HBM (T read).
+template <int NT>
+__global__ void __launch_bounds__(256) k_dft_y(const __bf16* __restrict__ T, const float* __restrict__ Gre,
+                                               const float* __restrict__ Gim, float* __restrict__ out, long images,
+                                               int N, int m) {
+    extern __shared__ __attribute__((aligned(16))) __bf16 sm[];
+    const int KS = N / 32, M2 = 2 * m, TS = N + 8;
+    __bf16* Gs = sm;
+    __bf16* Tt = Gs + (size_t)2 * NT * KS * 512;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    stage_gtable<NT>(Gs, Gre, Gim, N, M2, 256);
+    for (long img = blockIdx.x; img < images; img += gridDim.x) {
+        __syncthreads();  // the tables are staged / the previous image's T is read
+        // y on the lanes: a lane's 8 columns of one y go to 8 rows of Tt
+        for (int e = threadIdx.x; e < N * NT * 2; e += 256) {
+            const int y = e % N, c8 = e / N;
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(T + ((size_t)img * N + y) * (NT * 16) + c8 * 8);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int ky = mt * 16 + (lane >> 4) * 4 + q;
-                if (ky < M2 && kx < m) out[((img * M2 + ky) * m + kx) * 2 + ri] = ri ? p[q] + s[q] : p[q] - s[q];
-            }
+            for (int j = 0; j < 8; j++) Tt[(c8 * 8 + j) * TS + y] = v[j];
         }
+        __syncthreads();
+        ydft_tasks<NT>(Gs, Tt, out + img * M2 * m * 2, KS, TS, m, wave, 4, lane);
     }
 }
 
@@ -988,6 +1134,25 @@ static hipError_t dft2_launch(const float* h, const float* F, long sfk, long sfn
     // few images: 16 waves on a CU's one image (256 of 256^2: 22 us against 25)
     if (images <= 256) return dft2_launch_t<NT, 1024>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
     return dft2_launch_t<NT, 512>(h, F, sfk, sfn, Gre, Gim, out, images, N, m, st);
+}
+template <int NT>
+static hipError_t dft_y_launch(const __bf16* T, const float* Gre, const float* Gim, float* out, long images, int N, int m,
+                               hipStream_t st) {
+    const size_t lds = ((size_t)2 * NT * (N / 32) * 512 + (size_t)32 * (N + 8)) * sizeof(__bf16);
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void*)k_dft_y<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const long res = 256 * (160 * 1024 / (long)lds < 4 ? 160 * 1024 / (long)lds : 4);
+    const long turns = (images + res - 1) / res;  // the same number of images a workgroup
+    k_dft_y<NT><<<(unsigned)((images + turns - 1) / turns), 256, lds, st>>>(T, Gre, Gim, out, images, N, m);
+    return hipGetLastError();
+}
+hipError_t launch_dft_y(const void* T, const float* Gre, const float* Gim, float* out, long images, int N, int m,
+                        hipStream_t st) {
+    if (images <= 0) return hipSuccess;
+    return m <= 8 ? dft_y_launch<1>((const __bf16*)T, Gre, Gim, out, images, N, m, st)
+                  : dft_y_launch<2>((const __bf16*)T, Gre, Gim, out, images, N, m, st);
 }
 hipError_t launch_dft2(const float* h, const float* F, long sfk, long sfn, const float* Gre, const float* Gim,
                        float* out, long images, int N, int m, hipStream_t st) {

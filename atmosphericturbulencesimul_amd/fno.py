@@ -85,15 +85,24 @@ class Ops:
                 and (K2 == 0 or (rowlen <= 512 and K2 <= 64 and K2 % 4 == 0)))
 
     def pointwise(self, W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U=None, K2=0, F=None, sfk=0, sfx=0, bias=None,
-                  pre=None, act=0):
+                  pre=None, act=0, D=None, dsk=0, dsn=0, m=0, T=None):
         """out = act(W h [+ U F] [+ bias]) over [C][nrows][rowlen] images; act 0
-        identity, 1 GELU (pre keeps its argument), 2 times GELU'(pre)"""
+        identity, 1 GELU (pre keeps its argument), 2 times GELU'(pre).  T: also
+        the transform of out along x (table D, m modes), for spectral"""
         n = nrows * rowlen
         if (h.numel() < Cin * n or out.numel() < Cout * n or W.numel() <= (Cout - 1) * swm + (Cin - 1) * swk
                 or (bias is not None and bias.numel() < Cout) or (pre is not None and pre.numel() != out.numel())
                 or (U is not None and (U.numel() < Cout * nrows * K2
                                        or F.numel() <= (K2 - 1) * sfk + (rowlen - 1) * sfx))):
             raise ValueError(f"pointwise operands out of bounds ({Cout} x {Cin} channels, {nrows} rows of {rowlen})")
+        if T is not None:
+            if (T.numel() < Cout * nrows * 16 * ((m + 7) // 8) or T.element_size() != 2
+                    or D.numel() <= (rowlen - 1) * dsk + (2 * m - 1) * dsn):
+                raise ValueError(f"pointwise transform out of bounds ({Cout} channels, {nrows} rows, {m} modes)")
+            self.ctx._chk(self.L.atsim_nn_map_dft(self.ctx.h, _p(W), swm, swk, Cout, Cin, _p(h), _p(out), nrows, rowlen,
+                                                  _p(U), K2, _p(F), sfk, sfx, _p(bias), _p(pre), act, _p(D), dsk, dsn, m,
+                                                  _p(T)))
+            return
         self.ctx._chk(self.L.atsim_nn_pointwise(self.ctx.h, _p(W), swm, swk, Cout, Cin, _p(h), _p(out), nrows, rowlen,
                                                 _p(U), K2, _p(F), sfk, sfx, _p(bias), _p(pre), act))
 
@@ -116,13 +125,25 @@ class Ops:
         return (C_ <= 64 and N % 32 == 0 and 2 * m <= N <= 1024 and m <= 32 and lds <= 160 * 1024
                 and h.data_ptr() % 16 == 0 and R.data_ptr() % 8 == 0)
 
-    def spectral(self, h, F, sfk, sfn, Gre, Gim, R, adjoint, B, O, U, C_, S, N, m):
-        """B = G (h F), O = R B per mode (adjoint: R^H B), U = G^H O"""
+    @staticmethod
+    def rows_ok(C_, N, m):
+        """the sizes at which pointwise takes T and spectral begins from it"""
+        return C_ <= 32 and m <= 16 and N % 32 == 0 and N <= 512
+
+    def spectral(self, h, F, sfk, sfn, Gre, Gim, R, adjoint, B, O, U, C_, S, N, m, T=None):
+        """B = G (h F), O = R B per mode (adjoint: R^H B), U = G^H O; T: h F as
+        pointwise left it"""
         sp = C_ * S * 4 * m * m
         if (h.numel() < C_ * S * N * N or F.numel() <= (N - 1) * sfk + (2 * m - 1) * sfn or Gre.numel() < 2 * m * N
                 or Gim.numel() < 2 * m * N or R.numel() < 4 * m * m * C_ * C_ or B.numel() < sp or O.numel() < sp
                 or U.numel() < C_ * S * N * 2 * m):
             raise ValueError(f"spectral operands out of bounds ({C_} channels, {S} samples of {N}^2, {m} modes)")
+        if T is not None:
+            if T.numel() < C_ * S * N * 16 * ((m + 7) // 8):
+                raise ValueError(f"spectral rows out of bounds ({C_} channels, {S} samples of {N}^2, {m} modes)")
+            self.ctx._chk(self.L.atsim_nn_spectral_rows(self.ctx.h, _p(T), _p(Gre), _p(Gim), _p(R), int(adjoint), _p(B),
+                                                        _p(O), _p(U), C_, S, N, m))
+            return
         self.ctx._chk(self.L.atsim_nn_spectral_fwd(self.ctx.h, _p(h), _p(F), sfk, sfn, _p(Gre), _p(Gim), _p(R),
                                                    int(adjoint), _p(B), _p(O), _p(U), C_, S, N, m))
 
@@ -267,19 +288,33 @@ class FNO:
         self.Fx, self.Gre, self.Gim, self.Fxi = f(Fx), f(np.cos(ay)), f(-np.sin(ay)), f(Fxi)
 
     # ---------------------------------------------------------------- building blocks
-    def _pointwise(self, Wt, h, out, Cout, Cin, SP, bias=None, pre=None, gelu=False):
+    def _rows(self, out, R, Cin, S, K2, tensors, adjoint=False):
+        """The transform along x that the pass writing out is to leave for the
+        spectral path of out with R (adjoint: the backward path's table), as the
+        last arguments of Ops.pointwise, if both passes take these sizes"""
+        N, m, Cw = self.N, self.m, self.width
+        if not (self.ops.rows_ok(Cw, N, m) and self.ops.spectral_ok(Cw, N, m, out, R)
+                and self.ops.pointwise_ok(Cw, Cin, N, (out,) + tensors, K2)):
+            return {}
+        torch = _torch()
+        D = (self.Fxi, 1, N) if adjoint else (self.Fx, 2 * m, 1)
+        T = torch.empty((Cw * S * N, 16 * ((m + 7) // 8)), dtype=torch.bfloat16, device=self.dev)
+        return dict(D=D[0], dsk=D[1], dsn=D[2], m=m, T=T)
+
+    def _pointwise(self, Wt, h, out, Cout, Cin, SP, bias=None, pre=None, gelu=False, rows={}):
         # out[o][q] = act(sum_i W[o][i] h[i][q] + bias[o])
         if self.ops.pointwise_ok(Cout, Cin, self.N, (h, out, pre)):
-            self.ops.pointwise(Wt, Cin, 1, Cout, Cin, h, out, SP // self.N, self.N, bias=bias, pre=pre, act=int(gelu))
+            self.ops.pointwise(Wt, Cin, 1, Cout, Cin, h, out, SP // self.N, self.N, bias=bias, pre=pre, act=int(gelu),
+                               **rows)
             return
         self.ops.gemm(Cout, SP, Cin, 1, Wt, 0, 0, Cin, 1, h, 0, 0, SP, 1, out, 0, 0, SP, 1, bias=bias, pre=pre,
                       gelu=gelu)
 
-    def _pointwise_t(self, Wt, dy, out, Cout, Cin, SP, pre=None):
+    def _pointwise_t(self, Wt, dy, out, Cout, Cin, SP, pre=None, rows={}):
         # out[i][q] = sum_o W[o][i] dy[o][q], times GELU'(pre[i][q]) if pre is given
         if self.ops.pointwise_ok(Cin, Cout, self.N, (dy, out, pre)):
             self.ops.pointwise(Wt, 1, Cin, Cin, Cout, dy, out, SP // self.N, self.N, pre=pre,
-                               act=2 if pre is not None else 0)
+                               act=2 if pre is not None else 0, **rows)
             return
         self.ops.gemm(Cin, SP, Cout, 1, Wt, 0, 0, 1, Cin, dy, 0, 0, SP, 1, out, 0, 0, SP, 1)
         if pre is not None:
@@ -297,9 +332,10 @@ class FNO:
         self.ops.gemm(Cout, Cin, kc, nb, dy, 0, kc, SP, 1, h, 0, kc, 1, SP, part, 0, Cout * Cin, Cin, 1)
         self.ops.reduce(part, gW, nb, Cout * Cin)
 
-    def _spectral(self, h, R, S):
+    def _spectral(self, h, R, S, T=None):
         """U [C][S][N][2m], the retained spectrum of K h transformed back along y,
-        and the retained spectrum B [C][S][2m][m][2] of h"""
+        and the retained spectrum B [C][S][2m][m][2] of h (T: h's transform along
+        x, from the pass that wrote h)"""
         torch = _torch()
         N, m, Cw = self.N, self.m, self.width
         rows = Cw * S * N
@@ -308,7 +344,7 @@ class FNO:
         O = torch.empty_like(B)
         U = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
         if self.ops.spectral_ok(Cw, N, m, h, R):
-            self.ops.spectral(h, self.Fx, 2 * m, 1, self.Gre, self.Gim, R, False, B, O, U, Cw, S, N, m)
+            self.ops.spectral(h, self.Fx, 2 * m, 1, self.Gre, self.Gim, R, False, B, O, U, Cw, S, N, m, T)
             return U, B
         T1 = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
         self.ops.gemm(rows, 2 * m, N, 1, h, 0, 0, N, 1, self.Fx, 0, 0, 2 * m, 1, T1, 0, 0, 2 * m, 1)
@@ -317,13 +353,14 @@ class FNO:
         self._cmat_left_inv(O, U, cs)
         return U, B
 
-    def _map_add(self, W, swm, swk, h, U, F, sfk, sfx, out, SP, bias=None, pre=None, act=0):
+    def _map_add(self, W, swm, swk, h, U, F, sfk, sfx, out, SP, bias=None, pre=None, act=0, rows={}):
         """out = act(W h + U F + bias): a block's 1x1 map with the inverse x
         transform of its spectral path (U, table F) in the same pass; act as
         Ops.pointwise"""
         N, K2, Cw = self.N, 2 * self.m, self.width
         if self.ops.pointwise_ok(Cw, Cw, N, (h, out, pre, U), K2):
-            self.ops.pointwise(W, swm, swk, Cw, Cw, h, out, SP // N, N, U, K2, F, sfk, sfx, bias, pre, act)
+            self.ops.pointwise(W, swm, swk, Cw, Cw, h, out, SP // N, N, U, K2, F, sfk, sfx, bias, pre, act,
+                               **rows)
             return
         g = self.ops.gemm
         g(Cw * SP // N, N, K2, 1, U, 0, 0, K2, 1, F, 0, 0, sfk, sfx, out, 0, 0, N, 1)
@@ -366,8 +403,9 @@ class FNO:
         g(Cw, S, Cw, nm, R, 0, *ra, B, 1, *bb, O, 1, *cc)
         g(Cw, S, Cw, nm, R, 1, *ra, B, 0, *bb, O, 1, *cc, beta=1.0)
 
-    def _spectral_backward(self, g_out, R, B, S, dR):
-        """dR (written) from the upstream gradient g_out [C][S][N][N]; returns dT1
+    def _spectral_backward(self, g_out, R, B, S, dR, T=None):
+        """dR (written) from the upstream gradient g_out [C][S][N][N] (T: its
+        transform along x, from the pass that wrote it); returns dT1
         [C][S][N][2m], whose product with Fx^T is the gradient of h"""
         torch = _torch()
         N, m, Cw = self.N, self.m, self.width
@@ -379,7 +417,8 @@ class FNO:
             dO = torch.empty((Cw, S, 2 * m, m, 2), dtype=torch.float32, device=self.dev)
             dB = torch.empty_like(dO)
             dT1 = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
-            self.ops.spectral(g_out, self.Fxi, 1, N, self.Gre, self.Gim, R, True, dO, dB, dT1, Cw, S, N, m)
+            self.ops.spectral(g_out, self.Fxi, 1, N, self.Gre, self.Gim, R, True, dO, dB, dT1, Cw, S, N, m,
+                              T)
             self.ops.mix_grad(dO, B, dR, Cw, S, m)
             return dT1
         dU = torch.empty((rows, 2 * m), dtype=torch.float32, device=self.dev)
@@ -419,11 +458,12 @@ class FNO:
         Cw, p, ops = self.width, self.param, self.ops
         cache = {"x": x, "S": S}
         h = torch.empty((Cw, S, self.N, self.N), dtype=torch.float32, device=self.dev)
-        self._pointwise(p["Lw"], x, h, Cw, self.cin, SP, bias=p["Lb"])
+        rows = self._rows(h, p["R0"], self.cin, S, 0, (x,)) if self.blocks > 0 else {}
+        self._pointwise(p["Lw"], x, h, Cw, self.cin, SP, bias=p["Lb"], rows=rows)
         for b in range(self.blocks):
             # hn = act(W h + K h + B): the 1x1 map adds the spectral path's
             # inverse x transform, its bias and activation in one pass
-            U, B = self._spectral(h, p[f"R{b}"], S)
+            U, B = self._spectral(h, p[f"R{b}"], S, rows.get("T"))
             if not keep and b == self.blocks - 1 and self.cout <= 16 and self.hidden <= 64 \
                     and ops.pointwise_ok(Cw, Cw, N, (h, U), 2 * self.m):
                 # nothing is kept: the last map and both projections in one pass
@@ -433,8 +473,9 @@ class FNO:
                 return y
             hn = torch.empty_like(h)
             pre = torch.empty_like(h) if keep else None
+            rows = self._rows(hn, p[f"R{b + 1}"], Cw, S, 2 * self.m, (h, pre, U)) if b < self.blocks - 1 else {}
             self._map_add(p[f"W{b}"], Cw, 1, h, U, self.Fxi, N, 1, hn, SP, bias=p[f"B{b}"], pre=pre,
-                          act=int(b < self.blocks - 1))
+                          act=int(b < self.blocks - 1), rows=rows)
             if keep:
                 cache[f"h{b}"], cache[f"pre{b}"], cache[f"B{b}"] = h, pre, B
             h = hn
@@ -472,17 +513,22 @@ class FNO:
         self._weight_grad(dq1, c["hL"], g["Q1"], H, Cw, SP)
         ops.bias_grad(dq1, g["q1b"], H, SP)
         dh = torch.empty_like(c["hL"])
-        self._pointwise_t(p["Q1"], dq1, dh, H, Cw, SP)
+        nb = self.blocks
+        rows = self._rows(dh, p[f"R{nb - 1}"], H, S, 0, (dq1,), True) if nb > 0 else {}
+        self._pointwise_t(p["Q1"], dq1, dh, H, Cw, SP, rows=rows)
         for b in reversed(range(self.blocks)):
             dpre = dh  # times GELU' already: by the pass that wrote it
             h = c[f"h{b}"]
             ops.bias_grad(dpre, g[f"B{b}"], Cw, SP)
             self._weight_grad(dpre, h, g[f"W{b}"], Cw, Cw, SP)
             dhn = torch.empty_like(h)
-            dT1 = self._spectral_backward(dpre, p[f"R{b}"], c[f"B{b}"], S, g[f"R{b}"])
+            dT1 = self._spectral_backward(dpre, p[f"R{b}"], c[f"B{b}"], S, g[f"R{b}"],
+                                          rows.get("T"))
             # W^T dpre + dT1 Fx^T, times the GELU' of the block before
+            pre = c[f"pre{b - 1}"] if b > 0 else None
+            rows = self._rows(dhn, p[f"R{b - 1}"], Cw, S, 2 * self.m, (dpre, pre, dT1), True) if b > 0 else {}
             self._map_add(p[f"W{b}"], 1, Cw, dpre, dT1, self.Fx, 1, 2 * self.m, dhn, SP,
-                          pre=c[f"pre{b - 1}"] if b > 0 else None, act=2 if b > 0 else 0)
+                          pre=pre, act=2 if b > 0 else 0, rows=rows)
             dh = dhn
         self._weight_grad(dh, c["x"], g["Lw"], Cw, self.cin, SP)
         ops.bias_grad(dh, g["Lb"], Cw, SP)

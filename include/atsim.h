@@ -418,6 +418,18 @@ int atsim_nn_tail(atsim_ctx *ctx, const float *W, long C, const float *h, long n
 int atsim_nn_spectral_fwd(atsim_ctx *ctx, const float *h, const float *F, long sfk, long sfn, const float *Gre,
                           const float *Gim, const float *R, int adjoint, float *B, float *O, float *U, long C,
                           long S, long N, long m);
+/* atsim_nn_pointwise with, in the same pass, the transform of out along x that
+ * the next block's atsim_nn_spectral_fwd would begin with (table D[x dsk + c
+ * dsn], m modes): T receives it as BF16 [Cout][nrows][16 ceil(m / 8)], the
+ * operand of atsim_nn_spectral_rows, which gives what atsim_nn_spectral_fwd
+ * gives from out.  Cout <= 32, m <= 16, K2 <= 32, rows of a multiple of 32
+ * pixels and at most 512, T 16-byte aligned, and the conditions of
+ * atsim_nn_pointwise (ATSIM_EUNSUPPORTED otherwise). */
+int atsim_nn_map_dft(atsim_ctx *ctx, const float *W, long swm, long swk, long Cout, long Cin, const float *h,
+                     float *out, long nrows, long rowlen, const float *U, long K2, const float *F, long sfk, long sfx,
+                     const float *bias, float *pre, int act, const float *D, long dsk, long dsn, long m, void *T);
+int atsim_nn_spectral_rows(atsim_ctx *ctx, const void *T, const float *Gre, const float *Gim, const float *R,
+                           int adjoint, float *B, float *O, float *U, long C, long S, long N, long m);
 /* dR = dO B^H per mode over the samples: dO and B [C][S][2m][m], dR
  * [2m m][C][C], complex.  C <= 64, 8-byte aligned (ATSIM_EUNSUPPORTED
  * otherwise). */

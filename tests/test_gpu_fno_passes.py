@@ -68,6 +68,46 @@ def test_pointwise_refuses_what_it_does_not_take(ctx):
         assert L.atsim_nn_pointwise(*a) == -4  # ATSIM_EUNSUPPORTED
 
 
+# the transform of out left by the pass that writes it: the spectral path from it
+# against the spectral path from out, bit for bit.  Edges of the 16-column tiles
+# (8, 9 and 16 modes), of the 64-pixel groups, channels over one tile and one
+# step, rows that do not fill the workgroups, the longest rows.
+@pytest.mark.parametrize("C,Cin,S,N,m,act,spec", [(1, 1, 1, 32, 1, 0, False), (16, 33, 1, 32, 8, 1, True),
+                                                  (17, 32, 2, 96, 9, 2, False), (32, 64, 1, 160, 16, 0, False),
+                                                  (32, 32, 5, 64, 16, 1, True), (24, 24, 1, 512, 12, 2, True)])
+def test_map_leaves_the_transform_along_x(ctx, C, Cin, S, N, m, act, spec):
+    import torch
+    from atmosphericturbulencesimul_amd.fno import FNO, Ops
+    print(f"map_dft C={C} Cin={Cin} S={S} N={N} m={m} act={act}", flush=True)
+    rng = np.random.default_rng(C + N)
+    ops = Ops(ctx)
+    net = FNO(ctx, N, 2, 2, width=C, modes=m, blocks=1, hidden=4, seed=1)
+    f32 = lambda *s: _dev(rng.standard_normal(s))[0]
+    W, h, b, pre, U = f32(C, Cin), f32(Cin, S, N, N), f32(C), f32(C, S, N, N), f32(C * S * N, 2 * m)
+    kw = dict(U=U, K2=2 * m, F=net.Fxi, sfk=N, sfx=1) if spec else {}
+    outs, specs = [], []
+    for rows in (False, True):
+        out = torch.full((C, S, N, N), np.nan, dtype=torch.float32, device="cuda")
+        T = torch.full((C * S * N, 16 * ((m + 7) // 8)), np.nan, dtype=torch.bfloat16, device="cuda") if rows else None
+        torch.cuda.synchronize()
+        ops.pointwise(W, Cin, 1, C, Cin, h, out, S * N, N, bias=b, pre=pre if act else None, act=act,
+                      **kw, **(dict(D=net.Fx, dsk=2 * m, dsn=1, m=m, T=T) if rows else {}))
+        B, O = (torch.zeros((C, S, 2 * m, m, 2), dtype=torch.float32, device="cuda") for _ in range(2))
+        Us = torch.zeros((C * S * N, 2 * m), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        ops.spectral(out, net.Fx, 2 * m, 1, net.Gre, net.Gim, net.param["R0"], rows, B, O, Us, C, S, N, m, T)
+        ctx.sync()
+        outs.append(out.cpu().numpy())
+        specs.append(B.cpu().numpy())
+    assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
+    assert np.abs(specs[0]).max() > 0 and np.array_equal(specs[0], specs[1])
+    # refused: more channels, more modes, rows of another length
+    for C_, m_, N_ in ((33, m, N), (C, 17, N), (C, m, 48), (C, m, 544)):
+        assert not ops.rows_ok(C_, N_, m_)
+        assert ctx.L.atsim_nn_map_dft(ctx.h, W.data_ptr(), 1, 1, C_, 1, h.data_ptr(), h.data_ptr(), 1, N_, None, 0, None,
+                                      0, 0, None, None, 0, net.Fx.data_ptr(), 0, 0, m_, T.data_ptr()) == -4
+
+
 # the fused passes against the general GEMM path, bit for bit: edges of the
 # 16-mode tiles, the 32-value steps, channels over one step, odd sample counts
 @pytest.mark.parametrize("N,m,width,S,hidden", [(32, 1, 8, 1, 16), (32, 16, 32, 3, 64), (64, 5, 17, 2, 33),

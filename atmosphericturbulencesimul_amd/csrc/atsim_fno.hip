@@ -268,8 +268,16 @@ __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
+// The matrix row that row i of an MFMA row tile rt stands for.  CHAIN: pairs of
+// tiles hold 32 rows in the order in which a lane's results of both tiles are
+// the 8 values of the next product's operand (4 (l / 16) + q of tile 0 and 1 ->
+// 8 (l / 16) + 0 .. 7), so that products follow one another in registers.
+template <bool CHAIN>
+__device__ __forceinline__ int tile_row(int rt, int i) {
+    return CHAIN ? 32 * (rt >> 1) + 8 * (i >> 2) + 4 * (rt & 1) + (i & 3) : rt * 16 + i;
+}
 // a wave's operands of an M x K matrix (element strides sm, sk)
-template <int RT, int KT>
+template <int RT, int KT, bool CHAIN = false>
 __device__ __forceinline__ void matrix_operands(bf16x8 (&wa)[RT][KT], const float* __restrict__ W, long sm, long sk,
                                                 int M, int K, int lm, int lk) {
 #pragma unroll
@@ -279,14 +287,14 @@ __device__ __forceinline__ void matrix_operands(bf16x8 (&wa)[RT][KT], const floa
             float v[8];
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                v[j] = W[min(rt * 16 + lm, M - 1) * sm + min(kt * 32 + lk + j, K - 1) * sk];
+                v[j] = W[min(tile_row<CHAIN>(rt, lm), M - 1) * sm + min(kt * 32 + lk + j, K - 1) * sk];
                 if (kt * 32 + lk + j >= K) v[j] = 0.f;
             }
             wa[rt][kt] = to_bf16x8(v);
         }
 }
 // the spectrum operands of row r of every channel
-template <int RT, int KU>
+template <int RT, int KU, bool CHAIN = false>
 __device__ __forceinline__ void spectrum_operands(bf16x8 (&ua)[RT][KU], const float* __restrict__ U, long nrows,
                                                   long r, int C, int K2, int lm, int lk) {
 #pragma unroll
@@ -294,7 +302,7 @@ __device__ __forceinline__ void spectrum_operands(bf16x8 (&ua)[RT][KU], const fl
 #pragma unroll
         for (int ku = 0; ku < KU; ku++) {
             const int k = ku * 32 + lk;
-            const float* up = U + ((long)min(rt * 16 + lm, C - 1) * nrows + r) * K2;
+            const float* up = U + ((long)min(tile_row<CHAIN>(rt, lm), C - 1) * nrows + r) * K2;
             const float4 a = *reinterpret_cast<const float4*>(up + min(k, K2 - 4));
             const float4 b = *reinterpret_cast<const float4*>(up + min(k + 4, K2 - 4));
             float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
@@ -491,6 +499,12 @@ __global__ void __launch_bounds__(256, point_waves(RT, KT, KU)) k_pointwise(Poin
     }
 }
 
+// Workgroups of a launch whose waves walk their units: as many as can be
+// resident (each stages the tables once), each with the same number of turns.
+static unsigned turns_grid(long wg, long resident) {
+    const long turns = (wg + resident - 1) / resident;
+    return (unsigned)(turns > 0 ? (wg + turns - 1) / turns : 1);
+}
 template <int RT, int KT, int KU, int NT>
 static hipError_t point_dft_launch(const PointArgs& g, hipStream_t st) {
     const size_t lds = ((size_t)KU * ((g.rowlen + 63) / 64) * 2048 + (size_t)(g.rowlen / 32) * NT * 512 +
@@ -500,10 +514,8 @@ static hipError_t point_dft_launch(const PointArgs& g, hipStream_t st) {
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    // the resident workgroups, each with the same number of rows a wave
-    const long wg = (g.nrows + 3) / 4, res = 256 * (160 * 1024 / (long)lds < 4 ? 160 * 1024 / (long)lds : 4);
-    const long turns = (wg + res - 1) / res;
-    k_pointwise<RT, KT, KU, NT><<<(unsigned)((wg + turns - 1) / turns), 256, lds, st>>>(g);
+    const long cap = 160 * 1024 / (long)lds, wv = point_waves(RT, KT, KU);
+    k_pointwise<RT, KT, KU, NT><<<turns_grid((g.nrows + 3) / 4, 256 * (cap < wv ? cap : wv)), 256, lds, st>>>(g);
     return hipGetLastError();
 }
 template <int RT, int KT, int KU>
@@ -512,8 +524,7 @@ static hipError_t point_launch(const PointArgs& g, hipStream_t st) {
         if (g.T) return g.dm <= 8 ? point_dft_launch<RT, KT, KU, 1>(g, st) : point_dft_launch<RT, KT, KU, 2>(g, st);
     }
     const long wg = (g.nrows * ((g.rowlen + 63) / 64) + 3) / 4;
-    // as many workgroups as can be resident (each stages F once)
-    const unsigned grid = (unsigned)(wg < 1024 ? (wg > 0 ? wg : 1) : 1024);
+    const unsigned grid = turns_grid(wg, 256 * (RT * KT == 1 ? 4 : point_waves(RT, KT, KU)));
     const size_t lds = (size_t)KU * ((g.rowlen + 63) / 64) * 256 * 8 * sizeof(__bf16);
     k_pointwise<RT, KT, KU, 0><<<grid, 256, lds, st>>>(g);
     return hipGetLastError();
@@ -531,61 +542,50 @@ static hipError_t point_kt(const PointArgs& g, hipStream_t st) {
 
 // The network's tail for inference, in one pass over the pixels: the last
 // block's map h' = W h + U F + bias (no activation), q = GELU(Q1 h' + q1b),
-// y = Q2 q + q2b, without writing h' and q.  Per pixel t of its lanes' fours a
-// wave passes h' and q through its own LDS rows (BF16, as the next product's
-// operand).  Products, sums and roundings as the three k_pointwise passes: the
+// y = Q2 q + q2b, without writing h' and q: their rows are taken in tile_row's
+// order, so that each product's results are the next one's operand (BF16) in the
+// same lane.  Products, sums and roundings as the three k_pointwise passes: the
 // same results.  Bound: VALU (64 GELUs a pixel).  50 images of 256^2, 32 and 64
-// channels: 248 us, where the three passes took 194 + 276 + 207 us and wrote and
-// read 1.3 GB between them.
+// channels: 222 us, where operands passed through LDS took 255 and the three
+// passes 194 + 276 + 207 us, with 1.3 GB written and read between them.
 struct TailArgs {
     PointArgs b;     // the block's map (act 0, no pre; out unused)
     const float *Q1, *q1b, *Q2, *q2b;
     int H, cout;
     float* y;        // [cout][nrows][rowlen]
 };
-template <int RT, int RH, int KU>
-__global__ void __launch_bounds__(256) k_tail(TailArgs g) {
-    constexpr int KT = (RT + 1) / 2, KH = (RH + 1) / 2, PS = 64 + 8;
+// KT, KH: steps of 32 channels of h and h', and of q
+template <int KT, int KH, int KU>
+__global__ void __launch_bounds__(256, (KT == 1 ? 2 : 1)) k_tail(TailArgs g) {
+    constexpr int RT = 2 * KT, RH = 2 * KH;
     extern __shared__ __attribute__((aligned(16))) __bf16 Fs[];
-    __shared__ __attribute__((aligned(16))) __bf16 X[4][16][PS];  // [wave][pixel][channel]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lm = lane & 15, lk = (lane >> 4) * 8, lr = (lane >> 4) * 4;
     const int C = g.b.Cout;
     const long SP = g.b.nrows * g.b.rowlen;
     const int ngrp = (g.b.rowlen + 63) / 64;
     stage_xtable<KU>(Fs, g.b.F, g.b.sfk, g.b.sfx, g.b.K2, g.b.rowlen);
-    for (int e = threadIdx.x; e < 4 * 16 * PS; e += 256) (&X[0][0][0])[e] = (__bf16)0.f;  // channels past the last stay 0
     __syncthreads();
     bf16x8 wa[RT][KT], q1[RH][KT], q2[1][KH];
-    matrix_operands<RT, KT>(wa, g.b.W, g.b.swm, g.b.swk, C, g.b.Cin, lm, lk);
-    matrix_operands<RH, KT>(q1, g.Q1, C, 1, g.H, C, lm, lk);
+    matrix_operands<RT, KT, true>(wa, g.b.W, g.b.swm, g.b.swk, C, g.b.Cin, lm, lk);
+    matrix_operands<RH, KT, true>(q1, g.Q1, C, 1, g.H, C, lm, lk);
     matrix_operands<1, KH>(q2, g.Q2, g.H, 1, g.cout, g.H, lm, lk);
-    float b0[RT][4], b1[RH][4], b2[4];
+    float b0[KT][8], b1[KH][8], b2[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
+    for (int j = 0; j < 8; j++) {
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) b0[rt][q] = g.b.bias[min(rt * 16 + lr + q, C - 1)];
+        for (int k = 0; k < KT; k++) b0[k][j] = g.b.bias[min(k * 32 + lk + j, C - 1)];
 #pragma unroll
-        for (int rt = 0; rt < RH; rt++) b1[rt][q] = g.q1b[min(rt * 16 + lr + q, g.H - 1)];
-        b2[q] = g.q2b[min(lr + q, g.cout - 1)];
+        for (int k = 0; k < KH; k++) b1[k][j] = g.q1b[min(k * 32 + lk + j, g.H - 1)];
     }
-    // the D layout's 4 channels of one pixel into the wave's rows, and back as
-    // an operand of the next product.  Channels past n stay zero.
-    auto put = [&](int c, int n, const float (&v)[4]) {
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (c + q < n) X[wave][lm][c + q] = (__bf16)v[q];
-    };
-    auto put4 = [&](int c, const float (&v)[4]) {
-        const bf16x4 t = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-        *reinterpret_cast<bf16x4*>(&X[wave][lm][c]) = t;
-    };
+    for (int q = 0; q < 4; q++) b2[q] = g.q2b[min(lr + q, g.cout - 1)];
     const long units = g.b.nrows * ngrp;
     for (long u = (long)blockIdx.x * 4 + wave; u < units; u += (long)gridDim.x * 4) {
         const long r = u / ngrp;
         const int x0 = (int)(u - r * ngrp) * 64;
         bf16x8 ua[RT][KU];
-        spectrum_operands<RT, KU>(ua, g.b.U, g.b.nrows, r, C, g.b.K2, lm, lk);
+        spectrum_operands<RT, KU, true>(ua, g.b.U, g.b.nrows, r, C, g.b.K2, lm, lk);
         const bool in = x0 + 4 * lm < g.b.rowlen;
         const long p = r * g.b.rowlen + min(x0 + 4 * lm, g.b.rowlen - 4);
         float4 hv[KT][8];
@@ -593,54 +593,53 @@ __global__ void __launch_bounds__(256) k_tail(TailArgs g) {
         float yv[4][4];  // [t][row]
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            bf16x8 hb[KT];
+            bf16x8 hb[KT], xb[KT];
             pixel_operands<KT>(hb, hv, t, g.b.Cin, lk);
-            wave_fence();
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f}, sp = acc;
+            for (int k = 0; k < KT; k++) {
+                float v[8];  // channels 32 k + lk + 0 .. 7, zero past the last
 #pragma unroll
-                for (int kt = 0; kt < KT; kt++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[rt][kt], hb[kt], acc, 0, 0, 0);
+                for (int i = 0; i < 2; i++) {
+                    const int rt = 2 * k + i;
+                    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, sp = acc;
 #pragma unroll
-                for (int ku = 0; ku < KU; ku++)
-                    sp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        ua[rt][ku],
-                        *reinterpret_cast<const bf16x8*>(Fs + ((size_t)((ku * ngrp + (x0 >> 6)) * 4 + t) * 64 + lane) * 8),
-                        sp, 0, 0, 0);
-                acc += sp;
-                const float v[4] = {acc[0] + b0[rt][0], acc[1] + b0[rt][1], acc[2] + b0[rt][2], acc[3] + b0[rt][3]};
-                if (C == RT * 16) put4(rt * 16 + lr, v);
-                else put(rt * 16 + lr, C, v);
+                    for (int kt = 0; kt < KT; kt++)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[rt][kt], hb[kt], acc, 0, 0, 0);
+#pragma unroll
+                    for (int ku = 0; ku < KU; ku++)
+                        sp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            ua[rt][ku],
+                            *reinterpret_cast<const bf16x8*>(Fs + ((size_t)((ku * ngrp + (x0 >> 6)) * 4 + t) * 64 + lane) * 8),
+                            sp, 0, 0, 0);
+                    acc += sp;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        v[4 * i + q] = acc[q] + b0[k][4 * i + q];
+                        if (k * 32 + lk + 4 * i + q >= C) v[4 * i + q] = 0.f;
+                    }
+                }
+                xb[k] = to_bf16x8(v);
             }
-            // channels C .. 32 KT - 1 hold q's of the pixel before: their products must be zero
-            if (C < KT * 32)
-                for (int c = C + (lane >> 4); c < KT * 32; c += 4) X[wave][lm][c] = (__bf16)0.f;
-            wave_fence();
-            bf16x8 xb[KT];
+            f32x4 y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) xb[kt] = *reinterpret_cast<const bf16x8*>(&X[wave][lm][kt * 32 + lk]);
-            wave_fence();
+            for (int k = 0; k < KH; k++) {
+                float v[8];
 #pragma unroll
-            for (int rt = 0; rt < RH; rt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                for (int i = 0; i < 2; i++) {
+                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int kt = 0; kt < KT; kt++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q1[rt][kt], xb[kt], acc, 0, 0, 0);
-                float v[4];
+                    for (int kt = 0; kt < KT; kt++)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q1[2 * k + i][kt], xb[kt], acc, 0, 0, 0);
 #pragma unroll
-                for (int q = 0; q < 4; q++) v[q] = gelu_t(acc[q] + b1[rt][q], nullptr);
-                if (g.H == RH * 16) put4(rt * 16 + lr, v);
-                else put(rt * 16 + lr, g.H, v);
+                    for (int q = 0; q < 4; q++) {
+                        v[4 * i + q] = gelu_t(acc[q] + b1[k][4 * i + q], nullptr);
+                        if (k * 32 + lk + 4 * i + q >= g.H) v[4 * i + q] = 0.f;
+                    }
+                }
+                y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q2[0][k], to_bf16x8(v), y, 0, 0, 0);
             }
-            if (g.H < KH * 32)
-                for (int c = g.H + (lane >> 4); c < KH * 32; c += 4) X[wave][lm][c] = (__bf16)0.f;
-            wave_fence();
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kt = 0; kt < KH; kt++)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    q2[0][kt], *reinterpret_cast<const bf16x8*>(&X[wave][lm][kt * 32 + lk]), acc, 0, 0, 0);
-#pragma unroll
-            for (int q = 0; q < 4; q++) yv[t][q] = acc[q] + b2[q];
+            for (int q = 0; q < 4; q++) yv[t][q] = y[q] + b2[q];
         }
         if (!in) continue;
 #pragma unroll
@@ -651,22 +650,17 @@ __global__ void __launch_bounds__(256) k_tail(TailArgs g) {
     }
 }
 
-template <int RT, int RH, int KU>
+template <int KT, int KH, int KU>
 static hipError_t tail_launch(const TailArgs& g, hipStream_t st) {
     const long wg = (g.b.nrows * ((g.b.rowlen + 63) / 64) + 3) / 4;
-    const size_t lds = (size_t)KU * ((g.b.rowlen + 63) / 64) * 256 * 8 * sizeof(__bf16);
-    if (lds + sizeof(__bf16) * 4 * 16 * 72 > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_tail<RT, RH, KU>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    k_tail<RT, RH, KU><<<(unsigned)(wg < 1024 ? wg : 1024), 256, lds, st>>>(g);
+    const size_t lds = (size_t)KU * ((g.b.rowlen + 63) / 64) * 256 * 8 * sizeof(__bf16);  // 64 KB at most
+    k_tail<KT, KH, KU><<<turns_grid(wg, 256 * (KT == 1 ? 2 : 1)), 256, lds, st>>>(g);
     return hipGetLastError();
 }
-template <int RT>
-static hipError_t tail_rt(const TailArgs& g, hipStream_t st) {
-    if (g.b.K2 <= 32) return g.H <= 32 ? tail_launch<RT, 2, 1>(g, st) : tail_launch<RT, 4, 1>(g, st);
-    return g.H <= 32 ? tail_launch<RT, 2, 2>(g, st) : tail_launch<RT, 4, 2>(g, st);
+template <int KT>
+static hipError_t tail_kt(const TailArgs& g, hipStream_t st) {
+    if (g.b.K2 <= 32) return g.H <= 32 ? tail_launch<KT, 1, 1>(g, st) : tail_launch<KT, 2, 1>(g, st);
+    return g.H <= 32 ? tail_launch<KT, 1, 2>(g, st) : tail_launch<KT, 2, 2>(g, st);
 }
 hipError_t launch_tail(const float* W, int C, const float* h, long nrows, int rowlen, const float* U, int K2,
                        const float* F, long sfk, long sfx, const float* bias, const float* Q1, const float* q1b, int H,
@@ -680,12 +674,7 @@ hipError_t launch_tail(const float* W, int C, const float* h, long nrows, int ro
     g.H = H;
     g.cout = cout;
     g.y = y;
-    switch ((C + 15) / 16) {
-        case 1: return tail_rt<1>(g, st);
-        case 2: return tail_rt<2>(g, st);
-        case 3: return tail_rt<3>(g, st);
-        default: return tail_rt<4>(g, st);
-    }
+    return C <= 32 ? tail_kt<1>(g, st) : tail_kt<2>(g, st);
 }
 
 // Channel maps of at most 64 in and out channels over rows of a multiple of 4
@@ -1144,8 +1133,7 @@ static hipError_t dft_y_launch(const __bf16* T, const float* Gre, const float* G
         if (e != hipSuccess) return e;
     }
     const long res = 256 * (160 * 1024 / (long)lds < 4 ? 160 * 1024 / (long)lds : 4);
-    const long turns = (images + res - 1) / res;  // the same number of images a workgroup
-    k_dft_y<NT><<<(unsigned)((images + turns - 1) / turns), 256, lds, st>>>(T, Gre, Gim, out, images, N, m);
+    k_dft_y<NT><<<turns_grid(images, res), 256, lds, st>>>(T, Gre, Gim, out, images, N, m);
     return hipGetLastError();
 }
 hipError_t launch_dft_y(const void* T, const float* Gre, const float* Gim, float* out, long images, int N, int m,

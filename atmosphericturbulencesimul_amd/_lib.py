@@ -113,6 +113,10 @@ _SIGS = {
     "atsim_nn_map_dft": (C.c_int, [C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_long, C.c_void_p, C.c_void_p,
                                    C.c_long, C.c_long, C.c_void_p, C.c_long, C.c_void_p, C.c_long, C.c_long, C.c_void_p,
                                    C.c_void_p, C.c_int, C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_void_p]),
+    "atsim_nn_lift_map_dft": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_void_p, C.c_long, C.c_long,
+                                        C.c_long, C.c_long, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_void_p,
+                                        C.c_long, C.c_void_p, C.c_long, C.c_long, C.c_void_p, C.c_void_p, C.c_int,
+                                        C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_void_p]),
     "atsim_nn_spectral_rows": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p,
                                          C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_long]),
     "atsim_nn_mix_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long]),

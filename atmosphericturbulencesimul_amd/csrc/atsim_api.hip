@@ -2235,22 +2235,30 @@ int atsim_nn_pointwise(atsim_ctx* c, const float* W, long swm, long swk, long Co
     return ATSIM_OK;
 }
 
-int atsim_nn_map_dft(atsim_ctx* c, const float* W, long swm, long swk, long Cout, long Cin, const float* h, float* out,
-                     long nrows, long rowlen, const float* U, long K2, const float* F, long sfk, long sfx,
-                     const float* bias, float* pre, int act, const float* D, long dsk, long dsn, long m, void* T) {
-    if (!c || !W || !h || !out || !D || !T || Cout <= 0 || Cin <= 0 || nrows <= 0 || rowlen <= 0 || m <= 0)
+int atsim_nn_lift_map_dft(atsim_ctx* c, const float* L, const float* Lb, long Cl, const float* W, long swm, long swk,
+                          long Cout, long Cin, const float* h, float* out, long nrows, long rowlen, const float* U, long K2,
+                          const float* F, long sfk, long sfx, const float* bias, float* pre, int act, const float* D,
+                          long dsk, long dsn, long m, void* T) {
+    if (!c || !W || !h || !D || !T || Cout <= 0 || Cin <= 0 || nrows <= 0 || rowlen <= 0 || m <= 0)
         return ATSIM_EINVAL;
     if (swm < 0 || swk < 0 || act < 0 || act > 2 || (act == 2 && !pre) || (U && (!F || sfk < 0 || sfx < 0)) || dsk < 0 ||
-        dsn < 0)
+        dsn < 0 || (L && (!Lb || !U || Cl <= 0)))
         return fail(c, ATSIM_EINVAL, "map and transform: invalid operands");
     if (!pointwise_supported(h, out, pre, U, Cout, Cin, nrows, rowlen, K2) ||
-        !point_dft_supported(T, Cout, rowlen, m, U ? K2 : 0))
+        !point_dft_supported(T, Cout, rowlen, m, U ? K2 : 0) || (L && (Cin > 32 || Cl > 32)))
         return fail(c, ATSIM_EUNSUPPORTED, "map and transform: %ld x %ld channels over rows of %ld, %ld modes", Cout, Cin,
                     rowlen, m);
     c->work_gen++;
     HIPCHK(c, launch_pointwise(W, swm, swk, (int)Cout, (int)Cin, h, out, nrows, (int)rowlen, U, U ? (int)K2 : 0, F, sfk,
-                               sfx, bias, pre, act, c->stream, D, dsk, dsn, (int)m, T));
+                               sfx, bias, pre, act, c->stream, D, dsk, dsn, (int)m, T, L, Lb, (int)Cl));
     return ATSIM_OK;
+}
+
+int atsim_nn_map_dft(atsim_ctx* c, const float* W, long swm, long swk, long Cout, long Cin, const float* h, float* out,
+                     long nrows, long rowlen, const float* U, long K2, const float* F, long sfk, long sfx,
+                     const float* bias, float* pre, int act, const float* D, long dsk, long dsn, long m, void* T) {
+    return atsim_nn_lift_map_dft(c, nullptr, nullptr, 0, W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U, K2, F, sfk, sfx,
+                                 bias, pre, act, D, dsk, dsn, m, T);
 }
 
 int atsim_nn_spectral_rows(atsim_ctx* c, const void* T, const float* Gre, const float* Gim, const float* R, int adjoint,

@@ -230,7 +230,9 @@ struct PointArgs {
     const float* D;  // table of the transform of out along x (NT > 0): D[x dsk + c dsn], dm modes
     long dsk, dsn;
     int dm;
-    __bf16* T;       // its result [Cout][nrows][16 NT]
+    __bf16* T;       // its result [Cout][nrows][16 NT]; out may then be null
+    const float *L, *Lb;  // h = L x + Lb ([Cin][cl], x in h's place)
+    int cl;
 };
 
 // F [K2][rowlen] staged as MFMA operands [KU][64-pixel group][t][lane][8]
@@ -352,8 +354,15 @@ constexpr int point_waves(int RT, int KT, int KU) {
 // HBM about equally; channel tiles one after the other, 16 of them live at a time,
 // leave room for 3 waves a SIMD (all tiles at once: 2 waves, 264 us; the
 // next pixels loaded ahead: scratch, 254 us).
-template <int RT, int KT, int KU, int NT>
+//
+// LIFT: the map's input is itself a channel map of x (at most 32 channels), made
+// in registers as the operand (tile_row's order) where the pass that would write
+// it only leaves its transform (out null): inference needs the first image of
+// a network nowhere else.  The same frames from 14 channels: 69 + 219 us, where
+// the lift and the first map took 138 + 231.
+template <int RT, int KT, int KU, int NT, bool LIFT>
 __global__ void __launch_bounds__(256, point_waves(RT, KT, KU)) k_pointwise(PointArgs g) {
+    static_assert(!LIFT || KT == 1, "one step of lifted channels");
     extern __shared__ __attribute__((aligned(16))) __bf16 Fs[];  // F as MFMA operands: [KU][64-pixel group][4][lane][8]
     constexpr int XS = 64 + 8;
     __bf16* Ds = Fs + (size_t)KU * ((g.rowlen + 63) / 64) * 2048;                       // [k step][NT][lane][8]
@@ -375,6 +384,13 @@ __global__ void __launch_bounds__(256, point_waves(RT, KT, KU)) k_pointwise(Poin
 #pragma unroll
         for (int q = 0; q < 4; q++)
             bias[rt][q] = g.bias ? g.bias[min(rt * 16 + (lane >> 4) * 4 + q, g.Cout - 1)] : 0.f;
+    bf16x8 la[2][1];
+    float lb[8];
+    if constexpr (LIFT) {
+        matrix_operands<2, 1, true>(la, g.L, g.cl, 1, g.Cin, g.cl, lm, lk);
+#pragma unroll
+        for (int j = 0; j < 8; j++) lb[j] = g.Lb[min(lk + j, g.Cin - 1)];
+    }
     f32x4 tx[RT][NT > 0 ? NT : 1];  // the row's transform: columns 4 (l / 16) .. + 3, channel l % 16
     bf16x8 ua[RT][KU > 0 ? KU : 1];
     const long units = NT > 0 ? g.nrows : g.nrows * ngrp, stride = (long)gridDim.x * 4;
@@ -388,10 +404,27 @@ __global__ void __launch_bounds__(256, point_waves(RT, KT, KU)) k_pointwise(Poin
         const bool in = x0 + 4 * lm < g.rowlen;
         const long p = r * g.rowlen + min(x0 + 4 * lm, g.rowlen - 4);
         float4 hv[KT][8];
-        load_channels<KT>(hv, g.h, SP, p, g.Cin, lk);
+        load_channels<KT>(hv, g.h, SP, p, LIFT ? g.cl : g.Cin, lk);
         bf16x8 hb[4][KT];
 #pragma unroll
-        for (int t = 0; t < 4; t++) pixel_operands<KT>(hb[t], hv, t, g.Cin, lk);
+        for (int t = 0; t < 4; t++) pixel_operands<KT>(hb[t], hv, t, LIFT ? g.cl : g.Cin, lk);
+        if constexpr (LIFT) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                    const f32x4 a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la[i][0], hb[t][0], z, 0, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        v[4 * i + q] = a[q] + lb[4 * i + q];
+                        if (lk + 4 * i + q >= g.Cin) v[4 * i + q] = 0.f;
+                    }
+                }
+                hb[t][0] = to_bf16x8(v);
+            }
+        }
         if (NT == 0 || grp == 0) {
             if constexpr (KU > 0) spectrum_operands<RT, KU>(ua, g.U, g.nrows, r, g.Cout, g.K2, lm, lk);
 #pragma unroll
@@ -460,7 +493,7 @@ __global__ void __launch_bounds__(256, point_waves(RT, KT, KU)) k_pointwise(Poin
                 } else if (g.pre) {
                     *reinterpret_cast<float4*>(g.pre + o) = v;
                 }
-                *reinterpret_cast<float4*>(g.out + o) = v;
+                if (NT == 0 || g.out) *reinterpret_cast<float4*>(g.out + o) = v;
                 if constexpr (NT > 0) {
                     const bf16x4 t = {(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
                     *reinterpret_cast<bf16x4*>(Xs + c * XS + 4 * lm) = t;
@@ -505,28 +538,33 @@ static unsigned turns_grid(long wg, long resident) {
     const long turns = (wg + resident - 1) / resident;
     return (unsigned)(turns > 0 ? (wg + turns - 1) / turns : 1);
 }
-template <int RT, int KT, int KU, int NT>
+template <int RT, int KT, int KU, int NT, bool LIFT>
 static hipError_t point_dft_launch(const PointArgs& g, hipStream_t st) {
     const size_t lds = ((size_t)KU * ((g.rowlen + 63) / 64) * 2048 + (size_t)(g.rowlen / 32) * NT * 512 +
                         4 * RT * 16 * (64 + 8)) * sizeof(__bf16);
     if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_pointwise<RT, KT, KU, NT>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_pointwise<RT, KT, KU, NT, LIFT>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
     const long cap = 160 * 1024 / (long)lds, wv = point_waves(RT, KT, KU);
-    k_pointwise<RT, KT, KU, NT><<<turns_grid((g.nrows + 3) / 4, 256 * (cap < wv ? cap : wv)), 256, lds, st>>>(g);
+    k_pointwise<RT, KT, KU, NT, LIFT><<<turns_grid((g.nrows + 3) / 4, 256 * (cap < wv ? cap : wv)), 256, lds, st>>>(g);
     return hipGetLastError();
 }
 template <int RT, int KT, int KU>
 static hipError_t point_launch(const PointArgs& g, hipStream_t st) {
     if constexpr (RT <= 2 && KU <= 1) {
-        if (g.T) return g.dm <= 8 ? point_dft_launch<RT, KT, KU, 1>(g, st) : point_dft_launch<RT, KT, KU, 2>(g, st);
+        if constexpr (KT == 1 && KU == 1)
+            if (g.T && g.L)
+                return g.dm <= 8 ? point_dft_launch<RT, 1, 1, 1, true>(g, st) : point_dft_launch<RT, 1, 1, 2, true>(g, st);
+        if (g.T)
+            return g.dm <= 8 ? point_dft_launch<RT, KT, KU, 1, false>(g, st)
+                             : point_dft_launch<RT, KT, KU, 2, false>(g, st);
     }
     const long wg = (g.nrows * ((g.rowlen + 63) / 64) + 3) / 4;
     const unsigned grid = turns_grid(wg, 256 * (RT * KT == 1 ? 4 : point_waves(RT, KT, KU)));
     const size_t lds = (size_t)KU * ((g.rowlen + 63) / 64) * 256 * 8 * sizeof(__bf16);
-    k_pointwise<RT, KT, KU, 0><<<grid, 256, lds, st>>>(g);
+    k_pointwise<RT, KT, KU, 0, false><<<grid, 256, lds, st>>>(g);
     return hipGetLastError();
 }
 
@@ -698,9 +736,10 @@ bool point_dft_supported(const void* T, long Cout, long rowlen, long dm, long K2
 hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Cin, const float* h, float* out,
                             long nrows, int rowlen, const float* U, int K2, const float* F, long sfk, long sfx,
                             const float* bias, float* pre, int act, hipStream_t st, const float* D, long dsk, long dsn,
-                            int dm, void* T) {
+                            int dm, void* T, const float* L, const float* Lb, int cl) {
     if (!pointwise_supported(h, out, pre, U, Cout, Cin, nrows, rowlen, K2)) return hipErrorInvalidValue;
     if (T && !point_dft_supported(T, Cout, rowlen, dm, K2)) return hipErrorInvalidValue;
+    if (L && (!T || !U || !Lb || Cin > 32 || cl < 1 || cl > 32)) return hipErrorInvalidValue;
     if (!U && !T) {  // no rows to tell apart: the image as rows of 64 pixels
         const long SP = nrows * rowlen;
         if (SP % 64 == 0) {
@@ -709,7 +748,7 @@ hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Ci
         }
     }
     const PointArgs g{W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U, K2, F, sfk, sfx, bias, pre, act,
-                      D, dsk, dsn, dm, (__bf16*)T};
+                      D, dsk, dsn, dm, (__bf16*)T, L, Lb, cl};
     switch ((Cout + 15) / 16) {
         case 1: return point_kt<1>(g, st);
         case 2: return point_kt<2>(g, st);

@@ -157,9 +157,11 @@ bool pointwise_supported(const float* h, const float* out, const float* pre, con
 hipError_t launch_pointwise(const float* W, long swm, long swk, int Cout, int Cin, const float* h, float* out,
                             long nrows, int rowlen, const float* U, int K2, const float* F, long sfk, long sfx,
                             const float* bias, float* pre, int act, hipStream_t st, const float* D = nullptr,
-                            long dsk = 0, long dsn = 0, int dm = 0, void* T = nullptr);
+                            long dsk = 0, long dsn = 0, int dm = 0, void* T = nullptr,
+                            const float* L = nullptr, const float* Lb = nullptr, int cl = 0);
 // sizes at which launch_pointwise also transforms out along x (T, BF16
-// [Cout][nrows][16 or 32 columns]; table D, dm modes), and the rest of that
+// [Cout][nrows][16 or 32 columns]; table D, dm modes; out may be null), its input
+// being L x + Lb of cl channels x in h's place if L is given, and the rest of that
 // transform; see k_dft_y
 bool point_dft_supported(const void* T, long Cout, long rowlen, long dm, long K2);
 hipError_t launch_dft_y(const void* T, const float* Gre, const float* Gim, float* out, long images, int N, int m,

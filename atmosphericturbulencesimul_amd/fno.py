@@ -85,13 +85,20 @@ class Ops:
                 and (K2 == 0 or (rowlen <= 512 and K2 <= 64 and K2 % 4 == 0)))
 
     def pointwise(self, W, swm, swk, Cout, Cin, h, out, nrows, rowlen, U=None, K2=0, F=None, sfk=0, sfx=0, bias=None,
-                  pre=None, act=0, D=None, dsk=0, dsn=0, m=0, T=None):
+                  pre=None, act=0, D=None, dsk=0, dsn=0, m=0, T=None, L=None, Lb=None, Cl=0):
         """out = act(W h [+ U F] [+ bias]) over [C][nrows][rowlen] images; act 0
         identity, 1 GELU (pre keeps its argument), 2 times GELU'(pre).  T: also
-        the transform of out along x (table D, m modes), for spectral"""
+        the transform of out along x (table D, m modes), for spectral (out may
+        be None); L: the map's input is L h + Lb of Cl channels h"""
         n = nrows * rowlen
-        if (h.numel() < Cin * n or out.numel() < Cout * n or W.numel() <= (Cout - 1) * swm + (Cin - 1) * swk
-                or (bias is not None and bias.numel() < Cout) or (pre is not None and pre.numel() != out.numel())
+        if L is not None and (T is None or U is None or L.numel() < Cin * Cl or Lb.numel() < Cin):
+            raise ValueError(f"pointwise lift out of bounds ({Cin} x {Cl} channels)")
+        if out is None and T is None:
+            raise ValueError("pointwise without an output")
+        no = Cout * n if out is None else out.numel()
+        if (h.numel() < (Cin if L is None else Cl) * n or no < Cout * n
+                or W.numel() <= (Cout - 1) * swm + (Cin - 1) * swk
+                or (bias is not None and bias.numel() < Cout) or (pre is not None and pre.numel() != no)
                 or (U is not None and (U.numel() < Cout * nrows * K2
                                        or F.numel() <= (K2 - 1) * sfk + (rowlen - 1) * sfx))):
             raise ValueError(f"pointwise operands out of bounds ({Cout} x {Cin} channels, {nrows} rows of {rowlen})")
@@ -99,9 +106,9 @@ class Ops:
             if (T.numel() < Cout * nrows * 16 * ((m + 7) // 8) or T.element_size() != 2
                     or D.numel() <= (rowlen - 1) * dsk + (2 * m - 1) * dsn):
                 raise ValueError(f"pointwise transform out of bounds ({Cout} channels, {nrows} rows, {m} modes)")
-            self.ctx._chk(self.L.atsim_nn_map_dft(self.ctx.h, _p(W), swm, swk, Cout, Cin, _p(h), _p(out), nrows, rowlen,
-                                                  _p(U), K2, _p(F), sfk, sfx, _p(bias), _p(pre), act, _p(D), dsk, dsn, m,
-                                                  _p(T)))
+            self.ctx._chk(self.L.atsim_nn_lift_map_dft(self.ctx.h, _p(L), _p(Lb), Cl, _p(W), swm, swk, Cout, Cin, _p(h),
+                                                       _p(out), nrows, rowlen, _p(U), K2, _p(F), sfk, sfx, _p(bias),
+                                                       _p(pre), act, _p(D), dsk, dsn, m, _p(T)))
             return
         self.ctx._chk(self.L.atsim_nn_pointwise(self.ctx.h, _p(W), swm, swk, Cout, Cin, _p(h), _p(out), nrows, rowlen,
                                                 _p(U), K2, _p(F), sfk, sfx, _p(bias), _p(pre), act))
@@ -457,10 +464,23 @@ class FNO:
         SP = S * N * N
         Cw, p, ops = self.width, self.param, self.ops
         cache = {"x": x, "S": S}
+        first = 0
         h = torch.empty((Cw, S, self.N, self.N), dtype=torch.float32, device=self.dev)
-        rows = self._rows(h, p["R0"], self.cin, S, 0, (x,)) if self.blocks > 0 else {}
-        self._pointwise(p["Lw"], x, h, Cw, self.cin, SP, bias=p["Lb"], rows=rows)
-        for b in range(self.blocks):
+        # nothing is kept: the first image is not written, the lift leaves its
+        # transform and block 0's map makes it again from x
+        lift = {} if keep or self.blocks < 2 or self.cin > 32 else \
+            self._rows(h, p["R1"], self.cin, S, 2 * self.m, (x,))
+        if lift and self.ops.spectral_ok(Cw, N, self.m, h, p["R0"]):
+            ops.pointwise(p["Lw"], self.cin, 1, Cw, self.cin, x, None, S * N, N, bias=p["Lb"], **lift)
+            U, _ = self._spectral(h, p["R0"], S, lift["T"])
+            rows = self._rows(h, p["R1"], self.cin, S, 2 * self.m, (x, U))
+            ops.pointwise(p["W0"], Cw, 1, Cw, Cw, x, h, S * N, N, U, 2 * self.m, self.Fxi, N, 1, p["B0"], None,
+                          1, **rows, L=p["Lw"], Lb=p["Lb"], Cl=self.cin)
+            first = 1
+        else:
+            rows = self._rows(h, p["R0"], self.cin, S, 0, (x,)) if self.blocks > 0 else {}
+            self._pointwise(p["Lw"], x, h, Cw, self.cin, SP, bias=p["Lb"], rows=rows)
+        for b in range(first, self.blocks):
             # hn = act(W h + K h + B): the 1x1 map adds the spectral path's
             # inverse x transform, its bias and activation in one pass
             U, B = self._spectral(h, p[f"R{b}"], S, rows.get("T"))

@@ -422,12 +422,19 @@ int atsim_nn_spectral_fwd(atsim_ctx *ctx, const float *h, const float *F, long s
  * the next block's atsim_nn_spectral_fwd would begin with (table D[x dsk + c
  * dsn], m modes): T receives it as BF16 [Cout][nrows][16 ceil(m / 8)], the
  * operand of atsim_nn_spectral_rows, which gives what atsim_nn_spectral_fwd
- * gives from out.  Cout <= 32, m <= 16, K2 <= 32, rows of a multiple of 32
+ * gives from out; out may be null.  Cout <= 32, m <= 16, K2 <= 32, rows of a multiple of 32
  * pixels and at most 512, T 16-byte aligned, and the conditions of
  * atsim_nn_pointwise (ATSIM_EUNSUPPORTED otherwise). */
 int atsim_nn_map_dft(atsim_ctx *ctx, const float *W, long swm, long swk, long Cout, long Cin, const float *h,
                      float *out, long nrows, long rowlen, const float *U, long K2, const float *F, long sfk, long sfx,
                      const float *bias, float *pre, int act, const float *D, long dsk, long dsn, long m, void *T);
+/* the same where the map's input is L h + Lb of the Cl channels of h (L
+ * row-major Cin x Cl), which is not written; with U, Cin and Cl <= 32.  L may be
+ * null: atsim_nn_map_dft. */
+int atsim_nn_lift_map_dft(atsim_ctx *ctx, const float *L, const float *Lb, long Cl, const float *W, long swm, long swk,
+                          long Cout, long Cin, const float *h, float *out, long nrows, long rowlen, const float *U,
+                          long K2, const float *F, long sfk, long sfx, const float *bias, float *pre, int act,
+                          const float *D, long dsk, long dsn, long m, void *T);
 int atsim_nn_spectral_rows(atsim_ctx *ctx, const void *T, const float *Gre, const float *Gim, const float *R,
                            int adjoint, float *B, float *O, float *U, long C, long S, long N, long m);
 /* dR = dO B^H per mode over the samples: dO and B [C][S][2m][m], dR

@@ -3,7 +3,12 @@
 //
 // Every linear map of the network -- the truncated DFTs along x and y, the
 // per-mode complex channel mixing, the 1x1 channel maps -- and every product
-// of its backward pass is one strided, batched GEMM
+// of its backward pass is a matrix product on the matrix cores with BF16
+// operands and FP32 sums.  At the sizes the network is used at, passes of their
+// own make them: k_pointwise and k_tail (channel maps with the inverse x
+// transform, bias, activation, and the next forward x transform), k_dft2 /
+// k_dft_y, k_mix and k_idft_y (spectral path), k_mix_grad and k_weight_grad.
+// Other sizes and alignments take k_gemm_bf16, a strided, batched GEMM
 //     C[b] = alpha * A[b] (M x K) * B[b] (K x N) + beta * C[b]
 // with arbitrary element strides, so transposes, real/imaginary views and
 // channel-major / mode-major layouts cost nothing.  Operands are FP32 in

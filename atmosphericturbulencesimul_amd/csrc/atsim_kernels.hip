@@ -7,17 +7,19 @@
 //  k_row_fresnel   the frame's x pass over several wavelengths of one row:
 //                  optionally the x factor of the gap before a layer group,
 //                  the group's screen, the x factor of the gap after it.
+//  k_row_screen    the same for the passes after the first, the screen read
+//                  from sampled phase planes, in one-wave workgroups.
 //  k_col_screen(_split)  the frame's y pass: y factor, screen (from sampled
 //                  phase planes), y factor.  With the x and y factors of a
 //                  gap commuting, gaps alternate x-first / y-first and a
 //                  frame makes one pass over the fields per gap.
-//  k_layer_phase   FP64 phase planes of the layers column passes apply.
+//  k_layer_phase   FP64 phase planes of the layers those passes apply.
 //  k_permut        quadrant swap (fft.c:570-792).
 //  k_noise         Philox4x32-10 + Box-Muller complex Gaussian noise.
 //  k_synth_row     von Karman spectral filter on the noise in the
 //                  quadrant-swapped layout (AtmosphericTurbulence.c:643-784) and
 //                  its transform along x.
-//  k_lag_sums, k_strfn  FP64 structure-function reductions
+//  k_lag_sums, k_lag_fit, k_strfn  FP64 structure-function reductions
 //                  (AT.c:790-847, 2246-2270).
 //  k_extract       crop, amplitude, phase, geometric-phase unwrap
 //                  (AT.c:3418-3476), block sums of the science-lambda rule

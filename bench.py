@@ -655,8 +655,8 @@ def main():
     # Algorithmic bytes of every Fresnel pass of a frame, by kind: one c64
     # read + write of every field (the first pass creates the field: write
     # only) and, per direction, one f32 read of the footprint of each layer
-    # whose screen a row pass applies, or one f64 read of the sampled phase
-    # plane of each layer a column pass applies (the phase kernel reads the
+    # whose screen the first pass applies, or one f64 read of the sampled phase
+    # plane of each layer a later pass applies (the phase kernel reads the
     # f32 footprint and writes the f64 plane).  Layer groups top -> bottom as
     # the library forms them; the last group is applied by the extraction.
     sli = list(np.asarray(setup["sli"]))
@@ -671,7 +671,7 @@ def main():
     field_rw, field_w, foot = 16.0 * N * N * F, 8.0 * N * N * F, 4.0 * N * N * wl["D"]
     passes = []  # (kind, bytes)
     if fused:
-        nslots = sum(lcount[k] for k in range(1, G, 2))
+        nslots = sum(lcount[k] for k in range(1, G))
         passes.append(("phase", 3.0 * foot * nslots))
         for k in range(G + 1):
             rows = k % 2 == 0
@@ -679,10 +679,8 @@ def main():
                 passes.append(("row", field_w + foot * lcount[0]))
             elif k == G:
                 passes.append(("row" if rows else "col", field_rw))
-            elif rows:
-                passes.append(("row2", field_rw + foot * lcount[k]))
             else:
-                passes.append(("col2", field_rw + 2.0 * foot * lcount[k]))
+                passes.append(("row2" if rows else "col2", field_rw + 2.0 * foot * lcount[k]))
     else:
         for g in range(G):
             passes.append(("row", (field_w if g == 0 else field_rw) + foot * lcount[g]))
@@ -708,10 +706,10 @@ def main():
     c2e = ctx.get_tuning("col2_e") or (32 if 256 <= N <= 2048 else 16)
     ce = ctx.get_tuning("col_e") or 16
     cc = ctx.get_tuning("col_c") or (8 if N == 2048 else 16)
+    cs = 256 <= N <= 2048 and cc in (8, 16) if ce == 32 else (ctx.get_tuning("col_e") == 0 and N == 2048 and F > 1)
     kernel_names = {"row": f"k_row_fresnel<{N}> (x pass: screen phase, FFT, transfer function, IFFT)",
-                    "col": (f"k_col_split<{N}, 8, 32>" if ce == 32 and 256 <= N <= 2048 and cc in (8, 16)
-                            else f"k_col<{N}, 1, 0, {cc}>") + " (y pass: FFT, transfer function, IFFT)",
-                    "row2": f"k_row_fresnel<{N}, false, true> (x pass: FFT, transfer function, IFFT, screen "
+                    "col": (f"k_col_split<{N}, 1, 0, 8, 32>" if cs else f"k_col<{N}, 1, 0, {cc}>") + " (y pass: FFT, transfer function, IFFT)",
+                    "row2": f"k_row_screen<{N}> (x pass: FFT, transfer function, IFFT, screen "
                             "phase, FFT, transfer function, IFFT)",
                     "col2": (f"k_col_screen_split<{N}, 8, 32>" if c2e == 32 else f"k_col_screen<{N}>") +
                             " (y pass: FFT, transfer function, IFFT, screen phase, FFT, transfer function, IFFT)"}

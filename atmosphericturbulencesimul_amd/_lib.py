@@ -122,6 +122,8 @@ _SIGS = {
     "atsim_nn_mix_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long, C.c_long]),
     "atsim_nn_weight_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long, C.c_long,
                                        C.c_long, C.c_long]),
+    "atsim_nn_weight_bias_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
+                                            C.c_void_p, C.c_long, C.c_long, C.c_long, C.c_long]),
     "atsim_nn_tail": (C.c_int, [C.c_void_p, C.c_void_p, C.c_long, C.c_void_p, C.c_long, C.c_long, C.c_void_p, C.c_long,
                                 C.c_void_p, C.c_long, C.c_long, C.c_void_p, C.c_void_p, C.c_void_p, C.c_long,
                                 C.c_void_p, C.c_void_p, C.c_long, C.c_void_p]),

@@ -66,13 +66,13 @@ struct atsim_ctx {
     long mg_frames = 0;
     hipEvent_t mg_fork = nullptr;
     float2* fresnel_tab = nullptr;  // [8192] transfer factor of the running Fresnel step
-    // work space of calls on the context stream (ctx_scratch), kept between them
+    // work space of calls on the context stream (Scratch), kept between them
     void* scratch = nullptr;
     size_t scratch_cap = 0;
     double* nn_loss_host = nullptr;  // pinned: partial sums of a loss read later
     hipEvent_t nn_loss_ev = nullptr;
     double* nn_part = nullptr;  // 256 partial sums of the network's loss reduction
-    float* nn_bias = nullptr;   // per-chunk partial sums of bias gradients
+    double* nn_bias = nullptr;  // per-chunk partial sums of bias gradients
     size_t nn_bias_cap = 0;
 };
 
@@ -2299,15 +2299,20 @@ int atsim_nn_mix_grad(atsim_ctx* c, const float* dO, const float* B, float* dR, 
     return ATSIM_OK;
 }
 
-int atsim_nn_weight_grad(atsim_ctx* c, const float* dy, const float* h, float* part, float* gW, long Cout, long Cin,
-                         long SP, long kc) {
-    if (!c || !dy || !h || !part || !gW || Cout <= 0 || Cin <= 0 || SP <= 0 || kc <= 0) return ATSIM_EINVAL;
+int atsim_nn_weight_bias_grad(atsim_ctx* c, const float* dy, const float* h, float* part, float* gW, double* bpart,
+                              float* gb, long Cout, long Cin, long SP, long kc) {
+    if (!c || !dy || !h || !part || !gW || (bpart != nullptr) != (gb != nullptr) || Cout <= 0 || Cin <= 0 || SP <= 0 || kc <= 0) return ATSIM_EINVAL;
     if (!weight_grad_supported(dy, h, Cout, Cin, SP, kc))
         return fail(c, ATSIM_EUNSUPPORTED, "weight_grad: %ld x %ld channels, %ld pixels by %ld", Cout, Cin, SP, kc);
     c->work_gen++;
-    HIPCHK(c, launch_weight_grad(dy, h, part, (int)Cout, (int)Cin, SP, (int)kc, c->stream));
-    HIPCHK(c, launch_reduce_batches(part, gW, SP / kc, Cout * Cin, 0, c->stream));
+    HIPCHK(c, launch_weight_grad(dy, h, part, bpart, (int)Cout, (int)Cin, SP, (int)kc, c->stream));
+    HIPCHK(c, launch_reduce_batches(part, gW, SP / kc, Cout * Cin, 0, bpart, gb, bpart ? Cout : 0, c->stream));
     return ATSIM_OK;
+}
+
+int atsim_nn_weight_grad(atsim_ctx* c, const float* dy, const float* h, float* part, float* gW, long Cout, long Cin,
+                         long SP, long kc) {
+    return atsim_nn_weight_bias_grad(c, dy, h, part, gW, nullptr, nullptr, Cout, Cin, SP, kc);
 }
 
 int atsim_nn_tail(atsim_ctx* c, const float* W, long C, const float* h, long nrows, long rowlen, const float* U,
@@ -2343,7 +2348,7 @@ int atsim_nn_bias_grad(atsim_ctx* c, const float* dy, float* db, long S, long C,
     if (!c || !dy || !db || S <= 0 || C <= 0 || P <= 0) return ATSIM_EINVAL;
     c->work_gen++;
     const int nchunk = 64;
-    const size_t need = sizeof(float) * nchunk * C;
+    const size_t need = sizeof(double) * nchunk * C;
     if (c->nn_bias_cap < need) {
         if (c->nn_bias) hipFree(c->nn_bias);
         c->nn_bias = nullptr;
@@ -2352,7 +2357,7 @@ int atsim_nn_bias_grad(atsim_ctx* c, const float* dy, float* db, long S, long C,
         c->nn_bias_cap = need;
     }
     HIPCHK(c, launch_bias_grad(dy, c->nn_bias, S, C, P, nchunk, c->stream));
-    HIPCHK(c, launch_reduce_batches(c->nn_bias, db, nchunk, C, accumulate, c->stream));
+    HIPCHK(c, launch_reduce_batches(nullptr, nullptr, nchunk, 0, accumulate, c->nn_bias, db, C, c->stream));
     return ATSIM_OK;
 }
 
@@ -2399,7 +2404,7 @@ int atsim_nn_mse_end(atsim_ctx* c, long n, double* loss) {
 int atsim_nn_reduce_batches(atsim_ctx* c, const float* part, float* out, long nb, long n, int accumulate) {
     if (!c || !part || !out || nb <= 0 || n <= 0) return ATSIM_EINVAL;
     c->work_gen++;
-    HIPCHK(c, launch_reduce_batches(part, out, nb, n, accumulate, c->stream));
+    HIPCHK(c, launch_reduce_batches(part, out, nb, n, accumulate, nullptr, nullptr, 0, c->stream));
     return ATSIM_OK;
 }
 

@@ -1057,10 +1057,13 @@ __global__ void __launch_bounds__(256) k_mix_grad(const float* __restrict__ dO, 
 // (both operands are contiguous along the sum), the loads of UN k steps in flight.
 // Order and results as k_gemm_bf16.  Bound: HBM.  32 x 32 channels over 524 288
 // pixels (134 MB): 34 us, 64 x 32 76 us, against 45 and 92 with one tile a wave
-// and 53 through k_gemm_bf16's LDS staging.
+// and 53 through k_gemm_bf16's LDS staging.  With bpart also the chunk's sums of
+// dy, bpart[chunk][o], in FP64 from the same loads: a pass of its own reads dy
+// again (12 us for 67 MB).
 template <int RT, int CT>
 __global__ void __launch_bounds__(64) k_weight_grad(const float* __restrict__ dy, const float* __restrict__ h,
-                                                    float* __restrict__ part, int Cout, int Cin, long SP, int kc) {
+                                                    float* __restrict__ part, double* __restrict__ bpart, int Cout,
+                                                    int Cin, long SP, int kc) {
     constexpr int UN = RT + CT <= 4 ? 4 : RT + CT <= 6 ? 2 : 1;
     const int lane = threadIdx.x, lm = lane & 15, lk = (lane >> 4) * 8;
     const float *a[RT], *b[CT];
@@ -1073,6 +1076,9 @@ __global__ void __launch_bounds__(64) k_weight_grad(const float* __restrict__ dy
     for (int r = 0; r < RT; r++)
 #pragma unroll
         for (int q = 0; q < CT; q++) acc[r][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    double bs[RT];
+#pragma unroll
+    for (int r = 0; r < RT; r++) bs[r] = 0.0;
     float4 v[UN][RT + CT][2];
     auto fetch = [&](int k0) {
 #pragma unroll
@@ -1094,6 +1100,9 @@ __global__ void __launch_bounds__(64) k_weight_grad(const float* __restrict__ dy
                 const float x[8] = {v[s][t][0].x, v[s][t][0].y, v[s][t][0].z, v[s][t][0].w,
                                     v[s][t][1].x, v[s][t][1].y, v[s][t][1].z, v[s][t][1].w};
                 o[s][t] = to_bf16x8(x);
+                if (t < RT && bpart)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) bs[t < RT ? t : 0] += (double)x[j];
             }
         fetch(min(k0 + 32 * UN, kc - 32 * UN));  // the next steps' loads beside the products
 #pragma unroll
@@ -1112,6 +1121,13 @@ __global__ void __launch_bounds__(64) k_weight_grad(const float* __restrict__ dy
                 const int oo = r * 16 + (lane >> 4) * 4 + q, i = c * 16 + lm;
                 if (oo < Cout && i < Cin) part[((long)blockIdx.x * Cout + oo) * Cin + i] = acc[r][c][q];
             }
+    if (!bpart) return;
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        bs[r] += __shfl_xor(bs[r], 16);
+        bs[r] += __shfl_xor(bs[r], 32);
+        if (lane < 16 && r * 16 + lm < Cout) bpart[(long)blockIdx.x * Cout + r * 16 + lm] = bs[r];
+    }
 }
 
 // at most 64 channels each way, chunks of a multiple of 128 pixels, 16-byte
@@ -1120,13 +1136,13 @@ bool weight_grad_supported(const float* dy, const float* h, long Cout, long Cin,
     return Cout >= 1 && Cout <= 64 && Cin >= 1 && Cin <= 64 && kc >= 128 && kc % 128 == 0 && kc <= (1L << 24) &&
            SP % kc == 0 && SP / kc < (1L << 31) && (((uintptr_t)dy | (uintptr_t)h) & 15) == 0;
 }
-hipError_t launch_weight_grad(const float* dy, const float* h, float* part, int Cout, int Cin, long SP, int kc,
-                              hipStream_t st) {
+hipError_t launch_weight_grad(const float* dy, const float* h, float* part, double* bpart, int Cout, int Cin, long SP,
+                              int kc, hipStream_t st) {
     const unsigned grid = (unsigned)(SP / kc);
     switch ((Cout + 15) / 16 * 4 + (Cin + 15) / 16 - 5) {
 #define X(RT, CT)                                                                       \
     case (RT - 1) * 4 + CT - 1:                                                         \
-        k_weight_grad<RT, CT><<<grid, 64, 0, st>>>(dy, h, part, Cout, Cin, SP, kc);     \
+        k_weight_grad<RT, CT><<<grid, 64, 0, st>>>(dy, h, part, bpart, Cout, Cin, SP, kc);     \
         return hipGetLastError();
         X(1, 1) X(1, 2) X(1, 3) X(1, 4) X(2, 1) X(2, 2) X(2, 3) X(2, 4)
         X(3, 1) X(3, 2) X(3, 3) X(3, 4) X(4, 1) X(4, 2) X(4, 3) X(4, 4)
@@ -1270,9 +1286,9 @@ __global__ void k_gelu_bwd(const float* __restrict__ pre, const float* __restric
 }
 
 // partial[chunk][c] = sum of dy[s][c][p] over this workgroup's chunk of
-// the S * P values of channel c (FP64); the chunks are summed by
-// k_reduce_batches in a fixed order
-__global__ void __launch_bounds__(256) k_bias_grad(const float* __restrict__ dy, float* __restrict__ partial, long S,
+// the S * P values of channel c, in FP64 as are the chunks' sums
+// (k_reduce_batches)
+__global__ void __launch_bounds__(256) k_bias_grad(const float* __restrict__ dy, double* __restrict__ partial, long S,
                                                    long C, long P) {
     const long c = blockIdx.x, nchunk = gridDim.y, chunk = blockIdx.y;
     const long n = S * P, per = (n + nchunk - 1) / nchunk;
@@ -1302,7 +1318,7 @@ __global__ void __launch_bounds__(256) k_bias_grad(const float* __restrict__ dy,
         if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[chunk * C + c] = (float)red[0];
+    if (threadIdx.x == 0) partial[chunk * C + c] = red[0];
 }
 
 // mean squared error over n elements: partial sums of (pred - target)^2 and
@@ -1361,11 +1377,28 @@ __global__ void k_adam_many(AdamTensors p, float lr, float b1, float b2, float e
 // A workgroup takes 64 outputs: all four waves load 128 partials of each ahead
 // into LDS, and its first wave adds them, so that the chain of dependent adds
 // waits for LDS and not for memory (512 partials of 1 024 outputs: 7 us, against
-// 66 with one thread walking each output's partials in memory).
+// 66 with one thread walking each output's partials in memory).  A workgroup past
+// those takes one bias gradient bout[c], the sum of bpart[b nbias + c] in FP64.
 constexpr int RED_B = 128;
 __global__ void __launch_bounds__(256) k_reduce_batches(const float* __restrict__ part, float* __restrict__ out,
-                                                        long nb, long n, int accumulate) {
-    __shared__ float P[RED_B][64];
+                                                        long nb, long n, int accumulate,
+                                                        const double* __restrict__ bpart, float* __restrict__ bout,
+                                                        long nbias) {
+    __shared__ __attribute__((aligned(16))) float P[RED_B][64];
+    if (blockIdx.x >= (n + 63) / 64) {
+        const long c = blockIdx.x - (n + 63) / 64;
+        double acc = 0.0;
+        for (long b = threadIdx.x; b < nb; b += 256) acc += bpart[b * nbias + c];
+        double* red = reinterpret_cast<double*>(&P[0][0]);
+        red[threadIdx.x] = acc;
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) bout[c] = accumulate ? bout[c] + (float)red[0] : (float)red[0];
+        return;
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const long i = blockIdx.x * 64L + lane, ic = min(i, n - 1);
     float v[RED_B / 4];
@@ -1459,7 +1492,7 @@ hipError_t launch_gelu_bwd(const float* pre, const float* dy, float* dx, long n,
     k_gelu_bwd<<<grid_for(n), 256, 0, st>>>(pre, dy, dx, n);
     return hipGetLastError();
 }
-hipError_t launch_bias_grad(const float* dy, float* partial, long S, long C, long P, int nchunk, hipStream_t st) {
+hipError_t launch_bias_grad(const float* dy, double* partial, long S, long C, long P, int nchunk, hipStream_t st) {
     k_bias_grad<<<dim3((unsigned)C, (unsigned)nchunk), 256, 0, st>>>(dy, partial, S, C, P);
     return hipGetLastError();
 }
@@ -1468,8 +1501,9 @@ hipError_t launch_mse(const float* pred, const float* target, float* grad, long 
     k_mse<<<nblk, 256, 0, st>>>(pred, target, grad, n, partial);
     return hipGetLastError();
 }
-hipError_t launch_reduce_batches(const float* part, float* out, long nb, long n, int accumulate, hipStream_t st) {
-    k_reduce_batches<<<(unsigned)((n + 63) / 64), 256, 0, st>>>(part, out, nb, n, accumulate);
+hipError_t launch_reduce_batches(const float* part, float* out, long nb, long n, int accumulate, const double* bpart,
+                                 float* bout, long nbias, hipStream_t st) {
+    k_reduce_batches<<<(unsigned)((n + 63) / 64 + nbias), 256, 0, st>>>(part, out, nb, n, accumulate, bpart, bout, nbias);
     return hipGetLastError();
 }
 hipError_t launch_nn_pairs(const float* screens, const double* sc, const float* pha, const float* amp, long D, long L,

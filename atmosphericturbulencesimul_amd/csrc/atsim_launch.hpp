@@ -182,15 +182,16 @@ hipError_t launch_idft_y(const float* Gre, const float* Gim, const float* O, flo
 hipError_t launch_mix(const float* R, const float* B, float* out, int C, int S, int nm, bool adj, hipStream_t st);
 hipError_t launch_mix_grad(const float* dO, const float* B, float* dR, int C, int S, int nm, hipStream_t st);
 bool weight_grad_supported(const float* dy, const float* h, long Cout, long Cin, long SP, long kc);
-hipError_t launch_weight_grad(const float* dy, const float* h, float* part, int Cout, int Cin, long SP, int kc,
-                              hipStream_t st);
+hipError_t launch_weight_grad(const float* dy, const float* h, float* part, double* bpart, int Cout, int Cin, long SP,
+                              int kc, hipStream_t st);
 hipError_t launch_add_bias_act(const float* a, const float* b, const float* bias, float* pre, float* y, long C,
                                long P, long n, int gelu, hipStream_t st);
 hipError_t launch_gelu_bwd(const float* pre, const float* dy, float* dx, long n, hipStream_t st);
-hipError_t launch_bias_grad(const float* dy, float* partial, long S, long C, long P, int nchunk, hipStream_t st);
+hipError_t launch_bias_grad(const float* dy, double* partial, long S, long C, long P, int nchunk, hipStream_t st);
 hipError_t launch_mse(const float* pred, const float* target, float* grad, long n, double* partial, int nblk,
                       hipStream_t st);
-hipError_t launch_reduce_batches(const float* part, float* out, long nb, long n, int accumulate, hipStream_t st);
+hipError_t launch_reduce_batches(const float* part, float* out, long nb, long n, int accumulate, const double* bpart,
+                                 float* bout, long nbias, hipStream_t st);
 hipError_t launch_nn_pairs(const float* screens, const double* sc, const float* pha, const float* amp, long D, long L,
                            long N, long Stot, long s0, float* x, float* t, double xs, double xl, double cs, double ps,
                            hipStream_t st);

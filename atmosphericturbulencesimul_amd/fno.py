@@ -167,12 +167,15 @@ class Ops:
         return (Cout <= 64 and Cin <= 64 and kc % 128 == 0 and SP % kc == 0
                 and dy.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
 
-    def weight_grad(self, dy, h, part, gW, Cout, Cin, SP, kc):
-        """gW = dy h^T over SP pixels, in chunks of kc"""
+    def weight_grad(self, dy, h, part, gW, Cout, Cin, SP, kc, bpart=None, gb=None):
+        """gW = dy h^T over SP pixels, in chunks of kc (gb: also the sums of dy)"""
         if (dy.numel() < Cout * SP or h.numel() < Cin * SP or part.numel() < SP // kc * Cout * Cin
                 or gW.numel() < Cout * Cin):
             raise ValueError("weight_grad: operands too small")
-        self.ctx._chk(self.L.atsim_nn_weight_grad(self.ctx.h, _p(dy), _p(h), _p(part), _p(gW), Cout, Cin, SP, kc))
+        if gb is not None and (gb.numel() != Cout or bpart.numel() < SP // kc * Cout or bpart.element_size() != 8):
+            raise ValueError("weight_grad: bias operands too small")
+        self.ctx._chk(self.L.atsim_nn_weight_bias_grad(self.ctx.h, _p(dy), _p(h), _p(part), _p(gW), _p(bpart), _p(gb),
+                                                       Cout, Cin, SP, kc))
 
     def add_bias_act(self, a, b, bias, pre, y, Cc, P, gelu):
         n = a.numel()
@@ -327,17 +330,19 @@ class FNO:
         if pre is not None:
             self.ops.gelu_bwd(pre, out, out)
 
-    def _weight_grad(self, dy, h, gW, Cout, Cin, SP):
-        # gW[o][i] = sum_q dy[o][q] h[i][q], split over K chunks, partials summed in order
+    def _weight_grad(self, dy, h, gW, gb, Cout, Cin, SP):
+        # gW[o][i] = sum_q dy[o][q] h[i][q] and gb[o] = sum_q dy[o][q], split over K chunks, partials summed in order
         torch = _torch()
         kc = 1024 if SP % 1024 == 0 else SP
         nb = SP // kc
         part = torch.empty((nb, Cout, Cin), dtype=torch.float32, device=self.dev)
         if self.ops.weight_grad_ok(Cout, Cin, SP, kc, dy, h):
-            self.ops.weight_grad(dy, h, part, gW, Cout, Cin, SP, kc)
+            bpart = torch.empty((nb, Cout), dtype=torch.float64, device=self.dev)
+            self.ops.weight_grad(dy, h, part, gW, Cout, Cin, SP, kc, bpart, gb)
             return
         self.ops.gemm(Cout, Cin, kc, nb, dy, 0, kc, SP, 1, h, 0, kc, 1, SP, part, 0, Cout * Cin, Cin, 1)
         self.ops.reduce(part, gW, nb, Cout * Cin)
+        self.ops.bias_grad(dy, gb, Cout, SP)
 
     def _spectral(self, h, R, S, T=None):
         """U [C][S][N][2m], the retained spectrum of K h transformed back along y,
@@ -526,12 +531,10 @@ class FNO:
             ops.mse_begin(y, t, dy)
         else:
             ops.mse(y, t, dy, False)
-        self._weight_grad(dy, c["q1"], g["Q2"], self.cout, H, SP)
-        ops.bias_grad(dy, g["q2b"], self.cout, SP)
+        self._weight_grad(dy, c["q1"], g["Q2"], g["q2b"], self.cout, H, SP)
         dq1 = torch.empty_like(c["q1"])
         self._pointwise_t(p["Q2"], dy, dq1, self.cout, H, SP, pre=c["preq"])
-        self._weight_grad(dq1, c["hL"], g["Q1"], H, Cw, SP)
-        ops.bias_grad(dq1, g["q1b"], H, SP)
+        self._weight_grad(dq1, c["hL"], g["Q1"], g["q1b"], H, Cw, SP)
         dh = torch.empty_like(c["hL"])
         nb = self.blocks
         rows = self._rows(dh, p[f"R{nb - 1}"], H, S, 0, (dq1,), True) if nb > 0 else {}
@@ -539,8 +542,7 @@ class FNO:
         for b in reversed(range(self.blocks)):
             dpre = dh  # times GELU' already: by the pass that wrote it
             h = c[f"h{b}"]
-            ops.bias_grad(dpre, g[f"B{b}"], Cw, SP)
-            self._weight_grad(dpre, h, g[f"W{b}"], Cw, Cw, SP)
+            self._weight_grad(dpre, h, g[f"W{b}"], g[f"B{b}"], Cw, Cw, SP)
             dhn = torch.empty_like(h)
             dT1 = self._spectral_backward(dpre, p[f"R{b}"], c[f"B{b}"], S, g[f"R{b}"],
                                           rows.get("T"))
@@ -550,8 +552,7 @@ class FNO:
             self._map_add(p[f"W{b}"], 1, Cw, dpre, dT1, self.Fx, 1, 2 * self.m, dhn, SP,
                           pre=pre, act=2 if b > 0 else 0, rows=rows)
             dh = dhn
-        self._weight_grad(dh, c["x"], g["Lw"], Cw, self.cin, SP)
-        ops.bias_grad(dh, g["Lb"], Cw, SP)
+        self._weight_grad(dh, c["x"], g["Lw"], g["Lb"], Cw, self.cin, SP)
         return ops.mse_end(y.numel()) if want_loss else None
 
     @on_ctx_stream

@@ -448,6 +448,10 @@ int atsim_nn_mix_grad(atsim_ctx *ctx, const float *dO, const float *B, float *dR
  * (ATSIM_EUNSUPPORTED otherwise). */
 int atsim_nn_weight_grad(atsim_ctx *ctx, const float *dy, const float *h, float *part, float *gW, long Cout, long Cin,
                          long SP, long kc);
+/* the same with the bias gradient gb[o] = sum_q dy[o][q] from the same loads, in
+ * FP64 (bpart: SP / kc x Cout partial sums) */
+int atsim_nn_weight_bias_grad(atsim_ctx *ctx, const float *dy, const float *h, float *part, float *gW, double *bpart,
+                              float *gb, long Cout, long Cin, long SP, long kc);
 /* y = act(a + b + bias[c]) over n = S*C*P elements laid out [S][C][P]; b, bias
  * and pre may be NULL; pre keeps the activation's input; act = GELU (tanh
  * form) if gelu != 0, else identity. */

@@ -164,7 +164,7 @@ class Ops:
     def weight_grad_ok(Cout, Cin, SP, kc, dy, h):
         """the sizes and alignments atsim_nn_weight_grad takes; the others go
         through gemm and reduce"""
-        return (Cout <= 64 and Cin <= 64 and kc % 128 == 0 and SP % kc == 0
+        return (Cout <= 64 and Cin <= 64 and kc % 128 == 0 and kc <= 1 << 24 and SP % kc == 0
                 and dy.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
 
     def weight_grad(self, dy, h, part, gW, Cout, Cin, SP, kc, bpart=None, gb=None):

@@ -102,6 +102,43 @@ static int fail(atsim_ctx* c, int code, const char* fmt, ...) {
         if (e_ != hipSuccess) return fail((ctx), ATSIM_EHIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
+// The context's device as the calling thread's current one for a scope: device
+// memory, events and streams are made on the current device, whatever stream
+// they are for, and a program with contexts on several devices calls with any
+// of them current.
+struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(const atsim_ctx* c) {
+        int now = -1;
+        if (hipGetDevice(&now) == hipSuccess && now != c->device && hipSetDevice(c->device) == hipSuccess) prev = now;
+    }
+    ~OnDevice() {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+};
+// Device memory of the context; *p is null after a failure, which leaves no
+// error behind for a later hipGetLastError.
+template <class T>
+static hipError_t device_malloc(atsim_ctx* c, T** p, size_t bytes) {
+    OnDevice on(c);
+    hipError_t e = hipMalloc((void**)p, bytes);
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();
+    }
+    return e;
+}
+static hipError_t device_event(atsim_ctx* c, hipEvent_t* e, unsigned flags = hipEventDisableTiming) {
+    OnDevice on(c);
+    return hipEventCreateWithFlags(e, flags);
+}
+static hipError_t device_stream(atsim_ctx* c, hipStream_t* s) {
+    OnDevice on(c);
+    return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+}
+
 // Work space of one call, used on the context stream only (the next call's
 // kernels follow this one's): the context's own block, grown as needed and kept
 // up to SCRATCH_KEEP bytes (an 8192^2 master), so that a call does not wait for
@@ -128,11 +165,8 @@ struct Scratch {
             if (c->scratch) (void)hipFree(c->scratch);
             c->scratch = nullptr;
             c->scratch_cap = 0;
-            e = hipMalloc(&c->scratch, bytes);
-            if (e != hipSuccess) {
-                c->scratch = nullptr;
-                return e;
-            }
+            e = device_malloc(c, &c->scratch, bytes);
+            if (e != hipSuccess) return e;
             c->scratch_cap = bytes;
         }
         p = c->scratch;
@@ -167,7 +201,7 @@ static int get_twiddles(atsim_ctx* c, long n, float2** out) {
             }
     }
     float2* d = nullptr;
-    HIPCHK(c, hipMalloc(&d, sizeof(float2) * (n + extra)));
+    HIPCHK(c, device_malloc(c, &d, sizeof(float2) * (n + extra)));
     HIPCHK(c, copy_on_stream(c, d, h.data(), sizeof(float2) * (n + extra)));
     c->twiddles[n] = d;
     *out = d;
@@ -326,8 +360,7 @@ int atsim_malloc(atsim_ctx* c, void** ptr, size_t nbytes) {
     if (!c || !ptr) return ATSIM_EINVAL;
     *ptr = nullptr;
     HIPCHK(c, hipSetDevice(c->device));
-    if (hipMalloc(ptr, nbytes > 0 ? nbytes : 1) != hipSuccess) {
-        (void)hipGetLastError();
+    if (device_malloc(c, ptr, nbytes > 0 ? nbytes : 1) != hipSuccess) {
         return fail(c, ATSIM_ENOMEM, "cannot allocate %zu device bytes", nbytes);
     }
     return ATSIM_OK;
@@ -367,10 +400,10 @@ int atsim_host_free(atsim_ctx* c, void* ptr) {
 
 static int copy_stream_init(atsim_ctx* c) {
     if (c->copy_stream) return ATSIM_OK;
-    HIPCHK(c, hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
+    HIPCHK(c, device_stream(c, &c->copy_stream));
     for (int i = 0; i < ATSIM_COPY_SLOTS; i++) {
-        HIPCHK(c, hipEventCreateWithFlags(&c->copy_ready[i], hipEventDisableTiming));
-        HIPCHK(c, hipEventCreateWithFlags(&c->copy_done[i], hipEventDisableTiming));
+        HIPCHK(c, device_event(c, &c->copy_ready[i]));
+        HIPCHK(c, device_event(c, &c->copy_done[i]));
     }
     return ATSIM_OK;
 }
@@ -590,7 +623,7 @@ static int line_plan(atsim_ctx* c, long L, long nlines, int sign, LinePlan* out)
         for (long k = 0; k < M; k++)
             h[(size_t)(L + k)] = make_float2((float)(dr[(size_t)k] / M), (float)(di[(size_t)k] / M));
         float2* d = nullptr;
-        HIPCHK(c, hipMalloc(&d, sizeof(float2) * h.size()));
+        HIPCHK(c, device_malloc(c, &d, sizeof(float2) * h.size()));
         if (hipError_t e = copy_on_stream(c, d, h.data(), sizeof(float2) * h.size())) {
             hipFree(d);
             return fail(c, ATSIM_EHIP, "fft: table upload: %s", hipGetErrorString(e));
@@ -636,7 +669,7 @@ int atsim_fresnel(atsim_ctx* c, const void* d_in, void* d_out, long n, long nbat
     if (int r = get_twiddles(c, n, &tw)) return r;
     // the transfer factor is made on the device, in the context's own table (one
     // call's kernels follow the other's on the stream); the row pass reads d_in
-    if (!c->fresnel_tab) HIPCHK(c, hipMalloc(&c->fresnel_tab, sizeof(float2) * 8192));
+    if (!c->fresnel_tab) HIPCHK(c, device_malloc(c, &c->fresnel_tab, sizeof(float2) * 8192));
     HIPCHK(c, launch_fresnel_tables(c->fresnel_tab, nullptr, n, dx, lambda, z, z, 0, 1, 1, c->stream));
     HIPCHK(c, launch_row(n, OP_FRESNEL, 0, (const float2*)d_in, n * n, (float2*)d_out, nbatch, c->fresnel_tab, 1, tw,
                          c->stream));
@@ -1014,7 +1047,7 @@ enum {
 static hipEvent_t prof_event(atsim_sim* s) {
     if (s->ev_used == s->ev_pool.size()) {
         hipEvent_t e;
-        if (hipEventCreate(&e) != hipSuccess) return nullptr;
+        if (device_event(s->ctx, &e, hipEventDefault) != hipSuccess) return nullptr;
         s->ev_pool.push_back(e);
     }
     return s->ev_pool[s->ev_used++];
@@ -1138,8 +1171,7 @@ static int pipeline_init(atsim_sim* s) {
     const size_t nn = (size_t)s->N * s->N;
     auto alloc = [&](void** p, size_t bytes) {
         if (*p) return ATSIM_OK;
-        if (hipMalloc(p, bytes) != hipSuccess) {
-            *p = nullptr;
+        if (device_malloc(c, p, bytes) != hipSuccess) {
             return fail(c, ATSIM_ENOMEM, "pipeline: cannot allocate %zu bytes for a second buffer set", bytes);
         }
         return ATSIM_OK;
@@ -1154,11 +1186,11 @@ static int pipeline_init(atsim_sim* s) {
         if (int r = alloc((void**)&s->bsum_buf[1], sizeof(double) * bsum_doubles(F, nb))) return r;
     }
     for (int p = 0; p < 2; p++) {
-        if (!s->ev_head[p]) HIPCHK(c, hipEventCreateWithFlags(&s->ev_head[p], hipEventDisableTiming));
-        if (!s->ev_tail[p]) HIPCHK(c, hipEventCreateWithFlags(&s->ev_tail[p], hipEventDisableTiming));
+        if (!s->ev_head[p]) HIPCHK(c, device_event(c, &s->ev_head[p]));
+        if (!s->ev_tail[p]) HIPCHK(c, device_event(c, &s->ev_tail[p]));
     }
-    if (!s->ev_sync) HIPCHK(c, hipEventCreateWithFlags(&s->ev_sync, hipEventDisableTiming));
-    HIPCHK(c, hipStreamCreateWithFlags(&s->hs, hipStreamNonBlocking));
+    if (!s->ev_sync) HIPCHK(c, device_event(c, &s->ev_sync));
+    HIPCHK(c, device_stream(c, &s->hs));
     s->head_sync = true;
     return ATSIM_OK;
 }
@@ -1215,7 +1247,7 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
     int r = ATSIM_OK;
 #define SIMALLOC(ptr, bytes)                                                                       \
     do {                                                                                           \
-        if (r == ATSIM_OK && hipMalloc((void**)&(ptr), (bytes)) != hipSuccess)                     \
+        if (r == ATSIM_OK && device_malloc(c, &(ptr), (bytes)) != hipSuccess)                      \
             r = fail(c, ATSIM_ENOMEM, "sim: cannot allocate %zu bytes for " #ptr, (size_t)(bytes)); \
     } while (0)
     SIMALLOC(s->masters, sizeof(float) * s->L * s->M * s->M);
@@ -1245,17 +1277,17 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
     }
     if (r == ATSIM_OK && hipHostMalloc((void**)&s->ls_host, sizeof(LayerSample) * s->D * s->L * atsim_sim::RING) != hipSuccess)
         r = fail(c, ATSIM_ENOMEM, "sim: pinned allocation failed");
-    if (r == ATSIM_OK && (hipEventCreateWithFlags(&s->ev_fork, hipEventDisableTiming) != hipSuccess ||
-                          hipEventCreateWithFlags(&s->ev_phase, hipEventDisableTiming) != hipSuccess))
+    if (r == ATSIM_OK && (device_event(c, &s->ev_fork) != hipSuccess ||
+                          device_event(c, &s->ev_phase) != hipSuccess))
         r = fail(c, ATSIM_EHIP, "sim: event creation failed");
     for (int k = 0; r == ATSIM_OK && k < atsim_sim::MAX_SETS - 1; k++)
-        if (hipStreamCreateWithFlags(&s->xs_stream[k], hipStreamNonBlocking) != hipSuccess ||
-            hipEventCreateWithFlags(&s->ev_first[k], hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&s->ev_join[k], hipEventDisableTiming) != hipSuccess)
+        if (device_stream(c, &s->xs_stream[k]) != hipSuccess ||
+            device_event(c, &s->ev_first[k]) != hipSuccess ||
+            device_event(c, &s->ev_join[k]) != hipSuccess)
             r = fail(c, ATSIM_EHIP, "sim: stream / event creation failed");
     if (r == ATSIM_OK) {
         s->ls_ev = new hipEvent_t[atsim_sim::RING];
-        for (int i = 0; i < atsim_sim::RING; i++) hipEventCreateWithFlags(&s->ls_ev[i], hipEventDisableTiming);
+        for (int i = 0; i < atsim_sim::RING; i++) device_event(c, &s->ls_ev[i]);
     }
     std::vector<int> flist;
     for (long dd = 0; dd < s->D; dd++)
@@ -1293,9 +1325,7 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
         make_slots(1);
         s->row_planes = true;
         if (!s->factored) make_extra();
-        if (hipMalloc((void**)&s->vq, sizeof(double) * s->nslots * s->D * nn) != hipSuccess) {
-            (void)hipGetLastError();
-            s->vq = nullptr;
+        if (device_malloc(c, &s->vq, sizeof(double) * s->nslots * s->D * nn) != hipSuccess) {
             s->row_planes = false;
             layer_slot.clear();
             make_slots(2);
@@ -1834,11 +1864,11 @@ int atsim_sims_frame(atsim_sim** sims, long n, float** d_pha, float** d_amp) {
     for (long k = 0; k < n; k++) {
         atsim_sim* s = sims[k];
         if (!s->own) {
-            HIPCHK(c, hipStreamCreateWithFlags(&s->own, hipStreamNonBlocking));
-            HIPCHK(c, hipEventCreateWithFlags(&s->own_done, hipEventDisableTiming));
+            HIPCHK(c, device_stream(c, &s->own));
+            HIPCHK(c, device_event(c, &s->own_done));
         }
     }
-    if (!c->mg_fork) HIPCHK(c, hipEventCreateWithFlags(&c->mg_fork, hipEventDisableTiming));
+    if (!c->mg_fork) HIPCHK(c, device_event(c, &c->mg_fork));
     for (long k = 0; k < n; k++)
         if (int r = advance_positions(sims[k], c->stream)) return r;
     // every simulation's frame on its own stream, forked from and joined to
@@ -1879,7 +1909,7 @@ int atsim_sim_synth_masters(atsim_sim* s, uint64_t seed, const double* outerscal
     atsim_ctx* c = s->ctx;
     if (!supported_n(s->M)) return fail(c, ATSIM_EUNSUPPORTED, "synth_masters: M=%ld unsupported", s->M);
     float2* noise = nullptr;
-    HIPCHK(c, hipMalloc(&noise, sizeof(float2) * s->M * s->M));
+    HIPCHK(c, device_malloc(c, &noise, sizeof(float2) * s->M * s->M));
     int r = ATSIM_OK;
     for (long l = 0; l < s->L && r == ATSIM_OK; l++) {
         r = atsim_noise_c64(c, noise, s->M * s->M, seed, (uint32_t)l);
@@ -1974,8 +2004,8 @@ int atsim_sim_autotune(atsim_sim* s, float* d_pha, float* d_amp, int frames, cha
     if (cand[4].empty()) cand[4].push_back(0);
     cand[5] = (N >= 256 && N <= 2048) ? std::vector<int>{16, 32} : std::vector<int>{16};
     hipEvent_t e0, e1;
-    HIPCHK(c, hipEventCreate(&e0));
-    if (hipEventCreate(&e1) != hipSuccess) {
+    HIPCHK(c, device_event(c, &e0, hipEventDefault));
+    if (device_event(c, &e1, hipEventDefault) != hipSuccess) {
         hipEventDestroy(e0);
         return fail(c, ATSIM_EHIP, "autotune: event creation failed");
     }
@@ -2095,8 +2125,8 @@ int atsim_sim_stats_enable(atsim_sim* s, int enable) {
     atsim_ctx* c = s->ctx;
     const long F = s->D * s->W;
     if (enable && !s->st_out) {
-        HIPCHK(c, hipMalloc(&s->st_part, sizeof(double) * F * STATS_PART_PER_FIELD));
-        HIPCHK(c, hipMalloc(&s->st_out, sizeof(double) * F * 4));
+        HIPCHK(c, device_malloc(c, &s->st_part, sizeof(double) * F * STATS_PART_PER_FIELD));
+        HIPCHK(c, device_malloc(c, &s->st_out, sizeof(double) * F * 4));
         HIPCHK(c, hipMemsetAsync(s->st_out, 0, sizeof(double) * F * 4, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
     }
@@ -2137,9 +2167,9 @@ int atsim_block_fixup(atsim_ctx* c, const double* bsum, long xs, double* peaks) 
     unsigned* d_max = nullptr;
     int* d_f = nullptr;
     int r = ATSIM_OK;
-    if (hipMalloc(&d_sum, sizeof(double) * nb * 2) != hipSuccess || hipMalloc(&d_bin, sizeof(double) * nb) != hipSuccess ||
-        hipMalloc(&d_ch, sizeof(double) * nb) != hipSuccess || hipMalloc(&d_max, sizeof(unsigned)) != hipSuccess ||
-        hipMalloc(&d_f, sizeof(int)) != hipSuccess)
+    if (device_malloc(c, &d_sum, sizeof(double) * nb * 2) != hipSuccess || device_malloc(c, &d_bin, sizeof(double) * nb) != hipSuccess ||
+        device_malloc(c, &d_ch, sizeof(double) * nb) != hipSuccess || device_malloc(c, &d_max, sizeof(unsigned)) != hipSuccess ||
+        device_malloc(c, &d_f, sizeof(int)) != hipSuccess)
         r = fail(c, ATSIM_ENOMEM, "block fix-up: out of device memory");
     const int f0 = 0;
     const unsigned z0 = 0u;
@@ -2169,8 +2199,8 @@ int atsim_block_counts(atsim_ctx* c, const double* peaks, long xs, float* counts
     unsigned* d_max = nullptr;
     int* d_f = nullptr;
     int r = ATSIM_OK;
-    if (hipMalloc(&d_bin, sizeof(double) * nb) != hipSuccess || hipMalloc(&d_ch, sizeof(float) * nb) != hipSuccess ||
-        hipMalloc(&d_max, sizeof(unsigned)) != hipSuccess || hipMalloc(&d_f, sizeof(int)) != hipSuccess)
+    if (device_malloc(c, &d_bin, sizeof(double) * nb) != hipSuccess || device_malloc(c, &d_ch, sizeof(float) * nb) != hipSuccess ||
+        device_malloc(c, &d_max, sizeof(unsigned)) != hipSuccess || device_malloc(c, &d_f, sizeof(int)) != hipSuccess)
         r = fail(c, ATSIM_ENOMEM, "block counts: out of device memory");
     const int f0 = 0;
     const unsigned z0 = 0u;
@@ -2248,6 +2278,7 @@ int atsim_nn_lift_map_dft(atsim_ctx* c, const float* L, const float* Lb, long Cl
         !point_dft_supported(T, Cout, rowlen, m, U ? K2 : 0) || (L && (Cin > 32 || Cl > 32)))
         return fail(c, ATSIM_EUNSUPPORTED, "map and transform: %ld x %ld channels over rows of %ld, %ld modes", Cout, Cin,
                     rowlen, m);
+    OnDevice on(c);  // the kernels' LDS limits are raised on the current device
     c->work_gen++;
     HIPCHK(c, launch_pointwise(W, swm, swk, (int)Cout, (int)Cin, h, out, nrows, (int)rowlen, U, U ? (int)K2 : 0, F, sfk,
                                sfx, bias, pre, act, c->stream, D, dsk, dsn, (int)m, T, L, Lb, (int)Cl));
@@ -2267,6 +2298,7 @@ int atsim_nn_spectral_rows(atsim_ctx* c, const void* T, const float* Gre, const 
     const long images = C * S;
     if (!spectral_supported((const float*)T, U, B, O, R, images, N, m, C, S) || !point_dft_supported(T, C, N, m, 0))
         return fail(c, ATSIM_EUNSUPPORTED, "spectral: %ld channels, %ld samples of %ld^2, %ld modes", C, S, N, m);
+    OnDevice on(c);  // the kernels' LDS limits are raised on the current device
     c->work_gen++;
     HIPCHK(c, launch_dft_y(T, Gre, Gim, B, images, (int)N, (int)m, c->stream));
     HIPCHK(c, launch_mix(R, B, O, (int)C, (int)S, (int)(2 * m * m), adjoint != 0, c->stream));
@@ -2283,6 +2315,7 @@ int atsim_nn_spectral_fwd(atsim_ctx* c, const float* h, const float* F, long sfk
     const long images = C * S;
     if (!spectral_supported(h, U, B, O, R, images, N, m, C, S))
         return fail(c, ATSIM_EUNSUPPORTED, "spectral: %ld channels, %ld samples of %ld^2, %ld modes", C, S, N, m);
+    OnDevice on(c);  // the kernels' LDS limits are raised on the current device
     c->work_gen++;
     HIPCHK(c, launch_dft2(h, F, sfk, sfn, Gre, Gim, B, images, (int)N, (int)m, c->stream));
     HIPCHK(c, launch_mix(R, B, O, (int)C, (int)S, (int)(2 * m * m), adjoint != 0, c->stream));
@@ -2353,7 +2386,7 @@ int atsim_nn_bias_grad(atsim_ctx* c, const float* dy, float* db, long S, long C,
         if (c->nn_bias) hipFree(c->nn_bias);
         c->nn_bias = nullptr;
         c->nn_bias_cap = 0;
-        HIPCHK(c, hipMalloc(&c->nn_bias, need));
+        HIPCHK(c, device_malloc(c, &c->nn_bias, need));
         c->nn_bias_cap = need;
     }
     HIPCHK(c, launch_bias_grad(dy, c->nn_bias, S, C, P, nchunk, c->stream));
@@ -2365,7 +2398,7 @@ int atsim_nn_mse(atsim_ctx* c, const float* pred, const float* target, float* gr
     if (!c || !pred || !target || n <= 0) return ATSIM_EINVAL;
     c->work_gen++;
     const int nblk = 256;
-    if (!c->nn_part) HIPCHK(c, hipMalloc(&c->nn_part, sizeof(double) * nblk));
+    if (!c->nn_part) HIPCHK(c, device_malloc(c, &c->nn_part, sizeof(double) * nblk));
     HIPCHK(c, launch_mse(pred, target, grad, n, c->nn_part, nblk, c->stream));
     if (loss) {
         std::vector<double> v;
@@ -2385,7 +2418,7 @@ int atsim_nn_mse_begin(atsim_ctx* c, const float* pred, const float* target, flo
             return fail(c, ATSIM_ENOMEM, "mse: cannot allocate pinned host memory");
         }
     }
-    if (!c->nn_loss_ev) HIPCHK(c, hipEventCreateWithFlags(&c->nn_loss_ev, hipEventDisableTiming));
+    if (!c->nn_loss_ev) HIPCHK(c, device_event(c, &c->nn_loss_ev));
     if (int r = atsim_nn_mse(c, pred, target, grad, n, nullptr)) return r;
     HIPCHK(c, hipMemcpyAsync(c->nn_loss_host, c->nn_part, sizeof(double) * 256, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipEventRecord(c->nn_loss_ev, c->stream));

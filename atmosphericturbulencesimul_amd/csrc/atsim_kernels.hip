@@ -1391,8 +1391,9 @@ __device__ __forceinline__ void planes_phase(double a, double vr, double vl, dou
     pl = a * vl;
     phi = fma(a, vr, pl);
 }
-// The same from the layers' phase planes (quarter turns): the sums of s_wl V_l
-// over the layers before the last group (other) and over it (last).
+// The same from the layers' samples V_l in quarter turns, from their phase planes
+// or made here (the same values, sums and order: the same bits): the sums of
+// s_wl V_l over the layers outside the last group (other) and over it (last).
 __device__ __forceinline__ void layers_phase(double other, double last, double& phi, double& pl) {
 #pragma clang fp contract(off)
     pl = last * 1.57079632679489661923;
@@ -1402,6 +1403,18 @@ __device__ __forceinline__ void layers_phase(double other, double last, double& 
 __device__ __forceinline__ double rotated_arg(float2 E, double rot) {
 #pragma clang fp contract(off)
     return (double)atan2_poly(E.y, E.x) + rot;
+}
+// |E| with the hardware square root (1 ulp), the sum of squares in one written
+// order: left to contraction, one of the extraction's variants squared y inside
+// the multiply-add and another x
+__device__ __forceinline__ float field_amplitude(float2 E) {
+#pragma clang fp contract(off)
+    return __builtin_amdgcn_sqrtf(fmaf(E.x, E.x, E.y * E.y));
+}
+// the reference-wavelength rule: the whole turns of phi added to the wrapped phase
+__device__ __forceinline__ double plain_unwrap(double phw, double phi) {
+#pragma clang fp contract(off)
+    return fma(2.0 * M_PI, trunc(fma(phi, 0.15915494309189533577, 1000.5)) - 1000.0, phw);
 }
 // the block rule's whole turns n = rint((PHI - ph) / 2 pi) and FP64
 // remainder r = PHI - ph - 2 pi n
@@ -1443,7 +1456,9 @@ __device__ __forceinline__ float wave_inclusive_sum(float x) {
 //
 // MODE 0 does all of that.  MODE 1 reads the pixel's samples from the layers'
 // phase planes, made beside the first pass, when every layer has one and the
-// multipliers do not factor (1024^2, 7 layers, 5 wavelengths: 42 us against 62).  When
+// multipliers do not factor (1024^2, 7 layers, 5 wavelengths: 42 us against 62);
+// both give the same bits, as frames with the planes and without (pipelined ones,
+// or where the planes do not fit) have to.  When
 // the phase multipliers factor as
 // s_wl = a_w b_l, the sums need the layers only through two planes per
 // direction, Vr = sum b_l v_l over the layers before the last group and Vl
@@ -1611,13 +1626,14 @@ __global__ void __launch_bounds__(EXT_T) k_extract(ExtractArgs a) {
         }
         __syncthreads();
         if (valid) {
-            // the pixel's FP64 sample of staged layer q: its 4 x-filtered rows
+            // the pixel's FP64 sample of staged layer q in quarter turns, as the
+            // phase planes hold it: its 4 x-filtered rows
             auto sample = [&](int q) {
                 const LayerSample& p = sls[l0 + q];
                 double v = 0.0;
 #pragma unroll
                 for (int b = 0; b < 4; b++) v = fma(p.wy[b], H[q][wv + b][lane], v);
-                return v;
+                return v * 0.63661977236758134308;
             };
             // staged layers lo .. hi - 1 belong to the last group (uniform
             // bounds).  Two loops with straight bodies: one branch per layer
@@ -1645,7 +1661,7 @@ __global__ void __launch_bounds__(EXT_T) k_extract(ExtractArgs a) {
     // (from the planes it is the total already)
     if (MODE == 0) {
 #pragma unroll
-        for (int w = 0; w < 8; w++) PHI[w] += PL[w];
+        for (int w = 0; w < 8; w++) layers_phase(PHI[w], PL[w], PHI[w], PL[w]);
     }
     const double inv2pi = 0.15915494309189533577;
     // block column of lane + 1 (-1: none, or the last lane) and whether this
@@ -1685,17 +1701,15 @@ __global__ void __launch_bounds__(EXT_T) k_extract(ExtractArgs a) {
                     a.pha[oi] = (float)PHI[w];
                     a.amp[oi] = 1.f;
                 } else {
-                    // |E| with the hardware square root (1 ulp); arg E with
-                    // the polynomial arctangent (< 4e-7 rad)
-                    a.amp[oi] = __builtin_amdgcn_sqrtf(E.x * E.x + E.y * E.y);
-                    // arg of the rotated field, not yet brought into (-pi, pi]
+                    a.amp[oi] = field_amplitude(E);
+                    // arg (the polynomial arctangent, < 4e-7 rad) of the rotated field, not yet brought into (-pi, pi]
                     const double ph = rotated_arg(E, rot);
                     if (!block_rule) {
                         // this rule adds whole turns of PHI alone to the phase
                         // in (-pi, pi] (AT.c:3456), so the rotated phase is
                         // wrapped first
                         const double phw = fma(-6.283185307179586477, rint(ph * inv2pi), ph);
-                        a.pha[oi] = (float)(phw + 2.0 * M_PI * unwrap_count(PHI[w] * inv2pi));
+                        a.pha[oi] = (float)plain_unwrap(phw, PHI[w]);
                     } else {
                         // whole turns of PHI - atan2 go into the phase now, the
                         // FP64 remainder (rounded to float) waits for the

@@ -705,17 +705,24 @@ int atsim_fresnel_nm(atsim_ctx* c, const void* d_in, void* d_out, long n0, long 
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return r;
     }
-    // even sides: rows, then columns with the factor and back, then rows back
+    // even sides: rows, then columns with the factor and back, then rows back.
+    // The first pass reads d_in row by row while it writes d_out: where the two
+    // overlap without being one, it reads a copy.
     LinePlan xf, xb, yf, yb;
     if (int r = line_plan(c, n0, n1 * nbatch, -1, &xf)) return r;
     if (int r = line_plan(c, n0, n1 * nbatch, +1, &xb)) return r;
     if (int r = line_plan(c, n1, n0 * nbatch, -1, &yf)) return r;
     if (int r = line_plan(c, n1, n0 * nbatch, +1, &yb)) return r;
+    const size_t bytes = sizeof(float2) * n0 * n1 * nbatch, factors = sizeof(double2) * (n0 + n1);
+    const uintptr_t ia = (uintptr_t)d_in, oa = (uintptr_t)d_out;
+    const bool copy = ia != oa && ia < oa + bytes && oa < ia + bytes;
     Scratch work(c);
-    HIPCHK(c, work.get(sizeof(double2) * (n0 + n1)));
+    HIPCHK(c, work.get(factors + (copy ? bytes : 0)));
     double2* h = (double2*)work.p;
+    const float2* src = copy ? (const float2*)(h + n0 + n1) : (const float2*)d_in;
+    if (copy) HIPCHK(c, hipMemcpyAsync(h + n0 + n1, d_in, bytes, hipMemcpyDeviceToDevice, c->stream));
     hipError_t e = launch_any_factor(h, h + n0, n0, n1, coeff, c->stream);
-    if (e == hipSuccess) e = launch_any_row(xf, -1, (const float2*)d_in, out, n1 * nbatch, c->stream);
+    if (e == hipSuccess) e = launch_any_row(xf, -1, src, out, n1 * nbatch, c->stream);
     if (e == hipSuccess) e = launch_any_col(yf, &yb, 0, out, n0, nbatch, h, h + n0, c->stream);
     if (e == hipSuccess) e = launch_any_row(xb, +1, out, out, n1 * nbatch, c->stream);
     if (e != hipSuccess) return fail(c, ATSIM_EHIP, "fresnel_nm: %s", hipGetErrorString(e));

@@ -177,7 +177,9 @@ int atsim_fresnel_noalloc(atsim_ctx *ctx, const void *d_in, void *d_out, long n,
 /* Fresnel_propagate_wavefront on any n0 x n1 shape (WFpropagate.c:68-152):
  * FFT, permut, e^{-i coeff ((ii - n0/2)^2 + (jj - n1/2)^2)} / (n0 n1) with
  * coeff = pi z lambda / (dx n0)^2 (n0 for both axes, as the reference),
- * permut, inverse FFT.  Square power-of-two images take atsim_fresnel. */
+ * permut, inverse FFT.  d_in and d_out may be the same memory, and (images that
+ * are no powers of two) may overlap.  Square power-of-two images take
+ * atsim_fresnel. */
 int atsim_fresnel_nm(atsim_ctx *ctx, const void *d_in, void *d_out, long n0, long n1, long nbatch,
                      double pupil_scale, double z, double lambda);
 /* Init_Fresnel_propagate_wavefront (WFpropagate.c:166-261): fills the

@@ -868,7 +868,8 @@ static hipError_t col_dispatch(int op, int dir, float2* data, long F, const floa
         // 32 elements per thread exchanging through half the LDS: twice the
         // columns (64 and 32 bytes of a row) in a workgroup (one Fresnel call on
         // 4 fields of 4096^2: 684 against 792 us; 8192^2: 966 against 1 038)
-        if (c <= 0) return col_split_launch<N, N == 4096 ? 8 : 4>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
+        if (c <= 0 && e != 16)
+            return col_split_launch<N, N == 4096 ? 8 : 4>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
     }
     if constexpr (N == 2048) {
         // two workgroups a CU instead of one (forward and backward transform of 4

@@ -61,14 +61,19 @@ int atsim_copy_wait(atsim_ctx *ctx, int slot);
 int atsim_stream_wait_copy(atsim_ctx *ctx, int slot);
 /* Launch-shape tuning of this context (0 restores the built-in default):
  *   "row_mw"  wavelength fields per workgroup of the row passes that sample
- *             the layers or apply none (1..8; default 8192 / n, at most 8)
- *   "col_c"   columns per column-pass workgroup (2, 4, 8, 16)
- *   "col_e"   elements per thread of the column Fresnel pass (16, or 32:
- *             8 columns per workgroup exchanging through half the LDS).
- *             32 applies only to Fresnel column passes with 256 <= n <= 2048
- *             and col_c 0, 8 or 16; plain FFT passes, other sizes and
- *             col_c 2 or 4 run the 16-element kernel (the value is kept and
- *             atsim_get_tuning returns it)
+ *             the layers themselves (1..8; default 8192 / n, at most 8): a
+ *             frame's first pass, unless it has one wavelength and phase planes,
+ *             every pass with gap_passes 2, and the passes between two gaps
+ *             where they have no phase planes.  Row passes that read planes or
+ *             apply no screen take workgroups of one wave where it holds a row
+ *   "col_c"   columns per workgroup of the column passes without a screen (2,
+ *             4, 8, 16; default by size and number of fields)
+ *   "col_e"   elements per thread of the column Fresnel pass: 16, or 32
+ *             (exchanging through half the LDS).  Default: 32 at n = 2048 from
+ *             2 fields on and from n = 4096 on, else 16.  32 is built for 256
+ *             <= n <= 2048 with col_c 0, 8 or 16 and for n >= 4096 with col_c
+ *             0; elsewhere the 16-element kernel runs (the value is kept and
+ *             atsim_get_tuning returns it).  Plain transforms take the defaults
  *   "streams" S = 2..4 (default 2): the Fresnel passes of S contiguous sets
  *             of the wavelengths run as S chains on S streams (set k started
  *             after set k - 1's first row pass) and join before the

@@ -54,6 +54,10 @@ struct atsim_ctx {
     // the simulation's own stream beside frame k's extraction and block
     // fix-up, which stay on the context stream (two buffer sets alternate)
     int pipeline = 0;
+    // 1: simulations keep phase planes for their row passes and, where the
+    // multipliers do not factor, for the extraction, where the memory allows;
+    // 2: for the column passes only
+    int row_planes = 1;
     unsigned tuning_gen = 0;  // bumped by every accepted atsim_set_tuning: captured frame graphs are stale
     // bumped by every call that enqueues device writes on the context stream:
     // a pipelined frame's passes then wait for that stream first
@@ -69,6 +73,8 @@ struct atsim_ctx {
     // work space of calls on the context stream (Scratch), kept between them
     void* scratch = nullptr;
     size_t scratch_cap = 0;
+    int scratch_users = 0;          // running calls that hold it
+    std::vector<atsim_sim*> sims;   // simulations on this context
     double* nn_loss_host = nullptr;  // pinned: partial sums of a loss read later
     hipEvent_t nn_loss_ev = nullptr;
     double* nn_part = nullptr;  // 256 partial sums of the network's loss reduction
@@ -118,16 +124,26 @@ struct OnDevice {
     OnDevice(const OnDevice&) = delete;
     OnDevice& operator=(const OnDevice&) = delete;
 };
+// Frees one block that is only kept for speed (the scratch block, then the
+// optional phase planes of a simulation); false when there is none left.
+static bool give_back(atsim_ctx* c);
 // Device memory of the context; *p is null after a failure, which leaves no
 // error behind for a later hipGetLastError.
 template <class T>
-static hipError_t device_malloc(atsim_ctx* c, T** p, size_t bytes) {
+static hipError_t plain_malloc(atsim_ctx* c, T** p, size_t bytes) {
     OnDevice on(c);
     hipError_t e = hipMalloc((void**)p, bytes);
     if (e != hipSuccess) {
         *p = nullptr;
         (void)hipGetLastError();
     }
+    return e;
+}
+// The same, giving back what the context can do without rather than failing.
+template <class T>
+static hipError_t device_malloc(atsim_ctx* c, T** p, size_t bytes) {
+    hipError_t e = plain_malloc(c, p, bytes);
+    while (e != hipSuccess && give_back(c)) e = plain_malloc(c, p, bytes);
     return e;
 }
 static hipError_t device_event(atsim_ctx* c, hipEvent_t* e, unsigned flags = hipEventDisableTiming) {
@@ -141,22 +157,31 @@ static hipError_t device_stream(atsim_ctx* c, hipStream_t* s) {
 
 // Work space of one call, used on the context stream only (the next call's
 // kernels follow this one's): the context's own block, grown as needed and kept
-// up to SCRATCH_KEEP bytes (an 8192^2 master), so that a call does not wait for
-// an allocation; more than that is allocated for the call alone.
+// up to SCRATCH_KEEP bytes (an 8192^2 master) until the memory is wanted, so that
+// a call does not wait for an allocation; more than that is allocated for the
+// call alone.
 static constexpr size_t SCRATCH_KEEP = (size_t)640 << 20;
 struct Scratch {
     atsim_ctx* c;
     void* p = nullptr;
-    bool own = false;
+    bool own = false, held = false;
     explicit Scratch(atsim_ctx* ctx) : c(ctx) {}
     ~Scratch() {
         if (own && p) (void)hipFreeAsync(p, c->stream);
+        if (held) c->scratch_users--;
     }
+    Scratch(const Scratch&) = delete;
+    Scratch& operator=(const Scratch&) = delete;
     hipError_t get(size_t bytes) {
-        if (bytes > SCRATCH_KEEP) {
+        if (bytes > SCRATCH_KEEP || c->scratch_users > 0) {
             own = true;
             hipError_t e = hipMallocAsync(&p, bytes, c->stream);
-            if (e != hipSuccess) p = nullptr;
+            while (e != hipSuccess) {
+                p = nullptr;
+                (void)hipGetLastError();
+                if (!give_back(c)) break;
+                e = hipMallocAsync(&p, bytes, c->stream);
+            }
             return e;
         }
         if (bytes > c->scratch_cap) {
@@ -169,6 +194,8 @@ struct Scratch {
             if (e != hipSuccess) return e;
             c->scratch_cap = bytes;
         }
+        held = true;
+        c->scratch_users++;
         p = c->scratch;
         return hipSuccess;
     }
@@ -462,6 +489,9 @@ int atsim_set_tuning(atsim_ctx* c, const char* key, int value) {
     } else if (!strcmp(key, "extract_planes")) {
         if (value < 0 || value > 2) return fail(c, ATSIM_EINVAL, "extract_planes must be 0, 1 or 2");
         c->extract_planes = value == 0 ? 1 : value;
+    } else if (!strcmp(key, "row_planes")) {
+        if (value < 0 || value > 2) return fail(c, ATSIM_EINVAL, "row_planes must be 0, 1 or 2");
+        c->row_planes = value == 0 ? 1 : value;
     } else if (!strcmp(key, "pipeline")) {
         if (value != 0 && value != 1) return fail(c, ATSIM_EINVAL, "pipeline must be 0 or 1");
         c->pipeline = value;
@@ -483,6 +513,7 @@ int atsim_get_tuning(atsim_ctx* c, const char* key) {
     if (!strcmp(key, "graph")) return c->graph;
     if (!strcmp(key, "extract_planes")) return c->extract_planes;
     if (!strcmp(key, "block_apply")) return c->block_apply;
+    if (!strcmp(key, "row_planes")) return c->row_planes;
     if (!strcmp(key, "pipeline")) return c->pipeline;
     return ATSIM_EINVAL;
 }
@@ -979,15 +1010,18 @@ struct atsim_sim {
     int* flist_dev = nullptr;
     // sampled phase planes of the layers whose screens the passes between two
     // gaps apply (one pass per gap; row_planes false: only the column passes):
-    // [nslots][D][N][N] FP64 quarter turns
+    // [nslots][D][N][N] FP64 quarter turns (set_planes)
     double* vq = nullptr;
     bool row_planes = false, gen_planes = false;
-    int* slot_layer_dev = nullptr;
+    int* slot_layer_dev = nullptr;  // [L], nslots of them used
     // nslots planes, the first pass_slots of them for the passes; the others (with
     // layer_slot_dev [L], the plane of each layer) for the extraction of
-    // multipliers that do not factor
+    // multipliers that do not factor (layer_planes)
     int nslots = 0, pass_slots = 0;
+    bool layer_planes = false;
     int* layer_slot_dev = nullptr;
+    unsigned planes_gen = 0;   // the context's tuning generation the planes were chosen at
+    bool replanned = false;    // the planes changed: the next frame runs eagerly
     int nblockfields = 0;
     int xs = 0;
     // per-frame output statistics (atsim_sim_stats_enable): partial sums and
@@ -1097,7 +1131,11 @@ static void sim_drop_graph(atsim_sim* s) {
 
 static void sim_free(atsim_sim* s) {
     if (!s) return;
-    if (s->ctx) hipStreamSynchronize(s->ctx->stream);
+    if (s->ctx) {
+        hipStreamSynchronize(s->ctx->stream);
+        auto& v = s->ctx->sims;
+        v.erase(std::remove(v.begin(), v.end(), s), v.end());
+    }
     if (s->hs) hipStreamSynchronize(s->hs);
     sim_drop_graph(s);
     if (s->own) hipStreamDestroy(s->own);
@@ -1143,6 +1181,129 @@ static void sim_free(atsim_sim* s) {
     hipFree(s->st_out);
     for (auto e : s->ev_pool) (void)hipEventDestroy(e);
     delete s;
+}
+
+// ------------------------------------------------------------------ phase planes
+// One pass per gap: pass k (0 <= k < G; columns for odd k) applies group k from
+// its layers' phase planes.  The column passes need them; the row passes can
+// sample their layers themselves, and so can the extraction, so their planes are
+// optional: they are taken last, where they and the second buffer set of
+// pipelined frames fit in half of the free memory, and given back when an
+// allocation of the context fails.
+struct PlanePlan {
+    std::vector<int> slot_layer;  // layer of each plane
+    std::vector<int> layer_slot;  // plane of each layer, if every layer has one for the extraction
+    std::vector<int> slot0;       // first plane of each group
+    int pass_slots = 0;
+    bool gen = false;             // the first pass has planes too
+};
+
+static bool uses_planes(const atsim_sim* s) {
+    return s->propagate && col_screen_supported(s->N) && s->groups.size() >= 3;
+}
+
+static PlanePlan plan_planes(const atsim_sim* s, bool all) {
+    PlanePlan p;
+    const long G = (long)s->groups.size() - 1;
+    p.slot0.assign(s->groups.size(), 0);
+    // one wavelength (one chain of passes, after the planes): group 0's too
+    p.gen = all && s->W == 1;
+    for (long k = p.gen ? 0 : 1; k < G; k += all ? 1 : 2) {
+        p.slot0[k] = (int)p.slot_layer.size();
+        for (int q = 0; q < s->groups[k].lcount; q++) p.slot_layer.push_back(s->groups[k].lfirst + q);
+    }
+    p.pass_slots = (int)p.slot_layer.size();
+    if (all && !s->factored) {
+        // a plane of every layer, those that no pass reads after the others
+        p.layer_slot.assign((size_t)s->L, -1);
+        for (size_t q = 0; q < p.slot_layer.size(); q++) p.layer_slot[p.slot_layer[q]] = (int)q;
+        for (long l = 0; l < s->L; l++)
+            if (p.layer_slot[l] < 0) {
+                p.layer_slot[l] = (int)p.slot_layer.size();
+                p.slot_layer.push_back((int)l);
+            }
+    }
+    return p;
+}
+
+static size_t planes_bytes(const atsim_sim* s, const PlanePlan& p) {
+    return sizeof(double) * p.slot_layer.size() * (size_t)s->D * s->N * s->N;
+}
+
+// Replace the planes by those of all passes (all) or of the column passes.
+// Without memory for them the simulation has none, and takes two passes per gap.
+static int set_planes(atsim_sim* s, bool all) {
+    atsim_ctx* c = s->ctx;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (s->hs) HIPCHK(c, hipStreamSynchronize(s->hs));
+    sim_drop_graph(s);
+    s->replanned = true;
+    s->head_sync = true;
+    if (s->vq) (void)hipFree(s->vq);
+    s->vq = nullptr;
+    s->nslots = s->pass_slots = 0;
+    s->row_planes = s->gen_planes = s->layer_planes = false;
+    const PlanePlan p = plan_planes(s, all);
+    if (plain_malloc(c, &s->vq, planes_bytes(s, p)) != hipSuccess)
+        return fail(c, ATSIM_ENOMEM, "sim: cannot allocate %zu bytes of phase planes", planes_bytes(s, p));
+    HIPCHK(c, copy_on_stream(c, s->slot_layer_dev, p.slot_layer.data(), sizeof(int) * p.slot_layer.size()));
+    if (!p.layer_slot.empty())
+        HIPCHK(c, copy_on_stream(c, s->layer_slot_dev, p.layer_slot.data(), sizeof(int) * p.layer_slot.size()));
+    for (size_t k = 0; k < p.slot0.size(); k++) s->groups[k].slot0 = p.slot0[k];
+    s->nslots = (int)p.slot_layer.size();
+    s->pass_slots = p.pass_slots;
+    s->row_planes = all;
+    s->gen_planes = p.gen;
+    s->layer_planes = !p.layer_slot.empty();
+    return ATSIM_OK;
+}
+
+// bytes of the second buffer set of pipelined frames that are not allocated yet
+static size_t second_set_bytes(const atsim_sim* s) {
+    const size_t nn = (size_t)s->N * s->N;
+    size_t b = 0;
+    if (s->fields_buf[0] && !s->fields_buf[1]) b += sizeof(float2) * s->D * s->W * nn;
+    if (s->vgeo_buf[0] && !s->vgeo_buf[1]) b += sizeof(double) * 2 * s->D * nn;
+    return b;
+}
+
+// The planes that the tuning asks for and the memory allows; called where the
+// tuning changed since they were last chosen.
+static int choose_planes(atsim_sim* s) {
+    atsim_ctx* c = s->ctx;
+    s->planes_gen = c->tuning_gen;
+    if (!uses_planes(s)) return ATSIM_OK;
+    bool want = c->row_planes == 1 && c->gap_passes == 1;
+    if (s->vq && want == s->row_planes) return ATSIM_OK;
+    if (want) {
+        OnDevice on(c);
+        size_t room = 0, total = 0;
+        HIPCHK(c, hipMemGetInfo(&room, &total));
+        want = planes_bytes(s, plan_planes(s, true)) + second_set_bytes(s) <= room / 2;
+        if (s->vq && !want) return ATSIM_OK;
+    }
+    if (want && set_planes(s, true) == ATSIM_OK) return ATSIM_OK;
+    int r = set_planes(s, false);
+    while (r == ATSIM_ENOMEM && give_back(c)) r = set_planes(s, false);
+    return r;
+}
+
+static bool give_back(atsim_ctx* c) {
+    if (c->scratch && c->scratch_users == 0) {
+        (void)hipStreamSynchronize(c->stream);
+        (void)hipFree(c->scratch);
+        c->scratch = nullptr;
+        c->scratch_cap = 0;
+        return true;
+    }
+    for (atsim_sim* s : c->sims)
+        if (s->row_planes) {
+            const std::string err = c->err;
+            (void)set_planes(s, false);
+            c->err = err;
+            return true;
+        }
+    return false;
 }
 
 extern "C" {
@@ -1301,46 +1462,9 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
         for (long w = 0; w < s->W; w++)
             if (s->unwrap[w] != 0 && s->amplitude) flist.push_back((int)(dd * s->W + w));
     s->nblockfields = (int)flist.size();
-    // one pass per gap: pass k (0 <= k < G; columns for odd k) applies group k
-    // from its layers' phase planes.  Without the memory for every group's planes
-    // only the column passes have them and the row passes sample the layers.
-    std::vector<int> slot_layer, layer_slot;
-    // multipliers that do not factor: a plane of every layer, those of the top and
-    // the last group after the others, for the extraction
-    auto make_extra = [&] {
-        s->pass_slots = s->nslots;
-        layer_slot.assign((size_t)s->L, -1);
-        for (size_t q = 0; q < slot_layer.size(); q++) layer_slot[slot_layer[q]] = (int)q;
-        for (long l = 0; l < s->L; l++)
-            if (layer_slot[l] < 0) {
-                layer_slot[l] = (int)slot_layer.size();
-                slot_layer.push_back((int)l);
-            }
-        s->nslots = (int)slot_layer.size();
-    };
-    auto make_slots = [&](long step) {
-        slot_layer.clear();
-        // one wavelength (one chain of passes, after the planes): group 0's too
-        s->gen_planes = step == 1 && s->W == 1;
-        for (long k = s->gen_planes ? 0 : 1; k < G; k += step) {
-            s->groups[k].slot0 = (int)slot_layer.size();
-            for (int q = 0; q < s->groups[k].lcount; q++) slot_layer.push_back(s->groups[k].lfirst + q);
-        }
-        s->nslots = (int)slot_layer.size();
-    };
-    if (r == ATSIM_OK && s->propagate && col_screen_supported(s->N) && G >= 2) {
-        make_slots(1);
-        s->row_planes = true;
-        if (!s->factored) make_extra();
-        if (device_malloc(c, &s->vq, sizeof(double) * s->nslots * s->D * nn) != hipSuccess) {
-            s->row_planes = false;
-            layer_slot.clear();
-            make_slots(2);
-            SIMALLOC(s->vq, sizeof(double) * s->nslots * s->D * nn);
-        }
-        SIMALLOC(s->slot_layer_dev, sizeof(int) * s->nslots);
-        if (!layer_slot.empty()) SIMALLOC(s->layer_slot_dev, sizeof(int) * s->L);
-        else s->pass_slots = s->nslots;
+    if (uses_planes(s)) {
+        SIMALLOC(s->slot_layer_dev, sizeof(int) * s->L);
+        if (!s->factored) SIMALLOC(s->layer_slot_dev, sizeof(int) * s->L);
     }
     s->xs = (int)(s->Nout / 20);
     if (s->nblockfields > 0) {
@@ -1382,18 +1506,16 @@ int atsim_sim_create(atsim_ctx* c, const atsim_sim_desc* d, atsim_sim** out) {
             copy_on_stream(c, s->blk, blk.data(), sizeof(int) * blk.size()) != hipSuccess ||
             (s->nblockfields > 0 &&
              (copy_on_stream(c, s->flist_dev, flist.data(), sizeof(int) * flist.size()) != hipSuccess ||
-              copy_on_stream(c, s->bstart, bstart.data(), sizeof(int) * bstart.size()) != hipSuccess)) ||
-            (s->layer_slot_dev &&
-             copy_on_stream(c, s->layer_slot_dev, layer_slot.data(), sizeof(int) * layer_slot.size()) != hipSuccess) ||
-            (s->nslots > 0 &&
-             copy_on_stream(c, s->slot_layer_dev, slot_layer.data(), sizeof(int) * slot_layer.size()) != hipSuccess))
+              copy_on_stream(c, s->bstart, bstart.data(), sizeof(int) * bstart.size()) != hipSuccess)))
             r = fail(c, ATSIM_EHIP, "sim: parameter upload failed");
     }
+    if (r == ATSIM_OK) r = choose_planes(s);  // last: into what the rest leaves
     if (r == ATSIM_OK && hipStreamSynchronize(c->stream) != hipSuccess) r = fail(c, ATSIM_EHIP, "sim: init sync failed");
     if (r != ATSIM_OK) {
         sim_free(s);
         return r;
     }
+    c->sims.push_back(s);
     *out = s;
     return ATSIM_OK;
 }
@@ -1607,7 +1729,7 @@ static int enqueue_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field
     const bool full = d_field != nullptr;
     // other multipliers: the extraction reads the layers' planes (one set of
     // them: not when the next frame's passes run beside it)
-    const bool layers = !s->factored && c->extract_planes == 1 && fused && s->layer_slot_dev && part == FRAME_ALL;
+    const bool layers = !s->factored && c->extract_planes == 1 && fused && s->layer_planes && part == FRAME_ALL;
     if (layers) {
         a.lv = s->vq;
         a.lslot = s->layer_slot_dev;
@@ -1808,8 +1930,13 @@ int atsim_sim_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field) {
         s->graph_gen = c->tuning_gen;
         retuned = true;
     }
-    const bool eager = !c->graph || s->prof || s->frames_done == 0 || retuned;
     const bool pipe = c->pipeline == 1 && s->propagate && !s->prof;
+    if (s->planes_gen != c->tuning_gen)
+        if (int r = choose_planes(s)) return r;
+    if (pipe)
+        if (int r = pipeline_init(s)) return r;
+    const bool eager = !c->graph || s->prof || s->frames_done == 0 || retuned || s->replanned;
+    s->replanned = false;
     if (!pipe) {
         // the whole frame on the context stream; a later pipelined frame's
         // passes wait for it
@@ -1830,7 +1957,6 @@ int atsim_sim_frame(atsim_sim* s, float* d_pha, float* d_amp, void* d_field) {
     // last read by the extraction of two frames back, so the passes wait for
     // it; they wait for the whole context stream when something other than
     // this simulation's frames wrote device memory there since its last frame.
-    if (int r = pipeline_init(s)) return r;
     const int p = s->parity ^ 1;
     use_buffers(s, p);
     hipStream_t hs = s->hs, ts = c->stream;
@@ -1876,6 +2002,9 @@ int atsim_sims_frame(atsim_sim** sims, long n, float** d_pha, float** d_amp) {
         }
     }
     if (!c->mg_fork) HIPCHK(c, device_event(c, &c->mg_fork));
+    for (long k = 0; k < n; k++)
+        if (sims[k]->planes_gen != c->tuning_gen)
+            if (int r = choose_planes(sims[k])) return r;
     for (long k = 0; k < n; k++)
         if (int r = advance_positions(sims[k], c->stream)) return r;
     // every simulation's frame on its own stream, forked from and joined to

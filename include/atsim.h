@@ -86,9 +86,17 @@ int atsim_stream_wait_copy(atsim_ctx *ctx, int slot);
  *             screen and the x (y) factor of the gap after it (n <= 4096,
  *             at least 2 gaps; the screens of the column passes' layers are
  *             sampled once per frame and direction into FP64 planes of
- *             n^2 x 8 bytes each, those of the row passes between two gaps
- *             too where the memory allows); 2: a row pass (screen, x factor) and a
+ *             n^2 x 8 bytes each); 2: a row pass (screen, x factor) and a
  *             column pass (y factor) per gap
+ *   "row_planes" 1 (default): with one pass per gap the row passes between two
+ *             gaps read such planes too, and with multipliers that do not
+ *             factor the extraction reads a plane of every layer, where these
+ *             planes and the second buffer set of "pipeline" fit in half of the
+ *             device's free memory; they are given back when a later allocation
+ *             of the context fails (atsim_malloc, another simulation, a second
+ *             buffer set, work space), and the frames after that are made as
+ *             with 2: the row passes and the extraction sample the layers
+ *             themselves.  The fields of both agree to their rounding
  *   "col2_e"  elements per thread of the column passes that apply a screen
  *             (16, or 32: 8 columns per workgroup exchanging through half
  *             the LDS, for 256 <= n <= 4096; default by size and fields)
@@ -103,10 +111,9 @@ int atsim_stream_wait_copy(atsim_ctx *ctx, int slot);
  *             layers before the last group and over the last group, 16 n^2
  *             bytes) by a kernel that runs beside the Fresnel passes, and
  *             the extraction reads them (PHI_w = a_w Vr + a_w Vl) instead of
- *             sampling every layer; with other multipliers and one pass per
- *             gap every layer is sampled into a phase plane and the extraction
- *             reads those (where the memory allows, and not in pipelined
- *             frames); 2: the extraction samples the layers
+ *             sampling every layer; with other multipliers it reads the layers'
+ *             planes of "row_planes" where there are any (not in pipelined
+ *             frames; the same bits); 2: the extraction samples the layers
  *   "block_apply" 1 (default): the final update of the block unwrap rule
  *             visits only the blocks where a count can be non-zero (from
  *             each block's largest |r|, kept by the extraction); 2: every

@@ -15,3 +15,63 @@ def test_column_elements(ctx, N, W):
     want = _frame(ctx, N, W, 1, True, gap_passes=2)
     for keys in (dict(col_e=16), dict(col_e=32), dict(col_c=2)):
         assert rel_l2(_frame(ctx, N, W, 1, True, gap_passes=2, **keys), want) < 5e-6
+
+
+# the row passes without phase planes (k_row_fresnel with a factor before the
+# group), as where the planes do not fit; every grid size, one to several
+# wavelengths a workgroup, groups of one and two layers
+@pytest.mark.parametrize("N,W,D", [(16, 1, 1), (16, 5, 3), (64, 8, 2), (128, 3, 1), (256, 5, 4), (512, 8, 1),
+                                   (1024, 1, 1), (1024, 5, 2), (2048, 3, 1), (4096, 1, 1)])
+@pytest.mark.parametrize("factored", [True, False])
+def test_rows_without_planes(ctx, N, W, D, factored):
+    print(f"rows without planes N={N} W={W} D={D} factored={factored}", flush=True)
+    want = _frame(ctx, N, W, D, factored, True)
+    for keys in (dict(), dict(streams=1), dict(row_mw=1), dict(pipeline=1)):
+        assert rel_l2(_frame(ctx, N, W, D, factored, True, row_planes=2, **keys), want) < 5e-6
+    assert rel_l2(_frame(ctx, N, W, D, factored, True, gap_passes=2, streams=1), want) < 5e-6
+
+
+# one simulation through the changes between frames, graphs replayed: each frame
+# agrees with the same frame of a simulation that never changes
+@pytest.mark.parametrize("factored", [True, False])
+@pytest.mark.parametrize("pipeline", [0, 1])
+def test_planes_changed_between_frames(factored, pipeline):
+    import numpy as np
+    from atmosphericturbulencesimul_amd.api import Context, Simulation
+    N, W, L = 256, 3, 6
+    lam = np.linspace(0.6e-6, 2.0e-6, W)
+    sc = np.array([[0.5e-6 / m * (1.0 if factored else 1.0 + 1e-3 * l * w) for l in range(L)]
+                   for w, m in enumerate(lam)])
+    x0 = np.array([[10.3 + l for l in range(L)]])
+
+    def make():
+        c = Context(0)
+        c.set_tuning("graph", 1)
+        s = Simulation(c, N, N, N, np.array([0.0, 4000.0, 8000.0, 12000.0]), [0, 0, 1, 2, 2, 3], lam, sc, [0] * W, x0,
+                       x0[:, ::-1], np.linspace(100.0, 900.0, L), np.linspace(-500.0, 700.0, L), 0.02, 0.001)
+        s.synth_masters(7, 400.0, 1.0)
+        s.normalize_masters(6.0, np.array([0.4, 0.2, 0.15, 0.1, 0.1, 0.05]))
+        return c, s
+
+    (c0, a), (c1, b) = make(), make()
+    c1.set_tuning("pipeline", pipeline)
+    for k in range(16):
+        if k in (3, 9):
+            c1.set_tuning("row_planes", 2)
+        if k in (6, 12):
+            c1.set_tuning("row_planes", 1)
+        if k == 13:
+            c1.set_tuning("gap_passes", 2)
+        if k == 14:
+            c1.set_tuning("gap_passes", 1)
+        want = [t.cpu().numpy() for t in a.frame()]
+        got = [t.cpu().numpy() for t in b.frame()]
+        print("frame", k, flush=True)
+        # (phases as unit vectors: a count of turns may hang on a rounding)
+        z = [amp * np.exp(1j * pha.astype(np.float64)) for pha, amp in (got, want)]
+        assert rel_l2(*z) < 5e-6, k
+        if k < 3:
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    for c, s in ((c0, a), (c1, b)):
+        s.close()
+        c.close()

@@ -2212,6 +2212,9 @@ __global__ void __launch_bounds__(64) k_block_apply_sparse(float* __restrict__ p
         need = apply_count(-R, peak) != 0.0 || apply_count(R, peak) != 0.0;
     }
     unsigned long long m = __ballot(need);
+    const int dd = f / max(rs.W, 1);
+    const double ga = rs.fields ? rs.geo_a[f - dd * rs.W] : 0.0;
+    float* const pf = pha + (size_t)f * Nout * Nout;
     while (m) {
         const int bb = blockIdx.x * 64 + (__ffsll((long long)m) - 1);
         m &= m - 1;
@@ -2219,41 +2222,46 @@ __global__ void __launch_bounds__(64) k_block_apply_sparse(float* __restrict__ p
         const int r0 = bstart[by], c0 = bstart[bx];
         const int w = bstart[bx + 1] - c0, n = (bstart[by + 1] - r0) * w;
         const double peak = bin[(size_t)f * nb + bb];
-        // 4 pixels of a lane at a time, their loads together (clamped to the
-        // block's last pixel; a block of 20 x 20 is two rounds instead of seven)
-        for (int e0 = lane; e0 < n; e0 += 256) {
-            size_t o[4];
-            float rf[4];
-            double vr[4], vl[4];
-            float2 E[4];
-            const int dd = f / max(rs.W, 1);
+        // UN pixels of a lane at a time, their loads together (clamped to the
+        // block's last pixel; a block of 20 x 20 is two rounds).  The phase is one
+        // of them: loaded under its own condition it is waited for pixel by pixel.
+        // One field, weak turbulence (few blocks visited): 2.3 us, with one pixel
+        // at a time 3.9; strong turbulence (every block; bound by the wave's own
+        // arithmetic, block after block): 1024^2 229 us against 234, 256^2 233
+        // against 245 (with the phase loaded late 261 and 266).
+        constexpr int UN = 4;
+        for (int e0 = lane; e0 < n; e0 += UN * 64) {
+            int o[UN];
+            float rf[UN], ph[UN];
+            double vr[UN], vl[UN];
+            float2 E[UN];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
+            for (int u = 0; u < UN; u++) {
                 const int e = min(e0 + u * 64, n - 1), q = e / w, jj = r0 + q, ii = c0 + (e - q * w);
-                o[u] = ((size_t)f * Nout + jj) * Nout + ii;
+                o[u] = jj * Nout + ii;
+                ph[u] = pf[o[u]];
                 if (rs.fields) {
                     // the extraction's remainder again, from the final field and
                     // the geometric phase's planes at the full-grid pixel
-                    const int jf = jj + rs.o, ifl = ii + rs.o;
-                    const size_t gi = ((size_t)dd * rs.N + jf) * rs.N + ifl;
-                    vr[u] = rs.vr[gi];
-                    vl[u] = rs.vl[gi];
-                    E[u] = rs.fields[((size_t)f * rs.N + jf) * rs.N + ifl];
+                    const size_t gi = (size_t)(jj + rs.o) * rs.N + (ii + rs.o), nn = (size_t)rs.N * rs.N;
+                    vr[u] = rs.vr[dd * nn + gi];
+                    vl[u] = rs.vl[dd * nn + gi];
+                    E[u] = rs.fields[f * nn + gi];
                 } else {
-                    rf[u] = dres[o[u]];
+                    rf[u] = dres[(size_t)f * Nout * Nout + o[u]];
                 }
             }
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
+            for (int u = 0; u < UN; u++) {
                 if (e0 + u * 64 >= n) continue;
                 if (rs.fields) {
                     double phi, pl, r;
-                    planes_phase(rs.geo_a[f - dd * rs.W], vr[u], vl[u], phi, pl);
+                    planes_phase(ga, vr[u], vl[u], phi, pl);
                     block_turns(phi, rotated_arg(E[u], rs.rot ? pl : 0.0), r);
                     rf[u] = (float)r;
                 }
                 const double cnt = apply_count(rf[u], peak);
-                if (cnt != 0.0) pha[o[u]] = (float)fma(2.0 * M_PI, cnt, (double)pha[o[u]]);
+                if (cnt != 0.0) pf[o[u]] = (float)fma(2.0 * M_PI, cnt, (double)ph[u]);
             }
         }
     }

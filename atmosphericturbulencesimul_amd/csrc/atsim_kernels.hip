@@ -261,12 +261,15 @@ struct RowCfg {
     static constexpr int ROWS = ROWS0 < N ? ROWS0 : N;
     static constexpr int THREADS = ROWS * T;
 };
-// columns per workgroup of a column pass with 16 elements per thread.  8 up to
-// 2048: from 512 on two workgroups then share a CU (one Fresnel call on 8 fields
-// of 1024^2: 82 us against 92 with 16 columns, 64 of 512^2: 117 against 124).
+// columns per workgroup of a column pass with 16 elements per thread: what the
+// LDS of a CU holds twice from 512 to 1024 (one Fresnel call on 8 fields of
+// 1024^2: 82 us against 92 with 16 columns, 64 of 512^2: 117 against 124) and once
+// from 2048 on; 16 (128-byte row segments) up to 128, where a workgroup is a wave
+// or two whatever its columns (128 fields of 128^2: 11.9 us against 14.5 with 8,
+// of 64^2 7.5 against 8.0).
 template <int N>
 struct ColCfg {
-    static constexpr int C = N <= 2048 ? 8 : (N == 4096 ? 4 : 2);
+    static constexpr int C = N <= 128 ? 16 : N <= 2048 ? 8 : (N == 4096 ? 4 : 2);
 };
 
 // ------------------------------------------------------------------ passes
@@ -877,8 +880,9 @@ static hipError_t col_dispatch(int op, int dir, float2* data, long F, const floa
         if (c <= 0 && e != 16 && F > 1) return col_split_launch<N, 8>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
     }
     // 4 columns where 8 leave CUs without a workgroup (one field of 1024^2: 37
-    // against 39 us a call, 512^2: 31 against 32)
-    if (c <= 0) c = (ColCfg<N>::C == 8 && N / 8 * F < 256) ? 4 : ColCfg<N>::C;
+    // against 39 us a call, 512^2: 31 against 32); 16 at 256 from 64 fields on,
+    // where either fills the chip (128 fields: 27.0 us against 28.4; 32: equal)
+    if (c <= 0) c = ColCfg<N>::C != 8 ? ColCfg<N>::C : N / 8 * F < 256 ? 4 : N == 256 && F >= 64 ? 16 : 8;
     switch (c) {
         case 2: return col_launch<N, 2>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
         case 4: return col_launch<N, 4>(op, dir, data, F, tf, W, tw, wlo, wcnt, st);
@@ -1015,8 +1019,14 @@ hipError_t launch_col_screen(long n, float2* data, int D, const float2* tfp, con
     // workgroup or, at 1024, give a CU no more than two of its 8-wave ones.  Frames,
     // with 32 elements / 8 / 4 columns: 256^2 x 256 fields 868 / 818 / 914 us,
     // x 1 163 / 128 / 128; 512^2 x 32 568 / 478 / 495, x 1 240 / 175 / 166; 1024^2 x
-    // 32 2 152 / 2 110 / 2 213, x 8 594 / 536 / 522, x 1 303 / 249 / 236.
-    const bool few = n / 8 * F < 256 || (n == 1024 && n / 8 * F <= 512);
+    // 32 2 152 / 2 110 / 2 213, x 8 594 / 536 / 522, x 1 303 / 249 / 236.  The more
+    // planes a group has, the more the pass is their loads, which 32-byte segments
+    // make slow: at 1024 4 columns only up to 4 planes for two fields a launch and
+    // 2 for four (8 wavelengths on two streams, groups of 1 / 2 / 4 / 8 / 16
+    // layers: 437 / 449 / 498 / 669 / 940 us a frame with 4 columns, 437 / 450 / 483 /
+    // 616 / 879 with 8; 4 wavelengths: 355 / 363 / 386 / 506 / 771 and 362 / 367 /
+    // 390 / 502 / 753).
+    const bool few = n / 8 * F < 256 || (n == 1024 && n / 8 * F <= 512 && n / 8 * F * sa.lcount <= 1024);
 #define X(NN, CC)                                                                                     \
     case NN: return col_screen<NN, CC>(data, D, tfp, tf, tw, sa, vq, slot0, st);
     if (few) {

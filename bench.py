@@ -108,6 +108,46 @@ def read_valu():
     return read_pass_table("valu_headline_2048_10L_8lam.md", "wave_instructions_per_launch")
 
 
+def pass_kernels(N, W, D, lcount, get):
+    """the kernel of every kind of Fresnel pass of a frame (layer groups of
+    lcount layers, top to bottom; all fields in one launch, as profiled frames
+    run), by the library's own rules; get(key): the tuning in force"""
+    F, G = W * D, len(lcount) - 1
+    one = get("gap_passes") == 1 and N <= 4096 and G >= 2
+    planes = get("row_planes") == 1
+    # columns without a screen
+    c, e = get("col_c"), get("col_e")
+    if 256 <= N <= 2048 and e == 32 and c in (0, 8, 16):
+        col = f"k_col_split<{N}, 1, 0, {c or 8}, 32>"
+    elif c == 0 and e != 16 and (N >= 4096 or (N == 2048 and F > 1)):
+        col = f"k_col_split<{N}, 1, 0, {4 if N == 8192 else 8}, 32>"
+    else:
+        if N <= 128:
+            d = 16
+        elif N <= 2048:
+            d = 4 if N // 8 * F < 256 else 16 if N == 256 and F >= 64 else 8
+        else:
+            d = 4 if N == 4096 else 2
+        col = f"k_col<{N}, 1, 0, {c or d}, false>"
+    names = {"col": col}
+    sampled = f"k_row_fresnel<{N}, true, false>"
+    if not one:
+        names["row"] = sampled
+        return names
+    mw = 1024 // N if N < 2048 else 2 if N == 2048 else 1
+    names["row"] = f"k_row_screen<{N}, {mw}, true>" if planes and W == 1 else sampled
+    names["row2"] = f"k_row_screen<{N}, {mw}, false>" if planes else f"k_row_fresnel<{N}, false, true>"
+    # columns with a screen (of the first such group)
+    e2 = get("col2_e")
+    if N >= 256 and e2 != 16 and (e2 == 32 or N >= 4096 or (N == 2048 and F > 1)):
+        names["col2"] = f"k_col_screen_split<{N}, 8, 32>"
+    else:
+        few = N // 8 * F < 256 or (N == 1024 and N // 8 * F <= 512 and N // 8 * F * lcount[1] <= 1024)
+        w = 4 if few and N in (256, 512, 1024) else 16 if N <= 64 else 4 if N == 4096 else 8
+        names["col2"] = f"k_col_screen<{N}, {w}>"
+    return names
+
+
 def _fftw_backend():
     """Name of the FFT library a reference build on this host would use: FFTW
     (libfftw3f.so.3, src/fft/fft.c:52) if the host has it, else none"""
@@ -656,8 +696,8 @@ def main():
     # read + write of every field (the first pass creates the field: write
     # only) and, per direction, one f32 read of the footprint of each layer
     # whose screen the first pass applies, or one f64 read of the sampled phase
-    # plane of each layer a later pass applies (the phase kernel reads the
-    # f32 footprint and writes the f64 plane).  Layer groups top -> bottom as
+    # plane of each layer a later pass applies (with one wavelength the first
+    # too; the phase kernel reads the f32 footprint and writes the f64 plane).  Layer groups top -> bottom as
     # the library forms them; the last group is applied by the extraction.
     sli = list(np.asarray(setup["sli"]))
     L = wl["L"]
@@ -671,12 +711,12 @@ def main():
     field_rw, field_w, foot = 16.0 * N * N * F, 8.0 * N * N * F, 4.0 * N * N * wl["D"]
     passes = []  # (kind, bytes)
     if fused:
-        nslots = sum(lcount[k] for k in range(1, G))
+        nslots = sum(lcount[k] for k in range(0 if wl["W"] == 1 else 1, G))
         passes.append(("phase", 3.0 * foot * nslots))
         for k in range(G + 1):
             rows = k % 2 == 0
             if k == 0:
-                passes.append(("row", field_w + foot * lcount[0]))
+                passes.append(("row", field_w + foot * lcount[0] * (2 if wl["W"] == 1 else 1)))
             elif k == G:
                 passes.append(("row" if rows else "col", field_rw))
             else:
@@ -703,19 +743,19 @@ def main():
     frame_bytes = (sum(b for _, b in passes) + 8.0 * N * N * F) / F + 8.0 * wl["Nout"] ** 2
     if ctx.get_tuning("extract_planes") == 1:
         frame_bytes += (foot * L + 32.0 * N * N * wl["D"]) / F
-    c2e = ctx.get_tuning("col2_e") or (32 if 256 <= N <= 2048 else 16)
-    ce = ctx.get_tuning("col_e") or 16
-    cc = ctx.get_tuning("col_c") or (8 if N == 2048 else 16)
-    cs = 256 <= N <= 2048 and cc in (8, 16) if ce == 32 else (ctx.get_tuning("col_e") == 0 and N == 2048 and F > 1)
-    kernel_names = {"row": f"k_row_fresnel<{N}> (x pass: screen phase, FFT, transfer function, IFFT)",
-                    "col": (f"k_col_split<{N}, 1, 0, 8, 32>" if cs else f"k_col<{N}, 1, 0, {cc}>") + " (y pass: FFT, transfer function, IFFT)",
-                    "row2": f"k_row_screen<{N}> (x pass: FFT, transfer function, IFFT, screen "
-                            "phase, FFT, transfer function, IFFT)",
-                    "col2": (f"k_col_screen_split<{N}, 8, 32>" if c2e == 32 else f"k_col_screen<{N}>") +
-                            " (y pass: FFT, transfer function, IFFT, screen phase, FFT, transfer function, IFFT)"}
-    # the committed counter summaries were taken with the kernels named above
-    # (the default shapes); another pick of the autotuner has no summary
-    default_shapes = c2e == 32 and not (ce == 32) and cc == 8
+    names = pass_kernels(N, wl["W"], wl["D"], lcount, ctx.get_tuning)
+    what = {"row": "x pass: screen phase, FFT, transfer function, IFFT",
+            "col": "y pass: FFT, transfer function, IFFT",
+            "row2": "x pass: FFT, transfer function, IFFT, screen phase, FFT, transfer function, IFFT",
+            "col2": "y pass: FFT, transfer function, IFFT, screen phase, FFT, transfer function, IFFT",
+            "phase": "phase planes"}
+    kernel_names = {k: f"{names.get(k, 'k_layer_phase')} ({what[k]})" for k in kinds}
+    # the committed counter summaries were taken with the kernels that the
+    # default tuning chooses; a pass that another pick of the autotuner runs
+    # with another kernel has no summary
+    defaults = pass_kernels(N, wl["W"], wl["D"], lcount,
+                            lambda k: {"gap_passes": 1, "row_planes": 1}.get(k, 0))
+    default_shapes = names.get(dom) == defaults.get(dom) and ctx.get_tuning("row_mw") in (0, 4)
     traffic = None
     tr = read_traffic()
     if tr and dom in tr and default_shapes:

@@ -2233,23 +2233,23 @@ __global__ void __launch_bounds__(64) k_block_apply_sparse(float* __restrict__ p
         const int w = bstart[bx + 1] - c0, n = (bstart[by + 1] - r0) * w;
         const double peak = bin[(size_t)f * nb + bb];
         // UN pixels of a lane at a time, their loads together (clamped to the
-        // block's last pixel; a block of 20 x 20 is two rounds).  The phase is one
-        // of them: loaded under its own condition it is waited for pixel by pixel.
-        // One field, weak turbulence (few blocks visited): 2.3 us, with one pixel
-        // at a time 3.9; strong turbulence (every block; bound by the wave's own
-        // arithmetic, block after block): 1024^2 229 us against 234, 256^2 233
-        // against 245 (with the phase loaded late 261 and 266).
+        // block's last pixel; a block of 20 x 20 is two rounds), then those of the
+        // phases if one of the pixels changes: loaded under each pixel's own
+        // condition they would be waited for one by one.
+        // One field, weak turbulence (few blocks visited): 2.4 us, with one
+        // pixel at a time 3.9; strong turbulence (every block; bound by the wave's
+        // own arithmetic, block after block): 1024^2 237 us against 232, 256^2
+        // 239 against 244 (each phase under its own condition: 258 and 259).
         constexpr int UN = 4;
         for (int e0 = lane; e0 < n; e0 += UN * 64) {
             int o[UN];
             float rf[UN], ph[UN];
-            double vr[UN], vl[UN];
+            double vr[UN], vl[UN], cnt[UN];
             float2 E[UN];
 #pragma unroll
             for (int u = 0; u < UN; u++) {
                 const int e = min(e0 + u * 64, n - 1), q = e / w, jj = r0 + q, ii = c0 + (e - q * w);
                 o[u] = jj * Nout + ii;
-                ph[u] = pf[o[u]];
                 if (rs.fields) {
                     // the extraction's remainder again, from the final field and
                     // the geometric phase's planes at the full-grid pixel
@@ -2261,8 +2261,10 @@ __global__ void __launch_bounds__(64) k_block_apply_sparse(float* __restrict__ p
                     rf[u] = dres[(size_t)f * Nout * Nout + o[u]];
                 }
             }
+            bool any = false;
 #pragma unroll
             for (int u = 0; u < UN; u++) {
+                cnt[u] = 0.0;
                 if (e0 + u * 64 >= n) continue;
                 if (rs.fields) {
                     double phi, pl, r;
@@ -2270,9 +2272,15 @@ __global__ void __launch_bounds__(64) k_block_apply_sparse(float* __restrict__ p
                     block_turns(phi, rotated_arg(E[u], rs.rot ? pl : 0.0), r);
                     rf[u] = (float)r;
                 }
-                const double cnt = apply_count(rf[u], peak);
-                if (cnt != 0.0) pf[o[u]] = (float)fma(2.0 * M_PI, cnt, (double)ph[u]);
+                cnt[u] = apply_count(rf[u], peak);
+                any = any || cnt[u] != 0.0;
             }
+            if (!any) continue;
+#pragma unroll
+            for (int u = 0; u < UN; u++) ph[u] = pf[o[u]];
+#pragma unroll
+            for (int u = 0; u < UN; u++)
+                if (cnt[u] != 0.0) pf[o[u]] = (float)fma(2.0 * M_PI, cnt[u], (double)ph[u]);
         }
     }
 }

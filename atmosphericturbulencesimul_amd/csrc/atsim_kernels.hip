@@ -710,11 +710,11 @@ k_row_fresnel(float2* __restrict__ data, const float2* __restrict__ tf, const fl
 // once per frame by the sweep that makes the column passes'), x factor tfc of the
 // gap after it.  Bound: VALU issue, as far as the exchanges leave waves to issue
 // from: a workgroup is MW (row, wavelength) pairs, one wave up to 1024 (no wave
-// waits for another) and two rows at 2048, where k_row_fresnel, which samples the
-// layers for 8192 / N wavelengths at a time, has 8 waves at every barrier and 70 KB
-// of LDS.  Frames: 2048^2 x 8 2 381 -> 2 326 us (2 335 with one row, 2 366 with
-// four), 1024^2 x 5 319 -> 301 (306 with two rows), 512^2 x 128 2 111 -> 2 050 (2 083
-// with two waves).
+// waits for another) and two pairs of two waves each at 2048 (mostly two wavelengths
+// of one row), where k_row_fresnel, which samples the layers for 8192 / N
+// wavelengths at a time, has 8 waves at every barrier and 70 KB of LDS.  Frames:
+// 2048^2 x 8 2 381 -> 2 326 us (2 335 with one pair, 2 366 with four), 1024^2 x 5
+// 319 -> 301 (306 with two pairs), 512^2 x 128 2 111 -> 2 050 (2 083 with two waves).
 // GEN: the first pass of a frame whose planes are ready (no factor before the
 // group; the incoming field is 1).
 template <int N, int MW, bool GEN>
@@ -1002,7 +1002,8 @@ hipError_t launch_col_screen(long n, float2* data, int D, const float2* tfp, con
     const long F = (long)D * nw;
     // 32 elements per thread: asked for, or where the field is largest (4096), or
     // at 2048 from 2 fields on (8 fields: 2 321 us a frame against 2 365 with 16
-    // elements and 8 columns, 2 425 with 4; one field: 591 against 528)
+    // elements and 8 columns, 2 425 with 4; one field: 591 against 528; with 4 gaps
+    // 2, 3, 4 and 6 fields: 642 / 807 / 908 / 1 182 against 639 / 809 / 928 / 1 205)
     const bool split = n >= 256 && e != 16 && (e == 32 || n >= 4096 || (n == 2048 && F > 1));
     if (split) {
         switch (n) {

@@ -163,7 +163,7 @@ int atsim_row_fft_variant(atsim_ctx *ctx, void *d_data, long n, long nrows, int 
  * images take atsim_fft2d; otherwise each axis is transformed on its own,
  * power-of-two lengths directly and other lengths by Bluestein's chirp
  * convolution through power-of-two transforms (lengths up to 4096, or powers
- * of two up to 8192).  Works in the context's scratch memory. */
+ * of two up to 8192).  Keeps the tables of up to 64 lengths with the context. */
 int atsim_fft2d_nm(atsim_ctx *ctx, void *d_data, long n0, long n1, long nbatch, int sign);
 /* Quadrant swap of nbatch complex n0 x n1 images, permut (fft.c:570-792),
  * any size: for odd sizes the reference's swap loops are applied as their
